@@ -84,11 +84,11 @@ gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ 
     }
 }
 
-// Few rows (decode): the product is bound by reading W once, and the tiled kernel above would
+// Few rows (decode): the product is bound by reading W once, and tiles would
 // start N/64 workgroups for it. Here a wavefront owns one output column (WAVES columns a workgroup):
 // its lanes walk the column's weights in 16-byte steps (a wavefront's load is 1 KB of one row), the
 // activations of up to ROWS rows wait in LDS in chunks of F32R_KC floats, and a lane's partial sums
-// (k ascending) are added over the wavefront in a fixed order. More rows than ROWS take further passes over W.
+// (k ascending) are added over the wavefront in a fixed order. M is at most ROWS.
 // Needs K and the row strides in multiples of 4 floats and 16-byte aligned operands.
 #define F32R_KC 512      // 128 16-byte steps: two per lane
 
@@ -101,70 +101,233 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
     const int n = blockIdx.x * WAVES + wave;
     const float* wrow = W + static_cast<size_t>(min(n, N - 1)) * ldw;       // a surplus wavefront repeats the last column
     constexpr int STAGED = (ROWS * (F32R_KC / 4) + 64 * WAVES - 1) / (64 * WAVES);   // 16-byte steps of a chunk a thread stages
-    for (int m0 = 0; m0 < M; m0 += ROWS) {
-        float acc[ROWS];
+    float acc[ROWS];
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
-        // With a handful of wavefronts on a compute unit nothing hides a load's latency but the kernel itself:
-        // the weights and the activations of the next chunk are asked for before the chunk in LDS is used.
-        // A chunk is at most two 16-byte steps per lane (the second from a clamped address; its product is
-        // left out where it is past the chunk).
-        const int q0 = lane, q1 = lane + 64;
-        float4 w0, w1, v[STAGED];
-        auto fetch = [&](int kc0) {
-            const int quads = min(F32R_KC, K - kc0) / 4;
-            w0 = *reinterpret_cast<const float4*>(wrow + kc0 + 4 * min(q0, quads - 1));
-            w1 = *reinterpret_cast<const float4*>(wrow + kc0 + 4 * min(q1, quads - 1));
+    for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
+    // With a handful of wavefronts on a compute unit nothing hides a load's latency but the kernel itself:
+    // the weights and the activations of the next chunk are asked for before the chunk in LDS is used.
+    // A chunk is at most two 16-byte steps per lane (the second from a clamped address; its product is
+    // left out where it is past the chunk).
+    const int q0 = lane, q1 = lane + 64;
+    float4 w0, w1, v[STAGED];
+    auto fetch = [&](int kc0) {
+        const int quads = min(F32R_KC, K - kc0) / 4;
+        w0 = *reinterpret_cast<const float4*>(wrow + kc0 + 4 * min(q0, quads - 1));
+        w1 = *reinterpret_cast<const float4*>(wrow + kc0 + 4 * min(q1, quads - 1));
 #pragma unroll
-            for (int u = 0; u < STAGED; ++u) {
-                const int idx = tid + 64 * WAVES * u, r = idx / quads, q = idx % quads;
-                v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-                if (idx < ROWS * quads && m0 + r < M)
-                    v[u] = *reinterpret_cast<const float4*>(A + static_cast<size_t>(m0 + r) * lda + kc0 + 4 * q);
-            }
-        };
-        fetch(0);
-        for (int kc0 = 0; kc0 < K; kc0 += F32R_KC) {
-            const int quads = min(F32R_KC, K - kc0) / 4;
-            const float4 c0 = w0, c1 = w1;
-            __syncthreads();          // the chunk before has been read
+        for (int u = 0; u < STAGED; ++u) {
+            const int idx = tid + 64 * WAVES * u, r = idx / quads, q = idx % quads;
+            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (idx < ROWS * quads && r < M)
+                v[u] = *reinterpret_cast<const float4*>(A + static_cast<size_t>(r) * lda + kc0 + 4 * q);
+        }
+    };
+    fetch(0);
+    for (int kc0 = 0; kc0 < K; kc0 += F32R_KC) {
+        const int quads = min(F32R_KC, K - kc0) / 4;
+        const float4 c0 = w0, c1 = w1;
+        __syncthreads();          // the chunk before has been read
 #pragma unroll
-            for (int u = 0; u < STAGED; ++u) {
-                const int idx = tid + 64 * WAVES * u, r = idx / quads, q = idx % quads;
-                if (idx < ROWS * quads) *reinterpret_cast<float4*>(&a_s[r][4 * q]) = v[u];
-            }
-            if (kc0 + F32R_KC < K) fetch(kc0 + F32R_KC);
-            __syncthreads();
-            if (q0 < quads) {
+        for (int u = 0; u < STAGED; ++u) {
+            const int idx = tid + 64 * WAVES * u, r = idx / quads, q = idx % quads;
+            if (idx < ROWS * quads) *reinterpret_cast<float4*>(&a_s[r][4 * q]) = v[u];
+        }
+        if (kc0 + F32R_KC < K) fetch(kc0 + F32R_KC);
+        __syncthreads();
+        if (q0 < quads) {
 #pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    const float4 a4 = *reinterpret_cast<const float4*>(&a_s[r][4 * q0]);
-                    acc[r] = fmaf(a4.x, c0.x, acc[r]);
-                    acc[r] = fmaf(a4.y, c0.y, acc[r]);
-                    acc[r] = fmaf(a4.z, c0.z, acc[r]);
-                    acc[r] = fmaf(a4.w, c0.w, acc[r]);
-                }
-            }
-            if (q1 < quads) {
-#pragma unroll
-                for (int r = 0; r < ROWS; ++r) {
-                    const float4 a4 = *reinterpret_cast<const float4*>(&a_s[r][4 * q1]);
-                    acc[r] = fmaf(a4.x, c1.x, acc[r]);
-                    acc[r] = fmaf(a4.y, c1.y, acc[r]);
-                    acc[r] = fmaf(a4.z, c1.z, acc[r]);
-                    acc[r] = fmaf(a4.w, c1.w, acc[r]);
-                }
+            for (int r = 0; r < ROWS; ++r) {
+                const float4 a4 = *reinterpret_cast<const float4*>(&a_s[r][4 * q0]);
+                acc[r] = fmaf(a4.x, c0.x, acc[r]);
+                acc[r] = fmaf(a4.y, c0.y, acc[r]);
+                acc[r] = fmaf(a4.z, c0.z, acc[r]);
+                acc[r] = fmaf(a4.w, c0.w, acc[r]);
             }
         }
-        float mine = 0.f;
+        if (q1 < quads) {
 #pragma unroll
-        for (int r = 0; r < ROWS; ++r) {
-            const float t = wave_sum(acc[r]);
-            if (lane == r) mine = t;
+            for (int r = 0; r < ROWS; ++r) {
+                const float4 a4 = *reinterpret_cast<const float4*>(&a_s[r][4 * q1]);
+                acc[r] = fmaf(a4.x, c1.x, acc[r]);
+                acc[r] = fmaf(a4.y, c1.y, acc[r]);
+                acc[r] = fmaf(a4.z, c1.z, acc[r]);
+                acc[r] = fmaf(a4.w, c1.w, acc[r]);
+            }
         }
-        if (n < N && lane < ROWS && m0 + lane < M)
-            epilogue<float>(mode, mine, bias ? bias[n] : 0.f, C, static_cast<size_t>(m0 + lane) * ldc + n);
     }
+    float mine = 0.f;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        const float t = wave_sum(acc[r]);
+        if (lane == r) mine = t;
+    }
+    if (n < N && lane < ROWS && lane < M)
+        epilogue<float>(mode, mine, bias ? bias[n] : 0.f, C, static_cast<size_t>(lane) * ldc + n);
+}
+
+// More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). Four
+// wavefronts, two by two, of TM x TN tiles of 16 x 16 each share k tiles of 32 columns (a row's piece is one 128-byte line) in
+// LDS, double buffered with one barrier a tile; the loads of the two tiles behind the next are in flight in registers. KG such
+// groups take the 32-column parts of a KG times as wide k tile and add their sums in LDS: for few tiles, where the chain of
+// k tiles (LDS write, barrier, read, products: 0.34 us) is what a workgroup waits for. A lane's 16-byte read holds the k
+// columns of four matrix instructions (lane group l / 16 takes columns 4 (l / 16) to + 3 of 16, the same for both operands);
+// rows are an odd number of 16-byte pieces apart (16 lanes on 16 different groups of banks). The weights are the
+// instruction's first operand, so that a lane ends up with four neighbouring columns of one row. Sixteen columns are summed on
+// their own before they join an output's sum: the error against 64 bits is 1.2e-7 at K = 768 and 2.5e-7 at 3,072 (8.4e-8 and
+// 1.4e-7 with four groups and sums), where one chain of FMAs had 4.0e-7 and 9.4e-7 and the kernel for few rows below 8.0e-8 and 1.4e-7.
+// Bound by the matrix cores where the tiles fill the chip evenly, else by the units that take one tile more or by that chain.
+// 2,048 x 3,072 x 768: 91 us (106 TFLOP/s of the 155 a loop of these instructions reaches; a kernel of vector FMAs on 64 x 64
+// tiles took 134); 2,048 x 768 x 3,072: 99 (209); 570 x 768 x 3,072: 40 (197); 64 x 768 x 3,072: 24 (the kernel for few
+// rows: 59). Needs K and the row strides in multiples of 4 floats, 16-byte aligned operands.
+#define F32T_BK 32
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+template <int TM, int TN, int KG>
+__global__ void __launch_bounds__(256 * KG)
+gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, const float* __restrict__ bias,
+                      void* __restrict__ C, int ldc, int M, int N, int K, int mode, int tiles_m, int tiles_n, int down) {
+    constexpr int BM = 32 * TM, BN = 32 * TN, ROWS = BM + BN, BK = F32T_BK * KG, STRIDE = BK + 4;
+    constexpr int SUMS = TM * TN == 1 ? 4 : 1;      // an output's 16 columns in so many sums
+    constexpr int THREADS = 256 * KG, PIECES = BK / 4, STEP = THREADS / PIECES, LOADS = ROWS / STEP;      // STEP: rows that all threads load at once
+    static_assert(STEP == 32 && (KG == 1 || KG == 2 || KG == 4) && (KG - 1) * 4 * TM * TN * 64 * 4 <= 2 * ROWS * STRIDE, "the groups' sums fit the tiles' LDS");
+    __shared__ __attribute__((aligned(16))) float tile_s[2][ROWS * STRIDE];      // rows of A, then rows of W
+    const int tid = threadIdx.x, lane = tid % 64;
+    const int kg = __builtin_amdgcn_readfirstlane(tid / 256), wave = __builtin_amdgcn_readfirstlane(tid / 64 % 4);
+    // an XCD (workgroup id % 8) takes an even share of the tiles, neighbours in one direction: with `down` it walks down the
+    // rows of A for a few columns of tiles, else along the rows of W for a few rows of tiles
+    const int tiles = tiles_m * tiles_n, per = (tiles + 7) / 8, at = (blockIdx.x % 8) * per + blockIdx.x / 8;
+    if (blockIdx.x / 8 >= per || at >= tiles) return;
+    const int tm = down ? at % tiles_m : at / tiles_n, tn = down ? at / tiles_m : at % tiles_n;
+    const int m0 = tm * BM, n0 = tn * BN;
+    // a thread's 16-byte pieces of a tile: rows beyond the matrix read the last one and are never stored
+    const float* src[LOADS];
+    const int piece = 4 * (tid % PIECES), row0 = tid / PIECES;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const int row = row0 + STEP * i;
+        src[i] = (STEP * i < BM ? A + static_cast<size_t>(min(m0 + row, M - 1)) * lda : W + static_cast<size_t>(min(n0 + row - BM, N - 1)) * ldw) + piece;
+    }
+    float4 regs[2][LOADS];
+    auto fetch = [&](int set, int k0) {          // (columns beyond K: the row's last ones, zeroed when they are staged)
+        const int k = min(k0, K - 4 - piece);
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) regs[set][i] = *reinterpret_cast<const float4*>(src[i] + k);
+    };
+    auto stage = [&](int set, int buf, int k0) {
+        const bool ok = k0 + piece < K;
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i)
+            *reinterpret_cast<float4*>(&tile_s[buf][(row0 + STEP * i) * STRIDE + piece]) = ok ? regs[set][i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    };
+    f32x4v acc[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
+    const int wm = wave / 2, wn = wave % 2, row16 = lane % 16, quad = lane / 16;
+    const int a_off = (wm * TM * 16 + row16) * STRIDE + F32T_BK * kg + 4 * quad, w_off = (BM + wn * TN * 16 + row16) * STRIDE + F32T_BK * kg + 4 * quad;
+    auto multiply = [&](int buf) {
+#pragma unroll
+        for (int ks = 0; ks < F32T_BK / 16; ++ks) {
+            f32x4v fa[TM], fw[TN], sum[SUMS][TM][TN];
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const f32x4v*>(&tile_s[buf][a_off + i * 16 * STRIDE + ks * 16]);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const f32x4v*>(&tile_s[buf][w_off + j * 16 * STRIDE + ks * 16]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) {
+                        f32x4v& to = sum[e % SUMS][i][j];
+                        to = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][e], fa[i][e], e < SUMS ? f32x4v{0.f, 0.f, 0.f, 0.f} : to, 0, 0, 0);
+                    }
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) {
+                    if constexpr (SUMS == 4) acc[i][j] += (sum[0][i][j] + sum[1][i][j]) + (sum[2][i][j] + sum[3][i][j]);
+                    else acc[i][j] += sum[0][i][j];
+                }
+        }
+    };
+    const int nk = (K + BK - 1) / BK;
+    // tile t multiplies from buffer t % 2 while tile t + 1 is staged into the other one, whose readers (tile t - 1) passed the
+    // barrier before, and the loads of tile t + 3 go out into the registers that are free then (past the last tile: its own again)
+    fetch(0, 0);
+    fetch(1, min(1, nk - 1) * BK);
+    stage(0, 0, 0);
+    fetch(0, min(2, nk - 1) * BK);
+    lds_barrier();
+    for (int t = 0; t < nk; t += 2) {
+        stage(1, 1, (t + 1) * BK);
+        fetch(1, min(t + 3, nk - 1) * BK);
+        multiply(0);
+        lds_barrier();
+        if (t + 1 >= nk) break;
+        stage(0, 0, (t + 2) * BK);
+        fetch(0, min(t + 4, nk - 1) * BK);
+        multiply(1);
+        lds_barrier();
+    }
+    if constexpr (KG > 1) {          // the other groups leave their sums in LDS and go; group 0 adds them in their order
+        f32x4v* sums = reinterpret_cast<f32x4v*>(&tile_s[0][0]);
+        if (kg > 0) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j) sums[(((kg - 1) * 4 + wave) * TM * TN + i * TN + j) * 64 + lane] = acc[i][j];
+        }
+        lds_barrier();
+        if (kg > 0) return;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                auto other = [&](int g) { return sums[((g * 4 + wave) * TM * TN + i * TN + j) * 64 + lane]; };
+                if constexpr (KG == 4) acc[i][j] = (acc[i][j] + other(0)) + (other(1) + other(2));
+                else acc[i][j] += other(0);
+            }
+    }
+    // lane l holds columns 4 (l / 16) to + 3 of row l % 16 of every 16 x 16 tile
+    const bool vec = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 && (bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 15) == 0);
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+        const int m = m0 + (wm * TM + i) * 16 + row16;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) {
+            const int n = n0 + (wn * TN + j) * 16 + 4 * quad;
+            float* out = static_cast<float*>(C) + static_cast<size_t>(m) * ldc + n;
+            if (vec && n + 4 <= N) {
+                float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]}, o[4] = {0.f, 0.f, 0.f, 0.f};
+                if (bias != nullptr) {
+                    const float4 b = *reinterpret_cast<const float4*>(bias + n);
+                    v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
+                }
+                if (mode == EPI_ADD_RESIDUAL) {
+                    const float4 b = *reinterpret_cast<const float4*>(out);
+                    o[0] = b.x; o[1] = b.y; o[2] = b.z; o[3] = b.w;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+                    o[e] += mode == EPI_GELU_TANH ? gelu_tanh_precise(v[e]) : mode == EPI_GELU_ERF ? gelu_erf(v[e]) : mode == EPI_RELU2 ? relu2(v[e]) : v[e];
+                *reinterpret_cast<float4*>(out) = make_float4(o[0], o[1], o[2], o[3]);
+            } else {
+                for (int e = 0; e < 4 && n + e < N; ++e)
+                    epilogue<float>(mode, acc[i][j][e], bias ? bias[n + e] : 0.f, C, static_cast<size_t>(m) * ldc + n + e);
+            }
+        }
+    }
+}
+
+template <int TM, int TN, int KG>
+static void launch_f32_tiles(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int mode,
+                             hipStream_t stream) {
+    const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (N + 32 * TN - 1) / (32 * TN);
+    gemm_f32_tiles_kernel<TM, TN, KG><<<(tiles_m * tiles_n + 7) / 8 * 8, 256 * KG, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n,
+                                                                                             M > N ? 0 : 1);
 }
 
 // bfloat16 operands of any K, strides and alignment (what the matrix-core kernels of gemm_bf16.hip refuse:
@@ -208,7 +371,8 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
     if (M <= 0 || N <= 0) return 0;
     const bool quads = K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 &&
                        ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(W)) & 15) == 0;
-    if (M <= 64 && quads && K > 0) {
+    if (quads && K > 0 && (M <= 8 || (M <= 16 && N < 16384))) {
+        // (9 to 16 rows of a wide head: 73 us here, 55 on tiles at 50,257 columns.)
         // Workgroups start at a limited rate (a few hundred a microsecond over the chip): from 2,048 columns on
         // a workgroup takes eight instead of four, which also halves what is staged (sixteen lose again: at
         // 50,257 columns 54 us against 45).
@@ -224,6 +388,31 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
         MLLM_LAUNCH_CHECK();
         return 0;
     }
+    if (quads && K > 0) {
+        // Tiles of 32 x 32 shared by four groups up to 64 rows (whose sums are as exact as the kernel's for few rows) and while
+        // there are at most two a compute unit (570 x 768 x 3,072: 40 us, with two groups 43, with tiles of 64 x 32 44).
+        // Otherwise the shape whose fullest compute unit does least: its tiles times their size times what 32 x 32 outputs
+        // take there at K = 768 (in tenths of a microsecond, measured at 2,048 rows). Large tiles need several workgroups a unit
+        // to hide their barriers: 2,048 x 768 x 768 32 us with 64 x 32, 35 with 64 x 64 (384 tiles) and 64 x 96 (256).
+        const auto tiles = [&](int tm, int tn) { return static_cast<long>((M + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
+        const auto cost = [&](int tm, int tn, long from, int each) {
+            const long n = tiles(tm, tn);
+            return n < from ? (1L << 60) : ((n + 7) / 8 + 31) / 32 * tm * tn * each;
+        };
+        if (M <= 64 || tiles(1, 1) <= 512) {
+            launch_f32_tiles<1, 1, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+        } else {
+            const long c11 = cost(1, 1, 0, 44), c21 = cost(2, 1, 256, 40), c22 = cost(2, 2, 512, 36), c23 = cost(2, 3, 512, 37);
+            const long least = std::min(std::min(c11, c21), std::min(c22, c23));
+            if (least == c22) launch_f32_tiles<2, 2, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else if (least == c23) launch_f32_tiles<2, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else if (least == c21) launch_f32_tiles<2, 1, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else launch_f32_tiles<1, 1, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+        }
+        MLLM_LAUNCH_CHECK();
+        return 0;
+    }
+    // any K, strides and alignment
     dim3 grid((N + F32_BN - 1) / F32_BN, (M + F32_BM - 1) / F32_BM);
     gemm_f32_kernel<<<grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
     MLLM_LAUNCH_CHECK();

@@ -394,6 +394,37 @@ def test_linear_fp32_few_rows(ops, M, N, K, pad):
         assert (out.cpu().double() - ref).abs().max().item() <= 3e-5
 
 
+@pytest.mark.parametrize("M,N,K,pad", [(17, 40, 4, 0), (33, 97, 100, 4), (64, 193, 772, 0),     # 32 x 32 tiles, four groups
+                                       (9, 16400, 36, 0),                                       # few rows of a wide head
+                                       (800, 700, 132, 8),                                      # 32 x 32, two groups
+                                       (1025, 800, 260, 0),                                     # 64 x 32, two groups
+                                       (2049, 2308, 20, 4), (1900, 1500, 292, 0)])              # 64 x 96 and 64 x 64
+@pytest.mark.parametrize("epi", ["store", "gelu_tanh", "add_residual"])
+def test_linear_fp32_tiles(ops, M, N, K, pad, epi):
+    """Every tile shape of the 32-bit product at its edges (rows, columns and K that fill no tile, strides wider than the rows):
+    an output's products pass through at most 16 roundings, one for each further 16 columns, and a few to join groups, bias and
+    residual, so its error is at most that many units of 2^-24 of the sum of their magnitudes (GELU: at most 1.13 times as
+    steep, and 8 units of its own result). A row of infinities leaves the others as they are."""
+    g = torch.Generator().manual_seed(M + K)
+    a, w, b = _rand((M, K + pad), torch.float32, g), _rand((N, K + pad), torch.float32, g, 0.1), _rand((N,), torch.float32, g)
+    a[M // 2] = float("inf")
+    old = _rand((M, N + pad), torch.float32, g)
+    out = old.to(DEV)
+    ops.linear(a.to(DEV)[:, :K], w.to(DEV)[:, :K], b.to(DEV), out[:, :N], epi)
+    assert torch.equal(out[:, N:].cpu(), old[:, N:])
+    keep = torch.arange(M) != M // 2
+    a64, w64 = a[keep, :K].double(), w[:, :K].double()
+    want = a64 @ w64.T + b.double()
+    size = a64.abs() @ w64.abs().T + b.double().abs()
+    if epi == "gelu_tanh":
+        want = 0.5 * want * (1.0 + torch.tanh(0.7978845608 * (want + 0.044715 * want ** 3)))
+    elif epi == "add_residual":
+        want, size = want + old[keep, :N].double(), size + old[keep, :N].double().abs()
+    limit = 2.0 ** -24 * (1.13 * (16 + -(-K // 16) + 8) * size + 8 * want.abs())
+    assert ((out[:, :N].cpu()[keep].double() - want).abs() <= limit).all()
+    assert not torch.isfinite(out[M // 2, :N]).any() or epi == "gelu_tanh"
+
+
 @pytest.mark.parametrize("M, N, K", [(4, 8, 36), (70, 33, 44), (9, 5, 7)])
 def test_linear_bf16_takes_any_k_through_the_plain_kernel(ops, M, N, K):
     """A K that is no multiple of 8 (the matrix-core kernels read 16 bytes at a time) runs on the plain kernel."""
