@@ -233,8 +233,12 @@ static void check_linear(int64_t M, int64_t K, int a_dtype, const Tensor2& w, co
              (long long)out.rows, (long long)out.cols, dtype_name(out.dtype));
 }
 
-// Whether the product kernel that runs for these rows writes keys and values to the pages in its epilogue.
-static bool scatter_is_fused(int dtype, int64_t rows) { return dtype == BF16 && rows > 64; }
+static void check_scatter(const KvScatter& kv, int dtype, int64_t N, int epilogue, const char* what) {
+    if (epilogue != STORE) fail("%s: the key/value scatter needs the plain store", what);
+    check_pages(kv.k_pages, kv.v_pages, dtype, what);
+    const int kv_dim = static_cast<int>(kv.k_pages.cols);
+    if (N != kv.q_cols + 2 * kv_dim) fail("%s: %lld columns are not %d + 2 x %d", what, (long long)N, kv.q_cols, kv_dim);
+}
 
 void linear(const Tensor2& a, const Tensor2& w, const float* bias, const Tensor2& out, int epilogue,
             const KvScatter* kv, hipStream_t stream) {
@@ -242,11 +246,13 @@ void linear(const Tensor2& a, const Tensor2& w, const float* bias, const Tensor2
     const int64_t M = a.rows, K = a.cols, N = w.rows;
     check_linear(M, K, a.dtype, w, out, epilogue, "linear");
     if (kv != nullptr) {
-        if (epilogue != STORE) fail("linear: the key/value scatter needs the plain store");
-        check_pages(kv->k_pages, kv->v_pages, a.dtype, "linear (key/value scatter)");
+        check_scatter(*kv, a.dtype, N, epilogue, "linear (key/value scatter)");
         const int kv_dim = static_cast<int>(kv->k_pages.cols);
-        if (N != kv->q_cols + 2 * kv_dim) fail("linear: %lld columns are not %d + 2 x %d", (long long)N, kv->q_cols, kv_dim);
-        if (!scatter_is_fused(a.dtype, M)) {
+        // The matrix-core kernels write keys and values to the pages in their epilogues. Up to 64 rows, operands or widths that they
+        // do not take go through a product and a copy.
+        const bool fits = kv->q_cols % 4 == 0 && kv_dim % 4 == 0 && K % 8 == 0 && a.stride % 8 == 0 && w.stride % 8 == 0 &&
+                          aligned(a.data, 16) && aligned(w.data, 16);
+        if (a.dtype != BF16 || (M <= 64 && !fits)) {
             linear(a, w, bias, out, epilogue, nullptr, stream);
             kv_append(out, kv->q_cols, kv->q_cols + kv_dim, kv->k_pages, kv->v_pages, kv->slots, stream);
             return;
@@ -374,11 +380,20 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
     // (More rows than that: the norm is a kernel of its own. Normalising in the tiled product while it stages
     // its rows was measured at 64 to 256 rows and lost: every workgroup of a row tile has to pull the tile's
     // fp32 rows through its own L1 for the statistics, 6.5 us at 64 rows of 768, more than the norm's kernel.)
-    if (kv == nullptr && w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
-        (beta == nullptr || aligned(beta, 16))) {
-        const int rc = mllm_ln_gemm_bf16(static_cast<const float*>(x.data), static_cast<int>(x.stride), rows, gamma, beta, eps,
-                                         w.data, static_cast<int>(w.stride), bias, out.data, static_cast<int>(out.stride),
-                                         static_cast<int>(M), static_cast<int>(w.rows), static_cast<int>(K), epilogue, stream);
+    if (w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
+        (beta == nullptr || aligned(beta, 16)) && (kv == nullptr || aligned(w.data, 16))) {
+        int rc;
+        if (kv != nullptr) {
+            check_scatter(*kv, w.dtype, w.rows, epilogue, "ln_linear (key/value scatter)");
+            rc = mllm_ln_gemm_bf16_kv(static_cast<const float*>(x.data), static_cast<int>(x.stride), rows, gamma, beta, eps, w.data,
+                                      static_cast<int>(w.stride), bias, out.data, static_cast<int>(out.stride), static_cast<int>(M),
+                                      static_cast<int>(w.rows), static_cast<int>(K), kv->slots, kv->k_pages.data, kv->v_pages.data, kv->q_cols,
+                                      static_cast<int>(kv->k_pages.cols), stream);
+        } else {
+            rc = mllm_ln_gemm_bf16(static_cast<const float*>(x.data), static_cast<int>(x.stride), rows, gamma, beta, eps,
+                                   w.data, static_cast<int>(w.stride), bias, out.data, static_cast<int>(out.stride),
+                                   static_cast<int>(M), static_cast<int>(w.rows), static_cast<int>(K), epilogue, stream);
+        }
         if (rc == 0) return;
         if (rc != -2) check(rc, "ln_linear");
     }

@@ -448,8 +448,6 @@ struct SplitStates {
     float4 o[MERGE_MAX_SPLITS][2];        // 8 elements of the unnormalised output
 };
 
-struct NoExtra {};
-
 template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false>
 __global__ void __launch_bounds__(ASRC == A_NORMED ? 512 : (ASRC == A_GLOBAL || ASRC == A_MERGED ? 768 : 1024))
 gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: what the first loads need
@@ -466,8 +464,9 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
                  int n_splits = 1, int a_heads = 1, int a_head_dim = 8,
                  // A_NORMED: != 0: the norm does not centre (RMS norm: x / sqrt(mean(x^2) + eps) * gamma)
                  int rms = 0,
-                 // THROUGH (mode EPI_THROUGH): the norms the result passes and the copy it leaves
-                 typename std::conditional<THROUGH, MllmStreamAdd, NoExtra>::type add = {}) {
+                 // THROUGH (mode EPI_THROUGH): the norms the result passes and the copy it leaves; otherwise (plain store of
+                 // a split-K kernel) the pages that its key and value columns go to as well
+                 typename std::conditional<THROUGH, MllmStreamAdd, KvScatter>::type add = {}) {
     static_assert(!THROUGH || (SPLIT_K && MT == 1 && ASRC == A_GLOBAL), "results through norms: split-K kernels of one row tile");
     // NT > 1 (SPLIT_K, MT == 1): the workgroup owns cols_per_wg <= 16 NT columns, NT tiles that share
     // the rows of A, the last one possibly narrower: for products with more than 256 tiles, whose
@@ -540,11 +539,12 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     // accumulator order): requested now so that their latency hides behind the product.
     bool ep_ok[NT];
     size_t ep_idx[NT];
+    int ep_col[NT], ep_slot = -1;
     float ep_bias[NT], ep_old[NT];
     MllmNormColumn ep_norm[NT], ep_next[NT];
     float ep_alpha = 0.f, ep_alpha2 = 0.f;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) { ep_ok[t] = false; ep_idx[t] = 0; ep_bias[t] = 0.f; ep_old[t] = 0.f; }
+    for (int t = 0; t < NT; ++t) { ep_ok[t] = false; ep_idx[t] = 0; ep_col[t] = 0; ep_bias[t] = 0.f; ep_old[t] = 0.f; }
     if (SPLIT_K && MT == 1 && wave < 4) {
         // (loads without a per-lane condition: outputs beyond M or N read the last row or column)
         const int m = m_base + 4 * (lane / 16) + wave;
@@ -552,6 +552,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         for (int t = 0; t < NT; ++t) {
             const int ct = 16 * t + lane % 16, nn = n0 + ct;
             ep_ok[t] = m < M && nn < N && ct < cols_per_wg;
+            ep_col[t] = nn;
             ep_idx[t] = static_cast<size_t>(min(m, M - 1)) * ldc + min(nn, N - 1);
             if (bias) ep_bias[t] = bias[min(nn, N - 1)];
             if (THROUGH || mode == EPI_ADD_RESIDUAL) ep_old[t] = static_cast<const float*>(C)[ep_idx[t]];
@@ -564,6 +565,8 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         if constexpr (THROUGH) {
             if (add.norm.weight != nullptr) ep_alpha = add.norm.alpha[0];
             if (add.next.weight != nullptr) ep_alpha2 = add.next.alpha[0];
+        } else {
+            if (add.slots != nullptr) ep_slot = add.slots[min(m, M - 1)];
         }
     }
 
@@ -986,7 +989,14 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
                     if (add.copy != nullptr)
                         static_cast<bf16_t*>(add.copy)[ep_idx[t]] = float_to_bf16(mllm_norm_column(x, add.next.weight != nullptr, ep_alpha2, ep_next[t]));
                 } else if (mode == EPI_ADD_RESIDUAL) static_cast<float*>(C)[ep_idx[t]] = ep_old[t] + r;
-                else epilogue<bf16_t>(mode, r, 0.f, C, ep_idx[t]);
+                else {
+                    epilogue<bf16_t>(mode, r, 0.f, C, ep_idx[t]);
+                    if (ep_slot >= 0 && ep_col[t] >= add.q_cols) {      // (only with slots: the row's place in the pages)
+                        const int c = ep_col[t] - add.q_cols;
+                        bf16_t* dst = c < add.kv_dim ? add.k_pages + c : add.v_pages + (c - add.kv_dim);
+                        dst[static_cast<size_t>(ep_slot) * add.kv_dim] = float_to_bf16(r);
+                    }
+                }
             }
         }
         return;
@@ -1018,11 +1028,13 @@ template <bool LN_FUSED, bool MERGED = false>
 static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const float* bias, void* C, int ldc,
                          int M, int N, int K, int mode, const float* gamma, const float* beta, float eps,
                          const int* rows, hipStream_t stream, void* workspace = nullptr, size_t workspace_bytes = 0,
-                         MergedA merged = MergedA{}, int rms = 0, const MllmStreamAdd* through = nullptr) {
+                         MergedA merged = MergedA{}, int rms = 0, const MllmStreamAdd* through = nullptr,
+                         KvScatter kv = KvScatter{}) {
     static_assert(!(LN_FUSED && MERGED), "one source of A");
     const int tiles = (N + 15) / 16;
     const bool split_k = tiles < 1024;
     if (through != nullptr && (LN_FUSED || MERGED || !split_k)) return -2;
+    if (kv.slots != nullptr && (through != nullptr || !split_k || mode != EPI_STORE)) return -2;
     // Narrow products: 16 rows per workgroup and one workgroup per 16 rows (more workgroups, each
     // reading only its rows). Wide products: every wavefront keeps all rows of its tile in
     // registers (up to 4 accumulators), so the weights are streamed once.
@@ -1104,7 +1116,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         if (e != hipSuccess) return static_cast<int>(e);                                               \
         kernel<<<grid, block, staged_bytes, stream>>>(W, ldw, N, K, M, col_blocks, row_blocks, 16, 1, A, lda, mode, \
                                                       bias, C, ldc, gamma, beta, eps, rows, nullptr, nullptr, \
-                                                      nullptr, nullptr, 1, 1, 8, 0, NoExtra{});                   \
+                                                      nullptr, nullptr, 1, 1, 8, 0, KvScatter{});                 \
         break;                                                                                         \
     }
         switch (mt) {
@@ -1142,7 +1154,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         if constexpr (ASRC == A_GLOBAL) {                                                              \
             if (through != nullptr) { SKINNY_KERNEL(SPLIT, UV, A2, NTV, true, *through); break; }      \
         }                                                                                              \
-        SKINNY_KERNEL(SPLIT, UV, A2, NTV, false, NoExtra{});                                           \
+        SKINNY_KERNEL(SPLIT, UV, A2, NTV, false, kv);                                                  \
     } while (0)
     if (split_k) {
         // a chunk holds all k blocks of a wavefront when they are at most 3 (4 without the fused
@@ -1210,7 +1222,6 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
     if ((reinterpret_cast<uintptr_t>(A) & 15) || (reinterpret_cast<uintptr_t>(W) & 15)) return -1;
     const bf16_t* a = static_cast<const bf16_t*>(A);
     const bf16_t* w = static_cast<const bf16_t*>(W);
-    const bool scatter = kv.slots != nullptr;       // only the many-row kernel scatters
     // Which kernel for up to 256 rows. Up to 16 rows (one row block) and for the widest products (the
     // logits head) the weight-streaming kernel, always. In between both are priced, in microseconds,
     // by formulas fitted to measurements on the products of GPT-2 small to XL at 24 to 256 rows: the
@@ -1228,8 +1239,12 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
         return streaming <= tiled;
     };
     const bool few_rows = M <= 16 || (M <= 64 && col_tiles >= 1024) || (M <= 256 && streaming_is_faster());
-    if (!scatter && few_rows && launch_skinny<false>(A, lda, w, ldw, bias, C, ldc, M, N, K, mode, nullptr, nullptr,
-                                                    0.f, nullptr, stream, workspace, workspace_bytes, MergedA{}, 0, through) == 0) {
+    // (Keys and values leave the weight-streaming kernel two bytes a lane, in rows of 32: up to 64 rows that costs less than the
+    // copy it saves (a prompt of 7 tokens of GPT-2 small, with the norm inside as well: 443 -> 384 us), from 65 rows on the tiled
+    // kernel's whole rows are faster again: 529 us a prompt of 65 tokens against 544.)
+    if (few_rows && (kv.slots == nullptr || M <= 64) && launch_skinny<false>(A, lda, w, ldw, bias, C, ldc, M, N, K, mode, nullptr,
+                                                                                nullptr, 0.f, nullptr, stream, workspace, workspace_bytes,
+                                                                                MergedA{}, 0, through, kv) == 0) {
         // few rows: weight-streaming kernel
     } else if (M <= 32) {
         launch_tiled<1, 4, 1, 1, 64, 3>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through);
@@ -1349,7 +1364,23 @@ int mllm_ln_gemm_bf16(const float* x, int ldx, const int* rows, const float* gam
     return 0;
 }
 
-// The same with an RMS norm in front of the product: C = epilogue((x / sqrt(mean(x^2) + eps) * gamma) W^T + bias).
+// The norm and the product with the key/value scatter of mllm_gemm_bf16_kv (plain bf16 store, mode 0); return codes of both.
+int mllm_ln_gemm_bf16_kv(const float* x, int ldx, const int* rows, const float* gamma, const float* beta, float eps, const void* W, int ldw,
+                         const float* bias, void* C, int ldc, int M, int N, int K, const int* slots, void* k_pages, void* v_pages, int q_cols,
+                         int kv_dim, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (slots == nullptr || q_cols < 0 || kv_dim <= 0 || N != q_cols + 2 * kv_dim) return -1;
+    if (K % 8 != 0 || ldw % 8 != 0 || (reinterpret_cast<uintptr_t>(W) & 15)) return -1;
+    if (M > 64) return -2;
+    const KvScatter kv{slots, static_cast<bf16_t*>(k_pages), static_cast<bf16_t*>(v_pages), q_cols, kv_dim};
+    int rc = launch_skinny<true>(x, ldx, static_cast<const bf16_t*>(W), ldw, bias, C, ldc, M, N, K, EPI_STORE, gamma, beta, eps, rows, stream,
+                                 nullptr, 0, MergedA{}, 0, nullptr, kv);
+    if (rc != 0) return rc;
+    MLLM_LAUNCH_CHECK();
+    return 0;
+}
+
+// mllm_ln_gemm_bf16 with an RMS norm in front of the product: C = epilogue((x / sqrt(mean(x^2) + eps) * gamma) W^T + bias).
 int mllm_rms_gemm_bf16(const float* x, int ldx, const int* rows, const float* gamma, float eps, const void* W, int ldw,
                        const float* bias, void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;

@@ -256,6 +256,15 @@ def test_ln_linear_scatters_keys_and_values(ops, M, H, Hkv, dh, K):
     assert torch.equal(kp.cpu(), kr) and torch.equal(vp.cpu(), vr)
 
 
+@pytest.mark.parametrize("M,H,Hkv,dh,K", [(1, 12, 12, 64, 768), (7, 12, 3, 64, 768), (16, 25, 25, 64, 1600),     # (two column tiles a workgroup)
+                                          (17, 12, 12, 64, 768), (32, 5, 1, 40, 96), (33, 6, 2, 32, 200),
+                                          (9, 3, 3, 10, 64), (40, 3, 3, 10, 64),                     # widths that are no multiple of 4
+                                          (3, 2, 2, 16, 100)])                                       # K that is no multiple of 8
+def test_ln_linear_scatters_few_rows(ops, M, H, Hkv, dh, K):
+    """The same from the few-row product's epilogue (with the norm inside up to 32 rows), and where it does not take the sizes."""
+    test_ln_linear_scatters_keys_and_values(ops, M, H, Hkv, dh, K)
+
+
 @pytest.mark.parametrize("M", [1, 8, 16, 17, 48, 64])
 @pytest.mark.parametrize("N,K", [(2304, 768), (768, 3072), (1000, 96), (50257, 768), (72, 1600), (4800, 1600),
                                  (1600, 6400), (1024, 4096),
