@@ -407,7 +407,7 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
 // attention
 // ---------------------------------------------------------------------------------------------
 // How many workgroups share one (token, head) pair's keys, and wavefronts per workgroup.
-static void decode_launch_shape(int pairs, int max_ctx_len, bool unmerged, int* nsplit, int* waves, bool* merge_kernel) {
+static void decode_launch_shape(int pairs, int max_ctx_len, int keys_per_wave, bool unmerged, int* nsplit, int* waves, bool* merge_kernel) {
     const Tuning& t = tuning();
     *merge_kernel = false;
     if (t.decode_nsplit > 0) { *nsplit = t.decode_nsplit; *waves = t.decode_waves; return; }
@@ -443,9 +443,11 @@ static void decode_launch_shape(int pairs, int max_ctx_len, bool unmerged, int* 
     // One workgroup per pair: merging splits in the kernel (fences, a second merge) costs about 3 us,
     // more than the parallelism gains below about 2,000 keys (measured at 12 to 96 pairs). Few pairs get
     // more wavefronts each instead (measured: 12 are 1 to 3 % of a decode step faster than 8 up to 200
-    // pairs at GPT-2 small to XL sizes, 3 % slower from 384 pairs).
+    // pairs at GPT-2 small to XL sizes, 3 % slower from 384 pairs). More wavefronts than the keys occupy (each takes
+    // `keys_per_wave` at a time) only lengthen the merge: one prompt of 100 tokens and 64 new ones takes 22.5 ms with 12
+    // wavefronts, 21.6 with 4 (21.65 with 3, 22.0 with 6).
     *nsplit = 1;
-    *waves = pairs >= 512 ? 4 : pairs > 256 ? 6 : 12;
+    *waves = std::min(pairs >= 512 ? 4 : pairs > 256 ? 6 : 12, std::max(4, (max_ctx_len + keys_per_wave - 1) / keys_per_wave));
 }
 
 static bool pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
@@ -561,7 +563,7 @@ bool paged_attention(const AttentionArgs& a, AttentionSplits* splits, hipStream_
                         a.head_dim % 8 == 0 && tuning().decode_nsplit == 0;
         int nsplit = 1, waves = 12;
         bool merge_kernel = false;
-        decode_launch_shape(pairs, a.max_ctx_len, unmerged, &nsplit, &waves, &merge_kernel);
+        decode_launch_shape(pairs, a.max_ctx_len, 512 / lpk, unmerged, &nsplit, &waves, &merge_kernel);      // (8 rows a lane group: the kernel's UNR)
         // (sigmoid weights have no sum to divide by afterwards: the kernel merges its own splits, however many)
         // (nor does the merge kernel know a gate of one value per head)
         if (a.shape != nullptr && (a.shape->sigmoid || (a.gate != nullptr && a.shape->gate_per_head))) merge_kernel = false;
