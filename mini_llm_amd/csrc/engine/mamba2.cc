@@ -62,8 +62,8 @@ public:
         Tensor2 xbc = arena.tensor(F32, T, channels_);
         conv_silu(proj, inner_, conv_, conv_bias_, st, xbc, s);
         StageTimes::get().mark("conv", s);
-        // (the scan leaves its result as shares, one per slice of the state's rows; the norm adds them)
-        const int parts = ssm_scan_parts(N_);
+        // (the scan may leave its result as shares, one per slice of the state's rows; the norm adds them)
+        const int parts = ssm_scan_parts(xbc, P_, N_);
         Tensor2 y(arena.take(static_cast<size_t>(parts) * T * inner_ * 4), F32, T, inner_);
         // (portions longer than a chunk are scanned chunk by chunk side by side: room for the chunks' states)
         const size_t ws_floats = step.max_q_len > 64 ? ssm_scan_workspace_floats(T, step.n_seqs, H_, P_, N_) : 0;
@@ -77,7 +77,7 @@ public:
         StageTimes::get().mark("out_proj", s);
     }
     size_t workspace_bytes(int tokens) const override {
-        return static_cast<size_t>(tokens) * ((in_.out_features() + 4) * 4 + channels_ * 4 + ssm_scan_parts(N_) * inner_ * 4 + inner_ * dtype_size(dtype_)) +
+        return static_cast<size_t>(tokens) * ((in_.out_features() + 4) * 4 + channels_ * 4 + (N_ + 31) / 32 * inner_ * 4 + inner_ * dtype_size(dtype_)) +
                ssm_scan_workspace_floats(tokens, 1, H_, P_, N_) * 4 + 8192;
     }
     CacheNeed cache_need() const override {

@@ -160,7 +160,7 @@ void ssm_scan(const Tensor2& xbc, const Tensor2& proj, int dt_col, const float* 
                         stream), "ssm_scan");
 }
 
-int ssm_scan_parts(int N) { return mllm_ssm_scan_parts(N); }
+int ssm_scan_parts(const Tensor2& xbc, int P, int N) { return mllm_ssm_scan_parts(static_cast<const float*>(xbc.data), i32(xbc.stride), P, N); }
 
 size_t ssm_scan_workspace_floats(int tokens, int n_seqs, int H, int P, int N) {
     return mllm_ssm_scan_workspace_floats(tokens, n_seqs, H, P, N);

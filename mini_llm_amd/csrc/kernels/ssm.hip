@@ -343,113 +343,386 @@ ssm_scan_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict_
     }
 }
 
-// The same scan with the chunk's operands staged in LDS first: x [chunk][64], B and C of the slice [chunk][NS]
-// and the raw step sizes, all requested at once with 16-byte loads, so that the token loop waits for no memory
-// (one token ahead is not enough to cover a load that another XCD's kernel wrote a moment ago). Needs 16-byte
-// aligned rows and column offsets (the launcher checks) and chunk <= CH.
+// The scan of sequences of at most CH tokens (decoding, short portions; longer ones leave at once and go through the chunk
+// kernels below): one workgroup per (sequence, head, 64 values of p), a wavefront per slice of NS rows n (more
+// than four slices: in rounds). A wavefront's operands are staged in LDS first, x [CH][64], B and C of the slice [CH][NS] and the raw step sizes, all requested at once
+// with 16-byte loads, so that the token loop waits for no memory (one token ahead is not enough to cover a load that another
+// XCD's kernel wrote a moment ago). The slices' sums over n meet in LDS and are added in the order of the slices, so y leaves
+// whole. Needs 16-byte aligned rows and column offsets. Bound by the state that it reads and writes, and at eight sequences
+// (12.6 MB, 24 heads of 128 x 64) by the chain of one launch: 7.2 us a layer. LDS: floats a wavefront takes.
+template <int NS, int CH> constexpr int ssm_short_floats() { return CH * 64 + 2 * CH * NS + 2 * CH; }
 template <int NS, int CH>
-__global__ void __launch_bounds__(64)
-ssm_scan_staged_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict__ raw_dt, int ldd,
-                       const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
-                       const int* __restrict__ cu_q, const int* __restrict__ state_slots, int n_seqs, float* __restrict__ state,
-                       size_t slot_floats, size_t scan_offset, float* __restrict__ y, int ldy, size_t part_stride, int H, int P,
-                       int N, int G, int n_slices, int write, int chunk, float* __restrict__ chunk_state,
-                       float* __restrict__ cumlog) {
-    __shared__ __attribute__((aligned(16))) float xs[CH][64];
-    __shared__ __attribute__((aligned(16))) float Bs[CH][NS];
-    __shared__ __attribute__((aligned(16))) float Cs[CH][NS];
-    __shared__ float dts[64], as[64];                 // step size and decay of the chunk's tokens
-    const int lane = threadIdx.x;
-    const int h = blockIdx.y, slice = blockIdx.x % n_slices, p0 = (blockIdx.x / n_slices) * 64, p = p0 + lane;
-    const ChunkOf co = chunk_of(blockIdx.z, cu_q, n_seqs, chunk, chunk_state != nullptr);
-    if (co.b < 0) return;
-    const int slot = state_slots[co.b];
-    if (slot < 0) return;
+__global__ void __launch_bounds__(256)
+ssm_short_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict__ raw_dt, int ldd,
+                 const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
+                 const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ state,
+                 size_t slot_floats, size_t scan_offset, float* __restrict__ y, int ldy, int H, int P, int N, int G, int write) {
+    extern __shared__ __attribute__((aligned(16))) float short_s[];
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), waves = blockDim.x / 64;
+    const int h = blockIdx.y, p0 = blockIdx.x * 64, p = p0 + lane, b = blockIdx.z;
+    const int t0 = cu_q[b], nt = cu_q[b + 1] - t0;
+    const int slot = state_slots[b];
+    if (slot < 0 || nt < 1 || nt > CH) return;                 // (the whole workgroup)
     const bool p_ok = p < P;
     const int pc = p_ok ? p : P - 1;
     const int g = h / (H / G), inner = H * P;
-    const int n0 = slice * NS, nn = min(NS, N - n0);
-    const int t0 = cu_q[co.b] + co.k * chunk, t1 = min(t0 + chunk, cu_q[co.b + 1]), nt = t1 - t0;
-    float* sp = state + static_cast<size_t>(slot) * slot_floats + scan_offset + (static_cast<size_t>(h) * N + n0) * P + pc;
-    float S[NS];
+    const int n_slices = (N + NS - 1) / NS;
+    float* xs = short_s + wave * ssm_short_floats<NS, CH>();
+    float *Bs = xs + CH * 64, *Cs = Bs + CH * NS, *dts = Cs + CH * NS, *as = dts + CH;      // dts, as: the tokens' step sizes and decays
+    for (int s0 = 0; s0 < n_slices; s0 += waves) {
+        const int slice = s0 + wave;
+        if (slice < n_slices) {
+            const int n0 = slice * NS, nn = min(NS, N - n0);
+            float* sp = state + static_cast<size_t>(slot) * slot_floats + scan_offset + (static_cast<size_t>(h) * N + n0) * P + pc;
+            float S[NS];
 #pragma unroll
-    for (int j = 0; j < NS; ++j) S[j] = sp[static_cast<size_t>(min(j, nn - 1)) * P];
-    // Staging: quads of 4 floats, a fixed number per lane (CH * 16 quads of x, CH * NS / 4 of B and of C over 64
-    // lanes), all requested before the first is written to LDS; tokens beyond the chunk's end repeat its last one,
-    // a quad beyond the row's end (P or N no multiple of the tile) the row's last one.
-    const int pq = min(64, P - p0) / 4, nq = nn / 4;           // whole quads of x and of B, C in this tile
-    {
-        float4 xq[CH / 4];
+            for (int j = 0; j < NS; ++j) S[j] = sp[static_cast<size_t>(min(j, nn - 1)) * P];
+            // Staging: quads of 4 floats, a fixed number per lane (CH * 16 quads of x, CH * NS / 4 of B and of C over 64
+            // lanes), all requested before the first is written to LDS; tokens beyond the sequence's end repeat its last one,
+            // a quad beyond the row's end (P or N no multiple of the tile) the row's last one.
+            const int pq = min(64, P - p0) / 4, nq = nn / 4;           // whole quads of x and of B, C in this tile
+            {
+                constexpr int XQ = CH * 16 / 64, BQ = CH * (NS / 4) / 64;
+                float4 xq[XQ], bq[BQ], cq[BQ];
 #pragma unroll
-        for (int u = 0; u < CH / 4; ++u) {
-            const int e = lane + 64 * u, tt = min(e / 16, nt - 1), q = min(e % 16, pq - 1);
-            xq[u] = *reinterpret_cast<const float4*>(xbc + static_cast<size_t>(t0 + tt) * ldx + h * P + p0 + 4 * q);
+                for (int u = 0; u < XQ; ++u) {
+                    const int e = lane + 64 * u, tt = min(e / 16, nt - 1), q = min(e % 16, pq - 1);
+                    xq[u] = *reinterpret_cast<const float4*>(xbc + static_cast<size_t>(t0 + tt) * ldx + h * P + p0 + 4 * q);
+                }
+#pragma unroll
+                for (int u = 0; u < BQ; ++u) {
+                    const int e = lane + 64 * u, tt = min(e / (NS / 4), nt - 1), q = min(e % (NS / 4), nq - 1);
+                    const float* row = xbc + static_cast<size_t>(t0 + tt) * ldx + inner + g * N + n0 + 4 * q;
+                    bq[u] = *reinterpret_cast<const float4*>(row);
+                    cq[u] = *reinterpret_cast<const float4*>(row + G * N);
+                }
+#pragma unroll
+                for (int u = 0; u < XQ; ++u) {
+                    const int e = lane + 64 * u;
+                    *reinterpret_cast<float4*>(&xs[e / 16 * 64 + 4 * (e % 16)]) = xq[u];
+                }
+#pragma unroll
+                for (int u = 0; u < BQ; ++u) {
+                    const int e = lane + 64 * u, qi = e % (NS / 4);
+                    const bool real = qi < nq;                          // rows of the slice beyond N count as zeros
+                    *reinterpret_cast<float4*>(&Bs[e / (NS / 4) * NS + 4 * qi]) = real ? bq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+                    *reinterpret_cast<float4*>(&Cs[e / (NS / 4) * NS + 4 * qi]) = real ? cq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+                }
+            }
+            // step sizes and decays are the same for every lane: lane t works them out for token t, once (softplus, two exponentials)
+            const float neg_rate = -expf(A_log[h]), skip = slice == 0 ? Dskip[h] : 0.f;
+            {
+                static_assert(CH <= 64, "one lane per token");
+                const float dt = softplus_precise(raw_dt[static_cast<size_t>(t0 + min(lane, nt - 1)) * ldd + h] + dt_bias[h]);
+                if (lane < CH) {
+                    dts[lane] = dt;
+                    as[lane] = expf(neg_rate * dt);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < NS; ++j) S[j] = j < nn ? S[j] : 0.f;
+            wave_lds_sync();
+            for (int tt = 0; tt < nt; ++tt) {
+                const float xv = xs[tt * 64 + lane];
+                const float a = as[tt], dx = dts[tt] * xv;
+                float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int j = 0; j < NS; j += 4) {
+                    const float4 b4 = *reinterpret_cast<const float4*>(&Bs[tt * NS + j]), c4 = *reinterpret_cast<const float4*>(&Cs[tt * NS + j]);
+                    S[j] = a * S[j] + dx * b4.x;         acc[0] += S[j] * c4.x;
+                    S[j + 1] = a * S[j + 1] + dx * b4.y; acc[1] += S[j + 1] * c4.y;
+                    S[j + 2] = a * S[j + 2] + dx * b4.z; acc[2] += S[j + 2] * c4.z;
+                    S[j + 3] = a * S[j + 3] + dx * b4.w; acc[3] += S[j + 3] * c4.w;
+                }
+                xs[tt * 64 + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]) + skip * xv;      // the slice's share of y, in x's place
+            }
+            if (write && p_ok) {
+#pragma unroll
+                for (int j = 0; j < NS; ++j)
+                    if (j < nn) sp[static_cast<size_t>(j) * P] = S[j];
+            }
         }
-        constexpr int BQ = CH * (NS / 4) / 64;
-        float4 bq[BQ], cq[BQ];
+        __syncthreads();
+        for (int i = threadIdx.x; i < nt * 64; i += blockDim.x) {
+            if (p0 + i % 64 >= P) continue;
+            float* out = y + static_cast<size_t>(t0 + i / 64) * ldy + h * P + p0 + i % 64;
+            float v = s0 > 0 ? *out + short_s[i] : short_s[i];       // (an element's every round is the same thread's)
+            for (int k = 1; k < min(waves, n_slices - s0); ++k) v += short_s[k * ssm_short_floats<NS, CH>() + i];
+            *out = v;
+        }
+        if (s0 + waves < n_slices) __syncthreads();                  // the shares have been read
+    }
+}
+
+// A portion of several chunks of SSM_TILE tokens in matrix form, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32). With cum_t
+// the logarithm of the decay accumulated from the chunk's start to token t:
+//   state kernel:  L[n, p] = sum_s exp(cum_last - cum_s) dt_s B[s, n] x[s, p]          what the chunk adds to the state
+//   join kernel:   S_0 = the slot's state, S_(k+1) = exp(cum_last of chunk k) S_k + L_k; S_k takes L_k's place, the last goes back
+//   output kernel: y[t, p] = sum_(s <= t) (C_t . B_s) exp(cum_t - cum_s) dt_s x[s, p] + exp(cum_t) sum_n C[t, n] S_k[n, p] + D x[t, p]
+// The same sums as token by token in another order; every exponent is at most 0. One workgroup of four wavefronts per (chunk,
+// head, 64 values of p). n is walked in slices of SSM_NS rows that pass through LDS, the next slice's loads in flight during the
+// products of one (45 KB of LDS: three workgroups a unit). Rows in LDS are an odd number of 16-byte pieces apart for operands read
+// four k at a time, and 4 floats more than a multiple of 64 for those read one k at a time (16 neighbouring columns of four rows
+// 4 apart): neither conflicts. A token after the other, as the short kernel does it, was bound by its chain of 64 tokens:
+// 2,048 tokens of 24 heads of 128 x 64 took 85 us for the chunks and 45 to join them; the three kernels take 16.0, 11.7 and 28.0 us.
+// Needs 16-byte aligned rows and column offsets.
+#define SSM_TILE 64
+#define SSM_NS 32
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+// Step sizes and accumulated decays of a chunk's nt tokens, worked out by one wavefront (lane t: token t; past the end: dt 0).
+// The logarithms are summed in double: their differences are small numbers between large ones (in 32 bits the logits of a small
+// model were 5.8e-6 from the exact ones where the scan token by token is 1.5e-6 away, with this at most 1.5e-6).
+__device__ __forceinline__ void chunk_decays(const float* raw_dt, int ldd, int t0, int nt, int h, const float* dt_bias, const float* A_log, int lane,
+                                             float* dt_s, double* cum_s) {
+    const float dt = softplus_precise(raw_dt[static_cast<size_t>(t0 + min(lane, nt - 1)) * ldd + h] + dt_bias[h]);
+    double run = lane < nt ? -static_cast<double>(expf(A_log[h])) * dt : 0.0;
 #pragma unroll
-        for (int u = 0; u < BQ; ++u) {
-            const int e = lane + 64 * u, tt = min(e / (NS / 4), nt - 1), q = min(e % (NS / 4), nq - 1);
-            const float* row = xbc + static_cast<size_t>(t0 + tt) * ldx + inner + g * N + n0 + 4 * q;
+    for (int off = 1; off < 64; off *= 2) {
+        const double up = __shfl_up(run, off, 64);
+        if (lane >= off) run += up;
+    }
+    dt_s[lane] = lane < nt ? dt : 0.f;
+    cum_s[lane] = run;
+}
+
+__global__ void __launch_bounds__(256)
+ssm_chunk_state_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict__ raw_dt, int ldd, const float* __restrict__ dt_bias,
+                       const float* __restrict__ A_log, const int* __restrict__ cu_q, const int* __restrict__ state_slots, int n_seqs, int H, int P,
+                       int N, int G, float* __restrict__ chunk_state, float* __restrict__ cumlog) {
+    __shared__ __attribute__((aligned(16))) float Xs[SSM_TILE][68], Bs[SSM_TILE][SSM_NS + 4];
+    __shared__ float dt_s[64];
+    __shared__ double cum_s[64];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64, col = lane % 16, quad = lane / 16;
+    const int h = blockIdx.y, p0 = blockIdx.x * 64;
+    const ChunkOf co = chunk_of(blockIdx.z, cu_q, n_seqs, SSM_TILE, true);
+    if (co.b < 0 || co.n_chunks < 2 || state_slots[co.b] < 0) return;
+    const int g = h / (H / G), inner = H * P;
+    const int t0 = cu_q[co.b] + co.k * SSM_TILE, nt = min(t0 + SSM_TILE, cu_q[co.b + 1]) - t0;
+    if (wave == 0) chunk_decays(raw_dt, ldd, t0, nt, h, dt_bias, A_log, lane, dt_s, cum_s);
+    const int pq = min(64, P - p0) / 4;
+    float4 xq[4], bq[2];
+    const float* b_row = xbc + inner + g * N;
+    auto fetch = [&](int n0) {
+        const int nq = min(SSM_NS, N - n0) / 4;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + 256 * u;
+            bq[u] = *reinterpret_cast<const float4*>(b_row + static_cast<size_t>(t0 + min(e / 8, nt - 1)) * ldx + n0 + 4 * min(e % 8, nq - 1));
+        }
+    };
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+        const int e = tid + 256 * u;
+        xq[u] = *reinterpret_cast<const float4*>(xbc + static_cast<size_t>(t0 + min(e / 16, nt - 1)) * ldx + h * P + p0 + 4 * min(e % 16, pq - 1));
+    }
+    fetch(0);
+    __syncthreads();
+    if (tid == 0) cumlog[static_cast<size_t>(t0 + nt - 1) * H + h] = static_cast<float>(cum_s[63]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {          // (tokens past the chunk's end have dt 0)
+        const int e = tid + 256 * u, s = e / 16;
+        const float w = s < nt && e % 16 < pq ? expf(static_cast<float>(cum_s[63] - cum_s[s])) * dt_s[s] : 0.f;
+        *reinterpret_cast<float4*>(&Xs[s][4 * (e % 16)]) = w != 0.f ? make_float4(w * xq[u].x, w * xq[u].y, w * xq[u].z, w * xq[u].w) : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    float* out = chunk_state + (static_cast<size_t>(co.first_chunk + co.k) * H + h) * N * P;
+    for (int n0 = 0; n0 < N; n0 += SSM_NS) {
+        const int nn = min(SSM_NS, N - n0);
+        if (n0 > 0) __syncthreads();          // the slice before has been read
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + 256 * u;
+            *reinterpret_cast<float4*>(&Bs[e / 8][4 * (e % 8)]) = e / 8 < nt && 4 * (e % 8) < nn ? bq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+        fetch(n0 + SSM_NS < N ? n0 + SSM_NS : n0);      // (past the last slice: it again, unused; under a condition it would be waited for here)
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);          // (the loads stay in front of the products)
+        f32x4 acc[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};      // rows n of two tiles, columns p of the wavefront's
+#pragma unroll
+        for (int s = 0; s < SSM_TILE; s += 16)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const int k = s + 4 * quad + e;
+                const float xv = Xs[k][16 * wave + col];
+#pragma unroll
+                for (int i = 0; i < 2; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x4f32(Bs[k][16 * i + col], xv, acc[i], 0, 0, 0);
+            }
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const int n = 16 * i + 4 * quad + r, p = p0 + 16 * wave + col;
+                if (n < nn && p < P) out[static_cast<size_t>(n0 + n) * P + p] = acc[i][r];
+            }
+    }
+}
+
+// One thread per element of a head's state; the chunks' sums are asked for four ahead.
+__global__ void __launch_bounds__(256)
+ssm_chunk_prefix_kernel(const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ state, size_t slot_floats,
+                        size_t scan_offset, int H, int NP, int write, float* __restrict__ chunk_state, const float* __restrict__ cumlog) {
+    const int b = blockIdx.z, h = blockIdx.y, i = blockIdx.x * 256 + threadIdx.x;
+    const int q0 = cu_q[b], q1 = cu_q[b + 1], n_chunks = (q1 - q0 + SSM_TILE - 1) / SSM_TILE;
+    const int slot = state_slots[b];
+    if (n_chunks < 2 || slot < 0) return;
+    int first = 0;
+    for (int k = 0; k < b; ++k) {
+        const int n = (cu_q[k + 1] - cu_q[k] + SSM_TILE - 1) / SSM_TILE;
+        if (n > 1) first += n;
+    }
+    if (i >= NP) return;
+    float* sp = state + static_cast<size_t>(slot) * slot_floats + scan_offset + static_cast<size_t>(h) * NP + i;
+    const size_t step = static_cast<size_t>(H) * NP;
+    float* at = chunk_state + static_cast<size_t>(first) * step + static_cast<size_t>(h) * NP + i;
+    float S = *sp;
+    for (int k0 = 0; k0 < n_chunks; k0 += 4) {
+        float L[4], a[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+            const int k = min(k0 + u, n_chunks - 1);
+            L[u] = at[k * step];
+            a[u] = cumlog[static_cast<size_t>(min(q0 + (k + 1) * SSM_TILE, q1) - 1) * H + h];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (k0 + u < n_chunks) {
+                at[(k0 + u) * step] = S;
+                S = expf(a[u]) * S + L[u];
+            }
+    }
+    if (write) *sp = S;
+}
+
+__global__ void __launch_bounds__(256)
+ssm_chunk_out_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict__ raw_dt, int ldd, const float* __restrict__ dt_bias,
+                     const float* __restrict__ A_log, const float* __restrict__ Dskip, const int* __restrict__ cu_q, const int* __restrict__ state_slots,
+                     int n_seqs, float* __restrict__ y, int ldy, int H, int P, int N, int G, const float* __restrict__ chunk_state) {
+    __shared__ __attribute__((aligned(16))) float Xs[SSM_TILE][68], Ps[SSM_NS][68];
+    // the slices of B and C; once they are read, a wavefront's weights [16 tokens][64 tokens before] lie in their place
+    __shared__ __attribute__((aligned(16))) float slices[2 * SSM_TILE * (SSM_NS + 4)];
+    static_assert(4 * 16 * 68 <= 2 * SSM_TILE * (SSM_NS + 4), "the weights fit the slices");
+    float (*Bs)[SSM_NS + 4] = reinterpret_cast<float (*)[SSM_NS + 4]>(slices), (*Cs)[SSM_NS + 4] = Bs + SSM_TILE;
+    float (*Ms)[16][68] = reinterpret_cast<float (*)[16][68]>(slices);
+    __shared__ float dt_s[64];
+    __shared__ double cum_s[64];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64, col = lane % 16, quad = lane / 16;
+    const int h = blockIdx.y, p0 = blockIdx.x * 64;
+    const ChunkOf co = chunk_of(blockIdx.z, cu_q, n_seqs, SSM_TILE, true);
+    if (co.b < 0 || co.n_chunks < 2 || state_slots[co.b] < 0) return;
+    const int g = h / (H / G), inner = H * P;
+    const int t0 = cu_q[co.b] + co.k * SSM_TILE, nt = min(t0 + SSM_TILE, cu_q[co.b + 1]) - t0;
+    const int pq = min(64, P - p0) / 4;
+    float4 xq[4], bq[2], cq[2], sq[2];
+    const float* b_row = xbc + inner + g * N;
+    const float* s_row = chunk_state + (static_cast<size_t>(co.first_chunk + co.k) * H + h) * N * P + p0;
+    auto fetch = [&](int n0) {
+        const int nn = min(SSM_NS, N - n0), nq = nn / 4;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + 256 * u;
+            const float* row = b_row + static_cast<size_t>(t0 + min(e / 8, nt - 1)) * ldx + n0 + 4 * min(e % 8, nq - 1);
             bq[u] = *reinterpret_cast<const float4*>(row);
             cq[u] = *reinterpret_cast<const float4*>(row + G * N);
+            sq[u] = *reinterpret_cast<const float4*>(s_row + static_cast<size_t>(n0 + min(e / 16, nn - 1)) * P + 4 * min(e % 16, pq - 1));
         }
+    };
+    fetch(0);
 #pragma unroll
-        for (int u = 0; u < CH / 4; ++u) {
-            const int e = lane + 64 * u;
-            *reinterpret_cast<float4*>(&xs[e / 16][4 * (e % 16)]) = xq[u];
+    for (int u = 0; u < 4; ++u) {
+        const int e = tid + 256 * u;
+        xq[u] = *reinterpret_cast<const float4*>(xbc + static_cast<size_t>(t0 + min(e / 16, nt - 1)) * ldx + h * P + p0 + 4 * min(e % 16, pq - 1));
+    }
+    if (wave == 0) chunk_decays(raw_dt, ldd, t0, nt, h, dt_bias, A_log, lane, dt_s, cum_s);
+    // the wavefront's tokens are rows 16 wave to + 15: gram, their products C_t . B_s with the tokens s of the tiles up to their own; acc, y
+    f32x4 gram[4], acc[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) gram[j] = acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int n0 = 0; n0 < N; n0 += SSM_NS) {
+        const int nn = min(SSM_NS, N - n0);
+        if (n0 > 0) __syncthreads();
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int e = tid + 256 * u;
+            const bool real = e / 8 < nt && 4 * (e % 8) < nn;
+            *reinterpret_cast<float4*>(&Bs[e / 8][4 * (e % 8)]) = real ? bq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+            *reinterpret_cast<float4*>(&Cs[e / 8][4 * (e % 8)]) = real ? cq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+            *reinterpret_cast<float4*>(&Ps[e / 16][4 * (e % 16)]) = e / 16 < nn && e % 16 < pq ? sq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
+        if (n0 == 0) {
 #pragma unroll
-        for (int u = 0; u < BQ; ++u) {
-            const int e = lane + 64 * u, qi = e % (NS / 4);
-            const bool real = qi < nq;                          // rows of the slice beyond N count as zeros
-            *reinterpret_cast<float4*>(&Bs[e / (NS / 4)][4 * qi]) = real ? bq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
-            *reinterpret_cast<float4*>(&Cs[e / (NS / 4)][4 * qi]) = real ? cq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+            for (int u = 0; u < 4; ++u) {
+                const int e = tid + 256 * u;
+                *reinterpret_cast<float4*>(&Xs[e / 16][4 * (e % 16)]) = e / 16 < nt && e % 16 < pq ? xq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+            }
+        }
+        fetch(n0 + SSM_NS < N ? n0 + SSM_NS : n0);      // (past the last slice: it again, unused; under a condition it would be waited for here)
+        __syncthreads();
+        __builtin_amdgcn_sched_barrier(0);          // (the loads stay in front of the products)
+#pragma unroll
+        for (int q = 0; q < SSM_NS; q += 16) {
+            // all operands first; products with tokens behind the wavefront's own, masked below, cost no more than the last
+            // wavefront's, which needs all of them
+            const f32x4 c4 = *reinterpret_cast<const f32x4*>(&Cs[16 * wave + col][q + 4 * quad]);
+            f32x4 b4[4];
+            float s4[4][4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) b4[j] = *reinterpret_cast<const f32x4*>(&Bs[16 * j + col][q + 4 * quad]);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s4[e][j] = Ps[q + 4 * quad + e][16 * j + col];
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) gram[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4[e], b4[j][e], gram[j], 0, 0, 0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(c4[e], s4[e][j], acc[j], 0, 0, 0);
         }
     }
-    // Step sizes and decays are the same for every lane: lane t works them out for token t of the chunk, once
-    // (softplus, two exponentials), and a running sum over the lanes gives the logarithm of the decay accumulated
-    // since the chunk began.
-    const float bias = dt_bias[h], neg_rate = -expf(A_log[h]), skip = slice == 0 ? Dskip[h] : 0.f;
-    {
-        static_assert(CH <= 64, "one lane per token of a chunk");
-        const float dt = softplus_precise(raw_dt[static_cast<size_t>(t0 + min(lane, nt - 1)) * ldd + h] + bias);
-        const float lg = lane < nt ? neg_rate * dt : 0.f;
-        float run = lg;
+    // (register r of a lane: row 4 quad + r, column col of a tile)
+    double cum_t[4];
 #pragma unroll
-        for (int off = 1; off < 64; off *= 2) {
-            const float up = __shfl_up(run, off, 64);
-            if (lane >= off) run += up;
-        }
-        dts[lane] = dt;
-        as[lane] = expf(lg);
-        if (co.n_chunks > 1 && blockIdx.x == 0 && lane < nt) cumlog[static_cast<size_t>(t0 + lane) * H + h] = run;
+    for (int r = 0; r < 4; ++r) cum_t[r] = cum_s[16 * wave + 4 * quad + r];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float seen = expf(static_cast<float>(cum_t[r]));
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[j][r] *= seen;
     }
+    __syncthreads();          // the last slice has been read
 #pragma unroll
-    for (int j = 0; j < NS; ++j) S[j] = (co.k == 0 && j < nn) ? S[j] : 0.f;
-    float* yp = y + slice * part_stride + h * P + pc;
+    for (int j = 0; j < 4; ++j) {
+        const int s = 16 * j + col;
+        const double cs = cum_s[s];
+        const float ds = dt_s[s];
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            Ms[wave][4 * quad + r][s] = s <= 16 * wave + 4 * quad + r ? gram[j][r] * expf(static_cast<float>(cum_t[r] - cs)) * ds : 0.f;
+    }
     wave_lds_sync();
-    for (int tt = 0; tt < nt; ++tt) {
-        const float xv = xs[tt][lane];
-        const float a = as[tt], dx = dts[tt] * xv;
-        float acc[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < NS; j += 4) {
-            const float4 b4 = *reinterpret_cast<const float4*>(&Bs[tt][j]), c4 = *reinterpret_cast<const float4*>(&Cs[tt][j]);
-            S[j] = a * S[j] + dx * b4.x;         acc[0] += S[j] * c4.x;
-            S[j + 1] = a * S[j + 1] + dx * b4.y; acc[1] += S[j + 1] * c4.y;
-            S[j + 2] = a * S[j + 2] + dx * b4.z; acc[2] += S[j + 2] * c4.z;
-            S[j + 3] = a * S[j + 3] + dx * b4.w; acc[3] += S[j + 3] * c4.w;
+    for (int i = 0; i < 4; ++i) {
+        const f32x4 m4 = *reinterpret_cast<const f32x4*>(&Ms[wave][col][16 * i + 4 * quad]);
+        float x4[4][4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) x4[e][j] = Xs[16 * i + 4 * quad + e][16 * j + col];
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(m4[e], x4[e][j], acc[j], 0, 0, 0);
+    }
+    const float skip = Dskip[h];
+#pragma unroll
+    for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int t = 16 * wave + 4 * quad + r, p = 16 * j + col;
+            if (t < nt && p0 + p < P) y[static_cast<size_t>(t0 + t) * ldy + h * P + p0 + p] = acc[j][r] + skip * Xs[t][p];
         }
-        if (p_ok) yp[static_cast<size_t>(t0 + tt) * ldy] = (acc[0] + acc[1]) + (acc[2] + acc[3]) + skip * xv;
-    }
-    if (!p_ok) return;
-    if (co.n_chunks > 1) sp = chunk_state + ((static_cast<size_t>(co.first_chunk + co.k) * H + h) * N + n0) * P + p;
-    if (write || co.n_chunks > 1) {
-#pragma unroll
-        for (int j = 0; j < NS; ++j)
-            if (j < nn) sp[static_cast<size_t>(j) * P] = S[j];
-    }
 }
 
 // What the chunks before chunk k of a portion contribute to it (see ssm_scan_kernel): with A_j the whole
@@ -680,12 +953,16 @@ size_t mllm_ssm_scan_workspace_floats(int T, int B, int H, int P, int N) {
     (void)B;
     return chunk_states(T) * H * P * N + static_cast<size_t>(T) * H;
 }
-// The scan leaves y as this many shares (see ssm_scan_kernel), part_stride floats apart.
-int mllm_ssm_scan_parts(int N) { return (N + SSM_SLICE - 1) / SSM_SLICE; }
+// Whether the kernels that read 16 bytes at a time take these rows: the short one and the ones in matrix form.
+static bool ssm_by_quads(const float* xbc, int ldx, int P, int N) {
+    return ldx % 4 == 0 && P % 4 == 0 && N % 4 == 0 && (reinterpret_cast<uintptr_t>(xbc) & 15) == 0;
+}
+// The scan leaves y as this many shares, part_stride floats apart: one, or one per slice of the state's rows (ssm_scan_kernel).
+int mllm_ssm_scan_parts(const float* xbc, int ldx, int P, int N) { return ssm_by_quads(xbc, ldx, P, N) ? 1 : (N + SSM_SLICE - 1) / SSM_SLICE; }
 
 // The scan over every sequence's portion (see the kernels). `workspace` (mllm_ssm_scan_workspace_floats floats)
 // is needed when a portion is longer than one chunk (max_q_len > 64). -1: H is no multiple of G, or the
-// workspace is missing.
+// workspace is missing or not 16-byte aligned.
 int mllm_ssm_scan(const float* xbc, int ldx, const float* raw_dt, int ldd, const float* dt_bias, const float* A_log,
                   const float* Dskip, const int* cu_q, const int* state_slots, float* state, size_t slot_floats,
                   size_t scan_offset, float* y, int ldy, size_t part_stride, int T, int B, int max_q_len, int H, int P, int N,
@@ -697,18 +974,39 @@ int mllm_ssm_scan(const float* xbc, int ldx, const float* raw_dt, int ldd, const
     const int n_chunks = chunked ? T / SSM_CHUNK + B : B;
     float* chunk_state = workspace;
     float* cumlog = workspace ? workspace + chunk_states(T) * H * P * N : nullptr;
-    const int n_slices = mllm_ssm_scan_parts(N);
+    const int n_slices = (N + SSM_SLICE - 1) / SSM_SLICE;
+    if (ssm_by_quads(xbc, ldx, P, N)) {
+        if (chunked && (reinterpret_cast<uintptr_t>(workspace) & 15)) return -1;
+        const int p_tiles = (P + 63) / 64, waves = std::min(n_slices, 4);
+#define SSM_SHORT(CH)                                                                                                  \
+    do {                                                                                                               \
+        constexpr int floats = ssm_short_floats<SSM_SLICE, CH>();                                                      \
+        auto kernel = ssm_short_kernel<SSM_SLICE, CH>;                                                                 \
+        static bool lds_allowed = 4 * floats * 4 <= 64 * 1024;      /* more has to be asked for once */                \
+        if (!lds_allowed) {                                                                                            \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * floats * 4); \
+            if (e != hipSuccess) return static_cast<int>(e);                                                           \
+            lds_allowed = true;                                                                                        \
+        }                                                                                                              \
+        kernel<<<dim3(p_tiles, H, B), 64 * waves, waves * floats * 4, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, Dskip, cu_q, state_slots, \
+                                                                                      state, slot_floats, scan_offset, y, ldy, H, P, N, G, write);     \
+    } while (0)
+        if (max_q_len <= 8) SSM_SHORT(8); else if (!chunked || T < static_cast<long>(B) * max_q_len) SSM_SHORT(SSM_CHUNK);      // (equally long portions: none)
+#undef SSM_SHORT
+        if (chunked) {
+            const dim3 tiles(p_tiles, H, n_chunks);
+            ssm_chunk_state_kernel<<<tiles, 256, 0, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, cu_q, state_slots, B, H, P, N, G, chunk_state, cumlog);
+            ssm_chunk_prefix_kernel<<<dim3((N * P + 255) / 256, H, B), 256, 0, stream>>>(cu_q, state_slots, state, slot_floats, scan_offset, H, N * P,
+                                                                                        write, chunk_state, cumlog);
+            ssm_chunk_out_kernel<<<tiles, 256, 0, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, Dskip, cu_q, state_slots, B, y, ldy, H, P, N, G, chunk_state);
+        }
+        MLLM_LAUNCH_CHECK();
+        return 0;
+    }
     const dim3 grid(((P + 63) / 64) * n_slices, H, n_chunks);
-    const bool aligned = ldx % 4 == 0 && P % 4 == 0 && N % 4 == 0 && (reinterpret_cast<uintptr_t>(xbc) & 15) == 0;
-    if (aligned)
-        ssm_scan_staged_kernel<SSM_SLICE, SSM_CHUNK><<<grid, 64, 0, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, Dskip, cu_q, state_slots,
-                                                                             B, state, slot_floats, scan_offset, y, ldy, part_stride, H, P, N,
-                                                                             G, n_slices, write, SSM_CHUNK, chunked ? chunk_state : nullptr,
-                                                                             cumlog);
-    else
-        ssm_scan_kernel<SSM_SLICE><<<grid, 64, 0, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, Dskip, cu_q, state_slots, B, state,
-                                                           slot_floats, scan_offset, y, ldy, part_stride, H, P, N, G, n_slices, write,
-                                                           SSM_CHUNK, chunked ? chunk_state : nullptr, cumlog);
+    ssm_scan_kernel<SSM_SLICE><<<grid, 64, 0, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, Dskip, cu_q, state_slots, B, state,
+                                                       slot_floats, scan_offset, y, ldy, part_stride, H, P, N, G, n_slices, write,
+                                                       SSM_CHUNK, chunked ? chunk_state : nullptr, cumlog);
     if (chunked)
         ssm_chunk_join_kernel<SSM_SLICE><<<grid, 64, 0, stream>>>(xbc, ldx, cu_q, state_slots, B, state, slot_floats, scan_offset, y,
                                                                  ldy, part_stride, H, P, N, G, n_slices, write, SSM_CHUNK,

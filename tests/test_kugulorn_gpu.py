@@ -221,3 +221,20 @@ def test_greedy_generation_through_the_engine(dirs, dtype):
                 row = pk.forward(cfg, w, ids)[-1]
                 assert float(row[t]) >= float(row.max()) - 0.08 * float(row.std()), (o, t)
                 ids.append(t)
+
+
+@pytest.mark.parametrize("heads,vdim,state,groups,conv", [(2, 64, 128, 1, 4), (3, 68, 36, 1, 4),      # a second tile of 4 columns; a slice of 4 rows
+                                                          (4, 8, 20, 2, 2), (2, 16, 160, 1, 9),      # five slices: two rounds; more taps than vector loads
+                                                          (2, 6, 10, 1, 3)])                         # sizes that are no whole 16 bytes
+@pytest.mark.parametrize("sizes", [(8, 9, 64), (65, 1, 200, 7), (63, 128, 129, 2)])
+def test_scan_portions_of_every_length(tmp_path, heads, vdim, state, groups, conv, sizes):
+    """The scan's kernels at their borders, in 32 bits: portions of at most 8 and 64 tokens, of several chunks and of one more
+    than that, side by side in one step and carried from step to step, with decoded tokens among them."""
+    from mini_llm_amd import write_random_model
+    cfg = kc.model([kc.mamba(heads=heads, vdim=vdim, state=state, groups=groups, conv=conv, norm_groups=1)], vocab=200, width=48)
+    write_random_model(dict(cfg), str(tmp_path), 5)
+    reqs = kc.requests(cfg["vocab"], [1, 8, 9, 64, 65, 129, 193, 280], seed=heads + state)
+    steps, _ = ru.trace_mixed(reqs, seed=state, max_live=4, tail=3, sizes=sizes)
+    runner = _runner(str(tmp_path), "float32", n_pages=ru.peak_tokens(steps) // 4)
+    kc.check_against_plain(str(tmp_path), reqs, steps, ru.run_in_process(runner, steps), "float32", cfg["vocab"], f"scan {sizes}")
+    assert runner.check() == ""
