@@ -41,6 +41,54 @@ __global__ void conv_silu_kernel(const float* __restrict__ proj, int ld, int col
     out[static_cast<size_t>(t) * ldo + ch] = silu_precise(acc);
 }
 
+// The same four channels a thread, all loads of a token asked for together, as in conv_residual_vec_kernel below (which see):
+// 2,048 tokens x 1,792 channels 14.3 us, one channel a thread 26.
+template <int TAPS>
+__global__ void conv_silu_vec_kernel(const float* __restrict__ in, int ld, int C, const float* __restrict__ w, const float* __restrict__ bias,
+                                     const int* __restrict__ token_seq, const int* __restrict__ cu_q, const int* __restrict__ state_slots,
+                                     float* __restrict__ state, size_t slot_floats, float* __restrict__ out, int ldo, long long total4, int carry) {
+    const long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= total4) return;
+    const int C4 = C / 4;
+    const int t = static_cast<int>(i / C4), ch = static_cast<int>(i % C4) * 4;
+    const int b = token_seq[t], slot = state_slots[b];
+    if (slot < 0) return;
+    const int first = cu_q[b], k = t - first;
+    float* carried = state + static_cast<size_t>(slot) * slot_floats;
+    float4 wf[TAPS], v[TAPS];             // wf: the four channels' taps one behind the other (4 * TAPS floats)
+    const float4 b4 = *reinterpret_cast<const float4*>(bias + ch);
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) wf[j] = *reinterpret_cast<const float4*>(w + static_cast<size_t>(ch) * TAPS + 4 * j);
+    if (k >= TAPS - 1) {
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) v[j] = *reinterpret_cast<const float4*>(in + static_cast<size_t>(t - (TAPS - 1 - j)) * ld + ch);
+    } else {
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+            const int idx = k - (TAPS - 1 - j);
+            v[j] = idx >= 0 ? *reinterpret_cast<const float4*>(in + static_cast<size_t>(first + idx) * ld + ch)
+                            : *reinterpret_cast<const float4*>(carried + static_cast<size_t>(TAPS - 1 + idx) * C + ch);
+        }
+    }
+    float wv[4 * TAPS];
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) { wv[4 * j] = wf[j].x; wv[4 * j + 1] = wf[j].y; wv[4 * j + 2] = wf[j].z; wv[4 * j + 3] = wf[j].w; }
+    float acc[4] = {b4.x, b4.y, b4.z, b4.w};
+#pragma unroll
+    for (int j = 0; j < TAPS; ++j) {
+        acc[0] += wv[0 * TAPS + j] * v[j].x;
+        acc[1] += wv[1 * TAPS + j] * v[j].y;
+        acc[2] += wv[2 * TAPS + j] * v[j].z;
+        acc[3] += wv[3 * TAPS + j] * v[j].w;
+    }
+    if (carry) {                          // (see above)
+#pragma unroll
+        for (int j = 1; j < TAPS; ++j) *reinterpret_cast<float4*>(carried + static_cast<size_t>(j - 1) * C + ch) = v[j];
+    }
+    *reinterpret_cast<float4*>(out + static_cast<size_t>(t) * ldo + ch) =
+        make_float4(silu_precise(acc[0]), silu_precise(acc[1]), silu_precise(acc[2]), silu_precise(acc[3]));
+}
+
 // out[t, ch] = in[t, ch] + sum_j w[ch, j] * in(t - (taps - 1 - j), ch): the convolution added onto its own input,
 // no bias and no activation, the result in the activation dtype. Carried rows as above. residual == 0: the
 // convolution alone, its input not added.
@@ -859,8 +907,20 @@ int mllm_conv_silu(const float* proj, int ld, int col0, int C, const float* w, c
     const long long total = static_cast<long long>(T) * C;
     // (one token a sequence: the convolution's kernel brings the carried rows up to date itself)
     const bool single = T == B && write && taps > 1;
-    conv_silu_kernel<<<static_cast<int>((total + 255) / 256), 256, 0, stream>>>(proj, ld, col0, C, w, bias, taps, token_seq, cu_q,
-                                                                                state_slots, state, slot_floats, out, ldo, total, single ? 1 : 0);
+    const bool vec = taps <= 8 && C % 4 == 0 && col0 % 4 == 0 && ld % 4 == 0 && ldo % 4 == 0 && slot_floats % 4 == 0 &&
+                     ((reinterpret_cast<uintptr_t>(proj) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(bias) |
+                       reinterpret_cast<uintptr_t>(state) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
+    if (vec) {
+        const long long total4 = total / 4;
+        const int blocks4 = static_cast<int>((total4 + 255) / 256);
+#define CSV(TAPS) case TAPS: conv_silu_vec_kernel<TAPS><<<blocks4, 256, 0, stream>>>(proj + col0, ld, C, w, bias, token_seq, cu_q, state_slots, state, \
+                                                                                    slot_floats, out, ldo, total4, single ? 1 : 0); break
+        switch (taps) { CSV(1); CSV(2); CSV(3); CSV(4); CSV(5); CSV(6); CSV(7); CSV(8); }
+#undef CSV
+    } else {
+        conv_silu_kernel<<<static_cast<int>((total + 255) / 256), 256, 0, stream>>>(proj, ld, col0, C, w, bias, taps, token_seq, cu_q,
+                                                                                    state_slots, state, slot_floats, out, ldo, total, single ? 1 : 0);
+    }
     MLLM_LAUNCH_CHECK();
     if (write && taps > 1 && !single) {
         const long long pairs = static_cast<long long>(B) * C;
