@@ -442,13 +442,14 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 enum { A_GLOBAL = 0, A_NORMED = 1, A_STAGED = 2, A_MERGED = 3 };
 #define MERGE_MAX_SPLITS 4      // splits of a pair that the merging load takes (registers: 10 per split and load)
 
-// The states of up to MERGE_MAX_SPLITS splits for 8 consecutive elements of one head of one token.
-struct SplitStates {
-    float2 ml[MERGE_MAX_SPLITS];          // maximum (base 2), sum
-    float4 o[MERGE_MAX_SPLITS][2];        // 8 elements of the unnormalised output
+// The states of MS splits for 8 consecutive elements of one head of one token.
+template <int MS> struct SplitStates {
+    float2 ml[MS];          // maximum (base 2), sum
+    float4 o[MS][2];        // 8 elements of the unnormalised output
 };
 
-template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false>
+template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false, int MS = MERGE_MAX_SPLITS,
+          bool ONE = false>
 __global__ void __launch_bounds__(ASRC == A_NORMED ? 512 : (ASRC == A_GLOBAL || ASRC == A_MERGED ? 768 : 1024))
 gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: what the first loads need
                  const bf16_t* __restrict__ W, int ldw, int N, int K, int M, int col_blocks, int row_blocks,
@@ -458,10 +459,10 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
                  void* __restrict__ C, int ldc, const float* __restrict__ gamma, const float* __restrict__ beta,
                  float eps, const int* __restrict__ rows, float* __restrict__ part_sums,
                  int* __restrict__ part_counters,
-                 // A_MERGED: the attention splits' states (layout: attention_decode.hip), their number,
+                 // A_MERGED: the states of the attention's MS splits (layout: attention_decode.hip),
                  // heads per token and head size (K = heads x head size)
                  const float* __restrict__ split_o = nullptr, const float* __restrict__ split_ml = nullptr,
-                 int n_splits = 1, int a_heads = 1, int a_head_dim = 8,
+                 int a_heads = 1, int a_head_dim = 8,
                  // A_NORMED: != 0: the norm does not centre (RMS norm: x / sqrt(mean(x^2) + eps) * gamma)
                  int rms = 0,
                  // THROUGH (mode EPI_THROUGH): the norms the result passes and the copy it leaves; otherwise (plain store of
@@ -595,28 +596,28 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
             arow[j] = A + static_cast<size_t>(arow_idx[j]) * lda;
         }
     }
-    // A_MERGED: requests the splits' states for the 8 elements from k on of row `row` (all loads together;
-    // splits beyond n_splits take the last one again and get no weight), and merges them later
-    auto fetch_splits = [&](SplitStates& st, int row, int k) {
+    // A_MERGED: requests the splits' states for the 8 elements from k on of row `row` (all loads together; n_splits is MS),
+    // and merges them later
+    auto fetch_splits = [&](SplitStates<MS>& st, int row, int k) {
         const int h = k / a_head_dim, e = k - h * a_head_dim;
         const size_t pair = static_cast<size_t>(row) * a_heads + h;
 #pragma unroll
-        for (int sidx = 0; sidx < MERGE_MAX_SPLITS; ++sidx) {
-            const size_t slot = pair * n_splits + min(sidx, n_splits - 1);
+        for (int sidx = 0; sidx < MS; ++sidx) {
+            const size_t slot = pair * MS + sidx;
             st.ml[sidx] = *reinterpret_cast<const float2*>(split_ml + slot * 2);
             const float4* src = reinterpret_cast<const float4*>(split_o + slot * a_head_dim + e);
             st.o[sidx][0] = src[0];
             st.o[sidx][1] = src[1];
         }
     };
-    auto merge_splits = [&](const SplitStates& st) -> bf16x8 {
+    auto merge_splits = [&](const SplitStates<MS>& st) -> bf16x8 {
         float mx = st.ml[0].x;
 #pragma unroll
-        for (int sidx = 1; sidx < MERGE_MAX_SPLITS; ++sidx) mx = fmaxf(mx, sidx < n_splits ? st.ml[sidx].x : mx);
+        for (int sidx = 1; sidx < MS; ++sidx) mx = fmaxf(mx, st.ml[sidx].x);
         float l = 0.f, o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int sidx = 0; sidx < MERGE_MAX_SPLITS; ++sidx) {
-            const float w = sidx < n_splits ? fast_exp2(st.ml[sidx].x - mx) : 0.f;
+        for (int sidx = 0; sidx < MS; ++sidx) {
+            const float w = fast_exp2(st.ml[sidx].x - mx);
             l = fmaf(w, st.ml[sidx].y, l);
             o[0] = fmaf(w, st.o[sidx][0].x, o[0]); o[1] = fmaf(w, st.o[sidx][0].y, o[1]);
             o[2] = fmaf(w, st.o[sidx][0].z, o[2]); o[3] = fmaf(w, st.o[sidx][0].w, o[3]);
@@ -636,7 +637,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         bf16x8 a[A_REGS ? (A_TWO ? U : U / 2) : 1];
     };
     // (A_MERGED) the states requested for a chunk's blocks, rows 0..7 and 8..15
-    SplitStates pending[ASRC == A_MERGED ? U / 2 : 1][ASRC == A_MERGED && A_TWO ? 2 : 1];
+    SplitStates<MS> pending[ASRC == A_MERGED ? U / 2 : 1][ASRC == A_MERGED && A_TWO ? 2 : 1];
     auto fetch_block_splits = [&](int h, int k0) {
         if (ASRC != A_MERGED) return;
 #pragma unroll
@@ -905,9 +906,12 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         lds_barrier();
     }
 
+    // ONE: the launcher knows that a chunk holds all of a wavefront's blocks, and a second one takes no registers. (With it the
+    // kernels of four blocks a wavefront, and those that merge splits, kept 76 to 1,220 bytes a lane in scratch memory.)
+    constexpr bool SINGLE = ONE || ASRC == A_MERGED;
     if (n_chunks == 0) {
         mma_some(c0, n_blocks, k_first);
-    } else if (n_chunks == 1) {
+    } else if (SINGLE || n_chunks == 1) {
         mma_chunk(c0, 0);
     } else if (n_chunks > 1) {
         // past the last chunk the prefetch takes chunk 0 again (long since arrived, never used)
@@ -918,7 +922,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
             if (ci + 1 < n_chunks) mma_chunk(c1, ci + 1);
         }
     }
-    {
+    if (!SINGLE) {
         // blocks left over: fewer than H, loaded together
         const int first = n_chunks * H, left = n_chunks > 0 ? n_blocks - first : 0;
         if (left > 0) load_left();
@@ -1116,7 +1120,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         if (e != hipSuccess) return static_cast<int>(e);                                               \
         kernel<<<grid, block, staged_bytes, stream>>>(W, ldw, N, K, M, col_blocks, row_blocks, 16, 1, A, lda, mode, \
                                                       bias, C, ldc, gamma, beta, eps, rows, nullptr, nullptr, \
-                                                      nullptr, nullptr, 1, 1, 8, 0, KvScatter{});                 \
+                                                      nullptr, nullptr, 1, 8, 0, KvScatter{});                    \
         break;                                                                                         \
     }
         switch (mt) {
@@ -1134,9 +1138,9 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     }
     if (smem > MAX_DYNAMIC_LDS) return -2;
     constexpr int ASRC = LN_FUSED ? A_NORMED : (MERGED ? A_MERGED : A_GLOBAL);
-#define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, ...)                                                \
+#define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...)                                      \
     do {                                                                                               \
-        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH>;                          \
+        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE>;                \
         static bool lds_allowed = false;      /* more than 64 KB of dynamic LDS has to be asked for once */ \
         if (!lds_allowed) {                                                                            \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                  \
@@ -1146,61 +1150,77 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         }                                                                                              \
         kernel<<<grid, block, smem, stream>>>(W, ldw, N, K, M, col_blocks, row_blocks, cols_per_wg, k_parts, A, lda, \
                                               mode, bias, C, ldc, gamma, beta, eps, rows, part_sums,      \
-                                              part_counters, merged.split_o, merged.split_ml, merged.n_splits, \
+                                              part_counters, merged.split_o, merged.split_ml,             \
                                               merged.heads, merged.head_dim, rms, __VA_ARGS__);        \
     } while (0)
-#define SKINNY_LAUNCH(SPLIT, UV, A2, NTV)                                                              \
+#define SKINNY_LAUNCH(SPLIT, UV, A2, NTV, ONE)                                                         \
     do {                                                                                               \
         if constexpr (ASRC == A_GLOBAL) {                                                              \
-            if (through != nullptr) { SKINNY_KERNEL(SPLIT, UV, A2, NTV, true, *through); break; }      \
+            if (through != nullptr) { SKINNY_KERNEL(SPLIT, UV, A2, NTV, true, MERGE_MAX_SPLITS, ONE, *through); break; } \
         }                                                                                              \
-        SKINNY_KERNEL(SPLIT, UV, A2, NTV, false, kv);                                                  \
+        SKINNY_KERNEL(SPLIT, UV, A2, NTV, false, MERGE_MAX_SPLITS, ONE, kv);                           \
+    } while (0)
+// one chunk of UV / 2 blocks, or several
+#define SKINNY_CHUNKS(UV, A2, NTV)                                                                     \
+    do {                                                                                               \
+        if (per_wave <= UV / 2) SKINNY_LAUNCH(true, UV, A2, NTV, true);                                \
+        else SKINNY_LAUNCH(true, UV, A2, NTV, false);                                                  \
     } while (0)
     if (split_k) {
         // a chunk holds all k blocks of a wavefront when they are at most 3 (4 without the fused
-        // norm and with at most 8 rows): whole chunks only, so nothing is requested twice. The
-        // largest chunks of the kernels without the norm spill a few registers, and are still
-        // faster than smaller chunks (measured)
+        // norm and with at most 8 rows): whole chunks only, so nothing is requested twice, and
+        // one chunk's registers are enough. (The largest chunks of the kernels without the norm spill a few registers
+        // where a second one is in flight, and are still faster than smaller chunks.)
         const int per_wave = (k_blocks + nw - 1) / nw;
-        if (two_tiles) {
-            // (two tiles per chunk slot: half the blocks per chunk)
-            if (per_wave <= 1 || !LN_FUSED) SKINNY_LAUNCH(true, 2, false, 2);
-            else SKINNY_LAUNCH(true, 4, false, 2);
-        } else if (LN_FUSED) {
-            switch (std::min(per_wave, 3)) {
-                case 1: SKINNY_LAUNCH(true, 2, false, 1); break;
-                case 2: SKINNY_LAUNCH(true, 4, false, 1); break;
-                default: SKINNY_LAUNCH(true, 6, false, 1); break;
-            }
-        } else if (MERGED) {
+        if constexpr (MERGED) {
             // the splits' states of a whole chunk are in flight together: one chunk holds all of a
             // wavefront's k blocks, at most 3
             if (per_wave > 3) return -2;
-            if (M <= 8) {
-                switch (per_wave) {
-                    case 1: SKINNY_LAUNCH(true, 2, false, 1); break;
-                    case 2: SKINNY_LAUNCH(true, 4, false, 1); break;
-                    default: SKINNY_LAUNCH(true, 6, false, 1); break;
-                }
-            } else {
-                switch (per_wave) {
-                    case 1: SKINNY_LAUNCH(true, 2, true, 1); break;
-                    case 2: SKINNY_LAUNCH(true, 4, true, 1); break;
-                    default: SKINNY_LAUNCH(true, 6, true, 1); break;
-                }
+#define SKINNY_MERGED(MSV)                                                                             \
+    do {                                                                                               \
+        if (M <= 8) {                                                                                  \
+            switch (per_wave) {                                                                        \
+                case 1: SKINNY_KERNEL(true, 2, false, 1, false, MSV, true, kv); break;                       \
+                case 2: SKINNY_KERNEL(true, 4, false, 1, false, MSV, true, kv); break;                       \
+                default: SKINNY_KERNEL(true, 6, false, 1, false, MSV, true, kv); break;                      \
+            }                                                                                          \
+        } else {                                                                                       \
+            switch (per_wave) {                                                                        \
+                case 1: SKINNY_KERNEL(true, 2, true, 1, false, MSV, true, kv); break;                        \
+                case 2: SKINNY_KERNEL(true, 4, true, 1, false, MSV, true, kv); break;                        \
+                default: SKINNY_KERNEL(true, 6, true, 1, false, MSV, true, kv); break;                       \
+            }                                                                                          \
+        }                                                                                              \
+    } while (0)
+            switch (merged.n_splits) {
+                case 1: SKINNY_MERGED(1); break;
+                case 2: SKINNY_MERGED(2); break;
+                case 3: SKINNY_MERGED(3); break;
+                default: SKINNY_MERGED(4); break;
+            }
+#undef SKINNY_MERGED
+        } else if (two_tiles) {
+            // (two tiles per chunk slot: half the blocks per chunk)
+            if (per_wave <= 1 || !LN_FUSED) SKINNY_CHUNKS(2, false, 2);
+            else SKINNY_CHUNKS(4, false, 2);
+        } else if (LN_FUSED) {
+            switch (std::min(per_wave, 3)) {
+                case 1: SKINNY_LAUNCH(true, 2, false, 1, true); break;
+                case 2: SKINNY_LAUNCH(true, 4, false, 1, true); break;
+                default: SKINNY_CHUNKS(6, false, 1); break;
             }
         } else if (M <= 8) {
             switch (std::min(per_wave, 4)) {
-                case 1: SKINNY_LAUNCH(true, 2, false, 1); break;
-                case 2: SKINNY_LAUNCH(true, 4, false, 1); break;
-                case 3: SKINNY_LAUNCH(true, 6, false, 1); break;
-                default: SKINNY_LAUNCH(true, 8, false, 1); break;
+                case 1: SKINNY_LAUNCH(true, 2, false, 1, true); break;
+                case 2: SKINNY_LAUNCH(true, 4, false, 1, true); break;
+                case 3: SKINNY_LAUNCH(true, 6, false, 1, true); break;
+                default: SKINNY_CHUNKS(8, false, 1); break;
             }
         } else {
             switch (std::min(per_wave, 3)) {
-                case 1: SKINNY_LAUNCH(true, 2, true, 1); break;
-                case 2: SKINNY_LAUNCH(true, 4, true, 1); break;
-                default: SKINNY_LAUNCH(true, 6, true, 1); break;
+                case 1: SKINNY_LAUNCH(true, 2, true, 1, true); break;
+                case 2: SKINNY_LAUNCH(true, 4, true, 1, true); break;
+                default: SKINNY_CHUNKS(6, true, 1); break;
             }
         }
     } else {
@@ -1208,6 +1228,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         // staging them in LDS is faster than every workgroup normalising them again
         return -2;
     }
+#undef SKINNY_CHUNKS
 #undef SKINNY_LAUNCH
 #undef SKINNY_KERNEL
     return 0;
