@@ -48,6 +48,10 @@ int mllm_ln_gemm_bf16_kv(const float* x, int ldx, const int* rows, const float* 
                          void* k_pages, void* v_pages, int q_cols, int kv_dim, hipStream_t stream);
 int mllm_rms_gemm_bf16(const float* x, int ldx, const int* rows, const float* gamma, float eps, const void* W, int ldw,
                        const float* bias, void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream);
+int mllm_gated_gemm_bf16(const void* A, int lda, const void* gate, const void* up, int ldw, float limit, float alpha, void* C, int ldc,
+                         int M, int N, int K, hipStream_t stream);
+int mllm_rms_gated_gemm_bf16(const float* x, int ldx, const float* gamma, float eps, const void* gate, const void* up, int ldw, float limit,
+                             float alpha, void* C, int ldc, int M, int N, int K, hipStream_t stream);
 
 // attention.hip, attention_decode.hip, attention_prefill.hip
 int mllm_paged_attention_generic(const void* q, int q_stride, int q_col, const void* k_pages,

@@ -193,6 +193,10 @@ void rmsnorm_add(const Tensor2& y, const float* weight, const float* scale, floa
 // The same with a layer norm: x += mult * scale * ((y - mean) / sqrt(var + eps) * gamma + beta) (beta may be null).
 void layernorm_add(const Tensor2& y, const float* gamma, const float* beta, const float* scale, float mult, float eps, const Tensor2& x,
                    bool clear, hipStream_t stream, const Tensor2* copy = nullptr);
+// out = g sigmoid(alpha g) (u + 1), g = min(gate a, limit), u = clamp(up a, -limit, limit), the two products and the activation in
+// one kernel; with `weight`, a is the RMS norm of the fp32 rows. False: no such kernel for these sizes, and nothing was done.
+bool linear_gated(const Tensor2& a, const float* weight, float eps, const Tensor2& gate, const Tensor2& up, float limit, float alpha,
+                  const Tensor2& out, hipStream_t stream);
 // out = g sigmoid(alpha g) (u + 1), g = min(gate, limit), u = clamp(up, -limit, limit)
 void glu_clamped(const Tensor2& gate, const Tensor2& up, float limit, float alpha, const Tensor2& out, hipStream_t stream);
 void fill_zero(const Tensor2& x, hipStream_t stream);          // contiguous fp32, by a kernel

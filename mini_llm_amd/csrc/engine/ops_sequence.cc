@@ -103,6 +103,28 @@ void cast_stream(const Tensor2& x, const Tensor2& out, hipStream_t stream) {
     check(mllm_cast_bf16(static_cast<const float*>(x.data), out.data, static_cast<size_t>(x.rows) * x.cols, stream), "cast_stream");
 }
 
+bool linear_gated(const Tensor2& a, const float* weight, float eps, const Tensor2& gate, const Tensor2& up, float limit, float alpha,
+                  const Tensor2& out, hipStream_t stream) {
+    const int64_t M = a.rows, N = gate.rows, K = a.cols;
+    auto aligned = [](const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15) == 0; };
+    if (gate.dtype != BF16 || up.dtype != BF16 || out.dtype != BF16 || a.dtype != (weight != nullptr ? F32 : BF16)) return false;
+    if (up.rows != N || gate.cols != K || up.cols != K || out.rows != M || out.cols != N) fail("linear_gated: the shapes do not fit");
+    if (up.stride != gate.stride || gate.stride % 8 != 0 || K % 8 != 0 || !aligned(gate.data) || !aligned(up.data)) return false;
+    int rc;
+    if (weight != nullptr) {
+        if (M > tuning().ln_fuse_max_rows || !a.contiguous() || !aligned(weight)) return false;
+        rc = mllm_rms_gated_gemm_bf16(static_cast<const float*>(a.data), i32(a.stride), weight, eps, gate.data, up.data, i32(gate.stride), limit,
+                                      alpha, out.data, i32(out.stride), i32(M), i32(N), i32(K), stream);
+    } else {
+        if (a.stride % 8 != 0 || !aligned(a.data)) return false;
+        rc = mllm_gated_gemm_bf16(a.data, i32(a.stride), gate.data, up.data, i32(gate.stride), limit, alpha, out.data, i32(out.stride), i32(M),
+                                  i32(N), i32(K), stream);
+    }
+    if (rc == -2) return false;       // (the norm's product refuses sizes)
+    check(rc, "linear_gated");
+    return true;
+}
+
 void glu_clamped(const Tensor2& gate, const Tensor2& up, float limit, float alpha, const Tensor2& out, hipStream_t stream) {
     need_act(gate, "glu_clamped gate");
     if (up.dtype != gate.dtype || out.dtype != gate.dtype || up.rows != gate.rows || up.cols != gate.cols || out.rows != gate.rows ||

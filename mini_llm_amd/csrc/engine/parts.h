@@ -243,6 +243,12 @@ public:
     // (kv: a key/value scatter of the linear map, passed through to it)
     virtual void linear(const Tensor2& x, const Linear& lin, const Tensor2& out, int epilogue, const int* rows,
                         const KvScatter* kv, Arena& arena, hipStream_t s) const;
+    // out = gated activation of the two maps of norm(x) (linear_gated), the norm inside. False: no such kernel, nothing was done.
+    virtual bool linear_gated(const Tensor2& x, const Linear& gate, const Linear& up, float limit, float alpha, const Tensor2& out,
+                              hipStream_t s) const {
+        (void)x; (void)gate; (void)up; (void)limit; (void)alpha; (void)out; (void)s;
+        return false;
+    }
     // x += mult * scale * norm(y), row by row (y and x fp32 [rows, size]; scale per column or null); with
     // `clear`, y is zero afterwards; `copy` (optional) receives the new x in bfloat16. For arrangements with a norm
     // behind a sub-layer; a norm without it refuses.
@@ -264,6 +270,10 @@ public:
     explicit NormedInput(const Tensor2& h) : norm_(nullptr), x_(h), h_(h), have_(true) {}     // normalised already
     const Tensor2& tensor(Arena& arena, hipStream_t s);
     void linear(const Linear& lin, const Tensor2& out, int epilogue, const KvScatter* kv, Arena& arena, hipStream_t s);
+    // the norm inside, where it is still to be taken and the kernels allow it (see Norm::linear_gated)
+    bool linear_gated(const Linear& gate, const Linear& up, float limit, float alpha, const Tensor2& out, hipStream_t s) const {
+        return !have_ && norm_->linear_gated(x_, gate, up, limit, alpha, out, s);
+    }
     int64_t rows() const { return x_.rows; }
 
 private:

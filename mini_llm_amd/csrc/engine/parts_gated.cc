@@ -52,6 +52,10 @@ public:
         rms_linear(x, weight_, eps_, lin.weight, lin.bias, out, epilogue, rows, tmp, s);
         arena.release(mark);
     }
+    bool linear_gated(const Tensor2& x, const Linear& gate, const Linear& up, float limit, float alpha, const Tensor2& out,
+                      hipStream_t s) const override {
+        return x.cols == size_ && minillm::linear_gated(x, weight_, eps_, gate.weight, up.weight, limit, alpha, out, s);
+    }
     void add_scaled(const Tensor2& y, const float* scale, float mult, const Tensor2& x, bool clear, hipStream_t s,
                     const Tensor2* copy) const override {
         if (y.cols != size_) fail("rmsnorm: rows of %lld, the norm is %d wide", (long long)y.cols, size_);
@@ -400,18 +404,24 @@ public:
     }
     void forward(NormedInput& h, const StepView& step, const Tensor2& x, Arena& arena, hipStream_t s) const override {
         const int T = step.n_tokens, F = up_.out_features();
-        Tensor2 g = arena.tensor(dtype_, T, F), u = arena.tensor(dtype_, T, F);
-        if (T <= tuning().ln_fuse_max_rows) {
-            // few rows: each product normalises its input itself, and no norm kernel runs
-            h.linear(gate_, g, STORE, nullptr, arena, s);
-            h.linear(up_, u, STORE, nullptr, arena, s);
-        } else {
-            const Tensor2& in = h.tensor(arena, s);
-            gate_(in, g, STORE, nullptr, s);
-            up_(in, u, STORE, nullptr, s);
+        Tensor2 g = arena.tensor(dtype_, T, F);
+        // gate, up and the activation in one kernel where there is one (few rows: the norm inside as well)
+        const bool few = T <= tuning().ln_fuse_max_rows;
+        if (!(few && h.linear_gated(gate_, up_, limit_, alpha_, g, s)) &&
+            !(dtype_ == BF16 && linear_gated(h.tensor(arena, s), nullptr, 0.f, gate_.weight, up_.weight, limit_, alpha_, g, s))) {
+            Tensor2 u = arena.tensor(dtype_, T, F);
+            if (few) {
+                // few rows: each product normalises its input itself, and no norm kernel runs
+                h.linear(gate_, g, STORE, nullptr, arena, s);
+                h.linear(up_, u, STORE, nullptr, arena, s);
+            } else {
+                const Tensor2& in = h.tensor(arena, s);
+                gate_(in, g, STORE, nullptr, s);
+                up_(in, u, STORE, nullptr, s);
+            }
+            glu_clamped(g, u, limit_, alpha_, g, s);        // in place over the gate's rows
         }
         StageTimes::get().mark("fc1", s);
-        glu_clamped(g, u, limit_, alpha_, g, s);            // in place over the gate's rows
         down_(g, x, ADD_RESIDUAL, nullptr, s);
         StageTimes::get().mark("fc2", s);
     }

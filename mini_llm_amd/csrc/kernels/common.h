@@ -17,6 +17,7 @@
 #define EPI_GELU_ERF 2      // out[m,n] = gelu_erf(acc + bias)  (activation dtype)
 #define EPI_ADD_RESIDUAL 3  // res[m,n] += acc + bias           (fp32, in place)
 #define EPI_STORE_F32 4     // out[m,n] = acc + bias            (fp32)
+#define EPI_GATED 8         // out[m,n] = gated(acc of the gate's row n, acc of the up map's row n) (activation dtype)
 #define EPI_THROUGH 7       // x = res[m,n] += norm(acc + bias) (fp32, in place), then a bfloat16 copy of x or of another norm of x
                             // (tanh_norm.h; only the bfloat16 matrix-core kernels, which take the norms beside the mode)
 #define EPI_RELU2 6         // out[m,n] = max(acc + bias, 0)^2  (activation dtype; 5 is an activation of the gated kernels)

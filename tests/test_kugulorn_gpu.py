@@ -238,3 +238,45 @@ def test_scan_portions_of_every_length(tmp_path, heads, vdim, state, groups, con
     runner = _runner(str(tmp_path), "float32", n_pages=ru.peak_tokens(steps) // 4)
     kc.check_against_plain(str(tmp_path), reqs, steps, ru.run_in_process(runner, steps), "float32", cfg["vocab"], f"scan {sizes}")
     assert runner.check() == ""
+
+
+# (rows: one or two row tiles behind the norm, then the smallest and the larger tiles; columns: less than a tile, no whole tile,
+# whole ones; K with and without a remainder of the k tile)
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 32, 33, 64, 65, 130, 513])
+@pytest.mark.parametrize("ff,k", [(16, 64), (40, 72), (200, 768), (2048, 768), (1000, 1608), (200, 2112)])
+def test_gate_and_up_in_one_product(rows, ff, k):
+    """Gate, up map and clamped activation in one kernel, with the RMS norm inside (few rows) and without."""
+    import ctypes
+    import torch
+    from mini_llm_amd.kernels import ops
+    lib = ops.engine_library()
+    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    g = torch.Generator().manual_seed(rows * 7 + ff + k)
+    x = torch.randn(rows, k, generator=g)
+    gamma = 1 + 0.1 * torch.randn(k, generator=g)
+    gate, up = (torch.randn(ff, k, generator=g) * (2.0 / k ** 0.5) for _ in range(2))
+    gate, up = gate.bfloat16(), up.bfloat16()
+    limit, alpha, eps = 3.0, 1.702, 1e-5
+    fused = rows <= 32 and k <= 2048           # (wider norms stay outside)
+    a = (pk.rms_norm(x.double(), gamma.double(), eps) if fused else x).bfloat16()
+    gv, uv = (torch.clamp(a.double() @ gate.double().T, max=limit), torch.clamp(a.double() @ up.double().T, min=-limit, max=limit))
+    want = gv * torch.sigmoid(alpha * gv) * (uv + 1)
+    dev = [t.cuda() for t in (x, gamma, gate, up, a)]
+    out = torch.full((rows + 1, ff + 8), 7.0, dtype=torch.bfloat16, device="cuda")      # (what lies beside the result stays)
+    if fused:
+        fn = lib.mllm_rms_gated_gemm_bf16
+        fn.argtypes = [vp, i, vp, f, vp, vp, i, f, f, vp, i, i, i, i, vp]
+        rc = fn(dev[0].data_ptr(), k, dev[1].data_ptr(), eps, dev[2].data_ptr(), dev[3].data_ptr(), k, limit, alpha, out.data_ptr(), ff + 8, rows, ff, k, None)
+    else:
+        fn = lib.mllm_gated_gemm_bf16
+        fn.argtypes = [vp, i, vp, vp, i, f, f, vp, i, i, i, i, vp]
+        rc = fn(dev[4].data_ptr(), k, dev[2].data_ptr(), dev[3].data_ptr(), k, limit, alpha, out.data_ptr(), ff + 8, rows, ff, k, None)
+    assert rc == 0
+    torch.cuda.synchronize()
+    got = out.cpu().double()
+    assert (got[:, ff:] == 7).all() and (got[rows:] == 7).all()
+    # one rounding to bfloat16, fp32 sums; behind the norm a normalised value may round the other way: 2^-8 |h| |w| of a few of
+    # the K terms, times the slope of the activation (under 1.1 (limit + 1) in g, limit in u)
+    slack = 1e-4 if not fused else 4 * 2.0 ** -8 * 3 * float(gate.abs().max()) * 1.1 * (limit + 1)
+    err = (got[:rows, :ff] - want).abs() - 2.0 ** -8 * want.abs()
+    assert float(err.max()) <= slack, (float(err.max()), slack)
