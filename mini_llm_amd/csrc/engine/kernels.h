@@ -87,6 +87,8 @@ int mllm_rmsnorm_gate_after(const float* x, int ldx, const float* w, const float
 int mllm_softcap(float* x, size_t n, float cap, hipStream_t stream);
 int mllm_norm_add(float* y, const float* w, const float* beta, const float* scale, float mult, float eps, float* x, int n, int D,
                   int clear, int center, void* copy_bf16, hipStream_t stream);
+int mllm_rmsnorm_add_norm(float* y, const float* w, const float* scale, float mult, float eps, float* x, int n, int D, int clear,
+                          const float* next_w, float next_eps, void* out_bf16, hipStream_t stream);
 int mllm_rmsnorm_add_many(const float* y, size_t y_stride, const float* w, size_t w_stride, int n_in, float mult, float eps,
                           float* x, int n, int D, hipStream_t stream);
 int mllm_glu_clamped(const void* gate, int ldg, const void* up, int ldu, void* out, int ldo, int T, int F, float limit,

@@ -96,6 +96,7 @@ public:
                      hipStream_t s) const override {
         run(h, step, cache, x, write, arena, s, STORE_F32);
     }
+    bool sets_result() const override { return true; }
     void forward_through(NormedInput& h, const StepView& step, const CacheView& cache, const StreamAdd& add, bool write, Arena& arena,
                          hipStream_t s) const override {
         run(h, step, cache, add.x, write, arena, s, STORE_F32, &add);

@@ -49,6 +49,15 @@ public:
     }
     void forward(NormedInput& h, const StepView& step, const CacheView& cache, const Tensor2& x, bool write, Arena& arena,
                  hipStream_t s) const override {
+        run(h, step, cache, x, write, arena, s, ADD_RESIDUAL);
+    }
+    void forward_set(NormedInput& h, const StepView& step, const CacheView& cache, const Tensor2& x, bool write, Arena& arena,
+                     hipStream_t s) const override {
+        run(h, step, cache, x, write, arena, s, STORE_F32);
+    }
+    bool sets_result() const override { return true; }
+    void run(NormedInput& h, const StepView& step, const CacheView& cache, const Tensor2& x, bool write, Arena& arena, hipStream_t s,
+             int out_epilogue) const {
         if (!cache.has_state() || cache.state_bytes != slot_floats_ * 4) fail("mamba2 needs a state of %zu floats per request", slot_floats_);
         const int T = step.n_tokens, width = in_.out_features();
         // (rows padded to whole 16 bytes)
@@ -73,7 +82,7 @@ public:
         Tensor2 gated = arena.tensor(dtype_, T, inner_);
         const Tensor2 z(proj.data, F32, T, inner_, proj.stride);
         rmsnorm(y, norm_, eps_, norm_groups_, &z, gated, nullptr, s, parts, static_cast<size_t>(T) * inner_);
-        out_(gated, x, ADD_RESIDUAL, nullptr, s);
+        out_(gated, x, out_epilogue, nullptr, s);
         StageTimes::get().mark("out_proj", s);
     }
     size_t workspace_bytes(int tokens) const override {

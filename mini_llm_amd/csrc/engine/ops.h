@@ -190,6 +190,10 @@ void rms_linear(const Tensor2& x, const float* weight, float eps, const Tensor2&
 // `clear`: y is zero afterwards. `copy` (optional, x's shape): the new x in bfloat16.
 void rmsnorm_add(const Tensor2& y, const float* weight, const float* scale, float mult, float eps, const Tensor2& x,
                  bool clear, hipStream_t stream, const Tensor2* copy = nullptr);
+// The same, and out (bfloat16, x's shape) = the new x behind the RMS norm (next_weight, next_eps). False: no such kernel for these
+// sizes, and nothing was done.
+bool rmsnorm_add_norm(const Tensor2& y, const float* weight, const float* scale, float mult, float eps, const Tensor2& x, bool clear,
+                      const float* next_weight, float next_eps, const Tensor2& out, hipStream_t stream);
 // The same with a layer norm: x += mult * scale * ((y - mean) / sqrt(var + eps) * gamma + beta) (beta may be null).
 void layernorm_add(const Tensor2& y, const float* gamma, const float* beta, const float* scale, float mult, float eps, const Tensor2& x,
                    bool clear, hipStream_t stream, const Tensor2* copy = nullptr);

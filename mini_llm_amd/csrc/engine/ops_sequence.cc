@@ -91,6 +91,20 @@ void rmsnorm_add(const Tensor2& y, const float* weight, const float* scale, floa
     norm_add("rmsnorm_add", y, weight, nullptr, scale, mult, eps, x, clear, false, copy, stream);
 }
 
+bool rmsnorm_add_norm(const Tensor2& y, const float* weight, const float* scale, float mult, float eps, const Tensor2& x, bool clear,
+                      const float* next_weight, float next_eps, const Tensor2& out, hipStream_t stream) {
+    need_f32(y, "rmsnorm_add_norm");
+    need_f32(x, "rmsnorm_add_norm");
+    if (weight == nullptr || next_weight == nullptr) fail("rmsnorm_add_norm: a weight is missing");
+    if (!y.contiguous() || !x.contiguous() || y.rows != x.rows || y.cols != x.cols) fail("rmsnorm_add_norm: x and y must be contiguous float32 of one shape");
+    if (out.dtype != BF16 || !out.contiguous() || out.rows != x.rows || out.cols != x.cols) fail("rmsnorm_add_norm: out must be contiguous bfloat16 of x's shape");
+    const int rc = mllm_rmsnorm_add_norm(static_cast<float*>(y.data), weight, scale, mult, eps, static_cast<float*>(x.data), i32(x.rows), i32(x.cols),
+                                         clear ? 1 : 0, next_weight, next_eps, out.data, stream);
+    if (rc == -2) return false;
+    check(rc, "rmsnorm_add_norm");
+    return true;
+}
+
 void layernorm_add(const Tensor2& y, const float* gamma, const float* beta, const float* scale, float mult, float eps, const Tensor2& x,
                    bool clear, hipStream_t stream, const Tensor2* copy) {
     norm_add("layernorm_add", y, gamma, beta, scale, mult, eps, x, clear, true, copy, stream);

@@ -254,6 +254,15 @@ public:
     // behind a sub-layer; a norm without it refuses.
     virtual void add_scaled(const Tensor2& y, const float* scale, float mult, const Tensor2& x, bool clear,
                             hipStream_t s, const Tensor2* copy = nullptr) const;
+    // The same, and out (of the compute dtype, x's shape) = next(new x), in one kernel. False: no such kernel for the two, and
+    // nothing was done.
+    virtual bool add_scaled_then(const Tensor2& y, const float* scale, float mult, const Tensor2& x, bool clear, const Norm& next,
+                                 const Tensor2& out, hipStream_t s) const {
+        (void)y; (void)scale; (void)mult; (void)x; (void)clear; (void)next; (void)out; (void)s;
+        return false;
+    }
+    // The weight [size] and eps of an RMS norm; null: another kind.
+    virtual const float* rms_weight(float& eps) const { (void)eps; return nullptr; }
     // True: the norm has no statistics (every value of a row on its own) and `n` is it: what makes or reads the row's
     // values can apply it in passing.
     virtual bool pointwise(MllmTanhNorm& n) const { (void)n; return false; }
@@ -294,6 +303,7 @@ public:
         fill_zero(x, s);
         forward(h, step, cache, x, write, arena, s);
     }
+    virtual bool sets_result() const { return false; }       // whether forward_set() costs no more than forward()
     // The same with the output taken into the stream by `add` (a norm without statistics behind the mixer, the next
     // sub-layer's input): a mixer that ends in a product lets the product do it.
     virtual void forward_through(NormedInput& h, const StepView& step, const CacheView& cache, const StreamAdd& add, bool write,
@@ -329,6 +339,7 @@ public:
         fill_zero(x, s);
         forward(h, step, x, arena, s);
     }
+    virtual bool sets_result() const { return false; }       // as for mixers
     // The same with the result taken into the stream by `add`, as for mixers.
     virtual void forward_through(NormedInput& h, const StepView& step, const StreamAdd& add, Arena& arena, hipStream_t s) const {
         forward_set(h, step, add.y, arena, s);

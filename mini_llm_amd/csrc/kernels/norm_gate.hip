@@ -330,10 +330,15 @@ rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, const int* __restrict__
     }
 }
 
-template <int WAVES, bool CENTER>
+// NEXT: `copy` receives the new row behind the RMS norm that stands in front of the next sub-layer (next_w, next_eps) instead of
+// the row itself: the row is in registers, and a norm kernel of its own would read it again. Bound by memory: y and x once, x and
+// the copy written.
+template <int WAVES, bool CENTER, bool NEXT = false>
 __global__ void __launch_bounds__(64 * WAVES)
 rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const float* __restrict__ beta, const float* __restrict__ scale,
-                       float mult, float eps, float* __restrict__ x, int n, int D, int clear, bf16_t* __restrict__ copy) {
+                       float mult, float eps, float* __restrict__ x, int n, int D, int clear, bf16_t* __restrict__ copy,
+                       const float* __restrict__ next_w = nullptr, float next_eps = 0.f) {
+    static_assert(!(CENTER && NEXT), "the next norm stands behind RMS norms");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MLLM_WAVE), lane = threadIdx.x % MLLM_WAVE;
     const int r = blockIdx.x * WAVES + wave;
     if (r >= n) return;
@@ -343,6 +348,7 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const
     const float4* sr = reinterpret_cast<const float4*>(scale ? scale : w);
     const float4* br = reinterpret_cast<const float4*>(CENTER && beta ? beta : w);
     const int nq = D / 4, n_u = (nq + 63) / 64;
+    const float4* next_r = reinterpret_cast<const float4*>(next_w);
     float4 v[8], xx[8], ww[8], sc[8], bb[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u)
@@ -355,6 +361,7 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const
             ww[u] = wr[i];
             sc[u] = sr[i];
             if (CENTER) bb[u] = br[i];
+            if (NEXT) bb[u] = next_r[i];
         }
     if (CENTER) {
         float sum = 0.f;
@@ -371,6 +378,7 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const
     for (int u = 0; u < 8; ++u)
         if (u < n_u && lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
     const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(D) + eps);
+    float next_ss = 0.f;
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
         const int i = lane + 64 * u;
@@ -380,13 +388,29 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const
             if (CENTER && beta) { o.x += bb[u].x; o.y += bb[u].y; o.z += bb[u].z; o.w += bb[u].w; }
             const float4 now = make_float4(xx[u].x + s4.x * o.x, xx[u].y + s4.y * o.y, xx[u].z + s4.z * o.z, xx[u].w + s4.w * o.w);
             xr[i] = now;
-            if (copy) {
+            if (NEXT) {
+                xx[u] = now;
+                next_ss += (now.x * now.x + now.y * now.y) + (now.z * now.z + now.w * now.w);
+            } else if (copy) {
                 uint2 pk;
                 pk.x = pack_bf16x2(now.x, now.y);
                 pk.y = pack_bf16x2(now.z, now.w);
                 *reinterpret_cast<uint2*>(copy + static_cast<size_t>(r) * D + 4 * i) = pk;
             }
             if (clear) yr[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    }
+    if (NEXT) {
+        const float next_inv = 1.0f / sqrtf(wave_sum(next_ss) / static_cast<float>(D) + next_eps);
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+            const int i = lane + 64 * u;
+            if (u < n_u && i < nq) {
+                uint2 pk;
+                pk.x = pack_bf16x2(xx[u].x * next_inv * bb[u].x, xx[u].y * next_inv * bb[u].y);
+                pk.y = pack_bf16x2(xx[u].z * next_inv * bb[u].z, xx[u].w * next_inv * bb[u].w);
+                *reinterpret_cast<uint2*>(copy + static_cast<size_t>(r) * D + 4 * i) = pk;
+            }
         }
     }
 }
@@ -503,6 +527,21 @@ int mllm_norm_add(float* y, const float* w, const float* beta, const float* scal
     else if (vec) NORM_ADD(rmsnorm_add_vec_kernel, 4);
     else NORM_ADD(rmsnorm_add_kernel, 4);
 #undef NORM_ADD
+    MLLM_LAUNCH_CHECK();
+    return 0;
+}
+
+// x += mult * scale * rmsnorm(y) as mllm_norm_add, and out = bf16(x / sqrt(mean(x^2) + next_eps) * next_w) of the new rows.
+// -2: rows that are no multiple of 4 columns, of more than 2,048, or vectors that are not 16-byte aligned.
+int mllm_rmsnorm_add_norm(float* y, const float* w, const float* scale, float mult, float eps, float* x, int n, int D, int clear,
+                          const float* next_w, float next_eps, void* out_bf16, hipStream_t stream) {
+    if (n <= 0 || D <= 0) return 0;
+    bf16_t* out = static_cast<bf16_t*>(out_bf16);
+    if (D % 4 != 0 || D > 2048 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(scale) |
+                                    reinterpret_cast<uintptr_t>(next_w) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(y)) & 15) != 0)
+        return -2;
+    if (n >= 512) rmsnorm_add_vec_kernel<8, false, true><<<(n + 7) / 8, 512, 0, stream>>>(y, w, nullptr, scale, mult, eps, x, n, D, clear, out, next_w, next_eps);
+    else rmsnorm_add_vec_kernel<4, false, true><<<(n + 3) / 4, 256, 0, stream>>>(y, w, nullptr, scale, mult, eps, x, n, D, clear, out, next_w, next_eps);
     MLLM_LAUNCH_CHECK();
     return 0;
 }

@@ -280,3 +280,32 @@ def test_gate_and_up_in_one_product(rows, ff, k):
     slack = 1e-4 if not fused else 4 * 2.0 ** -8 * 3 * float(gate.abs().max()) * 1.1 * (limit + 1)
     err = (got[:rows, :ff] - want).abs() - 2.0 ** -8 * want.abs()
     assert float(err.max()) <= slack, (float(err.max()), slack)
+
+
+@pytest.mark.parametrize("rows,width", [(1, 4), (5, 68), (33, 256), (3, 260), (511, 768), (513, 768), (9, 2048)])
+def test_norm_behind_a_sub_layer_and_the_next_in_front(rows, width):
+    """x += mult scale rmsnorm(y) and the bfloat16 RMS norm of the new x, in one kernel."""
+    import ctypes
+    import torch
+    from mini_llm_amd.kernels import ops
+    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    fn = ops.engine_library().mllm_rmsnorm_add_norm
+    fn.argtypes = [vp, vp, vp, f, f, vp, i, i, i, vp, f, vp, vp]
+    g = torch.Generator().manual_seed(rows + width)
+    x, y = torch.randn(rows, width, generator=g), torch.randn(rows, width, generator=g)
+    w, scale, w2 = (1 + 0.2 * torch.randn(width, generator=g) for _ in range(3))
+    mult, eps, eps2 = 0.7, 1e-5, 1e-6
+    for clear in (0, 1):
+        xd, yd, out = x.cuda(), y.cuda(), torch.full((rows + 1, width), 7.0, dtype=torch.bfloat16, device="cuda")
+        dev = [t.cuda() for t in (w, scale, w2)]
+        assert fn(yd.data_ptr(), dev[0].data_ptr(), dev[1].data_ptr(), mult, eps, xd.data_ptr(), rows, width, clear, dev[2].data_ptr(), eps2, out.data_ptr(), None) == 0
+        torch.cuda.synchronize()
+        new = x.double() + mult * scale.double() * pk.rms_norm(y.double(), w.double(), eps)
+        want = pk.rms_norm(new, w2.double(), eps2)
+        # a row's fp32 sums of `width` squares (relative error under width / 2 * 2^-24 a sum), then one rounding to bfloat16
+        tol = (width / 2 + 16) * 2.0 ** -24
+        assert float((xd.cpu().double() - new).abs().max()) <= tol * (1 + float(new.abs().max()))
+        got = out.cpu().double()
+        assert (got[rows:] == 7).all()
+        assert float(((got[:rows] - want).abs() - 2.0 ** -8 * want.abs()).max()) <= 4 * tol * (1 + float(want.abs().max()))
+        assert torch.equal(yd.cpu(), torch.zeros_like(y) if clear else y)
