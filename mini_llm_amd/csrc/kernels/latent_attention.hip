@@ -401,12 +401,12 @@ latent_expand_kernel(const T* __restrict__ o_lat, int ldo, const T* __restrict__
 // (The widest sizes keep 128 accumulators, 70 query registers and a tile's staging registers a lane: they get the
 // whole register file, one wavefront per SIMD, which is also all their LDS allows.)
 template <int KS, int DT>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, (KS + DT > 30) ? 1 : 2)))
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((KS + DT > 30) ? 1 : 2, (KS + DT > 30) ? 1 : 2)))
 latent_prefill_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ vt_pages,
                       const int* __restrict__ block_tables, int max_blocks, const int* __restrict__ cu_q,
                       const int* __restrict__ ctx_len, int n_seqs, int H, int page_size, float scale_log2e, int window,
                       bf16_t* __restrict__ o_lat, int nsplit, float* __restrict__ partials, int single_tokens) {
-    constexpr int E = 32 * KS, R = 16 * DT, BN = 64, KSTRIDE = E + 8, VSTRIDE = BN + 8, CH = E / 8;
+    constexpr int E = 32 * KS, R = 16 * DT, BN = 64, KSTRIDE = E + 8, VSTRIDE = BN + 8;
     extern __shared__ __attribute__((aligned(16))) char smem[];
     bf16_t* Ks = reinterpret_cast<bf16_t*>(smem);                    // [BN][KSTRIDE]
     bf16_t* Vt = Ks + BN * KSTRIDE;                                  // [R][VSTRIDE]
@@ -465,66 +465,94 @@ latent_prefill_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ 
         kt_end = min(kt_end, kt_begin + per);
     }
     static_assert(DT % 2 == 0, "the transposed latent is staged in whole rounds of the workgroup");
+    // Staging. All loads of a tile are issued first (a fixed number per thread: 64 * E / 8 pieces of page rows
+    // over 256 threads are KS each, R * 8 pieces of the transposed latent DT / 2 each), then written to LDS: a
+    // load inside a loop of unknown length would be waited for before the next one is asked for. AHEAD: a tile's loads are
+    // issued while the tile before it is multiplied, where the registers allow it (not beside a latent of 512).
+    // Page rows, row-major; a key outside [k_lo, p_last] is replaced by one inside (always a held page; its
+    // scores are masked below). The latent transposed: 8 keys of one column a piece, keys outside the range
+    // set to zero.
+    u32x4 kreg[KS], vreg[DT / 2];
+    auto fetch = [&](int j_base) {
+        // (a thread keeps to one row, four threads a row: one page lookup, and all its addresses lie at constant distances;
+        // pieces dealt out along the rows cost the registers that the loads ahead need)
+        const int key = min(max(j_base + tid / 4, k_lo), p_last);
+        const size_t row = (static_cast<size_t>(sm_table[key >> shift]) << shift) + (key & (page_size - 1));
+        const bf16_t* krow = k_pages + row * E + 8 * (tid % 4);
+#pragma unroll
+        for (int u = 0; u < KS; ++u) kreg[u] = *reinterpret_cast<const u32x4*>(krow + 32 * u);
+        // (likewise one place in a page and every 32nd column of the latent)
+        const int key0 = j_base + 8 * (tid % 8);
+        const int pg = min(max(key0 >> shift, pg_lo), pg_hi);
+        const bf16_t* vcol = vt_pages + (static_cast<size_t>(sm_table[pg]) << shift) * R + tid / 8 * page_size + (key0 & (page_size - 1));
+#pragma unroll
+        for (int u = 0; u < DT / 2; ++u, vcol += 32 * page_size) vreg[u] = *reinterpret_cast<const u32x4*>(vcol);
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    constexpr bool AHEAD = KS + DT <= 30;
+    if (AHEAD && kt_begin < kt_end) fetch(kt_begin * BN);
     for (int kt = kt_begin; kt < kt_end; ++kt) {
         const int j_base = kt * BN;
-        // Staging. All loads of a tile are issued first (a fixed number per thread: 64 * E / 8 pieces of page rows
-        // over 256 threads are KS each, R * 8 pieces of the transposed latent DT / 2 each), then written to LDS: a
-        // load inside a loop of unknown length would be waited for before the next one is asked for.
-        // Page rows, row-major; a key outside [k_lo, p_last] is replaced by one inside (always a held page; its
-        // scores are masked below). The latent transposed: 8 keys of one column a piece, keys outside the range
-        // set to zero.
-        u32x4 kreg[KS], vreg[DT / 2];
+        if (!AHEAD) fetch(j_base);
+        lds_barrier();                             // the tile before is used up
 #pragma unroll
-        for (int u = 0; u < KS; ++u) {
-            const int idx = tid + 256 * u, j = idx / CH, c = idx % CH;
-            const int key = min(max(j_base + j, k_lo), p_last);
-            const size_t row = (static_cast<size_t>(sm_table[key >> shift]) << shift) + (key & (page_size - 1));
-            kreg[u] = *reinterpret_cast<const u32x4*>(k_pages + row * E + 8 * c);
+        for (int u = 0; u < KS; ++u) *reinterpret_cast<u32x4*>(Ks + tid / 4 * KSTRIDE + 32 * u + 8 * (tid % 4)) = kreg[u];
+        // (Within a slab of 32 keys the eight keys that one lane group multiplies lie side by side, see the slots below: keys
+        // 4 G .. 4 G + 3 and 16 + 4 G .. of it at 8 G; a fragment is then one read of 16 bytes at a constant distance.)
+        const int part = tid % 8, key0 = j_base + 8 * part, at = part / 4 * 32 + part % 2 * 16 + part % 4 / 2 * 4;
+        uint32_t keep[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int ka = key0 + 2 * e, kb = ka + 1;
+            keep[e] = ((ka >= k_lo && ka <= p_last) ? 0x0000ffffu : 0u) | ((kb >= k_lo && kb <= p_last) ? 0xffff0000u : 0u);
         }
 #pragma unroll
         for (int u = 0; u < DT / 2; ++u) {
-            const int idx = tid + 256 * u, col = idx / (BN / 8), part = idx % (BN / 8);
-            const int key0 = j_base + 8 * part;
-            const int pg = min(max(key0 >> shift, pg_lo), pg_hi);
-            vreg[u] = *reinterpret_cast<const u32x4*>(vt_pages + (static_cast<size_t>(sm_table[pg]) << shift) * R +
-                                                      static_cast<size_t>(col) * page_size + (key0 & (page_size - 1)));
+            bf16_t* dst = Vt + (tid / 8 + 32 * u) * VSTRIDE + at;
+            *reinterpret_cast<uint2*>(dst) = make_uint2(vreg[u][0] & keep[0], vreg[u][1] & keep[1]);
+            *reinterpret_cast<uint2*>(dst + 8) = make_uint2(vreg[u][2] & keep[2], vreg[u][3] & keep[3]);
         }
-        __syncthreads();                           // the tile before is used up
-#pragma unroll
-        for (int u = 0; u < KS; ++u) {
-            const int idx = tid + 256 * u, j = idx / CH, c = idx % CH;
-            *reinterpret_cast<u32x4*>(Ks + j * KSTRIDE + 8 * c) = kreg[u];
-        }
-#pragma unroll
-        for (int u = 0; u < DT / 2; ++u) {
-            const int idx = tid + 256 * u, col = idx / (BN / 8), part = idx % (BN / 8);
-            const int key0 = j_base + 8 * part;
-            u32x4 v = vreg[u];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int ka = key0 + 2 * e, kb = ka + 1;
-                const uint32_t keep = ((ka >= k_lo && ka <= p_last) ? 0x0000ffffu : 0u) | ((kb >= k_lo && kb <= p_last) ? 0xffff0000u : 0u);
-                v[e] &= keep;
-            }
-            *reinterpret_cast<u32x4*>(Vt + col * VSTRIDE + 8 * part) = v;
-        }
-        __syncthreads();
+        lds_barrier();
+        if (AHEAD && kt + 1 < kt_end) fetch(j_base + BN);
         // S^T: s[nt][r] is the score of key j_base + 16 nt + 4 G + r with this lane's query row
+        // The fragments are read from LDS four at a time, one group ahead of the matrix instructions, and the scheduling barriers
+        // keep it so: left alone the compiler reads one, waits for it, multiplies, and the kernel's time was those 68 round
+        // trips a tile (2 x 1,024 tokens, 12 heads, latent 256 + 32: 67.8 us; with the tile's loads ahead alone 65.1, with the
+        // fragments ahead as well 55.4; 8 single tokens at 130 keys 6.8 -> 6.0). The four sums run side by side, as one after the other each would wait for its own instructions.
         float s[4][4];
         float tile_max = -INFINITY;
+        f32x4 acc[4];
+#pragma unroll
+        for (int nt = 0; nt < 4; ++nt) acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        bf16x8 frag[2][4];
+        auto read_keys = [&](int ks, int set) {
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) frag[set][nt] = *reinterpret_cast<const bf16x8*>(Ks + (16 * nt + c16) * KSTRIDE + 32 * ks + 8 * G);
+        };
+        auto read_values = [&](int group, int set) {       // four (slab, dt) pairs, slab by slab
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int slab = (4 * group + i) / DT, dt = (4 * group + i) % DT;
+                frag[set][i] = *reinterpret_cast<const bf16x8*>(Vt + (16 * dt + c16) * VSTRIDE + 32 * slab + 8 * G);
+            }
+        };
+        read_keys(0, 0);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            if (ks + 1 < KS) read_keys(ks + 1, (ks + 1) & 1);
+            else read_values(0, KS & 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int nt = 0; nt < 4; ++nt) acc[nt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag[ks & 1][nt], qf[ks].v, acc[nt], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int nt = 0; nt < 4; ++nt) {
-            f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                const bf16x8 a = *reinterpret_cast<const bf16x8*>(Ks + (16 * nt + c16) * KSTRIDE + 32 * ks + 8 * G);
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, qf[ks].v, acc, 0, 0, 0);
-            }
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
                 const int j = j_base + 16 * nt + 4 * G + r;
                 const bool seen = q_ok && j <= p && (window <= 0 || j > p - window);
-                s[nt][r] = seen ? acc[r] : -INFINITY;
+                s[nt][r] = seen ? acc[nt][r] : -INFINITY;
                 tile_max = fmaxf(tile_max, s[nt][r]);
             }
         }
@@ -548,23 +576,24 @@ latent_prefill_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ 
             for (int r = 0; r < 4; ++r) o[dt][r] *= alpha;
         // O^T += C^T P^T over slabs of 32 keys: k slot i of lane group G stands for key 32 slab + 4 G + i
         // (i < 4) or 32 slab + 16 + 4 G + i - 4 (i >= 4) in both operands
+        Frag8 pf[2];
 #pragma unroll
         for (int slab = 0; slab < 2; ++slab) {
-            Frag8 pf;
-            pf.w[0] = pack_bf16x2(s[2 * slab][0], s[2 * slab][1]);
-            pf.w[1] = pack_bf16x2(s[2 * slab][2], s[2 * slab][3]);
-            pf.w[2] = pack_bf16x2(s[2 * slab + 1][0], s[2 * slab + 1][1]);
-            pf.w[3] = pack_bf16x2(s[2 * slab + 1][2], s[2 * slab + 1][3]);
+            pf[slab].w[0] = pack_bf16x2(s[2 * slab][0], s[2 * slab][1]);
+            pf[slab].w[1] = pack_bf16x2(s[2 * slab][2], s[2 * slab][3]);
+            pf[slab].w[2] = pack_bf16x2(s[2 * slab + 1][0], s[2 * slab + 1][1]);
+            pf[slab].w[3] = pack_bf16x2(s[2 * slab + 1][2], s[2 * slab + 1][3]);
+        }
 #pragma unroll
-            for (int dt = 0; dt < DT; ++dt) {
-                const uint32_t* vrow = reinterpret_cast<const uint32_t*>(Vt + (16 * dt + c16) * VSTRIDE);
-                Frag8 vf;
-                vf.w[0] = vrow[16 * slab + 2 * G];
-                vf.w[1] = vrow[16 * slab + 2 * G + 1];
-                vf.w[2] = vrow[16 * slab + 8 + 2 * G];
-                vf.w[3] = vrow[16 * slab + 8 + 2 * G + 1];
-                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf.v, pf.v, o[dt], 0, 0, 0);
+        for (int group = 0; group < DT / 2; ++group) {
+            if (group + 1 < DT / 2) read_values(group + 1, (KS + group + 1) & 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int slab = (4 * group + i) / DT, dt = (4 * group + i) % DT;
+                o[dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(frag[(KS + group) & 1][i], pf[slab].v, o[dt], 0, 0, 0);
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
     }
     l = rows_sum(l);
