@@ -286,6 +286,13 @@ def test_linear_bf16_few_rows(ops, M, N, K):
         assert err <= (2e-5 + 2e-5 * math.sqrt(K) if f32_out else 4e-2), (epi, err)
 
 
+@pytest.mark.parametrize("M", [1, 8, 9, 16])
+@pytest.mark.parametrize("N,K", [(96, 2304), (96, 2312), (96, 3072), (96, 3080), (96, 3136), (40, 64), (40, 5056), (4104, 768), (4104, 776), (4104, 832)])
+def test_linear_bf16_few_rows_at_the_chunks_borders(ops, M, N, K):
+    """A wavefront's blocks of K that fill one chunk, the next block, and part of one: kernels of one chunk and of several."""
+    test_linear_bf16_few_rows(ops, M, N, K)
+
+
 @pytest.mark.parametrize("M,N,K", [(65, 768, 768), (96, 2304, 768), (100, 1000, 96), (128, 768, 3072), (200, 72, 1600),
                                    (256, 768, 768), (256, 1024, 4096), (250, 40, 6400), (129, 2304, 768), (64, 6400, 1600)])
 def test_linear_bf16_up_to_256_rows(ops, M, N, K):
