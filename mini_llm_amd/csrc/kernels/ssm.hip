@@ -513,6 +513,9 @@ ssm_short_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict
 // four k at a time, and 4 floats more than a multiple of 64 for those read one k at a time (16 neighbouring columns of four rows
 // 4 apart): neither conflicts. A token after the other, as the short kernel does it, was bound by its chain of 64 tokens:
 // 2,048 tokens of 24 heads of 128 x 64 took 85 us for the chunks and 45 to join them; the three kernels take 16.0, 11.7 and 28.0 us.
+// A token's result must not depend on later ones: in the output kernel's second product their weights are 0, and 0 times an
+// infinity is no 0, so the product takes zeros in place of x that are not finite, and a loop that a chunk without any skips
+// adds these where they belong.
 // Needs 16-byte aligned rows and column offsets.
 #define SSM_TILE 64
 #define SSM_NS 32
@@ -653,6 +656,7 @@ ssm_chunk_out_kernel(const float* __restrict__ xbc, int ldx, const float* __rest
     float (*Ms)[16][68] = reinterpret_cast<float (*)[16][68]>(slices);
     __shared__ float dt_s[64];
     __shared__ double cum_s[64];
+    __shared__ int odd_s[4];          // whether a wavefront staged an x that is not finite
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64, col = lane % 16, quad = lane / 16;
     const int h = blockIdx.y, p0 = blockIdx.x * 64;
     const ChunkOf co = chunk_of(blockIdx.z, cu_q, n_seqs, SSM_TILE, true);
@@ -697,11 +701,23 @@ ssm_chunk_out_kernel(const float* __restrict__ xbc, int ldx, const float* __rest
             *reinterpret_cast<float4*>(&Ps[e / 16][4 * (e % 16)]) = e / 16 < nn && e % 16 < pq ? sq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
         }
         if (n0 == 0) {
+            bool odd = false;
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int e = tid + 256 * u;
-                *reinterpret_cast<float4*>(&Xs[e / 16][4 * (e % 16)]) = e / 16 < nt && e % 16 < pq ? xq[u] : make_float4(0.f, 0.f, 0.f, 0.f);
+                const bool real = e / 16 < nt && e % 16 < pq;
+                const float raw[4] = {xq[u].x, xq[u].y, xq[u].z, xq[u].w};
+                float x[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const bool finite = __builtin_isfinite(raw[i]);
+                    odd = odd || (real && !finite);
+                    x[i] = real && finite ? raw[i] : 0.f;
+                }
+                *reinterpret_cast<float4*>(&Xs[e / 16][4 * (e % 16)]) = make_float4(x[0], x[1], x[2], x[3]);
             }
+            const bool any_odd = __any(odd);
+            if (lane == 0) odd_s[wave] = any_odd ? 1 : 0;
         }
         fetch(n0 + SSM_NS < N ? n0 + SSM_NS : n0);      // (past the last slice: it again, unused; under a condition it would be waited for here)
         __syncthreads();
@@ -764,6 +780,21 @@ ssm_chunk_out_kernel(const float* __restrict__ xbc, int ldx, const float* __rest
             for (int j = 0; j < 4; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(m4[e], x4[e][j], acc[j], 0, 0, 0);
     }
     const float skip = Dskip[h];
+    if (odd_s[0] + odd_s[1] + odd_s[2] + odd_s[3] > 0) {          // infinities and NaN: to their own token and those behind it
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float* x_col = xbc + static_cast<size_t>(t0) * ldx + h * P + min(p0 + 16 * j + col, P - 1);
+            for (int s = 0; s < nt; ++s) {
+                const float x = x_col[static_cast<size_t>(s) * ldx];
+                if (__builtin_isfinite(x)) continue;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int t = 16 * wave + 4 * quad + r;
+                    if (s <= t) acc[j][r] += Ms[wave][4 * quad + r][s] * x + (s == t ? skip * x : 0.f);
+                }
+            }
+        }
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll

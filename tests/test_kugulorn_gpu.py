@@ -309,3 +309,71 @@ def test_norm_behind_a_sub_layer_and_the_next_in_front(rows, width):
         assert (got[rows:] == 7).all()
         assert float(((got[:rows] - want).abs() - 2.0 ** -8 * want.abs()).max()) <= 4 * tol * (1 + float(want.abs().max()))
         assert torch.equal(yd.cpu(), torch.zeros_like(y) if clear else y)
+
+
+def _scan_inputs(sizes, heads=2, vdim=68, state=36, seed=0):
+    """Inputs of the scan alone: x [T, H, P], B and C [T, 1, N], raw step sizes [T, H], and the heads' dt_bias, A_log and D."""
+    import torch
+    g = torch.Generator().manual_seed(seed)
+    T = sum(sizes)
+    made = [torch.randn(T, heads, vdim, generator=g), torch.randn(T, 1, state, generator=g), torch.randn(T, 1, state, generator=g),
+            torch.randn(T, heads, generator=g) - 2, 0.1 * torch.randn(heads, generator=g), 0.3 * torch.randn(heads, generator=g), torch.randn(heads, generator=g)]
+    return dict(zip(("x", "B", "C", "raw_dt", "dt_bias", "A_log", "D"), made))
+
+
+def _scan(sizes, given, workspace_floats_off=0):
+    """The scan's kernels alone over portions of these sizes, states that start at 0: (y [T, H, P], states [sequences, H, N, P])."""
+    import ctypes
+    import torch
+    from mini_llm_amd.kernels import ops
+    lib = ops.engine_library()
+    vp, i, sz = ctypes.c_void_p, ctypes.c_int, ctypes.c_size_t
+    fn, need = lib.mllm_ssm_scan, lib.mllm_ssm_scan_workspace_floats
+    need.argtypes, need.restype = [i] * 5, sz
+    fn.argtypes = [vp, i, vp, i, vp, vp, vp, vp, vp, vp, sz, sz, vp, i, sz, i, i, i, i, i, i, i, i, vp, vp]
+    T, H, P = given["x"].shape
+    N, b = given["B"].shape[-1], len(sizes)
+    xbc = torch.cat([given["x"].reshape(T, -1), given["B"][:, 0], given["C"][:, 0]], 1).cuda()
+    dev = [given[k].cuda() for k in ("raw_dt", "dt_bias", "A_log", "D")]
+    cu_q = torch.tensor(np.cumsum([0] + list(sizes)), dtype=torch.int32, device="cuda")
+    slots = torch.arange(b, dtype=torch.int32, device="cuda")
+    state = torch.zeros(b, H, N, P, device="cuda")
+    y = torch.full((T, H, P), 7.0, device="cuda")
+    ws = torch.full((need(T, b, H, P, N) + workspace_floats_off,), float("nan"), device="cuda")
+    rc = fn(xbc.data_ptr(), xbc.stride(0), dev[0].data_ptr(), H, *(d.data_ptr() for d in dev[1:]), cu_q.data_ptr(), slots.data_ptr(), state.data_ptr(),
+            H * N * P, 0, y.data_ptr(), H * P, T * H * P, T, b, max(sizes), H, P, N, 1, 1, ws.data_ptr() + 4 * workspace_floats_off, None)
+    assert rc == 0
+    torch.cuda.synchronize()
+    return y.cpu(), state.cpu()
+
+
+def _scan_plain(sizes, given, magnitudes=False):
+    """The same token by token in float64; `magnitudes`: of the terms' absolute values."""
+    import torch
+    d = {k: v.double() for k, v in given.items()}
+    dt = pk.softplus(d["raw_dt"] + d["dt_bias"])
+    ys, states, at = [], [], 0
+    for n in sizes:
+        part = [d[k][at:at + n].abs() if magnitudes else d[k][at:at + n] for k in ("x", "B", "C")]
+        y, s = pk.ssm_scan(*part, dt[at:at + n], d["A_log"], d["D"].abs() if magnitudes else d["D"], 1)
+        ys.append(y)
+        states.append(s)
+        at += n
+    return torch.cat(ys), torch.stack(states)
+
+
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")])
+@pytest.mark.parametrize("at", [0, 37, 63, 100, 199])
+def test_scan_keeps_tokens_before_a_non_finite_value(value, at):
+    """An infinite or NaN x (first, last and other tokens of a chunk) reaches its own token and those behind it in its column, as
+    token by token; every other value keeps its bits."""
+    import torch
+    sizes = (200, 70, 5)
+    given = _scan_inputs(sizes, seed=at)
+    before, _ = _scan(sizes, given)
+    given["x"][at, 1, 66] = value
+    got, _ = _scan(sizes, given)
+    want, _ = _scan_plain(sizes, given)
+    assert torch.equal(torch.isfinite(got), torch.isfinite(want)) and not torch.isfinite(got[at:200, 1, 66]).any()
+    kept = torch.isfinite(want)
+    assert torch.equal(got[kept], before[kept])
