@@ -527,7 +527,10 @@ typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ void chunk_decays(const float* raw_dt, int ldd, int t0, int nt, int h, const float* dt_bias, const float* A_log, int lane,
                                              float* dt_s, double* cum_s) {
     const float dt = softplus_precise(raw_dt[static_cast<size_t>(t0 + min(lane, nt - 1)) * ldd + h] + dt_bias[h]);
+    // (a decay of exp(-1000) is 0 in fp32 like any smaller one; without the bound an infinite rate or step size leaves differences
+    // of infinities, and a sum that holds a very large one has lost the small ones behind it. NaN stays.)
     double run = lane < nt ? -static_cast<double>(expf(A_log[h])) * dt : 0.0;
+    if (run < -1000.0) run = -1000.0;
 #pragma unroll
     for (int off = 1; off < 64; off *= 2) {
         const double up = __shfl_up(run, off, 64);

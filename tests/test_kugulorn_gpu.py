@@ -377,3 +377,19 @@ def test_scan_keeps_tokens_before_a_non_finite_value(value, at):
     assert torch.equal(torch.isfinite(got), torch.isfinite(want)) and not torch.isfinite(got[at:200, 1, 66]).any()
     kept = torch.isfinite(want)
     assert torch.equal(got[kept], before[kept])
+
+
+@pytest.mark.parametrize("log_rate,raw", [(0.3, 0.0), (100.0, 0.0), (20.0, 3.0), (1.0, 1e30), (3.0, 40.0), (-30.0, -2.0)])
+def test_scan_with_decays_of_any_size(log_rate, raw):
+    """Rates and step sizes whose decays underflow (infinite in 32 bits for the first head's log rate of 100), and faint ones, beside
+    a head of ordinary ones: every token forgets what it has to and nothing else. A sum's error is at most a rounding per term of its
+    magnitudes' sum (the state's rows, the tokens of a chunk) and one per unit of the decays' logarithms that still count."""
+    import torch
+    sizes = (200, 64, 130, 3)
+    given = _scan_inputs(sizes, seed=3)
+    given["A_log"][0] = log_rate
+    given["raw_dt"][20:180:7, 0] = raw
+    y, state = _scan(sizes, given)
+    for got, want, size in zip((y, state), _scan_plain(sizes, given), _scan_plain(sizes, given, magnitudes=True)):
+        assert torch.isfinite(got).all()
+        assert ((got.double() - want).abs() <= 2.0 ** -24 * (given["B"].shape[-1] + 64 + 200) * size).all()
