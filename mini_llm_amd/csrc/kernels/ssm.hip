@@ -574,10 +574,10 @@ ssm_chunk_state_kernel(const float* __restrict__ xbc, int ldx, const float* __re
     __syncthreads();
     if (tid == 0) cumlog[static_cast<size_t>(t0 + nt - 1) * H + h] = static_cast<float>(cum_s[63]);
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {          // (tokens past the chunk's end have dt 0)
+    for (int u = 0; u < 4; ++u) {          // (an infinity whose weight has underflowed stays one value that is not finite)
         const int e = tid + 256 * u, s = e / 16;
-        const float w = s < nt && e % 16 < pq ? expf(static_cast<float>(cum_s[63] - cum_s[s])) * dt_s[s] : 0.f;
-        *reinterpret_cast<float4*>(&Xs[s][4 * (e % 16)]) = w != 0.f ? make_float4(w * xq[u].x, w * xq[u].y, w * xq[u].z, w * xq[u].w) : make_float4(0.f, 0.f, 0.f, 0.f);
+        const float w = expf(static_cast<float>(cum_s[63] - cum_s[s])) * dt_s[s];
+        *reinterpret_cast<float4*>(&Xs[s][4 * (e % 16)]) = s < nt && e % 16 < pq ? make_float4(w * xq[u].x, w * xq[u].y, w * xq[u].z, w * xq[u].w) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
     float* out = chunk_state + (static_cast<size_t>(co.first_chunk + co.k) * H + h) * N * P;
     for (int n0 = 0; n0 < N; n0 += SSM_NS) {

@@ -379,6 +379,20 @@ def test_scan_keeps_tokens_before_a_non_finite_value(value, at):
     assert torch.equal(got[kept], before[kept])
 
 
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_scan_keeps_a_non_finite_value_in_the_state(value):
+    """Decays of about 1e-6 a token: at its chunk's end the token's weight has underflowed, but an infinite or NaN state stays one."""
+    import torch
+    sizes = (200, 70)
+    given = _scan_inputs(sizes, seed=8)
+    given["A_log"][:], given["raw_dt"][:] = 1.0, 5.0
+    given["x"][70, 1, 3] = value
+    y, state = _scan(sizes, given)
+    for got, want in zip((y, state), _scan_plain(sizes, given)):
+        assert torch.equal(torch.isfinite(got), torch.isfinite(want))
+    assert not torch.isfinite(y[70:200, 1, 3]).any() and not torch.isfinite(state[0, 1, :, 3]).any()
+
+
 @pytest.mark.parametrize("log_rate,raw", [(0.3, 0.0), (100.0, 0.0), (20.0, 3.0), (1.0, 1e30), (3.0, 40.0), (-30.0, -2.0)])
 def test_scan_with_decays_of_any_size(log_rate, raw):
     """Rates and step sizes whose decays underflow (infinite in 32 bits for the first head's log rate of 100), and faint ones, beside
