@@ -1045,7 +1045,7 @@ int mllm_stream_conv_single(float* x, int ldx, const float* y, int ldy, const fl
 static size_t chunk_states(int T) { return 2 * static_cast<size_t>(T) / SSM_CHUNK + 1; }
 size_t mllm_ssm_scan_workspace_floats(int T, int B, int H, int P, int N) {
     (void)B;
-    return chunk_states(T) * H * P * N + static_cast<size_t>(T) * H;
+    return chunk_states(T) * H * P * N + static_cast<size_t>(T) * H + 3;      // (3: the states start at a 16-byte border inside)
 }
 // Whether the kernels that read 16 bytes at a time take these rows: the short one and the ones in matrix form.
 static bool ssm_by_quads(const float* xbc, int ldx, int P, int N) {
@@ -1056,7 +1056,7 @@ int mllm_ssm_scan_parts(const float* xbc, int ldx, int P, int N) { return ssm_by
 
 // The scan over every sequence's portion (see the kernels). `workspace` (mllm_ssm_scan_workspace_floats floats)
 // is needed when a portion is longer than one chunk (max_q_len > 64). -1: H is no multiple of G, or the
-// workspace is missing or not 16-byte aligned.
+// workspace is missing.
 int mllm_ssm_scan(const float* xbc, int ldx, const float* raw_dt, int ldd, const float* dt_bias, const float* A_log,
                   const float* Dskip, const int* cu_q, const int* state_slots, float* state, size_t slot_floats,
                   size_t scan_offset, float* y, int ldy, size_t part_stride, int T, int B, int max_q_len, int H, int P, int N,
@@ -1066,11 +1066,10 @@ int mllm_ssm_scan(const float* xbc, int ldx, const float* raw_dt, int ldd, const
     const bool chunked = max_q_len > SSM_CHUNK;
     if (chunked && workspace == nullptr) return -1;
     const int n_chunks = chunked ? T / SSM_CHUNK + B : B;
-    float* chunk_state = workspace;
-    float* cumlog = workspace ? workspace + chunk_states(T) * H * P * N : nullptr;
+    float* chunk_state = reinterpret_cast<float*>((reinterpret_cast<uintptr_t>(workspace) + 15) & ~static_cast<uintptr_t>(15));
+    float* cumlog = workspace ? chunk_state + chunk_states(T) * H * P * N : nullptr;
     const int n_slices = (N + SSM_SLICE - 1) / SSM_SLICE;
     if (ssm_by_quads(xbc, ldx, P, N)) {
-        if (chunked && (reinterpret_cast<uintptr_t>(workspace) & 15)) return -1;
         const int p_tiles = (P + 63) / 64, waves = std::min(n_slices, 4);
 #define SSM_SHORT(CH)                                                                                                  \
     do {                                                                                                               \

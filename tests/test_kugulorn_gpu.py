@@ -407,3 +407,13 @@ def test_scan_with_decays_of_any_size(log_rate, raw):
     for got, want, size in zip((y, state), _scan_plain(sizes, given), _scan_plain(sizes, given, magnitudes=True)):
         assert torch.isfinite(got).all()
         assert ((got.double() - want).abs() <= 2.0 ** -24 * (given["B"].shape[-1] + 64 + 200) * size).all()
+
+
+def test_scan_takes_a_workspace_at_any_float():
+    """A workspace that starts off a 16-byte border (and is of the size asked for) is as good as any other."""
+    import torch
+    sizes = (200, 70)
+    given = _scan_inputs(sizes, seed=5)
+    first = _scan(sizes, given)
+    for off in (1, 2, 3):
+        assert all(torch.equal(a, b) for a, b in zip(first, _scan(sizes, given, off)))
