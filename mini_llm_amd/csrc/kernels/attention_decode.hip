@@ -390,14 +390,15 @@ __global__ void __launch_bounds__(MERGE_THREADS)
 merge_splits_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, int nsplit, int head_dim, int n_heads, T* __restrict__ out, int out_stride) {
     __shared__ __attribute__((aligned(16))) float4 o_s[MERGE_THREADS];
     __shared__ float2 ml_s[MERGE_THREADS];
-    const int pair = blockIdx.x, quads = head_dim / 4, groups = MERGE_THREADS / quads;
+    // (blockIdx.y: 4 MERGE_THREADS elements of heads wider than that)
+    const int pair = blockIdx.x, quad0 = blockIdx.y * MERGE_THREADS, quads = min(head_dim / 4 - quad0, MERGE_THREADS), groups = MERGE_THREADS / quads;
     const int quad = threadIdx.x % quads, group = threadIdx.x / quads;
     float m = -1.0e30f, l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
     if (group < groups) {
         for (int s = group; s < nsplit; s += groups) {
             const size_t slot = static_cast<size_t>(pair) * nsplit + s;
             const float2 ml = *reinterpret_cast<const float2*>(ws_ml + slot * 2);
-            const float4 v = *reinterpret_cast<const float4*>(ws_o + slot * head_dim + 4 * quad);
+            const float4 v = *reinterpret_cast<const float4*>(ws_o + slot * head_dim + 4 * (quad0 + quad));
             const float o2[4] = {v.x, v.y, v.z, v.w};
             merge_state<T, 4>(m, l, o, ml.x, ml.y, o2);
         }
@@ -413,7 +414,7 @@ merge_splits_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws
         merge_state<T, 4>(m, l, o, ml.x, ml.y, o2);
     }
     const float inv = 1.0f / l;
-    T* dst = out + static_cast<size_t>(pair / n_heads) * out_stride + (pair % n_heads) * head_dim + 4 * quad;
+    T* dst = out + static_cast<size_t>(pair / n_heads) * out_stride + (pair % n_heads) * head_dim + 4 * (quad0 + quad);
 #pragma unroll
     for (int k = 0; k < 4; ++k) dst[k] = from_float<T>(o[k] * inv);
 }
@@ -424,13 +425,14 @@ extern "C" {
 int mllm_merge_attention_splits(const float* ws, int n_q, int n_heads, int head_dim, int nsplit, void* out,
                                 int out_stride, int dtype, hipStream_t stream) {
     if (n_q <= 0) return 0;
-    if (head_dim % 4 != 0 || head_dim > 4 * MERGE_THREADS || nsplit < 1) return -1;
+    if (head_dim % 4 != 0 || nsplit < 1) return -1;
+    const dim3 grid(n_q * n_heads, (head_dim / 4 + MERGE_THREADS - 1) / MERGE_THREADS);
     const float* ws_o = ws;
     const float* ws_ml = ws + static_cast<size_t>(n_q) * n_heads * nsplit * head_dim;
     if (dtype == MLLM_F32)
-        merge_splits_kernel<float><<<n_q * n_heads, MERGE_THREADS, 0, stream>>>(ws_o, ws_ml, nsplit, head_dim, n_heads, static_cast<float*>(out), out_stride);
+        merge_splits_kernel<float><<<grid, MERGE_THREADS, 0, stream>>>(ws_o, ws_ml, nsplit, head_dim, n_heads, static_cast<float*>(out), out_stride);
     else
-        merge_splits_kernel<bf16_t><<<n_q * n_heads, MERGE_THREADS, 0, stream>>>(ws_o, ws_ml, nsplit, head_dim, n_heads, static_cast<bf16_t*>(out), out_stride);
+        merge_splits_kernel<bf16_t><<<grid, MERGE_THREADS, 0, stream>>>(ws_o, ws_ml, nsplit, head_dim, n_heads, static_cast<bf16_t*>(out), out_stride);
     MLLM_LAUNCH_CHECK();
     return 0;
 }

@@ -928,6 +928,44 @@ def test_sample_inverse_cdf(ops, V):
         assert lo - 1e-5 <= float(u[i]) <= hi + 1e-5, (i, got[i], lo, float(u[i]), hi)
 
 
+def _merge_splits(ops, ws, tokens, heads, head_dim, nsplit, out):
+    import ctypes
+    vp, i = ctypes.c_void_p, ctypes.c_int
+    fn = ops.engine_library().mllm_merge_attention_splits
+    fn.argtypes = [vp, i, i, i, i, vp, i, i, vp]
+    return fn(ws.data_ptr(), tokens, heads, head_dim, nsplit, out.data_ptr(), out.stride(0), 0 if out.dtype == torch.float32 else 1,
+              ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+
+
+# (256 threads are 1,024 / head_dim groups, each for every so-manieth split: one split, fewer than groups, as many, one more, several
+# rounds; head sizes that leave threads over, one group, and more elements than threads)
+@pytest.mark.parametrize("head_dim,nsplit", [(64, 1), (64, 15), (64, 16), (64, 17), (64, 64), (40, 25), (40, 26), (40, 60), (128, 9), (512, 2), (512, 9),
+                                             (516, 5), (1024, 3), (4, 64), (1100, 3), (2048, 2)])
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_merge_of_splits(ops, head_dim, nsplit, dtype):
+    """The states of splits (maximum base 2, sum, unnormalised output) joined, empty ones (maximum -1e30, sum 0) among them. A state
+    passes at most two exponentials and two products a merge, in 32 bits (with arguments of at most 40 in all: as many roundings)."""
+    tokens, heads, pad = 3, 2, 8
+    g = torch.Generator().manual_seed(head_dim + nsplit)
+    o = torch.randn(tokens, heads, nsplit, head_dim, generator=g)
+    m, l = 8 * torch.rand(tokens, heads, nsplit, generator=g), 1 + 30 * torch.rand(tokens, heads, nsplit, generator=g)
+    if nsplit > 1:
+        for t in range(tokens):
+            empty = [t % nsplit] if nsplit == 2 else [t % nsplit, nsplit - 1]
+            m[t, 1, empty], l[t, 1, empty], o[t, 1, empty] = -1.0e30, 0.0, 0.0
+    ws = torch.cat([o.reshape(-1), torch.stack([m, l], -1).reshape(-1)]).to(DEV)
+    out = torch.full((tokens, heads * head_dim + pad), 7.0, dtype=dtype, device=DEV)
+    assert _merge_splits(ops, ws, tokens, heads, head_dim, nsplit, out) == 0
+    w = torch.exp2(m.double() - m.double().amax(-1, keepdim=True))
+    total = (w * l.double()).sum(-1, keepdim=True)
+    want = ((w[..., None] * o.double()).sum(2) / total).reshape(tokens, -1)
+    size = ((w[..., None] * o.double().abs()).sum(2) / total).reshape(tokens, -1)
+    got = out.cpu().double()
+    limit = 2 * 2.0 ** -24 * (40 + 8 * nsplit) * size + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)
+    assert ((got[:, :heads * head_dim] - want).abs() <= limit).all()
+    assert (got[:, heads * head_dim:] == 7).all()
+
+
 def test_sample_edge_rows(ops):
     """All mass on one entry, a flat row, u at both ends, masses that underflow to zero."""
     V = 5000
