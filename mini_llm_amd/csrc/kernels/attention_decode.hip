@@ -425,7 +425,7 @@ extern "C" {
 int mllm_merge_attention_splits(const float* ws, int n_q, int n_heads, int head_dim, int nsplit, void* out,
                                 int out_stride, int dtype, hipStream_t stream) {
     if (n_q <= 0) return 0;
-    if (head_dim % 4 != 0 || nsplit < 1) return -1;
+    if (head_dim % 4 != 0 || head_dim < 4 || n_heads < 1 || nsplit < 1) return -1;
     const dim3 grid(n_q * n_heads, (head_dim / 4 + MERGE_THREADS - 1) / MERGE_THREADS);
     const float* ws_o = ws;
     const float* ws_ml = ws + static_cast<size_t>(n_q) * n_heads * nsplit * head_dim;

@@ -966,6 +966,13 @@ def test_merge_of_splits(ops, head_dim, nsplit, dtype):
     assert (got[:, heads * head_dim:] == 7).all()
 
 
+def test_merge_of_splits_refuses(ops):
+    ws, out = torch.zeros(64, device=DEV), torch.zeros(1, 64, device=DEV)
+    for tokens, heads, head_dim, nsplit in ((1, 1, 0, 1), (1, 1, -4, 1), (1, 1, 6, 1), (1, 0, 8, 1), (1, -1, 8, 1), (1, 1, 8, 0)):
+        assert _merge_splits(ops, ws, tokens, heads, head_dim, nsplit, out) == -1
+    assert _merge_splits(ops, ws, 0, 1, 8, 1, out) == 0
+
+
 def test_sample_edge_rows(ops):
     """All mass on one entry, a flat row, u at both ends, masses that underflow to zero."""
     V = 5000
