@@ -173,8 +173,10 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
 // columns of four matrix instructions (lane group l / 16 takes columns 4 (l / 16) to + 3 of 16, the same for both operands);
 // rows are an odd number of 16-byte pieces apart (16 lanes on 16 different groups of banks). The weights are the
 // instruction's first operand, so that a lane ends up with four neighbouring columns of one row. Sixteen columns are summed on
-// their own before they join an output's sum: the error against 64 bits is 1.2e-7 at K = 768 and 2.5e-7 at 3,072 (8.4e-8 and
-// 1.4e-7 with four groups and sums), where one chain of FMAs had 4.0e-7 and 9.4e-7 and the kernel for few rows below 8.0e-8 and 1.4e-7.
+// their own before they join an output's sum, with tiles of 16 x 16 a wavefront 32 columns in eight sums: the error against 64 bits
+// (2-norm over 2-norm, normal values) is 1.5e-7 at K = 768 and 2.0e-7 at 3,072, with eight sums and four groups 8.8e-8 and 1.2e-7,
+// where one chain of FMAs had 5.0e-7 and 9.9e-7 and the kernel for few rows has 9.3e-8 and 1.4e-7. (Four sums of 16 columns, 9.6e-8
+// and 1.5e-7, were a little less exact than that kernel, which took up to 64 rows before; up to K = 256 the two are alike.)
 // Bound by the matrix cores where the tiles fill the chip evenly, else by the units that take one tile more or by that chain.
 // 2,048 x 3,072 x 768: 91 us (106 TFLOP/s of the 155 a loop of these instructions reaches; a kernel of vector FMAs on 64 x 64
 // tiles took 134); 2,048 x 768 x 3,072: 99 (209); 570 x 768 x 3,072: 40 (197); 64 x 768 x 3,072: 24 (the kernel for few
@@ -226,10 +228,14 @@ gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restr
         for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
     const int wm = wave / 2, wn = wave % 2, row16 = lane % 16, quad = lane / 16;
     const int a_off = (wm * TM * 16 + row16) * STRIDE + F32T_BK * kg + 4 * quad, w_off = (BM + wn * TN * 16 + row16) * STRIDE + F32T_BK * kg + 4 * quad;
+    // TM x TN of 1: the 32 columns in eight sums of four that are added pairwise before they join; otherwise 16 columns in one sum each
     auto multiply = [&](int buf) {
+        constexpr int KS = F32T_BK / 16;
+        f32x4v sum[SUMS == 4 ? KS : 1][SUMS][TM][TN];
 #pragma unroll
-        for (int ks = 0; ks < F32T_BK / 16; ++ks) {
-            f32x4v fa[TM], fw[TN], sum[SUMS][TM][TN];
+        for (int ks = 0; ks < KS; ++ks) {
+            const int at = SUMS == 4 ? ks : 0;
+            f32x4v fa[TM], fw[TN];
 #pragma unroll
             for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const f32x4v*>(&tile_s[buf][a_off + i * 16 * STRIDE + ks * 16]);
 #pragma unroll
@@ -240,16 +246,20 @@ gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restr
                 for (int i = 0; i < TM; ++i)
 #pragma unroll
                     for (int j = 0; j < TN; ++j) {
-                        f32x4v& to = sum[e % SUMS][i][j];
+                        f32x4v& to = sum[at][e % SUMS][i][j];
                         to = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][e], fa[i][e], e < SUMS ? f32x4v{0.f, 0.f, 0.f, 0.f} : to, 0, 0, 0);
                     }
+            if constexpr (SUMS == 1) {
 #pragma unroll
-            for (int i = 0; i < TM; ++i)
+                for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) {
-                    if constexpr (SUMS == 4) acc[i][j] += (sum[0][i][j] + sum[1][i][j]) + (sum[2][i][j] + sum[3][i][j]);
-                    else acc[i][j] += sum[0][i][j];
-                }
+                    for (int j = 0; j < TN; ++j) acc[i][j] += sum[0][0][i][j];
+            }
+        }
+        if constexpr (SUMS == 4) {
+            static_assert(KS == 2, "two times four sums");
+            auto four = [&](int ks) { return (sum[ks][0][0][0] + sum[ks][1][0][0]) + (sum[ks][2][0][0] + sum[ks][3][0][0]); };
+            acc[0][0] += four(0) + four(1);
         }
     };
     const int nk = (K + BK - 1) / BK;
