@@ -441,6 +441,19 @@ def test_linear_fp32_tiles(ops, M, N, K, pad, epi):
     assert not torch.isfinite(out[M // 2, :N]).any() or epi == "gelu_tanh"
 
 
+@pytest.mark.parametrize("K", [768, 1600, 3072])
+def test_linear_fp32_is_as_exact_on_tiles_as_for_few_rows(ops, K):
+    """64 rows run on tiles, 16 at a time on the kernel for few rows: the former's error against 64 bits is no larger."""
+    g = torch.Generator().manual_seed(K)
+    a, w = _rand((64, K), torch.float32, g).to(DEV), _rand((768, K), torch.float32, g).to(DEV)
+    want, tiles, rows = a.double() @ w.double().T, torch.empty(64, 768, device=DEV), torch.empty(64, 768, device=DEV)
+    ops.linear(a, w, None, tiles, "store")
+    for m in range(0, 64, 16):
+        ops.linear(a[m:m + 16], w, None, rows[m:m + 16], "store")
+    assert not torch.equal(tiles, rows)
+    assert (tiles.double() - want).norm() <= (rows.double() - want).norm()
+
+
 @pytest.mark.parametrize("M, N, K", [(4, 8, 36), (70, 33, 44), (9, 5, 7)])
 def test_linear_bf16_takes_any_k_through_the_plain_kernel(ops, M, N, K):
     """A K that is no multiple of 8 (the matrix-core kernels read 16 bytes at a time) runs on the plain kernel."""
