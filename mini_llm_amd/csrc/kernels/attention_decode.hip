@@ -382,36 +382,60 @@ static int launch_decode(int lpk, dim3 grid, int waves, hipStream_t stream, cons
 
 // Merges the splits' states that `partial_out` left in the workspace into the attention output, for readers of the output
 // that do not merge while they load. One workgroup per (token, head): a thread takes 4 elements of every MERGE_THREADS /
-// (head_dim / 4)-th split, whose state it asks for at once, and the threads' states meet in LDS. (One thread per 4 elements
-// of all splits, in few workgroups, walked the splits one load after the other: 7.2 us for 12 heads of 64 in 15 splits, 3.0 us now.)
+// (head_dim / 4)-th split, whose states it asks for at once, and the threads' sums meet in LDS. Every split has one weight, against
+// the maximum of all, and a lone state gets it where the sums are added: so many roundings as in one sum over all splits, or fewer.
+// (One thread per 4 elements of all splits, in few workgroups, walked the splits one load after the other: 7.2 us for 12 heads of
+// 64 in 15 splits, 3.0 us now.)
 #define MERGE_THREADS 256
 template <typename T>
 __global__ void __launch_bounds__(MERGE_THREADS)
 merge_splits_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws_ml, int nsplit, int head_dim, int n_heads, T* __restrict__ out, int out_stride) {
     __shared__ __attribute__((aligned(16))) float4 o_s[MERGE_THREADS];
-    __shared__ float2 ml_s[MERGE_THREADS];
+    __shared__ float2 wl_s[MERGE_THREADS];          // weight still to be applied, sum
+    __shared__ float max_s[MERGE_THREADS / MLLM_WAVE];
     // (blockIdx.y: 4 MERGE_THREADS elements of heads wider than that)
     const int pair = blockIdx.x, quad0 = blockIdx.y * MERGE_THREADS, quads = min(head_dim / 4 - quad0, MERGE_THREADS), groups = MERGE_THREADS / quads;
     const int quad = threadIdx.x % quads, group = threadIdx.x / quads;
-    float m = -1.0e30f, l = 0.f, o[4] = {0.f, 0.f, 0.f, 0.f};
+    const float* state = ws_ml + static_cast<size_t>(pair) * nsplit * 2;
+    const float* values = ws_o + static_cast<size_t>(pair) * nsplit * head_dim + 4 * (quad0 + quad);
+    // (surplus threads and groups take the last split along and drop it)
+    int s = min(group, nsplit - 1);
+    float2 ml = *reinterpret_cast<const float2*>(state + 2 * s);
+    float4 v = *reinterpret_cast<const float4*>(values + static_cast<size_t>(s) * head_dim);
+    float mx = ml.x;
+    for (int i = threadIdx.x; i < nsplit; i += MERGE_THREADS) mx = fmaxf(mx, state[2 * i]);
+    mx = wave_max(mx);
+    if (threadIdx.x % MLLM_WAVE == 0) max_s[threadIdx.x / MLLM_WAVE] = mx;
+    __syncthreads();
+    mx = fmaxf(fmaxf(max_s[0], max_s[1]), fmaxf(max_s[2], max_s[3]));
+    float w = exp2_for<T>(ml.x - mx), l = ml.y, o[4] = {v.x, v.y, v.z, v.w};
     if (group < groups) {
-        for (int s = group; s < nsplit; s += groups) {
-            const size_t slot = static_cast<size_t>(pair) * nsplit + s;
-            const float2 ml = *reinterpret_cast<const float2*>(ws_ml + slot * 2);
-            const float4 v = *reinterpret_cast<const float4*>(ws_o + slot * head_dim + 4 * (quad0 + quad));
-            const float o2[4] = {v.x, v.y, v.z, v.w};
-            merge_state<T, 4>(m, l, o, ml.x, ml.y, o2);
+        if (s + groups < nsplit) {
+            l *= w;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) o[e] *= w;
+            for (s += groups; s < nsplit; s += groups) {
+                ml = *reinterpret_cast<const float2*>(state + 2 * s);
+                v = *reinterpret_cast<const float4*>(values + static_cast<size_t>(s) * head_dim);
+                w = exp2_for<T>(ml.x - mx);
+                l += w * ml.y;
+                o[0] += w * v.x; o[1] += w * v.y; o[2] += w * v.z; o[3] += w * v.w;
+            }
+            w = 1.f;
         }
         o_s[threadIdx.x] = make_float4(o[0], o[1], o[2], o[3]);
-        ml_s[threadIdx.x] = make_float2(m, l);
+        wl_s[threadIdx.x] = make_float2(w, l);
     }
     __syncthreads();
     if (group > 0) return;
+    l *= w;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) o[e] *= w;
     for (int g = 1; g < min(groups, nsplit); ++g) {
-        const float4 v = o_s[g * quads + quad];
-        const float2 ml = ml_s[g * quads + quad];
-        const float o2[4] = {v.x, v.y, v.z, v.w};
-        merge_state<T, 4>(m, l, o, ml.x, ml.y, o2);
+        v = o_s[g * quads + quad];
+        const float2 wl = wl_s[g * quads + quad];
+        l += wl.x * wl.y;
+        o[0] += wl.x * v.x; o[1] += wl.x * v.y; o[2] += wl.x * v.z; o[3] += wl.x * v.w;
     }
     const float inv = 1.0f / l;
     T* dst = out + static_cast<size_t>(pair / n_heads) * out_stride + (pair % n_heads) * head_dim + 4 * (quad0 + quad);

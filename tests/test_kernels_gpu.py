@@ -979,6 +979,29 @@ def test_merge_of_splits(ops, head_dim, nsplit, dtype):
     assert (got[:, heads * head_dim:] == 7).all()
 
 
+@pytest.mark.parametrize("nsplit", [9, 15, 17, 21, 33, 64])
+def test_merge_of_splits_rounds_no_more_than_one_weight_a_split(ops, nsplit):
+    """In 32 bits the error against float64 is no larger than that of one weight for every split, sums in their order
+    and the sum's reciprocal (the kernel's own last step, two roundings)."""
+    tokens, heads, head_dim = 64, 12, 64
+    g = torch.Generator().manual_seed(nsplit)
+    o = torch.randn(tokens, heads, nsplit, head_dim, generator=g)
+    m, l = torch.randn(tokens, heads, nsplit, generator=g), 1 + 30 * torch.rand(tokens, heads, nsplit, generator=g)
+    out = torch.empty(tokens, heads * head_dim, device=DEV)
+    assert _merge_splits(ops, torch.cat([o.reshape(-1), torch.stack([m, l], -1).reshape(-1)]).to(DEV), tokens, heads, head_dim, nsplit, out) == 0
+
+    def plain(dtype):
+        w = torch.exp2(m.to(dtype) - m.amax(-1, keepdim=True).to(dtype))
+        total, sums = torch.zeros(tokens, heads, 1, dtype=dtype), torch.zeros(tokens, heads, head_dim, dtype=dtype)
+        for s in range(nsplit):
+            total += (w * l.to(dtype))[..., s:s + 1]
+            sums += w[..., s:s + 1] * o[:, :, s].to(dtype)
+        return (sums * (1 / total)).reshape(tokens, -1)
+
+    want = plain(torch.float64)
+    assert (out.cpu().double() - want).norm() <= (plain(torch.float32).double() - want).norm()
+
+
 def test_merge_of_splits_refuses(ops):
     ws, out = torch.zeros(64, device=DEV), torch.zeros(1, 64, device=DEV)
     for tokens, heads, head_dim, nsplit in ((1, 1, 0, 1), (1, 1, -4, 1), (1, 1, 6, 1), (1, 0, 8, 1), (1, -1, 8, 1), (1, 1, 8, 0)):
