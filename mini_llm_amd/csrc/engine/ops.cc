@@ -407,7 +407,7 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
 // attention
 // ---------------------------------------------------------------------------------------------
 // How many workgroups share one (token, head) pair's keys, and wavefronts per workgroup.
-static void decode_launch_shape(int pairs, int max_ctx_len, int keys_per_wave, bool unmerged, int* nsplit, int* waves, bool* merge_kernel) {
+static void decode_launch_shape(int pairs, int max_ctx_len, int keys_per_wave, bool bf16, bool unmerged, int* nsplit, int* waves, bool* merge_kernel) {
     const Tuning& t = tuning();
     *merge_kernel = false;
     if (t.decode_nsplit > 0) { *nsplit = t.decode_nsplit; *waves = t.decode_waves; return; }
@@ -445,9 +445,17 @@ static void decode_launch_shape(int pairs, int max_ctx_len, int keys_per_wave, b
     // more wavefronts each instead (measured: 12 are 1 to 3 % of a decode step faster than 8 up to 200
     // pairs at GPT-2 small to XL sizes, 3 % slower from 384 pairs). More wavefronts than the keys occupy (each takes
     // `keys_per_wave` at a time) only lengthen the merge: one prompt of 100 tokens and 64 new ones takes 22.5 ms with 12
-    // wavefronts, 21.6 with 4 (21.65 with 3, 22.0 with 6).
+    // wavefronts, 21.6 with 4 (21.65 with 3, 22.0 with 6). A launch alone, as many as the keys occupy against all of them (us, heads
+    // of 64): bf16, 200 pairs: 5.8 / 7.6 at 164 keys, 7.2 / 8.1 at 320, 8.2 / 8.9 at 512, 9.55 / 9.60 at 600 (10), 9.9 / 9.9 at 660
+    // (11); 288 to 480 pairs: 7.0 / 8.7 at 128 keys, 9.3 / 9.9 at 257; 32 bits, 96 pairs: 6.5 / 7.6 at 164, 8.0 / 8.3 at 257 (9), 8.8
+    // / 8.9 at 321 (11). Nine lose where 16-bit keys of many pairs are streamed, as one SIMD unit of four then has a wavefront more
+    // than the others: 9.20 / 9.09 for 200 pairs at 520 keys, 11.1 / 11.0 for 256 with heads of 128 at 257; up to 144 pairs they
+    // win (8.9 / 9.0, 9.2 / 9.4).
     *nsplit = 1;
-    *waves = std::min(pairs >= 512 ? 4 : pairs > 256 ? 6 : 12, std::max(4, (max_ctx_len + keys_per_wave - 1) / keys_per_wave));
+    const int all = pairs >= 512 ? 4 : pairs > 256 ? 6 : 12;
+    int occupied = std::max(4, (max_ctx_len + keys_per_wave - 1) / keys_per_wave);
+    if (occupied == 9 && bf16 && pairs > 144) occupied = 12;
+    *waves = std::min(all, occupied);
 }
 
 static bool pow2(int v) { return v > 0 && (v & (v - 1)) == 0; }
@@ -563,7 +571,7 @@ bool paged_attention(const AttentionArgs& a, AttentionSplits* splits, hipStream_
                         a.head_dim % 8 == 0 && tuning().decode_nsplit == 0;
         int nsplit = 1, waves = 12;
         bool merge_kernel = false;
-        decode_launch_shape(pairs, a.max_ctx_len, 512 / lpk, unmerged, &nsplit, &waves, &merge_kernel);      // (8 rows a lane group: the kernel's UNR)
+        decode_launch_shape(pairs, a.max_ctx_len, 512 / lpk, a.q.dtype == BF16, unmerged, &nsplit, &waves, &merge_kernel);      // (8 rows a lane group: the kernel's UNR)
         // (sigmoid weights have no sum to divide by afterwards: the kernel merges its own splits, however many)
         // (nor does the merge kernel know a gate of one value per head)
         if (a.shape != nullptr && (a.shape->sigmoid || (a.gate != nullptr && a.shape->gate_per_head))) merge_kernel = false;

@@ -588,6 +588,20 @@ def test_paged_attention_decode_only(ops, dtype, H, Hkv, dh, page, window, shape
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("T,H,Hkv,dh", [(9, 16, 16, 64), (9, 17, 17, 64), (17, 12, 4, 64), (12, 25, 5, 64), (10, 16, 4, 128)])
+@pytest.mark.parametrize("blocks", [1, 4, 5, 8, 9, 10, 12, 13])
+def test_paged_attention_decode_wavefronts(ops, dtype, T, H, Hkv, dh, blocks):
+    """As many wavefronts as the longest context's keys occupy, within 4 to 12 and the limits by pairs: contexts on both sides of
+    every step of that rule, in one launch with short ones."""
+    per = 512 // (dh * (2 if dtype == torch.bfloat16 else 4) // 16)
+    g = torch.Generator().manual_seed(T * H + blocks)
+    for longest in (per * blocks, per * blocks + 1):
+        out, ref = _attention_case(ops, dtype, H, Hkv, dh, 16, [((longest - 1) // (1 + k % 3), 1) for k in range(T)], 0, g)
+        assert torch.isfinite(out).all()
+        assert (out - ref).abs().max() <= _tol(dtype, 2)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,Hkv,dh,page", [(4, 2, 64, 16), (6, 2, 128, 16), (3, 3, 32, 8), (5, 5, 48, 16), (2, 1, 40, 4)])
 @pytest.mark.parametrize("kind", ["window_bias", "chunk_gate", "sigmoid", "slope_sink", "window_keep"])
 def test_paged_attention_with_shaped_scores(ops, dtype, H, Hkv, dh, page, kind):
