@@ -282,6 +282,54 @@ def test_gate_and_up_in_one_product(rows, ff, k):
     assert float(err.max()) <= slack, (float(err.max()), slack)
 
 
+@pytest.mark.parametrize("rows", [1, 9, 17, 32, 33, 130, 300])
+@pytest.mark.parametrize("ff,k", [(1, 64), (5, 200), (18, 768), (1001, 72), (2050, 1608)])
+def test_gate_and_up_at_odd_sizes_to_the_last_rounding(rows, ff, k):
+    """The same for widths and row strides that fill no vector store, on rows so faint that eps counts in the norm, against a bound
+    that a rounding of gate or up before the activation exceeds: half a unit of the result in bfloat16, the fp32 sums' error and,
+    behind the norm, those of its values that lie so close to a border of bfloat16 that they may round either way."""
+    import ctypes
+    import torch
+    from mini_llm_amd.kernels import ops
+    lib = ops.engine_library()
+    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    g = torch.Generator().manual_seed(rows * 7 + ff + k)
+    x = 0.01 * torch.randn(rows, k, generator=g)
+    gamma = 1 + 0.1 * torch.randn(k, generator=g)
+    gate, up = ((torch.randn(ff, k, generator=g) * (2.0 / k ** 0.5)).bfloat16() for _ in range(2))
+    limit, alpha, eps = 3.0, 1.702, 1e-4            # (the rows' mean square is 1e-4 as well)
+    fused = rows <= 32
+    normed = pk.rms_norm(x.double(), gamma.double(), eps)
+    a = (normed if fused else 100 * x).bfloat16()
+    unsure = torch.zeros(rows, k, dtype=torch.float64)
+    if fused:          # the norm's relative error: a few roundings and half of those of a sum of k squares over 64 lanes
+        delta = (4 + (k / 64 + 8) / 2) * 2.0 ** -24
+        unsure = ((normed * (1 + delta)).bfloat16().double() - (normed * (1 - delta)).bfloat16().double()).abs()
+    gv, uv = a.double() @ gate.double().T, a.double() @ up.double().T
+    sums = [2.0 ** -24 * (k / 16 + 16) * (a.double().abs() @ w.double().abs().T) + unsure @ w.double().abs().T for w in (gate, up)]
+    gv, uv = torch.clamp(gv, max=limit), torch.clamp(uv, min=-limit, max=limit)
+    want = gv * torch.sigmoid(alpha * gv) * (uv + 1)
+    dev = [t.cuda() for t in (x, gamma, gate, up, a)]
+    stride = ff + 7 + ff % 2                         # (odd)
+    out = torch.full((rows + 1, stride), 7.0, dtype=torch.bfloat16, device="cuda")
+    if fused:
+        fn = lib.mllm_rms_gated_gemm_bf16
+        fn.argtypes = [vp, i, vp, f, vp, vp, i, f, f, vp, i, i, i, i, vp]
+        rc = fn(dev[0].data_ptr(), k, dev[1].data_ptr(), eps, dev[2].data_ptr(), dev[3].data_ptr(), k, limit, alpha, out.data_ptr(), stride, rows, ff, k, None)
+    else:
+        fn = lib.mllm_gated_gemm_bf16
+        fn.argtypes = [vp, i, vp, vp, i, f, f, vp, i, i, i, i, vp]
+        rc = fn(dev[4].data_ptr(), k, dev[2].data_ptr(), dev[3].data_ptr(), k, limit, alpha, out.data_ptr(), stride, rows, ff, k, None)
+    assert rc == 0
+    torch.cuda.synchronize()
+    got = out.cpu().double()
+    assert (got[:, ff:] == 7).all() and (got[rows:] == 7).all()
+    # (the activation's slope: under 1.1 (limit + 1) in g, at most limit in u; exponential and reciprocal to 2^-20)
+    half_unit = torch.ldexp(torch.ones_like(want), torch.frexp(want.abs() * (1 + 2.0 ** -9))[1] - 9)       # (8 bits)
+    bound = half_unit + 2.0 ** -18 * want.abs() + 1.1 * (limit + 1) * sums[0] + limit * sums[1]
+    assert ((got[:rows, :ff] - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("rows,width", [(1, 4), (5, 68), (33, 256), (3, 260), (511, 768), (513, 768), (9, 2048)])
 def test_norm_behind_a_sub_layer_and_the_next_in_front(rows, width):
     """x += mult scale rmsnorm(y) and the bfloat16 RMS norm of the new x, in one kernel."""
