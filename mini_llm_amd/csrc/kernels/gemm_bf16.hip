@@ -449,8 +449,8 @@ static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, con
 }
 
 // ---------------------------------------------------------------------------------------------
-// Few rows (decode; up to 64 rows always, up to 256 while the workgroups stay few, see the
-// dispatch). The product is bound by streaming W once, and how fast a compute
+// Few rows (decode; up to 16 rows and, of the widest products, 64 always; up to 256 where it is priced
+// lower than the tiles, see the dispatch). The product is bound by streaming W once, and how fast a compute
 // unit streams depends on the shape of a wavefront's load: 8 consecutive lanes take one 128-byte
 // line (8 weight rows x 1 line per load) at up to 90 GB/s per unit, but the MFMA operand layout
 // (consecutive lanes = consecutive weight rows, 4 lines per 4 lanes) at under 40 (measured). So

@@ -1,8 +1,7 @@
 // True fp32 matrix product for the 32-bit path: C[M,N] = A[M,K] * W[N,K]^T (+ bias, epilogue).
-// Plain FMA in fp32, every output accumulated over k in a fixed order, so a row's
-// result does not depend on which other rows share the launch (beyond the choice between the
-// two kernels below, which add in different orders). No reduced-precision matrix mode is
-// involved. Any M, N, K.
+// fp32 products summed in fp32, on the vector units or the fp32 matrix cores; no reduced-precision matrix mode is
+// involved. Every output is accumulated over k in an order that its kernel and tile shape fix, so which other
+// rows share the launch matters only through their number, which chooses between these. Any M, N, K.
 //
 // Same contract as the reference's bounds-safe kernel
 // (/root/reference/src/kernels/gemm.cu:238-392: alpha*acc + beta*old + bias, optional GELU),
