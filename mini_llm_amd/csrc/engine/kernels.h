@@ -112,7 +112,7 @@ int mllm_ssm_scan(const float* xbc, int ldx, const float* raw_dt, int ldd, const
                   const float* Dskip, const int* cu_q, const int* state_slots, float* state, size_t slot_floats,
                   size_t scan_offset, float* y, int ldy, size_t part_stride, int T, int B, int max_q_len, int H, int P, int N,
                   int G, int write, float* workspace, hipStream_t stream);
-int mllm_ssm_scan_parts(const float* xbc, int ldx, int P, int N);
+int mllm_ssm_scan_parts(const float* xbc, int ldx, int T, int max_q_len, int H, int P, int N);
 size_t mllm_ssm_scan_workspace_floats(int T, int B, int H, int P, int N);
 
 // latent_attention.hip

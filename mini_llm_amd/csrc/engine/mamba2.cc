@@ -72,7 +72,7 @@ public:
         conv_silu(proj, inner_, conv_, conv_bias_, st, xbc, s);
         StageTimes::get().mark("conv", s);
         // (the scan may leave its result as shares, one per slice of the state's rows; the norm adds them)
-        const int parts = ssm_scan_parts(xbc, P_, N_);
+        const int parts = ssm_scan_parts(xbc, step.max_q_len, H_, P_, N_);
         Tensor2 y(arena.take(static_cast<size_t>(parts) * T * inner_ * 4), F32, T, inner_);
         // (portions longer than a chunk are scanned chunk by chunk side by side: room for the chunks' states)
         const size_t ws_floats = step.max_q_len > 64 ? ssm_scan_workspace_floats(T, step.n_seqs, H_, P_, N_) : 0;

@@ -223,7 +223,7 @@ struct StateArgs {
 void conv_silu(const Tensor2& proj, int col0, const Tensor2& weight, const float* bias, const StateArgs& st,
                const Tensor2& out, hipStream_t stream);
 // The Mamba-2 scan (kernels/ssm.hip) over xbc [T, H*P + 2*G*N] and the raw step sizes (columns dt_col.. of
-// proj), state at `scan_offset` floats into the slot. y comes as ssm_scan_parts(xbc, P, N) shares, each [T, H*P] fp32
+// proj), state at `scan_offset` floats into the slot. y comes as ssm_scan_parts(xbc, ...) shares, each [T, H*P] fp32
 // and y.rows * y.stride floats after the one before (y is the first); their sum in the order of their index is
 // the result (rmsnorm adds them while it reads). Portions longer than a chunk are scanned chunk by chunk side by
 // side and joined, for which `workspace` (ssm_scan_workspace_floats floats) is needed.
@@ -231,7 +231,7 @@ void ssm_scan(const Tensor2& xbc, const Tensor2& proj, int dt_col, const float* 
               const float* skip, const StateArgs& st, size_t scan_offset, int H, int P, int N, int G, const Tensor2& y,
               float* workspace, size_t workspace_floats, hipStream_t stream);
 size_t ssm_scan_workspace_floats(int tokens, int n_seqs, int H, int P, int N);
-int ssm_scan_parts(const Tensor2& xbc, int P, int N);
+int ssm_scan_parts(const Tensor2& xbc, int max_q_len, int H, int P, int N);
 
 // -- latent attention --------------------------------------------------------------------------------
 struct LatentShape {

@@ -196,7 +196,9 @@ void ssm_scan(const Tensor2& xbc, const Tensor2& proj, int dt_col, const float* 
                         stream), "ssm_scan");
 }
 
-int ssm_scan_parts(const Tensor2& xbc, int P, int N) { return mllm_ssm_scan_parts(static_cast<const float*>(xbc.data), i32(xbc.stride), P, N); }
+int ssm_scan_parts(const Tensor2& xbc, int max_q_len, int H, int P, int N) {
+    return mllm_ssm_scan_parts(static_cast<const float*>(xbc.data), i32(xbc.stride), i32(xbc.rows), max_q_len > 0 ? max_q_len : i32(xbc.rows), H, P, N);
+}
 
 size_t ssm_scan_workspace_floats(int tokens, int n_seqs, int H, int P, int N) {
     return mllm_ssm_scan_workspace_floats(tokens, n_seqs, H, P, N);

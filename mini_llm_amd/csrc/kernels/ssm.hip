@@ -393,33 +393,36 @@ ssm_scan_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict_
 
 // The scan of sequences of at most CH tokens (decoding, short portions; longer ones leave at once and go through the chunk
 // kernels below): one workgroup per (sequence, head, 64 values of p), a wavefront per slice of NS rows n (more
-// than four slices: in rounds). A wavefront's operands are staged in LDS first, x [CH][64], B and C of the slice [CH][NS] and the raw step sizes, all requested at once
-// with 16-byte loads, so that the token loop waits for no memory (one token ahead is not enough to cover a load that another
-// XCD's kernel wrote a moment ago). The slices' sums over n meet in LDS and are added in the order of the slices, so y leaves
-// whole. Needs 16-byte aligned rows and column offsets. Bound by the state that it reads and writes, and at eight sequences
-// (12.6 MB, 24 heads of 128 x 64) by the chain of one launch: 7.2 us a layer. LDS: floats a wavefront takes.
+// slices than WAVES: in rounds). A wavefront's operands are staged in LDS first, x [CH][64], B and C of the slice [CH][NS] and the
+// raw step sizes, all requested at once with 16-byte loads, so that the token loop waits for no memory (one token ahead is not enough
+// to cover a load that another XCD's kernel wrote a moment ago). The slices' sums over n meet in LDS and are added in the order of
+// the slices, so y leaves whole. WAVES of 1: a workgroup per slice, which stores its share in y + slice * part_stride for the reader to
+// add. Needs 16-byte aligned rows and column offsets. Bound by the state that it reads and writes, at eight sequences
+// (12.6 MB, 24 heads of 128 x 64) by the chain of one launch: 7.2 us a layer, and from a dozen tokens on by the chain of tokens,
+// which sums that meet in LDS lengthen. LDS: floats a wavefront takes.
 template <int NS, int CH> constexpr int ssm_short_floats() { return CH * 64 + 2 * CH * NS + 2 * CH; }
-template <int NS, int CH>
-__global__ void __launch_bounds__(256)
+template <int NS, int CH, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES)
 ssm_short_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict__ raw_dt, int ldd,
                  const float* __restrict__ dt_bias, const float* __restrict__ A_log, const float* __restrict__ Dskip,
                  const int* __restrict__ cu_q, const int* __restrict__ state_slots, float* __restrict__ state,
-                 size_t slot_floats, size_t scan_offset, float* __restrict__ y, int ldy, int H, int P, int N, int G, int write) {
+                 size_t slot_floats, size_t scan_offset, float* __restrict__ y, int ldy, size_t part_stride, int H, int P, int N, int G, int write) {
+    constexpr bool SHARES = WAVES == 1;
     extern __shared__ __attribute__((aligned(16))) float short_s[];
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), waves = blockDim.x / 64;
-    const int h = blockIdx.y, p0 = blockIdx.x * 64, p = p0 + lane, b = blockIdx.z;
+    const int n_slices = (N + NS - 1) / NS;
+    const int h = blockIdx.y, p0 = (SHARES ? blockIdx.x / n_slices : blockIdx.x) * 64, p = p0 + lane, b = blockIdx.z;
     const int t0 = cu_q[b], nt = cu_q[b + 1] - t0;
     const int slot = state_slots[b];
     if (slot < 0 || nt < 1 || nt > CH) return;                 // (the whole workgroup)
     const bool p_ok = p < P;
     const int pc = p_ok ? p : P - 1;
     const int g = h / (H / G), inner = H * P;
-    const int n_slices = (N + NS - 1) / NS;
     float* xs = short_s + wave * ssm_short_floats<NS, CH>();
     float *Bs = xs + CH * 64, *Cs = Bs + CH * NS, *dts = Cs + CH * NS, *as = dts + CH;      // dts, as: the tokens' step sizes and decays
-    for (int s0 = 0; s0 < n_slices; s0 += waves) {
-        const int slice = s0 + wave;
-        if (slice < n_slices) {
+    for (int s0 = 0; s0 < (SHARES ? 1 : n_slices); s0 += waves) {
+        const int slice = SHARES ? blockIdx.x % n_slices : s0 + wave;
+        if (SHARES || slice < n_slices) {
             const int n0 = slice * NS, nn = min(NS, N - n0);
             float* sp = state + static_cast<size_t>(slot) * slot_floats + scan_offset + (static_cast<size_t>(h) * N + n0) * P + pc;
             float S[NS];
@@ -482,7 +485,9 @@ ssm_short_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict
                     S[j + 2] = a * S[j + 2] + dx * b4.z; acc[2] += S[j + 2] * c4.z;
                     S[j + 3] = a * S[j + 3] + dx * b4.w; acc[3] += S[j + 3] * c4.w;
                 }
-                xs[tt * 64 + lane] = (acc[0] + acc[1]) + (acc[2] + acc[3]) + skip * xv;      // the slice's share of y, in x's place
+                const float share = (acc[0] + acc[1]) + (acc[2] + acc[3]) + skip * xv;
+                if constexpr (!SHARES) xs[tt * 64 + lane] = share;      // in x's place
+                else if (p_ok) y[slice * part_stride + static_cast<size_t>(t0 + tt) * ldy + h * P + p] = share;
             }
             if (write && p_ok) {
 #pragma unroll
@@ -490,6 +495,7 @@ ssm_short_kernel(const float* __restrict__ xbc, int ldx, const float* __restrict
                     if (j < nn) sp[static_cast<size_t>(j) * P] = S[j];
             }
         }
+        if constexpr (SHARES) return;
         __syncthreads();
         for (int i = threadIdx.x; i < nt * 64; i += blockDim.x) {
             if (p0 + i % 64 >= P) continue;
@@ -1051,8 +1057,19 @@ size_t mllm_ssm_scan_workspace_floats(int T, int B, int H, int P, int N) {
 static bool ssm_by_quads(const float* xbc, int ldx, int P, int N) {
     return ldx % 4 == 0 && P % 4 == 0 && N % 4 == 0 && (reinterpret_cast<uintptr_t>(xbc) & 15) == 0;
 }
-// The scan leaves y as this many shares, part_stride floats apart: one, or one per slice of the state's rows (ssm_scan_kernel).
-int mllm_ssm_scan_parts(const float* xbc, int ldx, int P, int N) { return ssm_by_quads(xbc, ldx, P, N) ? 1 : (N + SSM_SLICE - 1) / SSM_SLICE; }
+// Whether the short kernel leaves a share per slice. One share costs every token's chain a store to LDS and the end a barrier, several are
+// written and read again: scan and norm, us, one share / one a slice: 24 heads of 128 x 64: 1 x 32 tokens 23.0 / 21.0, 1 x 64 34.8 / 31.2,
+// 8 x 32 24.5 / 25.4, 8 x 64 37.9 / 37.5; 24 heads of 64 x 64, 8 x 64: 36.6 / 33.6; 8 heads of 16 x 64 (a share either way), 8 x 64: 35.6 / 29.0;
+// 4 heads of 256 x 128 (one share in two rounds), 1 x 64: 61.5 / 44.6. Up to 8 tokens one share is even for one sequence (8 tokens: 13.1 / 12.9)
+// and ahead for several (8 x 8: 13.8 / 15.1; 64 x 1: 25.4 / 39.9).
+static bool ssm_shares(int T, int max_q_len, int H, int P, int n_slices) {
+    return max_q_len > 8 && max_q_len <= SSM_CHUNK && (n_slices > 4 || static_cast<double>(T) * H * P * (n_slices - 1) <= 1 << 20);
+}
+// The scan leaves y as this many shares, part_stride floats apart: one, or one per slice of the state's rows.
+int mllm_ssm_scan_parts(const float* xbc, int ldx, int T, int max_q_len, int H, int P, int N) {
+    const int n_slices = (N + SSM_SLICE - 1) / SSM_SLICE;
+    return ssm_by_quads(xbc, ldx, P, N) && !ssm_shares(T, max_q_len, H, P, n_slices) ? 1 : n_slices;
+}
 
 // The scan over every sequence's portion (see the kernels). `workspace` (mllm_ssm_scan_workspace_floats floats)
 // is needed when a portion is longer than one chunk (max_q_len > 64). -1: H is no multiple of G, or the
@@ -1070,21 +1087,28 @@ int mllm_ssm_scan(const float* xbc, int ldx, const float* raw_dt, int ldd, const
     float* cumlog = workspace ? chunk_state + chunk_states(T) * H * P * N : nullptr;
     const int n_slices = (N + SSM_SLICE - 1) / SSM_SLICE;
     if (ssm_by_quads(xbc, ldx, P, N)) {
-        const int p_tiles = (P + 63) / 64, waves = std::min(n_slices, 4);
-#define SSM_SHORT(CH)                                                                                                  \
+        const int p_tiles = (P + 63) / 64;
+#define SSM_SHORT(CH, WAVES)                                                                                           \
     do {                                                                                                               \
         constexpr int floats = ssm_short_floats<SSM_SLICE, CH>();                                                      \
-        auto kernel = ssm_short_kernel<SSM_SLICE, CH>;                                                                 \
-        static bool lds_allowed = 4 * floats * 4 <= 64 * 1024;      /* more has to be asked for once */                \
+        auto kernel = ssm_short_kernel<SSM_SLICE, CH, WAVES>;                                                          \
+        static bool lds_allowed = WAVES * floats * 4 <= 64 * 1024;      /* more has to be asked for once */            \
         if (!lds_allowed) {                                                                                            \
-            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, 4 * floats * 4); \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize, WAVES * floats * 4); \
             if (e != hipSuccess) return static_cast<int>(e);                                                           \
             lds_allowed = true;                                                                                        \
         }                                                                                                              \
-        kernel<<<dim3(p_tiles, H, B), 64 * waves, waves * floats * 4, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, Dskip, cu_q, state_slots, \
-                                                                                      state, slot_floats, scan_offset, y, ldy, H, P, N, G, write);     \
+        const int waves = std::min(n_slices, WAVES);                                                                   \
+        kernel<<<dim3(WAVES == 1 ? p_tiles * n_slices : p_tiles, H, B), 64 * waves, waves * floats * 4, stream>>>(xbc, ldx, raw_dt, ldd, dt_bias, A_log, \
+            Dskip, cu_q, state_slots, state, slot_floats, scan_offset, y, ldy, part_stride, H, P, N, G, write);        \
     } while (0)
-        if (max_q_len <= 8) SSM_SHORT(8); else if (!chunked || T < static_cast<long>(B) * max_q_len) SSM_SHORT(SSM_CHUNK);      // (equally long portions: none)
+        if (max_q_len <= 8) {
+            if (n_slices > 4) SSM_SHORT(8, 8); else SSM_SHORT(8, 4);
+        } else if (ssm_shares(T, max_q_len, H, P, n_slices)) {
+            SSM_SHORT(SSM_CHUNK, 1);
+        } else if (!chunked || T < static_cast<long>(B) * max_q_len) {      // (equally long portions of several chunks: none)
+            SSM_SHORT(SSM_CHUNK, 4);
+        }
 #undef SSM_SHORT
         if (chunked) {
             const dim3 tiles(p_tiles, H, n_chunks);

@@ -386,13 +386,16 @@ def _scan(sizes, given, workspace_floats_off=0):
     cu_q = torch.tensor(np.cumsum([0] + list(sizes)), dtype=torch.int32, device="cuda")
     slots = torch.arange(b, dtype=torch.int32, device="cuda")
     state = torch.zeros(b, H, N, P, device="cuda")
-    y = torch.full((T, H, P), 7.0, device="cuda")
+    shares = lib.mllm_ssm_scan_parts
+    shares.argtypes = [vp, i, i, i, i, i, i]
+    parts = shares(xbc.data_ptr(), xbc.stride(0), T, max(sizes), H, P, N)
+    y = torch.full((parts, T, H, P), 7.0, device="cuda")
     ws = torch.full((need(T, b, H, P, N) + workspace_floats_off,), float("nan"), device="cuda")
     rc = fn(xbc.data_ptr(), xbc.stride(0), dev[0].data_ptr(), H, *(d.data_ptr() for d in dev[1:]), cu_q.data_ptr(), slots.data_ptr(), state.data_ptr(),
             H * N * P, 0, y.data_ptr(), H * P, T * H * P, T, b, max(sizes), H, P, N, 1, 1, ws.data_ptr() + 4 * workspace_floats_off, None)
     assert rc == 0
     torch.cuda.synchronize()
-    return y.cpu(), state.cpu()
+    return y.sum(0).cpu(), state.cpu()
 
 
 def _scan_plain(sizes, given, magnitudes=False):
@@ -465,3 +468,14 @@ def test_scan_takes_a_workspace_at_any_float():
     first = _scan(sizes, given)
     for off in (1, 2, 3):
         assert all(torch.equal(a, b) for a, b in zip(first, _scan(sizes, given, off)))
+
+
+@pytest.mark.parametrize("sizes", [(64,), (9, 64, 1, 33), (64,) * 40, (8, 1, 5), (3,), (64, 65, 8)])
+@pytest.mark.parametrize("heads,vdim,state", [(2, 68, 36), (3, 64, 16), (24, 64, 64), (2, 64, 132), (1, 32, 260), (2, 36, 300)])
+def test_short_portions_leave_one_share_or_one_a_slice(sizes, heads, vdim, state):
+    """Portions of at most 64 tokens on both sides of the rule for shares, states of one slice of 32 rows to ten. A sum's error is at
+    most a rounding per term of its magnitudes' sum (the state's rows, the tokens) and one per unit of the decays' logarithms."""
+    import torch
+    given = _scan_inputs(sizes, heads, vdim, state, seed=state + len(sizes))
+    for got, want, size in zip(_scan(sizes, given), _scan_plain(sizes, given), _scan_plain(sizes, given, magnitudes=True)):
+        assert ((got.double() - want).abs() <= 2.0 ** -24 * (state + 64 + 200) * size).all()
