@@ -302,15 +302,44 @@ __device__ __forceinline__ ChunkOf chunk_of(int index, const int* cu_q, int n_se
     // (no portion longer than a chunk: chunk i is sequence i, and no walk over the sequences, whose every step
     // would wait for a load)
     if (!chunked) return ChunkOf{index < n_seqs ? index : -1, 0, 1, 0};
-    ChunkOf c{0, index, 0, 0};
-    for (; c.b < n_seqs; ++c.b) {
-        c.n_chunks = max(1, (cu_q[c.b + 1] - cu_q[c.b] + chunk - 1) / chunk);
-        if (c.k < c.n_chunks) return c;
-        c.k -= c.n_chunks;
-        if (c.n_chunks > 1) c.first_chunk += c.n_chunks;
+    if (n_seqs <= 8) {
+        ChunkOf c{0, index, 0, 0};
+        for (; c.b < n_seqs; ++c.b) {
+            c.n_chunks = max(1, (cu_q[c.b + 1] - cu_q[c.b] + chunk - 1) / chunk);
+            if (c.k < c.n_chunks) return c;
+            c.k -= c.n_chunks;
+            if (c.n_chunks > 1) c.first_chunk += c.n_chunks;
+        }
+        c.b = -1;
+        return c;
     }
-    c.b = -1;
-    return c;
+    // Many sequences: 64 at a time, one a lane, their lengths arrive together and are summed over the lanes. One after the other, every
+    // step waits for its load: 40 portions of 70 tokens, 24 heads of 128 x 64, scan and norm: 201 us > 158. (Up to eight the walk is
+    // 1 us shorter.)
+    const int lane = threadIdx.x % 64;
+    int chunks_before = 0, states_before = 0;
+    for (int b0 = 0; b0 < n_seqs; b0 += 64) {
+        const int b = b0 + lane;
+        const int n_tokens = cu_q[min(b + 1, n_seqs)] - cu_q[min(b, n_seqs)];
+        const int n = b < n_seqs ? max(1, (n_tokens + chunk - 1) / chunk) : 0;
+        int end = n;
+#pragma unroll
+        for (int off = 1; off < 64; off *= 2) {
+            const int up = __shfl_up(end, off, 64);
+            if (lane >= off) end += up;
+        }
+        const unsigned long long past = __ballot(chunks_before + end > index), single = __ballot(n == 1);
+        if (past != 0) {
+            const int at = __builtin_ctzll(past), n_chunks = __builtin_amdgcn_readlane(n, at);
+            const int before = __builtin_amdgcn_readlane(end, at) - n_chunks;
+            return ChunkOf{b0 + at, index - chunks_before - before, n_chunks,
+                           states_before + before - static_cast<int>(__popcll(single & ((1ull << at) - 1)))};
+        }
+        const int all = __builtin_amdgcn_readlane(end, 63);
+        chunks_before += all;
+        states_before += all - static_cast<int>(__popcll(single));
+    }
+    return ChunkOf{-1, 0, 0, 0};
 }
 
 template <int NS>
@@ -625,11 +654,15 @@ ssm_chunk_prefix_kernel(const int* __restrict__ cu_q, const int* __restrict__ st
     const int q0 = cu_q[b], q1 = cu_q[b + 1], n_chunks = (q1 - q0 + SSM_TILE - 1) / SSM_TILE;
     const int slot = state_slots[b];
     if (n_chunks < 2 || slot < 0) return;
-    int first = 0;
-    for (int k = 0; k < b; ++k) {
-        const int n = (cu_q[k + 1] - cu_q[k] + SSM_TILE - 1) / SSM_TILE;
-        if (n > 1) first += n;
+    int first = 0;          // the states in front of the sequence's: 64 sequences at a time, as in chunk_of
+    for (int k0 = 0; k0 < b; k0 += 64) {
+        const int k = k0 + threadIdx.x % 64, n = (cu_q[min(k + 1, b)] - cu_q[min(k, b)] + SSM_TILE - 1) / SSM_TILE;      // (from b on: 0)
+        int sum = n > 1 ? n : 0;
+#pragma unroll
+        for (int off = 32; off > 0; off /= 2) sum += __shfl_xor(sum, off, 64);
+        first += sum;
     }
+    first = __builtin_amdgcn_readfirstlane(first);
     if (i >= NP) return;
     float* sp = state + static_cast<size_t>(slot) * slot_floats + scan_offset + static_cast<size_t>(h) * NP + i;
     const size_t step = static_cast<size_t>(H) * NP;

@@ -479,3 +479,14 @@ def test_short_portions_leave_one_share_or_one_a_slice(sizes, heads, vdim, state
     given = _scan_inputs(sizes, heads, vdim, state, seed=state + len(sizes))
     for got, want, size in zip(_scan(sizes, given), _scan_plain(sizes, given), _scan_plain(sizes, given, magnitudes=True)):
         assert ((got.double() - want).abs() <= 2.0 ** -24 * (state + 64 + 200) * size).all()
+
+
+@pytest.mark.parametrize("sizes", [(70,) * 9, (1, 65, 64, 200, 3, 3, 128, 129, 1) * 8, (1,) * 64 + (130,), (1,) * 63 + (66, 66), (5,) * 130 + (70, 65)])
+@pytest.mark.parametrize("vdim,state", [(4, 4), (3, 5)])
+def test_scan_finds_chunks_among_many_portions(sizes, vdim, state):
+    """More than 8 sequences: their chunks are counted 64 at a time, on both sides of that and of portions of one chunk (in matrix form,
+    and at widths that only the scan token by token takes)."""
+    import torch
+    given = _scan_inputs(sizes, 1, vdim, state, seed=len(sizes))
+    for got, want, size in zip(_scan(sizes, given), _scan_plain(sizes, given), _scan_plain(sizes, given, magnitudes=True)):
+        assert ((got.double() - want).abs() <= 2.0 ** -24 * (state + 64 + 200) * size).all()
