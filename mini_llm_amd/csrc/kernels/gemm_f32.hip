@@ -397,21 +397,25 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
         MLLM_LAUNCH_CHECK();
         return 0;
     }
-    if (quads && K > 0) {
+    // Wide rows of an odd length leave the tiles an element at a time, which a short K does not hide: 130 x 50,257 x 64 35 us on tiles, 25 on
+    // vector FMAs, 2,048 x 50,257 x 64 346 / 239; 192 x 32,000 x 128 31.4 / 29.9 (at 192 columns 35.6 / 40.4), 192 x 16,384 x 64 13.8 / 13.4.
+    const bool odd_wide = M > 64 && ldc % 4 != 0 && N >= 16384 && K <= (N >= 32000 ? 128 : N >= 20000 ? 96 : 64);
+    if (quads && K > 0 && !odd_wide) {
         // Tiles of 32 x 32 shared by four groups up to 64 rows (whose sums are as exact as the kernel's for few rows) and while
         // there are at most two a compute unit (570 x 768 x 3,072: 40 us, with two groups 43, with tiles of 64 x 32 44).
         // Otherwise the shape whose fullest compute unit does least: its tiles times their size times what 32 x 32 outputs
-        // take there at K = 768 (in tenths of a microsecond, measured at 2,048 rows). Large tiles need several workgroups a unit
+        // take there at K = 768 (in tenths of a microsecond, measured at 2,048 rows). With two groups a sixth of that is there at
+        // any K, which shows up to 96 columns (130 x 50,304 x 96: 40 us with 32 x 32, 29 with 64 x 64; 65 x 50,304 x 256: 40.1, 41.5). Large tiles need several workgroups a unit
         // to hide their barriers: 2,048 x 768 x 768 32 us with 64 x 32, 35 with 64 x 64 (384 tiles) and 64 x 96 (256).
         const auto tiles = [&](int tm, int tn) { return static_cast<long>((M + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
-        const auto cost = [&](int tm, int tn, long from, int each) {
-            const long n = tiles(tm, tn);
-            return n < from ? (1L << 60) : ((n + 7) / 8 + 31) / 32 * tm * tn * each;
+        const auto cost = [&](int tm, int tn, int groups, long from, int each) {
+            const long n = tiles(tm, tn), k = K <= 96 ? K : 768;
+            return n < from ? (1L << 60) : ((n + 7) / 8 + 31) / 32 * tm * tn * each * (groups == 2 ? 5 * k + 768 : 6 * k);
         };
         if (M <= 64 || tiles(1, 1) <= 512) {
             launch_f32_tiles<1, 1, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
         } else {
-            const long c11 = cost(1, 1, 0, 44), c21 = cost(2, 1, 256, 40), c22 = cost(2, 2, 512, 36), c23 = cost(2, 3, 512, 37);
+            const long c11 = cost(1, 1, 2, 0, 44), c21 = cost(2, 1, 2, 256, 40), c22 = cost(2, 2, 1, 512, 36), c23 = cost(2, 3, 1, 512, 37);
             const long least = std::min(std::min(c11, c21), std::min(c22, c23));
             if (least == c22) launch_f32_tiles<2, 2, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
             else if (least == c23) launch_f32_tiles<2, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
@@ -421,7 +425,7 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
         MLLM_LAUNCH_CHECK();
         return 0;
     }
-    // any K, strides and alignment
+    // any K, strides and alignment, and short K (see above)
     dim3 grid((N + F32_BN - 1) / F32_BN, (M + F32_BM - 1) / F32_BM);
     gemm_f32_kernel<<<grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
     MLLM_LAUNCH_CHECK();

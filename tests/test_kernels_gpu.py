@@ -454,6 +454,21 @@ def test_linear_fp32_is_as_exact_on_tiles_as_for_few_rows(ops, K):
     assert (tiles.double() - want).norm() <= (rows.double() - want).norm()
 
 
+@pytest.mark.parametrize("N,K", [(16381, 64), (16385, 64), (16385, 68), (20001, 96), (32001, 128), (32001, 132), (16384, 96), (16384, 100), (20000, 16)])
+@pytest.mark.parametrize("M", [64, 65, 130])
+def test_linear_fp32_wide_rows_of_short_sums(ops, M, N, K):
+    """Both sides of the rules for wide results of short sums (odd rows off the tiles; the tiles' shapes): the error is at most one
+    rounding a term of the magnitudes' sum, and what stands beside the columns stays."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = _rand((M, K), torch.float32, g).to(DEV), _rand((N, K), torch.float32, g).to(DEV)
+    bias = _rand((N,), torch.float32, g).to(DEV)
+    out = torch.full((M, N + 4), 7.0, device=DEV)          # (a row stride as odd as N)
+    ops.linear(a, w, bias, out[:, :N], "store")
+    want, size = a.double() @ w.double().T + bias.double(), a.double().abs() @ w.double().abs().T + bias.double().abs()
+    assert ((out[:, :N].double() - want).abs() <= 2.0 ** -24 * (K + 2) * size).all()
+    assert (out[:, N:] == 7).all()
+
+
 @pytest.mark.parametrize("M, N, K", [(4, 8, 36), (70, 33, 44), (9, 5, 7)])
 def test_linear_bf16_takes_any_k_through_the_plain_kernel(ops, M, N, K):
     """A K that is no multiple of 8 (the matrix-core kernels read 16 bytes at a time) runs on the plain kernel."""
