@@ -380,8 +380,11 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
     // (More rows than that: the norm is a kernel of its own. Normalising in the tiled product while it stages
     // its rows was measured at 64 to 256 rows and lost: every workgroup of a row tile has to pull the tile's
     // fp32 rows through its own L1 for the statistics, 6.5 us at 64 rows of 768, more than the norm's kernel.)
+    // (Keys and values: 17 to 32 rows of more than 256 column tiles run in more than two rounds of workgroups, each normalising its rows
+    // again, and the norm and a product that writes the pages itself are shorter: a step of 17 tokens of GPT-2 XL takes 945 us so, 1,033 fused.)
+    const bool kv_fits = kv == nullptr || (aligned(w.data, 16) && (M <= 16 || w.rows <= 4096));
     if (w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
-        (beta == nullptr || aligned(beta, 16)) && (kv == nullptr || aligned(w.data, 16))) {
+        (beta == nullptr || aligned(beta, 16)) && kv_fits) {
         int rc;
         if (kv != nullptr) {
             check_scatter(*kv, w.dtype, w.rows, epilogue, "ln_linear (key/value scatter)");

@@ -258,6 +258,7 @@ def test_ln_linear_scatters_keys_and_values(ops, M, H, Hkv, dh, K):
 
 @pytest.mark.parametrize("M,H,Hkv,dh,K", [(1, 12, 12, 64, 768), (7, 12, 3, 64, 768), (16, 25, 25, 64, 1600),     # (two column tiles a workgroup)
                                           (17, 12, 12, 64, 768), (32, 5, 1, 40, 96), (33, 6, 2, 32, 200),
+                                          (17, 25, 25, 64, 1600), (32, 22, 21, 64, 256), (32, 22, 22, 64, 256),      # (both sides of 4,096 columns)
                                           (9, 3, 3, 10, 64), (40, 3, 3, 10, 64),                     # widths that are no multiple of 4
                                           (3, 2, 2, 16, 100)])                                       # K that is no multiple of 8
 def test_ln_linear_scatters_few_rows(ops, M, H, Hkv, dh, K):
