@@ -61,26 +61,39 @@ class RequestOutput:
     error: Optional[str] = None         # why a request failed
 
 
+class _Handle:
+    """A native engine's handle, destroyed with the last object that holds it. The engine and its runner both do; neither
+    holds the other for its life, so an engine that is let go without ``close`` frees its device memory at once and not
+    when the collector of cycles next runs."""
+
+    def __init__(self, lib, handle: int):
+        self._lib, self._h = lib, handle
+
+    def destroy(self) -> None:
+        h, self._h = self._h, None
+        if h:
+            self._lib.mllm_engine_destroy(h)
+
+    __del__ = destroy
+
+
 class Engine:
     def __init__(self, handle: int, options: EngineOptions):
         self._lib = native.lib()
         self._h = handle
+        self._held = _Handle(self._lib, handle)
         self.options = options
         cap = max(options.max_batch_num, 1) * 2 + 16
         self._ids = np.empty(cap, dtype=np.int64)
         self._toks = np.empty(cap, dtype=np.int32)
         self._fin = np.empty(cap, dtype=np.int32)
-        self.runner = Runner(_borrowed=self._lib.mllm_engine_runner(handle), _owner=self)
-
-    def __del__(self):
-        h, self._h = getattr(self, "_h", None), None
-        if h:
-            self._lib.mllm_engine_destroy(h)
+        self.runner = Runner(_borrowed=self._lib.mllm_engine_runner(handle), _owner=self._held)
 
     def close(self) -> None:
-        """Frees the model, the caches and the stream now (otherwise: when the object is collected)."""
+        """Frees the model, the caches and the stream now (otherwise: with the engine and every use of its runner)."""
         self.runner = None
-        self.__del__()
+        self._h = None
+        self._held.destroy()
 
     @staticmethod
     def _options(options: Optional[EngineOptions], kw) -> EngineOptions:

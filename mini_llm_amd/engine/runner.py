@@ -35,7 +35,7 @@ class Runner:
                  _borrowed: Optional[int] = None, _owner=None):
         self._lib = native.lib()
         self._box = None
-        self._owner = _owner            # keeps the engine alive while its runner is in use
+        self._owner = _owner            # keeps the native engine alive while its runner is in use
         if _borrowed is not None:
             self._h = _borrowed
         else:
