@@ -60,7 +60,7 @@ unsigned long long mllm_scratch_bytes(void) {
 }
 int mllm_release_scratch(hipStream_t stream) { return guarded([&] { release_scratch(stream); }); }
 // name: "decode_shape" (nsplit, waves; 0, 0 = automatic), "unmerged_shape", "merge_max_rows" (a), "ln_fuse_max_rows" (a), "long_context_splits" (a: 0 off, 1 on),
-// "qkv_attention", "latent_tiles", "scored_shared_kernels" (a: 0 off, 1 on), "halves_max_width" (a), "through_products" (a: 0 off, 1 on), "grouped_experts_rows" (a)
+// "latent_tiles", "scored_shared_kernels" (a: 0 off, 1 on), "halves_max_width" (a), "through_products" (a: 0 off, 1 on), "grouped_experts_rows" (a)
 int mllm_set_tuning(const char* name, int a, int b) {
     return guarded([&] {
         Tuning& t = tuning();
@@ -70,7 +70,6 @@ int mllm_set_tuning(const char* name, int a, int b) {
         else if (n == "merge_max_rows") t.merge_max_rows = a;
         else if (n == "ln_fuse_max_rows") t.ln_fuse_max_rows = a;
         else if (n == "long_context_splits") t.long_context_splits = a;
-        else if (n == "qkv_attention") t.qkv_attention = a;
         else if (n == "latent_tiles") t.latent_tiles = a;
         else if (n == "scored_shared_kernels") t.scored_shared_kernels = a;
         else if (n == "halves_max_width") t.halves_max_width = a;
@@ -84,12 +83,11 @@ int mllm_set_tuning(const char* name, int a, int b) {
 // were split over), "merge_kernel_launches", "prefill_tile_launches" (the bfloat16 matrix-core kernel), "tiled_f32_launches" (the 32-bit one),
 // "generic_attention_launches", "latent_tile_launches" and "latent_token_launches" (latent attention on the matrix cores / one
 // workgroup per token), "through_products" (products that took their result into the stream themselves), "grouped_experts"
-// (feed-forwards of routed experts run as grouped products), "qkv_attention" (attentions with the norm and the QKV product inside). -1: unknown name.
+// (feed-forwards of routed experts run as grouped products). -1: unknown name.
 long long mllm_get_seen(const char* name) {
     const Tuning::Seen& s = tuning().seen;
     const std::string n(name);
     if (n == "max_decode_splits") return s.max_decode_splits;
-    if (n == "qkv_attention") return s.qkv_attention;
     if (n == "merge_kernel_launches") return s.merge_kernel_launches;
     if (n == "prefill_tile_launches") return s.prefill_tile_launches;
     if (n == "tiled_f32_launches") return s.tiled_f32_launches;
@@ -144,11 +142,6 @@ int mllm_op_ln_linear(const Tensor2* x, const float* gamma, const float* beta, f
 // *unmerged = 1 and *splits filled when the result was left as splits (only with may_split)
 int mllm_op_paged_attention(const AttentionArgs* a, AttentionSplits* splits, int* unmerged, hipStream_t s) {
     return guarded([&] { *unmerged = paged_attention(*a, splits, s) ? 1 : 0; });
-}
-// *state = 0: no such kernel, nothing was done; 1: the result is in a->out; 2: *splits filled
-int mllm_op_ln_qkv_attention(const Tensor2* x, const float* gamma, const float* beta, float eps, const Tensor2* w, const float* bias,
-                             const AttentionArgs* a, AttentionSplits* splits, int* state, hipStream_t s) {
-    return guarded([&] { *state = !ln_qkv_attention(*x, gamma, beta, eps, *w, bias, *a, splits, s) ? 0 : splits->valid() ? 2 : 1; });
 }
 // A norm is {alpha, weight, bias} (weight null: none). copy, y, x0 and step may be null.
 int mllm_op_tanh_norm(const Tensor2* x, const MllmTanhNorm* norm, const Tensor2* out, const int* rows, hipStream_t s) {

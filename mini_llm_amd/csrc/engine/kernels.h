@@ -71,9 +71,6 @@ int mllm_decode_attention(const void* q, int q_stride, int q_col, const void* k_
                           int out_stride, float* ws, int* counters, int k_col, int v_col, const int* slots,
                           int partial_out, int dtype, hipStream_t stream, const MllmScoreShape* shape = nullptr,
                           const float* gate = nullptr, int ldg = 0);
-int mllm_ln_qkv_attention(const float* x, int ldx, const float* gamma, const float* beta, float eps, const void* w, int ldw, const float* bias,
-                          int K, void* k_pages, void* v_pages, const int* block_tables, int max_blocks, const int* positions, const int* slots,
-                          int n_q, int n_heads, int page_size, float scale, int nsplit, int keys, float* ws, void* out, int out_stride, hipStream_t stream);
 int mllm_merge_attention_splits(const float* ws, int n_q, int n_heads, int head_dim, int nsplit, void* out,
                                 int out_stride, int dtype, hipStream_t stream);
 int mllm_prefill_attention_bf16(const void* q, int q_stride, int q_col, const void* k_pages, const void* v_pages,

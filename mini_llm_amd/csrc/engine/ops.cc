@@ -99,9 +99,8 @@ void* gemm_workspace(hipStream_t s) { return scratch("gemm_workspace", GEMM_WORK
 
 void reserve_attention_scratch(int rows, int n_heads, int head_dim, hipStream_t stream) {
     if (rows < 1 || n_heads < 1 || head_dim < 1) return;
-    // (every launch shape keeps pairs x splits within max(8 x pairs, 256), and the one whose tokens' own keys are states too has one
-    // more for each of at most 32 pairs)
-    decode_partials(std::max<size_t>(static_cast<size_t>(rows) * n_heads * DECODE_MAX_SPLIT, 256 + 32) * (head_dim + 2), stream);
+    // (every launch shape keeps pairs x splits within max(8 x pairs, 256))
+    decode_partials(std::max<size_t>(static_cast<size_t>(rows) * n_heads * DECODE_MAX_SPLIT, 256) * (head_dim + 2), stream);
     decode_counters(static_cast<size_t>(rows) * n_heads, stream);
 }
 
@@ -620,54 +619,6 @@ bool paged_attention(const AttentionArgs& a, AttentionSplits* splits, hipStream_
                                        a.head_dim, a.page_size, a.scale, a.window, a.out.data, static_cast<int>(a.out.stride),
                                        a.q.dtype, stream), "paged_attention");
     return false;
-}
-
-bool ln_qkv_attention(const Tensor2& x, const float* gamma, const float* beta, float eps, const Tensor2& w, const float* bias,
-                      const AttentionArgs& a, AttentionSplits* splits, hipStream_t stream) {
-    const Tuning& t = tuning();
-    const int T = static_cast<int>(x.rows), pairs = T * a.n_heads;
-    const int64_t K = x.cols;
-    if (t.qkv_attention == 0 || t.decode_nsplit > 0 || t.unmerged_nsplit > 0) return false;
-    if (T < 1 || T != a.n_seqs || T != a.n_single || a.max_q_len != 1) return false;
-    if (!a.append || !a.may_split || splits == nullptr || a.shape != nullptr || a.gate != nullptr || a.window > 0) return false;
-    if (a.head_dim != 64 || a.n_heads < 1 || a.n_heads != a.n_kv_heads || a.slots == nullptr || a.block_tables == nullptr || a.positions == nullptr) return false;
-    if (w.dtype != BF16 || w.rows != 3ll * a.n_heads * 64 || w.cols != K || K % 64 != 0 || K > 2048 || w.stride % 8 != 0 || !aligned(w.data, 16)) return false;
-    if (x.dtype != F32 || x.stride % 4 != 0 || !aligned(x.data, 16) || gamma == nullptr || !aligned(gamma, 16) || (beta != nullptr && !aligned(beta, 16))) return false;
-    if (!pow2(a.page_size) || a.max_blocks < 1 || a.max_blocks > 4096 || !aligned(a.k_pages.data, 16) || !aligned(a.v_pages.data, 16)) return false;
-    check_pages(a.k_pages, a.v_pages, BF16, "ln_qkv_attention");
-    if (a.k_pages.cols != a.n_heads * 64 || a.k_pages.rows % a.page_size != 0) fail("ln_qkv_attention: the pages are %lld wide, %d expected", (long long)a.k_pages.cols, a.n_heads * 64);
-    if (a.out.rows != T || a.out.cols != a.n_heads * 64 || a.out.dtype != BF16) fail("ln_qkv_attention: out must be [%d, %d] bfloat16", T, a.n_heads * 64);
-    // One workgroup a compute unit (its registers leave no room for a second). From two a pair on, the pair's keys are split, over up to
-    // three of them, or, few pairs with long contexts, over all and a merge kernel. With one a pair every workgroup
-    // makes query, key and value, 3 x 128 K bytes of weights, which pays up to K = 768. A layer of a decode step with this kernel
-    // against norm, product and attention apart (us): width 768, 12 heads, 1 token at 500 keys 24.7 / 28.3, at 32,000 41.8 / 44.8; 8
-    // tokens at 20, 300 and 8,000 keys 24.0 / 27.0, 25.2 / 28.2, 58.3 / 62.4; one workgroup a pair: 16 tokens at 20, 800 and 8,000
-    // keys 26.8 / 31.2, 33.2 / 37.6, 93.8 / 97.2; width 1,024, 6 tokens at 300 keys 28.7 / 31.3 and 1,600, 4 tokens 39.6 / 42.0, but one
-    // workgroup a pair 48.3 / 48.0 (1,024, 16 tokens at 700 keys) and 52.9 / 49.6 (1,600, 10 tokens at 800). Three splits
-    // instead of two: 8.5 / 9.8 the kernel alone at 80 pairs.
-    const int most = 256 / pairs;
-    const bool spread = t.long_context_splits && std::min(most, a.max_ctx_len / 512) >= 8;
-    const int n = T > t.merge_max_rows ? 1 : spread ? std::min({most, a.max_ctx_len / 512, 63}) : std::min(most, 3);
-    if (most < 1 || (n == 1 && K > 768)) return false;
-    const int keys = (a.max_ctx_len - 1 + n - 1) / n;
-    float* ws = decode_partials(static_cast<size_t>(pairs) * (n + 1) * 66, stream);
-    check(mllm_ln_qkv_attention(static_cast<const float*>(x.data), static_cast<int>(x.stride), gamma, beta, eps, w.data, static_cast<int>(w.stride), bias,
-                                static_cast<int>(K), a.k_pages.data, a.v_pages.data, a.block_tables, a.max_blocks, a.positions, a.slots, T, a.n_heads,
-                                a.page_size, a.scale, n, keys, ws, a.out.data, static_cast<int>(a.out.stride), stream), "ln_qkv_attention");
-    tuning().seen.qkv_attention += 1;
-    tuning().seen.max_decode_splits = std::max(tuning().seen.max_decode_splits, n);
-    splits->ws = n > 1 ? ws : nullptr;
-    splits->n_tokens = T;
-    splits->n_heads = a.n_heads;
-    splits->head_dim = 64;
-    splits->nsplit = n + 1;
-    splits->dtype = BF16;
-    if (spread) {
-        tuning().seen.merge_kernel_launches += 1;
-        merge_splits(*splits, a.out, stream);
-        splits->ws = nullptr;
-    }
-    return true;
 }
 
 // ---------------------------------------------------------------------------------------------

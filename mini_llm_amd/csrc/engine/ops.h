@@ -116,7 +116,6 @@ struct Tuning {
     int unmerged_nsplit = 0, unmerged_waves = 0;      // > 0: forced shape of splits merged by the next product
     int merge_max_rows = 16;                          // tokens whose splits a product merges while loading
     int long_context_splits = 1;                      // 1: few pairs with long contexts are split over up to 256 workgroups
-    int qkv_attention = 1;                            // 1: norm, QKV product and attention of few single tokens may run as one kernel
     int ln_fuse_max_rows = 32;                        // rows up to which the norm is fused into the few-row product
     int latent_tiles = 1;                             // 1: latent attention's prompt portions may run on the matrix cores
     int scored_shared_kernels = 1;                    // 1: attention with shaped scores may run on the kernels the plain attention runs on
@@ -129,7 +128,6 @@ struct Tuning {
     // what the ops chose since the last reset (tests read it back instead of trusting the thresholds)
     struct Seen {
         int max_decode_splits = 0;                    // most workgroups a (token, head) pair's keys were split over
-        long long qkv_attention = 0;                  // attentions that made their queries, keys and values themselves
         long long merge_kernel_launches = 0, prefill_tile_launches = 0, tiled_f32_launches = 0, generic_attention_launches = 0;
         long long latent_tile_launches = 0, latent_token_launches = 0;      // latent attention: matrix-core kernel, one workgroup per token
         long long through_products = 0, grouped_experts = 0;                // products that took their result into the stream; routed experts as grouped products
@@ -176,12 +174,6 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
 // Causal attention of the step's queries over the pages. Returns true and fills *splits when the result is
 // left unmerged (only with may_split); otherwise `out` holds it.
 bool paged_attention(const AttentionArgs& a, AttentionSplits* splits, hipStream_t stream);
-// The attention of a step in which every sequence brings one token, from the rows in front of its layer norm: norm, QKV product
-// (w: queries, keys, values one behind the other) and attention in one kernel, the new keys and values written to the pages. `a` as for
-// paged_attention with append and may_split, without q and its columns. False: no such kernel for these sizes, and nothing was
-// done. True: as splits (valid()), or in a.out.
-bool ln_qkv_attention(const Tensor2& x, const float* gamma, const float* beta, float eps, const Tensor2& w, const float* bias,
-                      const AttentionArgs& a, AttentionSplits* splits, hipStream_t stream);
 
 // -- RMS norms, gated activation ---------------------------------------------------------------------
 // out[i, :] = x[rows ? rows[i] : i, :] / sqrt(mean(.^2) + eps) * weight, the columns in `groups` equal parts

@@ -159,9 +159,6 @@ public:
         ln_linear(x, gamma_, beta_, eps_, lin.weight, lin.bias, out, epilogue, rows, tmp, kv, s);
         arena.release(mark);
     }
-    bool attention(const Tensor2& x, const Linear& qkv, const AttentionArgs& a, AttentionSplits* splits, hipStream_t s) const override {
-        return x.cols == size_ && ln_qkv_attention(x, gamma_, beta_, eps_, qkv.weight, qkv.bias, a, splits, s);
-    }
     void add_scaled(const Tensor2& y, const float* scale, float mult, const Tensor2& x, bool clear, hipStream_t s,
                     const Tensor2* copy) const override {
         if (y.cols != size_) fail("layernorm: rows of %lld, the norm is %d wide", (long long)y.cols, size_);
@@ -204,7 +201,25 @@ public:
                  hipStream_t s) const override {
         if (!cache.has_pages()) fail("attention needs a cache of pages");
         const int T = step.n_tokens, g = cache.group;
+        Tensor2 qkv = arena.tensor(dtype_, T, q_dim_ + 2 * kv_dim_);
+        // Prompt portions: the QKV product is asked to put the new keys and values into the pages (how
+        // is the linear map's business). Single tokens: the attention kernel writes them.
+        // A position encoding that turns queries and keys does so on the qkv rows first: the keys are final
+        // only then, so they go to the pages afterwards (by the attention op), not from the product.
+        const bool scatter = write && step.max_q_len > 1 && !position_;
+        KvScatter kv;
+        if (scatter) {
+            kv.slots = step.slots[g];
+            kv.k_pages = cache.k_pages;
+            kv.v_pages = cache.v_pages;
+            kv.q_cols = q_dim_;
+        }
+        h.linear(qkv_, qkv, STORE, scatter ? &kv : nullptr, arena, s);
+        if (position_) position_->in_mixer(qkv, n_heads_, n_kv_heads_, head_dim_, step, s);
+        StageTimes::get().mark("qkv", s);
         AttentionArgs a;
+        a.q = qkv;
+        a.q_col = 0;
         a.n_heads = n_heads_;
         a.n_kv_heads = n_kv_heads_;
         a.head_dim = head_dim_;
@@ -223,38 +238,13 @@ public:
         a.ctx_len = step.ctx_len;
         a.max_q_len = step.max_q_len;
         a.max_ctx_len = step.max_ctx_len;
-        a.append = write ? 1 : 0;
+        a.append = (write && !scatter) ? 1 : 0;
         a.k_col = q_dim_;
         a.v_col = q_dim_ + kv_dim_;
         a.slots = step.slots[g];
         a.n_single = step.n_single;
         a.may_split = 1;
         AttentionSplits splits;
-        // Few single tokens: norm, QKV product and attention in one kernel (not where the stages are timed one by one).
-        if (write && !position_ && !StageTimes::get().enabled() && h.attention(qkv_, a, &splits, s)) {
-            if (splits.valid()) linear_from_splits(splits, out_.weight, out_.bias, x, ADD_RESIDUAL, a.out.data, s);
-            else out_(a.out, x, ADD_RESIDUAL, nullptr, s);
-            return;
-        }
-        Tensor2 qkv = arena.tensor(dtype_, T, q_dim_ + 2 * kv_dim_);
-        // Prompt portions: the QKV product is asked to put the new keys and values into the pages (how
-        // is the linear map's business). Single tokens: the attention kernel writes them.
-        // A position encoding that turns queries and keys does so on the qkv rows first: the keys are final
-        // only then, so they go to the pages afterwards (by the attention op), not from the product.
-        const bool scatter = write && step.max_q_len > 1 && !position_;
-        KvScatter kv;
-        if (scatter) {
-            kv.slots = step.slots[g];
-            kv.k_pages = cache.k_pages;
-            kv.v_pages = cache.v_pages;
-            kv.q_cols = q_dim_;
-        }
-        h.linear(qkv_, qkv, STORE, scatter ? &kv : nullptr, arena, s);
-        if (position_) position_->in_mixer(qkv, n_heads_, n_kv_heads_, head_dim_, step, s);
-        StageTimes::get().mark("qkv", s);
-        a.q = qkv;
-        a.q_col = 0;
-        a.append = (write && !scatter) ? 1 : 0;
         // (the result may come back unmerged, as the states of several workgroups per token and head:
         // the output projection takes either)
         const bool unmerged = paged_attention(a, &splits, s);

@@ -249,12 +249,6 @@ public:
         (void)x; (void)gate; (void)up; (void)limit; (void)alpha; (void)out; (void)s;
         return false;
     }
-    // The attention of single tokens from the rows in front of the norm, the norm and the QKV product inside (ops.h:
-    // ln_qkv_attention). False: no such kernel, nothing was done.
-    virtual bool attention(const Tensor2& x, const Linear& qkv, const AttentionArgs& a, AttentionSplits* splits, hipStream_t s) const {
-        (void)x; (void)qkv; (void)a; (void)splits; (void)s;
-        return false;
-    }
     // x += mult * scale * norm(y), row by row (y and x fp32 [rows, size]; scale per column or null); with
     // `clear`, y is zero afterwards; `copy` (optional) receives the new x in bfloat16. For arrangements with a norm
     // behind a sub-layer; a norm without it refuses.
@@ -288,9 +282,6 @@ public:
     // the norm inside, where it is still to be taken and the kernels allow it (see Norm::linear_gated)
     bool linear_gated(const Linear& gate, const Linear& up, float limit, float alpha, const Tensor2& out, hipStream_t s) const {
         return !have_ && norm_->linear_gated(x_, gate, up, limit, alpha, out, s);
-    }
-    bool attention(const Linear& qkv, const AttentionArgs& a, AttentionSplits* splits, hipStream_t s) const {
-        return !have_ && norm_->attention(x_, qkv, a, splits, s);
     }
     int64_t rows() const { return x_.rows; }
 

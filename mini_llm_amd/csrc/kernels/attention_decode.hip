@@ -6,10 +6,7 @@
 // the LPK partial dot products are summed with DPP shuffles, and every lane keeps the
 // running maximum, sum and its slice of the output for the keys of its lane group
 // (recurrence of /root/reference/src/kernels/prefill/flashattention.cu:129-178, in base 2).
-// Groups, wavefronts and splits are merged with the same (m, l, o) rule: within a wavefront every group is scaled to the largest
-// maximum and the sums are scattered over the lanes, between the wavefronts a thread adds one element of all (exchanging whole states
-// pairwise, twice, and scores as eight widened multiply-adds instead of four two-term ones cost 0.3 to 0.5 us more a launch: 192
-// pairs 10.8 > 10.4 us, 384 15.4 > 15.1, 96 pairs in 32 bits 8.5 > 8.0, all inside a decode step). The splits of a
+// Groups, wavefronts and splits are merged with the same (m, l, o) rule. The splits of a
 // (token, head) pair are merged either by the last workgroup to finish the pair, found through
 // an atomic counter (no workgroup ever waits for another), or, with `partial_out`, not here at
 // all: every workgroup leaves its state (maximum in base 2, sum, unnormalised output, fp32) in the
@@ -50,78 +47,6 @@ template <typename T>
 __device__ __forceinline__ uint4 load_stream16(const T* p) {
     const u32x4_nt v = __builtin_nontemporal_load(reinterpret_cast<const u32x4_nt*>(p));
     return make_uint4(v.x, v.y, v.z, v.w);
-}
-
-// A query's slice against 16 bytes of a key row: two bfloat16 products and their sum into fp32 in one instruction
-// (v_dot2_f32_bf16), or four fp32 multiply-adds.
-typedef __bf16 bf16x2_v __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ float dot_bf16x2(uint32_t a, uint32_t b, float acc) {
-    return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2_v, a), __builtin_bit_cast(bf16x2_v, b), acc, false);
-}
-template <typename T>
-__device__ __forceinline__ float dot16(const uint4& q, const uint4& k) {
-    if constexpr (sizeof(T) == 2) {
-        return dot_bf16x2(q.w, k.w, dot_bf16x2(q.z, k.z, dot_bf16x2(q.y, k.y, dot_bf16x2(q.x, k.x, 0.f))));
-    } else {
-        float a[4], b[4];
-        Vec16<float>::widen(q, a);
-        Vec16<float>::widen(k, b);
-        return fmaf(a[3], b[3], fmaf(a[2], b[2], fmaf(a[1], b[1], a[0] * b[0])));
-    }
-}
-
-// Sums o over the wavefront's groups of LPK lanes; of the N sums a lane keeps N / (64 / LPK), at least one, from number
-// group_kept<LPK, N>() on: at every step a lane hands half of what it still holds to its partner and takes the partner's share of
-// the other half, so that 8 values over 8 groups take 7 additions and 7 exchanges instead of 24 of each.
-template <int LPK, int N, int OFF = MLLM_WAVE / 2, int TOTAL = N>
-__device__ __forceinline__ void group_scatter(float (&o)[TOTAL]) {
-    if constexpr (OFF >= LPK) {
-        if constexpr (N > 1) {
-            constexpr int H = N / 2;
-#pragma unroll
-            for (int e = 0; e < H; ++e) {
-                if constexpr (OFF >= 16) {
-                    const unsigned a = __builtin_bit_cast(unsigned, o[e]), b = __builtin_bit_cast(unsigned, o[e + H]);
-                    const auto r = OFF == 32 ? __builtin_amdgcn_permlane32_swap(a, b, false, false) : __builtin_amdgcn_permlane16_swap(a, b, false, false);
-                    o[e] = __builtin_bit_cast(float, static_cast<unsigned>(r[0])) + __builtin_bit_cast(float, static_cast<unsigned>(r[1]));
-                } else {
-                    const bool high = threadIdx.x & OFF;
-                    const float given = high ? o[e] : o[e + H], kept = high ? o[e + H] : o[e];
-                    o[e] = kept + lane_xor(given, OFF);
-                }
-            }
-            group_scatter<LPK, H, OFF / 2, TOTAL>(o);
-        } else {
-            o[0] += lane_xor(o[0], OFF);
-            group_scatter<LPK, 1, OFF / 2, TOTAL>(o);
-        }
-    }
-}
-template <int LPK, int N, int OFF = MLLM_WAVE / 2>
-__device__ __forceinline__ int group_kept() {
-    if constexpr (OFF >= LPK && N > 1) return ((threadIdx.x & OFF) ? N / 2 : 0) + group_kept<LPK, N / 2, OFF / 2>();
-    else return 0;
-}
-constexpr int group_share(int lpk, int n) { return n * lpk > MLLM_WAVE ? n * lpk / MLLM_WAVE : 1; }
-
-// The states of a wavefront's lane groups (maximum, sum, slice of the output) as one, left in LDS: each is scaled to the largest
-// maximum, and what is left are plain sums.
-template <typename T, int LPK, int EPL>
-__device__ __forceinline__ void wave_state(float m, float l, float (&o)[EPL], float* sm_m, float* sm_l, float* sm_o) {
-    float mx = m;
-#pragma unroll
-    for (int off = LPK; off < MLLM_WAVE; off <<= 1) mx = fmaxf(mx, lane_xor(mx, off));
-    const float f = exp2_for<T>(m - mx);
-    l *= f;
-#pragma unroll
-    for (int off = LPK; off < MLLM_WAVE; off <<= 1) l += lane_xor(l, off);
-#pragma unroll
-    for (int e = 0; e < EPL; ++e) o[e] *= f;
-    group_scatter<LPK, EPL>(o);
-    const int lane = threadIdx.x % MLLM_WAVE, first = lane % LPK * EPL + group_kept<LPK, EPL>();
-#pragma unroll
-    for (int e = 0; e < group_share(LPK, EPL); ++e) sm_o[first + e] = o[e];
-    if (lane == 0) { *sm_m = mx; *sm_l = l; }
 }
 
 template <typename T, int N>
@@ -214,7 +139,10 @@ decode_attention_kernel(// the first 16 dwords arrive in registers with the wave
         for (int i = threadIdx.x; i < n_blk; i += blockDim.x) sm_table[i] = gtable[i];
     }
 
-    const uint4 qraw = load_raw16(q + static_cast<size_t>(t) * q_stride + q_col + h * DH + c * EPL);
+    float qf[EPL];
+    Vec16<T>::widen(load_raw16(q + static_cast<size_t>(t) * q_stride + q_col + h * DH + c * EPL), qf);
+#pragma unroll
+    for (int e = 0; e < EPL; ++e) qf[e] *= scale_log2e;
     uint4 k_own = make_uint4(0, 0, 0, 0), v_own = make_uint4(0, 0, 0, 0);
     const bool own_lanes = own_here && wave == 0 && g == 0;
     if (own_lanes) {
@@ -260,7 +188,12 @@ decode_attention_kernel(// the first 16 dwords arrive in registers with the wave
         float mx = NEG;
 #pragma unroll
         for (int u = 0; u < UNR; ++u) {
-            float d = group_sum<LPK>(dot16<T>(qraw, kraw[u])) * scale_log2e;
+            float kf[EPL];
+            Vec16<T>::widen(kraw[u], kf);
+            float d = 0.f;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) d = fmaf(qf[e], kf[e], d);
+            d = group_sum<LPK>(d);
             const bool valid = j0 + u * group_keys + g < ke_pages;
             if (SHAPED) d = mllm_shaped_score<sizeof(T) == 2>(d, shape, r1, r2, valid ? p - key_at(j0 + u * group_keys + g) : 0) * MLLM_LOG2E;
             if (SIGMOID) {
@@ -291,9 +224,13 @@ decode_attention_kernel(// the first 16 dwords arrive in registers with the wave
         m = mn;
     }
     if (own_lanes) {
-        float vf[EPL];
+        float kf[EPL], vf[EPL];
+        Vec16<T>::widen(k_own, kf);
         Vec16<T>::widen(v_own, vf);
-        float d = group_sum<LPK>(dot16<T>(qraw, k_own)) * scale_log2e;
+        float d = 0.f;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) d = fmaf(qf[e], kf[e], d);
+        d = group_sum<LPK>(d);
         if (SHAPED) d = mllm_shaped_score<sizeof(T) == 2>(d, shape, r1, r2, 0) * MLLM_LOG2E;
         const float mn = SIGMOID ? 0.f : fmaxf(m, d);
         const float a = SIGMOID ? 1.f : exp2_for<T>(m - mn);
@@ -303,37 +240,77 @@ decode_attention_kernel(// the first 16 dwords arrive in registers with the wave
         for (int e = 0; e < EPL; ++e) o[e] = o[e] * a + pj * vf[e];
         m = mn;
     }
-    // Merges the states of all lane groups and wavefronts; `done` gets every element of the result (unnormalised) with the maximum and
-    // the sum, each in a thread of its own.
-    auto block_merge = [&](auto&& done) {
-        wave_state<T, LPK, EPL>(m, l, o, &sm_m[wave], &sm_l[wave], sm_o[wave]);
+    // Merges the states of all lane groups and wavefronts; the result is valid in lane group 0
+    // of wavefront 0.
+    auto block_merge = [&]() {
+#pragma unroll
+        for (int off = LPK; off < MLLM_WAVE; off <<= 1) {
+            const float m2 = lane_xor(m, off), l2 = lane_xor(l, off);
+            float o2[EPL];
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) o2[e] = lane_xor(o[e], off);
+            merge_state<T, EPL>(m, l, o, m2, l2, o2);
+        }
+        __syncthreads();                      // earlier readers of the LDS arrays are done
+        if (g == 0) {
+            if (c == 0) { sm_m[wave] = m; sm_l[wave] = l; }
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) sm_o[wave][c * EPL + e] = o[e];
+        }
         __syncthreads();
-        for (int e = threadIdx.x; e < DH; e += blockDim.x) {
-            float mx = sm_m[0];
-            for (int w = 1; w < n_waves; ++w) mx = fmaxf(mx, sm_m[w]);
-            float sum = 0.f, v = 0.f;
-            for (int w = 0; w < n_waves; ++w) {
-                const float f = exp2_for<T>(sm_m[w] - mx);
-                sum = fmaf(f, sm_l[w], sum);
-                v = fmaf(f, sm_o[w][e], v);
+        if (wave == 0) {
+            // lane group G takes the state of wavefront G, G + KPW, ... (all reads at once), then
+            // the groups are merged as above
+            m = M0; l = 0.f;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) o[e] = 0.f;
+            for (int w = g; w < n_waves; w += KPW) {
+                float o2[EPL];
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) o2[e] = sm_o[w][c * EPL + e];
+                merge_state<T, EPL>(m, l, o, sm_m[w], sm_l[w], o2);
             }
-            done(e, mx, sum, v);
+#pragma unroll
+            for (int off = LPK; off < MLLM_WAVE; off <<= 1) {
+                const float m2 = lane_xor(m, off), l2 = lane_xor(l, off);
+                float o2[EPL];
+#pragma unroll
+                for (int e = 0; e < EPL; ++e) o2[e] = lane_xor(o[e], off);
+                merge_state<T, EPL>(m, l, o, m2, l2, o2);
+            }
         }
     };
-    auto finish = [&](int e, float, float sum, float v) {
-        float r = SIGMOID ? v : v / sum;
-        if (SHAPED && gate != nullptr) r *= 1.f / (1.f + __expf(-gate[static_cast<size_t>(t) * ldg + (shape.gate_per_head ? h : h * DH + e)]));
-        out[static_cast<size_t>(t) * out_stride + h * DH + e] = from_float<T>(r);
-    };
-    // (a split's state as it is: another kernel merges, or the last workgroup here)
-    auto leave = [&](int e, float mx, float sum, float v) {
+    block_merge();
+    T* op = out + static_cast<size_t>(t) * out_stride + h * DH + c * EPL;
+    if (partial_out) {
+        // the split's state as it is; whoever reads the workspace merges
         const size_t slot = static_cast<size_t>(pair) * nsplit + split;
-        ws_o[slot * DH + e] = v;
-        if (e == 0) { ws_ml[slot * 2] = mx; ws_ml[slot * 2 + 1] = sum; }
-    };
-    if (nsplit == 1 && !partial_out) { block_merge(finish); return; }
-    block_merge(leave);
-    if (partial_out) return;
+        if (wave == 0 && g == 0) {
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) ws_o[slot * DH + c * EPL + e] = o[e];
+            if (c == 0) { ws_ml[slot * 2] = m; ws_ml[slot * 2 + 1] = l; }
+        }
+        return;
+    }
+    if (nsplit == 1) {
+        if (wave == 0 && g == 0) {
+            const float inv = SIGMOID ? 1.f : 1.0f / l;
+#pragma unroll
+            for (int e = 0; e < EPL; ++e) {
+                float r = o[e] * inv;
+                if (SHAPED && gate != nullptr) r *= 1.f / (1.f + __expf(-gate[static_cast<size_t>(t) * ldg + (shape.gate_per_head ? h : h * DH + c * EPL + e)]));
+                op[e] = from_float<T>(r);
+            }
+        }
+        return;
+    }
+    // partial result of this split
+    const size_t slot = static_cast<size_t>(pair) * nsplit + split;
+    if (wave == 0 && g == 0) {
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) ws_o[slot * DH + c * EPL + e] = o[e];
+        if (c == 0) { ws_ml[slot * 2] = m; ws_ml[slot * 2 + 1] = l; }
+    }
     // One thread's fences order the partial results around the counter (after the barrier its
     // release covers every thread's stores); a fence in every thread would write back and
     // invalidate the L2 once per wavefront, tens of microseconds in all.
@@ -364,7 +341,16 @@ decode_attention_kernel(// the first 16 dwords arrive in registers with the wave
             merge_state<T, EPL>(m, l, o, m2, l2, o2);
         }
     }
-    block_merge(finish);
+    block_merge();
+    if (wave == 0 && g == 0) {
+        const float inv = SIGMOID ? 1.f : 1.0f / l;
+#pragma unroll
+        for (int e = 0; e < EPL; ++e) {
+            float r = o[e] * inv;
+            if (SHAPED && gate != nullptr) r *= 1.f / (1.f + __expf(-gate[static_cast<size_t>(t) * ldg + (shape.gate_per_head ? h : h * DH + c * EPL + e)]));
+            op[e] = from_float<T>(r);
+        }
+    }
     if (threadIdx.x == 0) counters[pair] = 0;     // ready for the next launch
 }
 
@@ -457,280 +443,6 @@ merge_splits_kernel(const float* __restrict__ ws_o, const float* __restrict__ ws
     for (int k = 0; k < 4; ++k) dst[k] = from_float<T>(o[k] * inv);
 }
 
-// ---------------------------------------------------------------------------------------------
-// Norm, QKV product and decode attention of few tokens in one kernel (bfloat16, heads of 64, as many key/value heads as query
-// heads, one token a sequence). At few rows the QKV product is a chain of latencies and so is the attention behind it, and between
-// the two stands the boundary of dependent kernels. Here every workgroup of a (token, head, split) makes the head's query itself: the norm
-// of the token's row, then 64 rows of the weights times it (98 KB at width 768, which the workgroups of a head share through
-// their XCD's L2), while the keys and values of its range are on their way from the pages. The new key is made by split 0, the new
-// value by split 1, and both go to the pages; nobody reads them back: the token's own key is a state of its own behind the
-// splits' (maximum = its score, sum 1, output = its value), which split 0 and split 1 leave together, and whoever merges the
-// states merges it like any other. One workgroup a pair makes all three, merges all itself and leaves the result. No workgroup waits
-// for another. Query, key and value are rounded to bfloat16 as the product of its own would leave them.
-// What bounds it is the chain launch, row, norm, product, scores, merge, and what a unit takes from its L2 (196 KB of weights and
-// 98 KB of keys and values a workgroup at 8 tokens and 768 keys). Measured in a decode step of width 768, 12 heads, against product and
-// attention as two kernels: 1 token at 130 keys 6.6 us (5.0 + 5.9), 8 tokens at 540 9.3 (5.2 + 7.6), 16 tokens of a queue 14.0 (6.1 + 10.4).
-// A wavefront owns 8 of the head's 64 columns of each product: 8 lanes share a weight row, one 128-byte line of it a load, so
-// that no sum crosses a wavefront. All of the first requests' weights are asked for behind the row and the norm's vectors, the
-// keys and values behind the weights: loads complete in that order, and each is waited for only where it is used.
-// ---------------------------------------------------------------------------------------------
-#define QKV_WAVES 8
-#define QKV_DH 64
-#define QKV_MAX_K 2048         // a thread takes four columns of the row
-
-struct QkvAttention {
-    const int* token_blocks;      // [T, max_blocks]
-    int max_blocks;
-    const int* positions;
-    int T, H, S;                  // tokens, heads, splits
-    unsigned per_s, per_t;        // 2^32 / S and 2^32 / T, rounded up: quotients of small numbers by one multiplication
-    const float* x;               // fp32 stream [T, K]
-    int ldx, K;
-    const float *gamma, *beta;
-    float eps;
-    const bf16_t* w;              // [3 H 64, K]
-    int ldw;
-    const float* bias;
-    bf16_t *k_pages, *v_pages;
-    int kv_dim, page_shift;
-    const int* slots;
-    float scale_log2e;
-    float *ws_o, *ws_ml;          // states of the splits, or
-    bf16_t* out;                  // the result
-    int out_stride;
-};
-
-struct QkvShared {
-    int table[DEC_TABLE_LDS];
-    uint4 x[QKV_MAX_K / 8 + 32];                             // the normalised row, zeros behind it
-    uint4 made[3][QKV_DH / 8];                               // query, and key and value where the workgroup makes them
-    float m[QKV_WAVES + 1], l[QKV_WAVES + 1], o[QKV_WAVES + 1][QKV_DH];
-    float sum[QKV_WAVES], sq[QKV_WAVES];
-};
-
-// CB: 128-byte lines of a weight row in one request, of which two are under way (TWO: they hold the whole row). UNR: groups of 64 keys
-// whose loads are in flight together. MATS: 1 the query, 2 and a key (split 0) or a value (split 1), 3 all three, and with them the
-// whole attention.
-template <int CB, bool TWO, int UNR, int MATS>
-__device__ __forceinline__ void qkv_attention_body(const QkvAttention& a, int t, int h, int split, QkvShared& sm) {
-    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
-    const int c = lane % 8, g = lane / 8;
-    const int K = a.K, nq = K / 4;
-    const int* table = a.token_blocks + static_cast<size_t>(t) * a.max_blocks;
-    // requested first: the table (every key's address hangs on it), the thread's own four columns of the row, the norm's vectors
-    const int tab = table[min(tid, a.max_blocks - 1)];
-    const int p = a.positions[t];
-    const int own = min(tid, nq - 1);
-    const float4 xt = reinterpret_cast<const float4*>(a.x + static_cast<size_t>(t) * a.ldx)[own], gt = reinterpret_cast<const float4*>(a.gamma)[own];
-    float4 bt = reinterpret_cast<const float4*>(a.beta != nullptr ? a.beta : a.gamma)[own];
-    if (a.beta == nullptr) bt = make_float4(0.f, 0.f, 0.f, 0.f);
-    __builtin_amdgcn_sched_barrier(0);
-    const int q_dim = a.H * QKV_DH, row = h * QKV_DH + wave * 8 + g;
-    const bf16_t* w[MATS];
-    float bias[MATS];
-#pragma unroll
-    for (int m = 0; m < MATS; ++m) {
-        const int r = row + (MATS == 2 && m == 1 && split == 1 ? 2 : m) * q_dim;
-        w[m] = a.w + static_cast<size_t>(r) * a.ldw;
-        bias[m] = a.bias != nullptr ? a.bias[r] : 0.f;
-    }
-    uint4 w0[MATS][CB], w1[MATS][CB];
-    auto load_weights = [&](uint4 (&wr)[MATS][CB], int chunk) {
-#pragma unroll
-        for (int i = 0; i < CB; ++i) {
-            const int k = min((chunk * CB + i) * 64, K - 64) + 8 * c;       // (lines beyond the row: its last one, against zeros)
-#pragma unroll
-            for (int m = 0; m < MATS; ++m) wr[m][i] = load_raw16(w[m] + k);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    load_weights(w0, 0);
-    load_weights(w1, 1);
-    if (tid < a.max_blocks) sm.table[tid] = tab;
-    for (int i = tid + 64 * QKV_WAVES; i < a.max_blocks; i += 64 * QKV_WAVES) sm.table[i] = table[i];
-    // the norm: the mean first, then the variance of the centred values
-    const float s = wave_sum(tid < nq ? (xt.x + xt.y) + (xt.z + xt.w) : 0.f);
-    if (lane == 0) sm.sum[wave] = s;
-    lds_barrier();
-
-    // the split's keys: those in the pages, positions 0 to p - 1
-    const int per = MATS == 3 ? p : (p + a.S - 1) / a.S, kb = split * per, ke = min(p, kb + per);
-    const size_t col = static_cast<size_t>(h) * QKV_DH + 8 * c;
-    const int mask = (1 << a.page_shift) - 1;
-    uint4 kraw[UNR], vraw[UNR];
-    auto load_keys = [&](int j0) {
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-            // (beyond the range: its last key again, masked when used; without a key before the token: the token's own row, dropped)
-            const int j = max(min(j0 + 64 * u + g, ke - 1), 0);
-            const size_t r = (static_cast<size_t>(sm.table[j >> a.page_shift]) << a.page_shift) + (j & mask);
-            kraw[u] = load_stream16(a.k_pages + r * a.kv_dim + col);
-            vraw[u] = load_stream16(a.v_pages + r * a.kv_dim + col);
-        }
-        __builtin_amdgcn_sched_barrier(0);
-    };
-    load_keys(kb + 8 * wave);
-
-    float mean = 0.f, var = 0.f;
-#pragma unroll
-    for (int i = 0; i < QKV_WAVES; ++i) mean += sm.sum[i];
-    mean /= static_cast<float>(K);
-    const float d0 = xt.x - mean, d1 = xt.y - mean, d2 = xt.z - mean, d3 = xt.w - mean;
-    const float q2 = wave_sum(tid < nq ? (d0 * d0 + d1 * d1) + (d2 * d2 + d3 * d3) : 0.f);
-    if (lane == 0) sm.sq[wave] = q2;
-    lds_barrier();
-#pragma unroll
-    for (int i = 0; i < QKV_WAVES; ++i) var += sm.sq[i];
-    const float inv = 1.0f / sqrtf(var / static_cast<float>(K) + a.eps);
-    {
-        uint2 pk = make_uint2(0, 0);           // (zeros behind the row, as far as whole requests of its weights reach)
-        if (tid < nq) {
-            pk.x = pack_bf16x2(d0 * inv * gt.x + bt.x, d1 * inv * gt.y + bt.y);
-            pk.y = pack_bf16x2(d2 * inv * gt.z + bt.z, d3 * inv * gt.w + bt.w);
-        }
-        reinterpret_cast<uint2*>(sm.x)[tid] = pk;
-        static_assert(64 * QKV_WAVES * 4 == QKV_MAX_K && (TWO ? 2 * CB : CB + 31) * 8 <= QKV_MAX_K / 8 + 32, "whole requests stay inside the row and its zeros");
-        if (!TWO && tid < 64) reinterpret_cast<uint2*>(sm.x)[QKV_MAX_K / 4 + tid] = make_uint2(0, 0);
-    }
-    lds_barrier();
-    float acc[MATS][2];
-#pragma unroll
-    for (int m = 0; m < MATS; ++m) acc[m][0] = acc[m][1] = 0.f;
-    auto use_weights = [&](const uint4 (&wr)[MATS][CB], int chunk) {
-#pragma unroll
-        for (int i = 0; i < CB; ++i) {
-            const uint4 xv = sm.x[(chunk * CB + i) * 8 + c];
-#pragma unroll
-            for (int m = 0; m < MATS; ++m) {
-                acc[m][0] = dot_bf16x2(wr[m][i].x, xv.x, acc[m][0]);
-                acc[m][1] = dot_bf16x2(wr[m][i].y, xv.y, acc[m][1]);
-                acc[m][0] = dot_bf16x2(wr[m][i].z, xv.z, acc[m][0]);
-                acc[m][1] = dot_bf16x2(wr[m][i].w, xv.w, acc[m][1]);
-            }
-        }
-    };
-    if constexpr (TWO) {
-        use_weights(w0, 0);
-        use_weights(w1, 1);
-    } else {
-        const int chunks = (K / 64 + CB - 1) / CB;
-        for (int i = 0; i < chunks; i += 2) {
-            // (past the end: the row's last line, long since arrived)
-            use_weights(w0, i);
-            load_weights(w0, i + 2);
-            if (i + 1 < chunks) use_weights(w1, i + 1);
-            load_weights(w1, i + 3);
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < MATS; ++m) {
-        const float v = group_sum<8>(acc[m][0] + acc[m][1]) + bias[m];
-        if (c == 0) reinterpret_cast<bf16_t*>(sm.made[m])[wave * 8 + g] = float_to_bf16(v);
-    }
-    lds_barrier();
-
-    const size_t pair = static_cast<size_t>(t) * a.H + h;
-    const int states = a.S + 1;
-    if (MATS > 1 && wave == 0) {
-        // the token's own key and value: to the pages, and as a state of their own
-        const int slot = a.slots[t];
-        const bf16_t mine = reinterpret_cast<const bf16_t*>(sm.made[1])[lane], mine_v = reinterpret_cast<const bf16_t*>(sm.made[MATS - 1])[lane];
-        const size_t at = static_cast<size_t>(slot) * a.kv_dim + h * QKV_DH + lane, own_state = pair * states + a.S;
-        if (slot >= 0 && split == 0) a.k_pages[at] = mine;
-        if (slot >= 0 && (MATS == 3 || split == 1)) a.v_pages[at] = mine_v;
-        if (split == 0) {
-            const float d = wave_sum(bf16_to_float(reinterpret_cast<const bf16_t*>(sm.made[0])[lane]) * bf16_to_float(mine)) * a.scale_log2e;
-            if (lane == 0) {
-                if (MATS == 3) { sm.m[QKV_WAVES] = d; sm.l[QKV_WAVES] = 1.f; }
-                else *reinterpret_cast<float2*>(a.ws_ml + own_state * 2) = make_float2(d, 1.f);
-            }
-        }
-        if (MATS == 3) sm.o[QKV_WAVES][lane] = bf16_to_float(mine_v);
-        else if (split == 1) a.ws_o[own_state * QKV_DH + lane] = bf16_to_float(mine_v);
-    }
-    const uint4 qraw = sm.made[0][c];
-    constexpr float NEG = -1.0e30f;
-    float m = NEG, l = 0.f, o[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) o[e] = 0.f;
-    for (int j0 = kb + 8 * wave, first = kb;;) {
-        float dot[UNR], mx = NEG;
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-            const float d = group_sum<8>(dot16<bf16_t>(qraw, kraw[u])) * a.scale_log2e;
-            dot[u] = j0 + 64 * u + g < ke ? d : NEG;
-            mx = fmaxf(mx, dot[u]);
-        }
-        const float mn = fmaxf(m, mx), f = fast_exp2(m - mn);
-        l *= f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] *= f;
-#pragma unroll
-        for (int u = 0; u < UNR; ++u) {
-            const float pj = dot[u] > NEG ? fast_exp2(dot[u] - mn) : 0.f;
-            float vf[8];
-            Vec16<bf16_t>::widen(vraw[u], vf);
-            l += pj;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) o[e] = fmaf(pj, vf[e], o[e]);
-        }
-        m = mn;
-        first += 64 * UNR;
-        if (first >= ke) break;
-        j0 += 64 * UNR;
-        load_keys(j0);
-    }
-    if (ke <= kb) {              // no keys: whatever was loaded is dropped
-        m = NEG; l = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) o[e] = 0.f;
-    }
-    wave_state<bf16_t, 8, 8>(m, l, o, &sm.m[wave], &sm.l[wave], sm.o[wave]);
-    lds_barrier();
-    if (wave != 0) return;
-    constexpr int N = MATS == 3 ? QKV_WAVES + 1 : QKV_WAVES;
-    float mx = sm.m[0];
-#pragma unroll
-    for (int i = 1; i < N; ++i) mx = fmaxf(mx, sm.m[i]);
-    l = 0.f;
-    float v = 0.f;
-#pragma unroll
-    for (int i = 0; i < N; ++i) {
-        const float f = fast_exp2(sm.m[i] - mx);
-        l = fmaf(f, sm.l[i], l);
-        v = fmaf(f, sm.o[i][lane], v);
-    }
-    if (MATS == 3) {
-        a.out[static_cast<size_t>(t) * a.out_stride + h * QKV_DH + lane] = float_to_bf16(v / l);
-    } else {
-        const size_t state = pair * states + split;
-        a.ws_o[state * QKV_DH + lane] = v;
-        if (lane == 0) *reinterpret_cast<float2*>(a.ws_ml + state * 2) = make_float2(mx, l);
-    }
-}
-
-template <int CB, bool TWO, int UNR, bool ALL>
-__global__ void __launch_bounds__(64 * QKV_WAVES)
-qkv_attention_kernel(QkvAttention a) {
-    __shared__ QkvShared sm;
-    // workgroups of one head on one XCD, as far as the counts allow: they share the head's weights
-    const unsigned per_xcd = gridDim.x / 8, i = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if (i >= static_cast<unsigned>(a.T * a.H * a.S)) return;
-    const int pair = a.S == 1 ? i : __umulhi(i, a.per_s), split = i - pair * a.S;
-    const int h = a.T == 1 ? pair : __umulhi(static_cast<unsigned>(pair), a.per_t), t = pair - h * a.T;
-    if constexpr (ALL) qkv_attention_body<CB, TWO, UNR, 3>(a, t, h, 0, sm);
-    else if (split < 2) qkv_attention_body<CB, TWO, UNR, 2>(a, t, h, split, sm);
-    else qkv_attention_body<CB, TWO, UNR, 1>(a, t, h, split, sm);
-}
-
-template <int CB, bool TWO, bool ALL>
-static void launch_qkv_attention(const QkvAttention& a, int groups, int keys, hipStream_t stream) {
-    if (keys <= 128) qkv_attention_kernel<CB, TWO, 2, ALL><<<groups, 64 * QKV_WAVES, 0, stream>>>(a);
-    else if (keys <= 256) qkv_attention_kernel<CB, TWO, 4, ALL><<<groups, 64 * QKV_WAVES, 0, stream>>>(a);
-    else if (keys <= 384) qkv_attention_kernel<CB, TWO, 6, ALL><<<groups, 64 * QKV_WAVES, 0, stream>>>(a);
-    else qkv_attention_kernel<CB, TWO, 8, ALL><<<groups, 64 * QKV_WAVES, 0, stream>>>(a);
-}
-
 extern "C" {
 
 // out[t, h * head_dim + e] from the states of `partial_out` (head_dim % 4 == 0).
@@ -797,46 +509,6 @@ int mllm_decode_attention(const void* q, int q_stride, int q_col, const void* k_
                                    n_heads, n_kv_heads, page_size, sl2, window, nsplit, (bf16_t*)out, out_stride,
                                    ws_o, ws_ml, counters, (bf16_t*)k_pages, (bf16_t*)v_pages, k_col, v_col, slots, partial_out, shape, gate, ldg);
     if (rc != 0) return rc;
-    MLLM_LAUNCH_CHECK();
-    return 0;
-}
-
-// Layer norm of the fp32 rows x [n_q, K], QKV product and decode attention over the pages in one kernel: n_q sequences that bring one
-// token each (row t of block_tables is token t's), heads of 64, as many key/value heads as query heads, w [3 n_heads 64, K] with
-// queries, keys and values one behind the other. The new keys and values go to rows slots[t] (>= 0) of the pages. nsplit 1: the result
-// goes to out (bfloat16). More: the states are left in ws as mllm_decode_attention's partial_out leaves them, nsplit + 1 of them a
-// pair, the last the token's own. keys: the most keys any split has. Returns 0, a HIP error code, or -1 for sizes the kernel
-// refuses: K must be a multiple of 64 up to 2,048 (nsplit 1: 768), ldw of 8, ldx of 4, page_size a power of two, max_blocks at most 4,096, all pairs' splits
-// at most 16,384 (operands 16-byte aligned).
-int mllm_ln_qkv_attention(const float* x, int ldx, const float* gamma, const float* beta, float eps, const void* w, int ldw, const float* bias,
-                          int K, void* k_pages, void* v_pages, const int* block_tables, int max_blocks, const int* positions, const int* slots,
-                          int n_q, int n_heads, int page_size, float scale, int nsplit, int keys, float* ws, void* out, int out_stride,
-                          hipStream_t stream) {
-    if (n_q <= 0) return 0;
-    if (K < 64 || K % 64 != 0 || K > (nsplit == 1 ? 768 : QKV_MAX_K) || ldw % 8 != 0 || ldx % 4 != 0 || n_heads < 1 || nsplit < 1 || max_blocks < 1 || max_blocks > DEC_TABLE_LDS) return -1;
-    if (page_size < 1 || (page_size & (page_size - 1)) != 0 || static_cast<long>(n_q) * n_heads * nsplit > 1 << 14) return -1;
-    QkvAttention a;
-    a.token_blocks = block_tables; a.max_blocks = max_blocks; a.positions = positions;
-    a.T = n_q; a.H = n_heads; a.S = nsplit;
-    // (exact below 2^16: the error of i ceil(2^32 / d) / 2^32 is less than i / 2^32, and i / d is 1 / d short of the next whole number)
-    a.per_s = static_cast<unsigned>(((1ull << 32) + nsplit - 1) / nsplit);
-    a.per_t = static_cast<unsigned>(((1ull << 32) + n_q - 1) / n_q);
-    a.x = x; a.ldx = ldx; a.K = K; a.gamma = gamma; a.beta = beta; a.eps = eps;
-    a.w = static_cast<const bf16_t*>(w); a.ldw = ldw; a.bias = bias;
-    a.k_pages = static_cast<bf16_t*>(k_pages); a.v_pages = static_cast<bf16_t*>(v_pages);
-    a.kv_dim = n_heads * QKV_DH; a.page_shift = __builtin_ctz(page_size); a.slots = slots;
-    a.scale_log2e = scale * MLLM_LOG2E;
-    a.ws_o = ws;
-    a.ws_ml = ws + static_cast<size_t>(n_q) * n_heads * (nsplit + 1) * QKV_DH;
-    a.out = static_cast<bf16_t*>(out); a.out_stride = out_stride;
-    const int groups = (n_q * n_heads * nsplit + 7) / 8 * 8;
-    if (nsplit == 1) {
-        launch_qkv_attention<6, true, true>(a, groups, keys, stream);
-    } else {
-        if (K <= 768) launch_qkv_attention<6, true, false>(a, groups, keys, stream);
-        else if (K <= 1024) launch_qkv_attention<8, true, false>(a, groups, keys, stream);
-        else launch_qkv_attention<5, false, false>(a, groups, keys, stream);
-    }
     MLLM_LAUNCH_CHECK();
     return 0;
 }

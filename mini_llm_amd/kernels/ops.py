@@ -82,8 +82,6 @@ def engine_library():
         "mllm_op_ln_linear": (_i, [T2p, _vp, _vp, _f, T2p, _vp, T2p, _i, _vp, _vp, _vp, _vp]),
         "mllm_op_paged_attention": (_i, [ctypes.POINTER(AttentionArgsC), ctypes.POINTER(AttentionSplitsC),
                                          ctypes.POINTER(_i), _vp]),
-        "mllm_op_ln_qkv_attention": (_i, [T2p, _vp, _vp, _f, T2p, _vp, ctypes.POINTER(AttentionArgsC), ctypes.POINTER(AttentionSplitsC),
-                                          ctypes.POINTER(_i), _vp]),
         "mllm_op_tanh_norm": (_i, [T2p, ctypes.POINTER(TanhNormC), T2p, _vp, _vp]),
         "mllm_op_stream_add": (_i, [T2p, T2p, T2p, _vp, T2p, ctypes.POINTER(TanhNormC), ctypes.POINTER(TanhNormC), _i, _vp]),
         "mllm_op_linear_stream_add": (_i, [T2p, T2p, _vp, T2p, T2p, T2p, ctypes.POINTER(TanhNormC), ctypes.POINTER(TanhNormC), _vp]),
@@ -194,11 +192,6 @@ def set_scored_shared_kernels(on: bool) -> None:
     """Whether attention with shaped scores may run on the kernels that plain attention runs on (default: on);
     off: every row goes through the one-wavefront-per-row kernel that takes any sizes."""
     _ok(engine_library().mllm_set_tuning(b"scored_shared_kernels", 1 if on else 0, 0))
-
-
-def set_qkv_attention(on: bool) -> None:
-    """Whether norm, QKV product and attention of few single tokens may run as one kernel (default: on)."""
-    _ok(engine_library().mllm_set_tuning(b"qkv_attention", 1 if on else 0, 0))
 
 
 def set_through_products(on: bool) -> None:
@@ -515,35 +508,6 @@ def paged_attention(q: torch.Tensor, q_col: int, n_heads: int, n_kv_heads: int, 
     if unmerged.value:
         return AttentionSplits(splits, q.device)
     return out
-
-
-def ln_qkv_attention(x: torch.Tensor, gamma: torch.Tensor, beta: Optional[torch.Tensor], eps: float, w: torch.Tensor, bias: Optional[torch.Tensor],
-                     n_heads: int, k_pages: torch.Tensor, v_pages: torch.Tensor, page_size: int, block_tables: torch.Tensor,
-                     positions: torch.Tensor, slots: torch.Tensor, max_ctx_len: int, scale: float, out: torch.Tensor):
-    """Layer norm of the fp32 rows ``x``, QKV product and attention of one new token per sequence (token t is row t of the block
-    tables) in one kernel, the new keys and values written to rows ``slots`` of the pages. None: no such kernel for these sizes, and
-    nothing was done; otherwise an ``AttentionSplits`` or ``out``."""
-    _gpu(x, gamma, beta, w, bias, k_pages, v_pages, block_tables, positions, slots, out)
-    T = x.shape[0]
-    if block_tables.dim() != 2 or block_tables.dtype != torch.int32 or not block_tables.is_contiguous() or block_tables.shape[0] != T:
-        raise KernelError("block_tables must be contiguous int32 [T, max_blocks]")
-    _i32(positions, "positions", T)
-    _i32(slots, "slots", T)
-    _f32vec(gamma, "gamma", x.shape[1])
-    _f32vec(beta, "beta", x.shape[1])
-    _f32vec(bias, "bias", w.shape[0])
-    a = AttentionArgsC()
-    a.n_heads = a.n_kv_heads = int(n_heads)
-    a.head_dim = out.shape[1] // int(n_heads)
-    a.k_pages, a.v_pages, a.page_size = t2(k_pages, "k_pages"), t2(v_pages, "v_pages"), int(page_size)
-    a.block_tables, a.n_seqs, a.max_blocks, a.n_single = block_tables.data_ptr(), T, block_tables.shape[1], T
-    a.positions, a.slots, a.scale, a.out = positions.data_ptr(), slots.data_ptr(), float(scale), t2(out, "out")
-    a.max_q_len, a.max_ctx_len, a.append, a.may_split = 1, int(max_ctx_len), 1, 1
-    push_tuning()
-    splits, state = AttentionSplitsC(), _i(0)
-    _ok(engine_library().mllm_op_ln_qkv_attention(ctypes.byref(t2(x, "x")), _p(gamma), _p(beta), float(eps), ctypes.byref(t2(w, "w")), _p(bias),
-                                                  ctypes.byref(a), ctypes.byref(splits), ctypes.byref(state), _stream()))
-    return None if state.value == 0 else out if state.value == 1 else AttentionSplits(splits, x.device)
 
 
 def argmax(logits: torch.Tensor, out: torch.Tensor) -> torch.Tensor:

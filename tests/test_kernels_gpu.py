@@ -1068,75 +1068,3 @@ def test_sample_frequencies_follow_softmax(ops):
     freq = torch.bincount(out.cpu().long(), minlength=4).double() / 4096
     p = torch.softmax(logits[0].double() / 0.8, 0)
     assert (freq - p).abs().max() < 4 * math.sqrt(0.25 / 4096)
-
-
-@pytest.mark.parametrize("lens", [(1,), (2, 1, 3), (17, 64, 65, 100), (129, 130, 5, 257, 256, 1, 400, 77), (700, 1000, 1024, 513, 1, 90), (8200,), (5000, 1)])
-@pytest.mark.parametrize("H,K,page,beta", [(12, 768, 16, True), (16, 1024, 4, True), (2, 64, 32, False), (3, 832, 16, True), (25, 1600, 16, True), (32, 2048, 8, False)])
-def test_ln_qkv_attention(ops, lens, H, K, page, beta):
-    """Norm, QKV product and attention of single tokens in one kernel: the result and what it leaves in the pages, against the same
-    with 64-bit sums. A key or value that is written or read is a bfloat16 (half a unit: 2^-9 of it), the normalised row that the weights
-    meet too, so the scores differ by about 2^-9 |q| |k| / sqrt(64) and the result by 2^-8 of the values: 1.6e-2 as for the other ops."""
-    g = torch.Generator().manual_seed(sum(lens) + H)
-    T, D = len(lens), H * 64
-    blocks = [(n + page - 1) // page for n in lens]
-    n_pages = sum(blocks) + 3
-    order = torch.randperm(n_pages, generator=g)
-    table = torch.zeros(T, max(blocks) + 1, dtype=torch.int32)
-    at = 0
-    for t, b in enumerate(blocks):
-        table[t, :b] = order[at:at + b].to(torch.int32)
-        at += b
-    x = _rand((T, K), torch.float32, g, 2.0)
-    gamma, bt = _rand((K,), torch.float32, g) * 0.1 + 1.0, _rand((K,), torch.float32, g, 0.1)
-    w, bias = _rand((3 * D, K), torch.bfloat16, g, K ** -0.5), _rand((3 * D,), torch.float32, g, 0.3)
-    kp, vp = (_rand((n_pages * page, D), torch.bfloat16, g) for _ in range(2))
-    slots = torch.tensor([int(table[t, (n - 1) // page]) * page + (n - 1) % page for t, n in enumerate(lens)], dtype=torch.int32)
-    kp[slots.long()] = float("nan")            # the tokens' own rows hold nothing yet
-    vp[slots.long()] = float("nan")
-    h = torch.nn.functional.layer_norm(x.double(), (K,), gamma.double(), bt.double() if beta else None, 1e-5).bfloat16().double()
-    q, k, v = ((h @ w.double().T + bias.double()).reshape(T, 3, H, 64)[:, i] for i in range(3))
-    k, v = k.bfloat16().double(), v.bfloat16().double()
-    want = torch.empty(T, H, 64, dtype=torch.double)
-    for t, n in enumerate(lens):
-        rows = (table[t, :blocks[t]].long()[:, None] * page + torch.arange(page)).reshape(-1)[:n - 1]
-        ks = torch.cat([kp[rows].double().reshape(-1, H, 64), k[t:t + 1]])
-        vs = torch.cat([vp[rows].double().reshape(-1, H, 64), v[t:t + 1]])
-        p = torch.softmax((q[t][None] * ks).sum(-1) * 0.125, 0)
-        want[t] = (p[..., None] * vs).sum(0)
-    dev = lambda a: a.to(DEV)
-    kd, vd, out = dev(kp), dev(vp), torch.empty(T, D, dtype=torch.bfloat16, device=DEV)
-    ops.reset_seen()
-    got = ops.ln_qkv_attention(dev(x), dev(gamma), dev(bt) if beta else None, 1e-5, dev(w), dev(bias), H, kd, vd, page, dev(table), dev(torch.tensor(lens, dtype=torch.int32) - 1),
-                               dev(slots), max(lens), 0.125, out)
-    if K > 768 and 256 // (T * H) == 1:
-        assert got is None
-        return
-    assert isinstance(got, ops.AttentionSplits) == (1 < min(256 // (T * H), max(max(lens) // 512, 3)) < 8)
-    assert ops.seen("qkv_attention") == 1 and ops.seen("merge_kernel_launches") == (1 if min(256 // (T * H), max(lens) // 512) >= 8 else 0)
-    result = (got.tensor() if isinstance(got, ops.AttentionSplits) else got).cpu().double().reshape(T, H, 64)
-    assert (result - want).abs().max() < _tol(torch.bfloat16)
-    for pages, before, new in ((kd, kp, k), (vd, vp, v)):
-        pages = pages.cpu()
-        assert (pages[slots.long()].double() - new.reshape(T, D)).abs().max() < 2.0 ** -7 * new.abs().max()
-        others = torch.ones(n_pages * page, dtype=torch.bool)
-        others[slots.long()] = False
-        assert torch.equal(pages[others], before[others])
-
-
-def test_ln_qkv_attention_leaves_other_steps_alone(ops):
-    """Heads, widths and pages that the kernel does not take are refused before anything is written."""
-    def call(H=2, dh=64, K=128, page=16, dtype=torch.bfloat16):
-        D, z = H * dh, lambda *s, dtype=torch.float32: torch.zeros(*s, dtype=dtype, device=DEV)
-        kp = torch.ones(4 * page, D, dtype=dtype, device=DEV)
-        got = ops.ln_qkv_attention(z(1, K), z(K) + 1, None, 1e-5, z(3 * D, K, dtype=dtype), None, H, kp, kp.clone(), page, z(1, 4, dtype=torch.int32),
-                                   z(1, dtype=torch.int32), z(1, dtype=torch.int32), 1, 0.125, z(1, D, dtype=dtype))
-        assert got is not None or bool((kp == 1).all())
-        return got
-    assert call() is not None
-    for other in (dict(dh=32), dict(K=96), dict(K=2112), dict(page=12), dict(dtype=torch.float32)):
-        assert call(**other) is None, other
-    try:
-        ops.set_qkv_attention(False)
-        assert call() is None
-    finally:
-        ops.set_qkv_attention(True)
