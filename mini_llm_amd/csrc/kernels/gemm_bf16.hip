@@ -19,15 +19,16 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 #define N_XCD 8       // accelerator dies of an MI355X, each with its own L2
 
 // ---------------------------------------------------------------------------------------------
-// Many rows (prefill): WM x WN wavefronts, each TM x TN MFMA tiles of 32x32. LDS is double
-// buffered (one barrier per k tile), global loads run DEPTH-1 tiles ahead in rotating register
-// sets, per-thread pointers only advance, and a K that is a multiple of the k tile takes a k loop
-// without checks, chosen at compile time (rows and columns beyond the matrices cost nothing there). Within a tile the memory instructions are spread between
-// the MFMA groups of its k steps, so that the matrix units work while they queue. For a long K
-// two such groups of wavefronts share a workgroup's tile, each on half of a twice as wide k tile,
-// and add their sums in LDS. The weight
-// fragment is the MFMA's A operand, so a lane's accumulator registers hold 4 consecutive columns
-// of one output row; the epilogue turns that, through LDS, into stores of whole rows.
+// Many rows (prefill): WM x WN wavefronts, each TM x TN MFMA tiles of 32x32. A k tile of both matrices lies in one of STAGES stages of
+// LDS, which loads fill without passing through registers (STAGES - 1 tiles ahead; one barrier a k tile); what an LDS read needs to be free of
+// bank conflicts is in the choice of the piece a lane asks for. For a long K two such groups of wavefronts may share a workgroup's
+// tile, each on half of a twice as wide k tile. The weight fragment is the MFMA's A operand, so a lane's accumulator registers hold 4
+// consecutive columns of one output row; the epilogue turns that, through LDS, into stores of whole rows.
+// Bound by the rate at which a compute unit takes tiles from its L2 and by what the matrix units wait around the barriers: at 2,048 x
+// 2,304 x 3,072 the products alone take 24.8 us, the loads alone 25.6, both 31.4. (With tiles loaded into registers and written to LDS from there,
+// at 78 bytes a clock, 40.3: 13 such instructions' time a k tile of 128x192. us, weights and rows cold, before / now: 2,048 x 2,304 x
+// 768 17.8 / 15.6 and x 3,072 x 768 18.2 / 16.6 in a step; alone 2,048 x 4,800 x 1,600 46.8 / 39.0, 2,048 x 6,400 x 1,600 58.4 / 48.0,
+// 2,048 x 1,600 x 6,400 60.0 / 45.4, 560 x 3,072 x 768 8.1 / 6.8, 256 x 3,072 x 768 6.5 / 5.2.)
 // ---------------------------------------------------------------------------------------------
 // Optional second destination of a plain bf16 store: columns [q_cols, q_cols + kv_dim) of output row
 // m also go to row slots[m] of the key pages and the next kv_dim columns to the value pages (the
@@ -93,12 +94,16 @@ __device__ __forceinline__ void through4(float* x, size_t idx, int n, const floa
 }
 
 template <int MODE>
+__device__ __forceinline__ float activated(float v) {
+    return MODE == EPI_GELU_TANH ? gelu_tanh(v) : MODE == EPI_GELU_ERF ? gelu_erf(v) : MODE == EPI_RELU2 ? relu2(v) : v;
+}
+template <int MODE>
 __device__ __forceinline__ void store4(void* C, size_t idx, const float (&v)[4], bool vec, int n_left) {
     // v: 4 consecutive columns of one row, bias already added; n_left: columns that exist (1..4)
     float o[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e)
-        o[e] = MODE == EPI_GELU_TANH ? gelu_tanh(v[e]) : MODE == EPI_GELU_ERF ? gelu_erf(v[e]) : MODE == EPI_RELU2 ? relu2(v[e]) : v[e];
+        o[e] = activated<MODE>(v[e]);
     if (MODE == EPI_ADD_RESIDUAL || MODE == EPI_STORE_F32) {
         float* c = static_cast<float*>(C) + idx;
         if (vec && n_left >= 4) {
@@ -124,37 +129,55 @@ __device__ __forceinline__ void store4(void* C, size_t idx, const float (&v)[4],
     }
 }
 
-template <int WM, int WN, int TM, int TN, int BKP, int DEPTH, bool EDGE, int MODE, int KG = 1>
+// One piece of a wavefront's loads straight into LDS: every lane's 16 bytes at base + offset go to lane-linear places from `lds` on. In
+// assembly, because a load into LDS that the compiler knows of makes it wait for all of them in front of the next LDS read:
+// whoever calls this waits (wait_loads) and passes a barrier before the bytes are read. It has no result register.
+__device__ __forceinline__ void load_to_lds(const unsigned char* base, unsigned offset, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(offset), "s"(base) : "memory");
+}
+// Waits until at most N of the wavefront's loads are under way (they end in their order) and its LDS reads are done, then for the others.
+template <int N>
+__device__ __forceinline__ void wait_loads_and_meet() {
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
+}
+
+template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG, bool HALVES, bool EDGE, int MODE>
 __global__ void __launch_bounds__(WM * WN * KG * 64)
 gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
                const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K,
                int tiles_m, int tiles_n, int xm, int xn, typename TiledExtra<MODE>::type kv) {
     // EPI_GATED: of a wavefront's TN column sub-tiles the even ones are the gate's and the odd ones the same 32 columns of the up
     // map, so that both values of an output lie in one register of one lane; N and the tile's columns count outputs.
-    constexpr bool GATED = MODE == EPI_GATED;
+    constexpr bool GATED = MODE == EPI_GATED, F32_OUT = MODE == EPI_ADD_RESIDUAL || MODE == EPI_STORE_F32 || MODE == EPI_THROUGH;
     static_assert(!GATED || TN % 2 == 0, "a wavefront holds whole pairs of sub-tiles");
     constexpr int PAIR = GATED ? 2 : 1;
-    // KG groups of WM x WN wavefronts share the tile: a k tile is KG * BKP wide and group g multiplies
-    // its g-th part, so a barrier interval covers KG times the depth; the groups' sums meet in LDS.
-    constexpr int NT = WM * WN * KG * 64;
-    constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
-    constexpr int BKT = BKP * KG;
-    constexpr int STRIDE = BKT + 8;
-    constexpr int CPR = BKT / 8;                      // 16-byte chunks per row
-    constexpr int KS = BKP / 16;                      // MFMA k steps per tile
-    constexpr int A_CH = (BM * CPR + NT - 1) / NT, W_CH = (BN * CPR + NT - 1) / NT, N_LOADS = A_CH + W_CH;
-    constexpr int EPI_STRIDE = 36;                    // floats per row of a 32x32 sub-tile in the epilogue
-    static_assert(KS % 2 == 0 && DEPTH >= 3, "the k loop alternates two fragment sets and three register sets");
-    constexpr int EPI_BASE = KG > 1 ? BM * BN : 0;    // floats: behind the groups' sums
-    static_assert(2 * (BM + BN) * STRIDE * 2 >= (EPI_BASE + WM * WN * 32 * EPI_STRIDE) * 4, "the tiles' LDS holds the epilogue's regions");
-    // one array: two buffers of A rows, two of W rows; the epilogue reuses it, a region per wavefront
-    __shared__ __attribute__((aligned(16))) bf16_t smem[2 * (BM + BN) * STRIDE];
+    // KG groups of WM x WN wavefronts share the tile: group g multiplies the g-th part of every k tile; their sums meet in LDS.
+    constexpr int NW = WM * WN * KG, BM = WM * TM * 32, BN = WN * TN * 32, ROWS = BM + BN;
+    constexpr int ROW_BYTES = BK * 2, PIECES = BK / 8;         // 16-byte pieces of a row of the k tile
+    constexpr int ROWS_PER_LOAD = 64 / PIECES;
+    constexpr int LOADS = ROWS / ROWS_PER_LOAD / NW;           // of a wavefront and k tile
+    static_assert(LOADS * ROWS_PER_LOAD * NW == ROWS && BM % ROWS_PER_LOAD == 0 && (PIECES == 8 || PIECES == 16), "whole loads");
+    static_assert(!GATED || 32 % ROWS_PER_LOAD == 0, "a load's rows belong to one map");
+    constexpr int KS = BK / 16 / KG;                           // MFMA k steps of a group and k tile
+    // HALVES: the 64-column blocks of K are summed in turn into two sums that are added at the end, as two groups (of 64 columns of a k
+    // tile of 128 each) do: which products do is a matter of their sizes alone (the dispatch), and so is every result's rounding.
+    static_assert(!HALVES || (KG == 1 && BK == 64), "one block a k tile");
+    static_assert(KG == 1 || (KG == 2 && BK == 128), "a group, a block of 64");
+    static_assert(KS % 2 == 0 && STAGES >= 3, "the k loop alternates two fragment sets and asks two tiles ahead");
+    constexpr int STAGE_BYTES = ROWS * ROW_BYTES;
+    constexpr bool APART = GATED && KG > 1;                    // both maps' sums go through LDS, as the groups' are still to be added
+    constexpr int EC = TN / PAIR * 32, EPI_STRIDE = EC * (APART ? 2 : 1) + 4;    // columns a wavefront stores; floats between their rows in LDS
+    constexpr int EPI_BYTES = NW * 32 * EPI_STRIDE * 4;
+    constexpr int V = F32_OUT ? 4 : 8, PER_ROW = EC / V, STEPS = 32 / KG * PER_ROW / 64;      // columns a lane stores at a time
+    static_assert(STEPS >= 1 && (KG == 1 || TM == 1), "two groups store half of the rows each");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[STAGES * STAGE_BYTES > EPI_BYTES ? STAGES * STAGE_BYTES : EPI_BYTES];
     __shared__ __attribute__((aligned(16))) float bias_s[BN];
-    bf16_t (*As)[BM * STRIDE] = reinterpret_cast<bf16_t (*)[BM * STRIDE]>(smem);
-    bf16_t (*Ws)[BN * STRIDE] = reinterpret_cast<bf16_t (*)[BN * STRIDE]>(smem + 2 * BM * STRIDE);
+    __shared__ int slot_s[BM];
+    static_assert(NW * 64 >= BN && NW * 64 >= BM, "a thread a column's bias, a thread a row's slot");
 
     const int tid = threadIdx.x, lane = tid % 64;
-    const int kg = tid / 64 / (WM * WN), wave = tid / 64 % (WM * WN);      // k group; wavefront within it
+    const int wid = __builtin_amdgcn_readfirstlane(tid / 64);
+    const int kg = wid / (WM * WN), wave = wid % (WM * WN);    // k group; wavefront within it
     const int wm = wave / WN, wn = wave % WN;
     // Workgroups are handed to the 8 XCDs round-robin and every XCD has an L2 of its own, so the
     // tiles of one XCD (workgroup id % 8) form one compact rectangle of the output: the rows of A
@@ -164,234 +187,245 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
     const int tm = (xcd / xn) * rect_m + local / rect_n, tn = (xcd % xn) * rect_n + local % rect_n;
     if (local >= rect_m * rect_n || tm >= tiles_m || tn >= tiles_n) return;      // padding of the grid
     const int m0 = tm * BM, n0 = tn * (BN / PAIR);
-    if (bias != nullptr)         // read again in the epilogue, after the k loop's barriers
-        for (int c = tid; c < BN; c += NT) bias_s[c] = n0 + c < N ? bias[n0 + c] : 0.f;
 
-    f32x16 acc[TM][TN];
+    // A k tile in LDS is its rows one behind the other (A's, then W's), without gaps, as the loads leave it: a load covers
+    // ROWS_PER_LOAD whole rows. Piece p of row r stands in place p ^ swizzle(r), so that the 16 lanes an LDS read serves at a time (16
+    // rows, one piece) fall on 16 different groups of banks; a lane asks for the piece whose place is its own.
+    auto swizzle = [](int row) { return PIECES == 8 ? (row >> 1) & 7 : row & 15; };
+    const unsigned char* base[LOADS];      // (uniform: a wavefront's load lies in one matrix)
+    unsigned offset[LOADS];
+#pragma unroll
+    for (int q = 0; q < LOADS; ++q) {
+        const int first = (wid * LOADS + q) * ROWS_PER_LOAD, row = first + lane / PIECES;
+        // (rows beyond the matrices: the last one; what is computed from it is never stored)
+        if (first < BM) {
+            base[q] = reinterpret_cast<const unsigned char*>(A + static_cast<size_t>(m0) * lda);
+            offset[q] = static_cast<unsigned>(min(row, M - 1 - m0)) * lda * 2;
+        } else {
+            const int w_row = row - BM, n = GATED ? w_row / 64 * 32 + w_row % 32 : w_row;
+            const bf16_t* map = W;
+            if constexpr (GATED) map = (first - BM) / 32 % 2 ? kv.up : W;
+            base[q] = reinterpret_cast<const unsigned char*>(map + static_cast<size_t>(n0) * ldw);
+            offset[q] = static_cast<unsigned>(min(n, N - 1 - n0)) * ldw * 2;
+        }
+        offset[q] += (lane % PIECES ^ swizzle(row)) * 16;
+    }
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem));
+    const int nk = (K + BK - 1) / BK, rest = K - (nk - 1) * BK;      // k tiles; columns of the last
+    auto fetch = [&](int q, int t, int stage) {                     // t: past the last tile, the last one again
+        t = min(t, nk - 1);
+        unsigned at = offset[q];
+        if (EDGE && t == nk - 1) {
+            // (pieces beyond K: the row's last one, against zeros)
+            const int piece = (lane % PIECES ^ swizzle((wid * LOADS + q) * ROWS_PER_LOAD + lane / PIECES)) * 16;
+            at += min(piece, rest * 2 - 16) - piece;
+        }
+        load_to_lds(base[q] + static_cast<size_t>(t) * ROW_BYTES, at, lds0 + stage * STAGE_BYTES + (wid * LOADS + q) * 1024);
+    };
+    // What the epilogue adds, asked for first and put into LDS behind the k loop.
+    float bias_r = 0.f;
+    int slot_r = -1;
+    if (bias != nullptr && tid < BN) bias_r = bias[min(n0 + tid, N - 1)];
+    if constexpr (MODE == EPI_STORE)
+        if (kv.slots != nullptr && tid < BM) slot_r = kv.slots[min(m0 + tid, M - 1)];
+    // The stream's old values: here too, unless registers are short, otherwise all of 32 rows together in the epilogue.
+    constexpr bool EARLY = MODE == EPI_ADD_RESIDUAL && !(HALVES && TM > 1);
+    const bool vec = (ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(C) & 15) == 0), vec8 = vec && ldc % 8 == 0;
+    float4 old[MODE == EPI_ADD_RESIDUAL ? (EARLY ? TM : 1) : 1][MODE == EPI_ADD_RESIDUAL ? STEPS : 1];
+    auto fetch_old = [&](int i) {
+#pragma unroll
+        for (int it = 0; it < (MODE == EPI_ADD_RESIDUAL ? STEPS : 0); ++it) {
+            const int idx = it * 64 + lane, m = m0 + (wm * TM + i) * 32 + 32 / KG * kg + idx / PER_ROW, n = n0 + wn * EC + idx % PER_ROW * V;
+            float4& o = old[EARLY ? i : 0][it];
+            o = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (vec && m < M && n + 4 <= N) o = *reinterpret_cast<const float4*>(static_cast<const float*>(C) + static_cast<size_t>(m) * ldc + n);
+        }
+    };
+    if constexpr (EARLY) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fetch_old(i);
+    }
+#pragma unroll
+    for (int s = 0; s < STAGES - 1; ++s)
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q) fetch(q, s, s);
+
+    f32x16 acc[TM][TN], acc2[TM][TN];      // (acc2: only with HALVES)
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
-
-    // per-thread chunk pointers (row fixed, k advances by BKP per tile) and LDS offsets
-    const bf16_t* pa[A_CH];
-    const bf16_t* pw[W_CH];
-    int la[A_CH], lw[W_CH];
-    bool va[A_CH], vw[W_CH];
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = acc2[i][j][r] = 0.f;
+    // two sets of MFMA operands: the fragments of k step ks+1 are read while step ks multiplies. A lane reads 8 elements of row
+    // lane % 32 of a sub-tile, from element 8 (lane / 32) of the k step on. (32 rows on the swizzle is the same.)
+    const int a_row = wm * TM * 32 + lane % 32, w_row = BM + wn * TN * 32 + lane % 32;
+    int a_at[KS], w_at[KS];
 #pragma unroll
-    for (int i = 0; i < A_CH; ++i) {
-        const int c = tid + i * NT, row = c / CPR, kc = c % CPR;
-        va[i] = (BM * CPR % NT == 0 || c < BM * CPR) && m0 + row < M;
-        pa[i] = A + static_cast<size_t>(va[i] ? m0 + row : 0) * lda + kc * 8;
-        la[i] = row * STRIDE + kc * 8;
+    for (int ks = 0; ks < KS; ++ks) {
+        const int piece = 2 * (kg * KS + ks) + lane / 32;
+        a_at[ks] = a_row * ROW_BYTES + (piece ^ swizzle(a_row)) * 16;
+        w_at[ks] = w_row * ROW_BYTES + (piece ^ swizzle(w_row)) * 16;
     }
-#pragma unroll
-    for (int i = 0; i < W_CH; ++i) {
-        const int c = tid + i * NT, row = c / CPR, kc = c % CPR;
-        const int n = n0 + (GATED ? row / 64 * 32 + row % 32 : row);
-        vw[i] = (BN * CPR % NT == 0 || c < BN * CPR) && n < N;
-        const bf16_t* rows = W;
-        if constexpr (GATED) rows = row / 32 % 2 ? kv.up : W;
-        pw[i] = rows + static_cast<size_t>(vw[i] ? n : 0) * ldw + kc * 8;
-        lw[i] = row * STRIDE + kc * 8;
-    }
-    struct TileRegs {
-        uint4 ra[A_CH], rw[W_CH];
-    };
-    TileRegs regs[DEPTH];
-    // (Rows of A or W beyond the matrix: the pointer stays on a row that exists, and what is computed
-    // from it lands in output rows or columns that are never stored. Only a K that is no multiple of
-    // the k tile needs care in the loop, EDGE: addresses clamped into the row, and zeros staged for
-    // what lies beyond K.)
-    // A tile's loads and its LDS writes are cut into KS portions (portion `part`, or all of them
-    // with part < 0), so that they can be issued between the MFMA groups of the tile in work.
-    // Every thread issues every load, with the address clamped into the matrix: the number of loads
-    // in flight is then the same on every path through the loop, and only so does the compiler wait
-    // for exactly the registers that are staged next while later loads stay in flight. What lies
-    // beyond K is zeroed when the tile is staged.
-    auto fetch = [&](TileRegs& t, int k0, int part) {
-#pragma unroll
-        for (int i = 0; i < A_CH; ++i) {
-            if (part >= 0 && i * KS / N_LOADS != part) continue;
-            const int kc8 = (tid + i * NT) % CPR * 8;
-            const int k = EDGE ? min(k0 + kc8, K - 8) - kc8 : k0;
-            t.ra[i] = *reinterpret_cast<const uint4*>(pa[i] + k);
-        }
-#pragma unroll
-        for (int i = 0; i < W_CH; ++i) {
-            if (part >= 0 && (A_CH + i) * KS / N_LOADS != part) continue;
-            const int kc8 = (tid + i * NT) % CPR * 8;
-            const int k = EDGE ? min(k0 + kc8, K - 8) - kc8 : k0;
-            t.rw[i] = *reinterpret_cast<const uint4*>(pw[i] + k);
-        }
-    };
-    auto stage = [&](const TileRegs& t, int buf, int k0, int part) {
-#pragma unroll
-        for (int i = 0; i < A_CH; ++i) {
-            if (part >= 0 && i * KS / N_LOADS != part) continue;
-            const int kc8 = (tid + i * NT) % CPR * 8;
-            const bool ok = !EDGE || k0 + kc8 < K;
-            if (BM * CPR % NT == 0 || tid + i * NT < BM * CPR)
-                *reinterpret_cast<uint4*>(&As[buf][la[i]]) = ok ? t.ra[i] : make_uint4(0, 0, 0, 0);
-        }
-#pragma unroll
-        for (int i = 0; i < W_CH; ++i) {
-            if (part >= 0 && (A_CH + i) * KS / N_LOADS != part) continue;
-            const int kc8 = (tid + i * NT) % CPR * 8;
-            const bool ok = !EDGE || k0 + kc8 < K;
-            if (BN * CPR % NT == 0 || tid + i * NT < BN * CPR)
-                *reinterpret_cast<uint4*>(&Ws[buf][lw[i]]) = ok ? t.rw[i] : make_uint4(0, 0, 0, 0);
-        }
-    };
-    // two sets of MFMA operands: the fragments of k step ks+1 are read while step ks multiplies
-    const int a_off = (wm * TM * 32 + lane % 32) * STRIDE + kg * BKP + 8 * (lane / 32);
-    const int w_off = (wn * TN * 32 + lane % 32) * STRIDE + kg * BKP + 8 * (lane / 32);
     bf16x8 fa[2][TM], fb[2][TN];
-    auto read_frags = [&](int buf, int ks, int set) {
+    auto read_frags = [&](int stage_at, int ks, int set) {
 #pragma unroll
-        for (int i = 0; i < TM; ++i)
-            fa[set][i] = *reinterpret_cast<const bf16x8*>(&As[buf][a_off + i * 32 * STRIDE + ks * 16]);
+        for (int i = 0; i < TM; ++i) fa[set][i] = *reinterpret_cast<const bf16x8*>(smem + stage_at + a_at[ks] + i * 32 * ROW_BYTES);
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
-            fb[set][j] = *reinterpret_cast<const bf16x8*>(&Ws[buf][w_off + j * 32 * STRIDE + ks * 16]);
+        for (int j = 0; j < TN; ++j) fb[set][j] = *reinterpret_cast<const bf16x8*>(smem + stage_at + w_at[ks] + j * 32 * ROW_BYTES);
     };
-    auto mma = [&](int set) {
+    auto mma = [&](int set, f32x16 (&sum)[TM][TN]) {
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j)
-                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[set][j], fa[set][i], acc[i][j], 0, 0, 0);
+                sum[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fb[set][j], fa[set][i], sum[i][j], 0, 0, 0);
+    };
+    auto zero_beyond = [&](int set, int ks) {                       // EDGE: the last tile's pieces beyond K
+        const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+        if ((2 * (kg * KS + ks) + lane / 32) * 8 >= rest) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i) fa[set][i] = zero;
+#pragma unroll
+            for (int j = 0; j < TN; ++j) fb[set][j] = zero;
+        }
     };
 
-    const int nk = (K + BKT - 1) / BKT;
-    // tiles 0 .. DEPTH-2 are requested (past the last tile: the last one again, never used);
-    // tile 0 is staged
-#pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d) fetch(regs[d], min(d, nk - 1) * BKT, -1);
-    stage(regs[0], 0, 0, -1);
-    lds_barrier();
+    // Tile t is in stage t % STAGES, the tiles up to t + STAGES - 2 are on their way. Every k step issues its share of the loads
+    // of tile t + STAGES - 1 (into the stage that tile t - 1 left: all wavefronts had read it when they last met), the fragment
+    // reads of the next k step and its MFMAs; the scheduling barriers keep that order. In front of the last step's MFMAs the
+    // wavefronts wait for tile t + 1 and meet, and read its first fragments: met behind them instead, all wavefronts would stand at the
+    // barrier and then for these reads with idle matrix units (36.5 > 31.4 us at 2,048 x 2,304 x 3,072).
+    wait_loads_and_meet<(STAGES - 2) * LOADS>();
     read_frags(0, 0, 0);
-    // Whole groups of DEPTH tiles run without a branch in the body (a load or a use of it under a
-    // condition would be moved or waited for conservatively); the last nk % DEPTH tiles, which
-    // fetch nothing any more, follow under conditions. In the body, tile t is in LDS buffer t%2
-    // and every k step issues, in this order: its share of the loads of tile t+DEPTH-1, its share
-    // of the LDS writes of tile t+1 (into the other buffer, whose last readers passed the barrier
-    // that ended the previous iteration), the fragment reads of the next k step, its MFMAs. The
-    // scheduling barriers keep that order: left alone, the compiler gathers the loads at the end
-    // of the iteration and the writes at its start, and a wavefront then issues nothing else while
-    // its memory instructions queue up.
-    const int n_groups = nk / DEPTH, n_tail = nk % DEPTH;
-    for (int g = 0; g < n_groups; ++g) {
+    int stage_at = 0, fetch_stage = STAGES - 1;
+    auto tile = [&](int t, f32x16 (&sum)[TM][TN]) {
+        const int next_at = stage_at == (STAGES - 1) * STAGE_BYTES ? 0 : stage_at + STAGE_BYTES;
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) {
-            const int t = g * DEPTH + d;
-            const int k_fetch = min(t + DEPTH - 1, nk - 1) * BKT;
+        for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                fetch(regs[(d + DEPTH - 1) % DEPTH], k_fetch, ks);
-                stage(regs[(d + 1) % DEPTH], (t + 1) & 1, (t + 1) * BKT, ks);
-                if (ks + 1 < KS) read_frags(t & 1, ks + 1, (ks + 1) & 1);
-                mma(ks & 1);
-                __builtin_amdgcn_sched_barrier(0);
+            for (int q = 0; q < LOADS; ++q)
+                if (q * KS / LOADS == ks) fetch(q, t + STAGES - 1, fetch_stage);
+            if (ks + 1 < KS) {
+                read_frags(stage_at, ks + 1, (ks + 1) & 1);
+            } else {
+                wait_loads_and_meet<(STAGES - 2) * LOADS>();
+                read_frags(next_at, 0, 0);
             }
-            lds_barrier();
-            read_frags((t + 1) & 1, 0, 0);
+            if (EDGE && t == nk - 1) zero_beyond(ks & 1, ks);
+            mma(ks & 1, sum);
+            __builtin_amdgcn_sched_barrier(0);
         }
-    }
-#pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d) {
-        const int t = n_groups * DEPTH + d;
-        if (d < n_tail) {
-            if (d + 1 < n_tail) stage(regs[(d + 1) % DEPTH], (t + 1) & 1, (t + 1) * BKT, -1);
-#pragma unroll
-            for (int ks = 0; ks < KS; ++ks) {
-                if (ks + 1 < KS) read_frags(t & 1, ks + 1, (ks + 1) & 1);
-                mma(ks & 1);
-            }
-            lds_barrier();
-            if (d + 1 < n_tail) read_frags((t + 1) & 1, 0, 0);
+        stage_at = next_at;
+        fetch_stage = fetch_stage == STAGES - 1 ? 0 : fetch_stage + 1;
+    };
+    if constexpr (HALVES) {
+        for (int t = 0; t < nk; t += 2) {
+            tile(t, acc);
+            if (t + 1 < nk) tile(t + 1, acc2);
         }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[i][j] += acc2[i][j];
+    } else {
+        for (int t = 0; t < nk; ++t) tile(t, acc);
     }
+    wait_loads_and_meet<0>();          // (nothing of the tiles is on its way or read any more)
+    if (tid < BN) bias_s[tid] = bias_r;
+    if (MODE == EPI_STORE && tid < BM) slot_s[tid] = slot_r;
 
     // With the weights as the A operand, register r of lane l holds output row l%32 and column
     // 8*(r/4) + 4*(l/32) + r%4 of a 32x32 sub-tile. Stored from there, one instruction would touch
-    // 16 bytes in each of 32 rows. So each sub-tile goes through the wavefront's own region of LDS
-    // (the tiles are done with theirs): written as the MFMA left it, read back with 8 lanes per row,
-    // and a store instruction then covers 8 whole rows of the sub-tile.
-    if constexpr (KG > 1) {
-        // the other groups leave their sums in LDS, register by register, and go; group 0 adds them
-        float4* sums = reinterpret_cast<float4*>(smem);
-        if (kg > 0) {
-#pragma unroll
-            for (int i = 0; i < TM; ++i)
-#pragma unroll
-                for (int j = 0; j < TN; ++j)
-#pragma unroll
-                    for (int g = 0; g < 4; ++g)
-                        sums[((wave * TM * TN + i * TN + j) * 4 + g) * 64 + lane] =
-                            make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-        }
-        lds_barrier();
-        if (kg > 0) return;
-        static_assert(KG == 2, "one other group's sums fit in front of the epilogue's regions");
-#pragma unroll
-        for (int i = 0; i < TM; ++i)
-#pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int g = 0; g < 4; ++g) {
-                    const float4 t = sums[((wave * TM * TN + i * TN + j) * 4 + g) * 64 + lane];
-                    acc[i][j][4 * g] += t.x; acc[i][j][4 * g + 1] += t.y; acc[i][j][4 * g + 2] += t.z; acc[i][j][4 * g + 3] += t.w;
-                }
-    }
-    const bool vec = (ldc % 4 == 0) && ((reinterpret_cast<uintptr_t>(C) & 15) == 0);
-    float* epi = reinterpret_cast<float*>(smem) + EPI_BASE + wave * (32 * EPI_STRIDE);
+    // 16 bytes in each of 32 rows. So the wavefront's 32 rows go through its own region of LDS: written as the MFMA left them,
+    // read back as whole rows, 16 bytes of output a lane.
+    // Two groups write both their sums, and each adds and stores half of the rows.
+    lds_barrier();                     // bias and slots
+    float* epi = reinterpret_cast<float*>(smem) + wid * (32 * EPI_STRIDE);
+    const float* other = KG > 1 ? reinterpret_cast<const float*>(smem) + wave * (32 * EPI_STRIDE) : epi;      // group 0's
+    const float* second = reinterpret_cast<const float*>(smem) + (WM * WN + wave) * (32 * EPI_STRIDE);        // group 1's
+    bool kv8 = false;                  // eight columns lie in one of the two parts and in 16 bytes
+    if constexpr (MODE == EPI_STORE) kv8 = kv.q_cols % 8 == 0 && kv.kv_dim % 8 == 0 && ((reinterpret_cast<uintptr_t>(kv.k_pages) | reinterpret_cast<uintptr_t>(kv.v_pages)) & 15) == 0;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
+        const int mb = m0 + (wm * TM + i) * 32, cb = wn * EC;      // first row; first column within the tile
+        if constexpr (MODE == EPI_ADD_RESIDUAL && !EARLY) fetch_old(i);
+        wave_lds_sync();          // the reads of the rows before are done
 #pragma unroll
-        for (int j = 0; j < TN; j += PAIR) {
-            if constexpr (GATED) {
+        for (int j = 0; j < TN; j += APART ? 1 : PAIR) {
+            if constexpr (GATED && !APART) {
 #pragma unroll
                 for (int r = 0; r < 16; ++r) acc[i][j][r] = gated_value(acc[i][j][r], acc[i][j + 1][r], kv);
             }
-            wave_lds_sync();          // the reads of the sub-tile before are done
+            const int column = APART ? j % 2 * EC + j / 2 * 32 : j / PAIR * 32;
 #pragma unroll
             for (int g = 0; g < 4; ++g)
-                *reinterpret_cast<float4*>(&epi[(lane % 32) * EPI_STRIDE + 8 * g + 4 * (lane / 32)]) =
+                *reinterpret_cast<float4*>(&epi[(lane % 32) * EPI_STRIDE + column + 8 * g + 4 * (lane / 32)]) =
                     make_float4(acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]);
-            wave_lds_sync();
-            const int mb = m0 + (wm * TM + i) * 32, nb = n0 + (wn * TN + j) / PAIR * 32;
+        }
+        if constexpr (KG > 1) lds_barrier(); else wave_lds_sync();
 #pragma unroll
-            for (int it = 0; it < 4; ++it) {
-                const int r = it * 8 + lane / 8, c4 = (lane % 8) * 4;
-                const int m = mb + r, n = nb + c4;
-                if (m >= M || n >= N) continue;
-                const int n_left = min(4, N - n);
-                const float4 t = *reinterpret_cast<const float4*>(&epi[r * EPI_STRIDE + c4]);
-                float v[4] = {t.x, t.y, t.z, t.w};
-                if (bias != nullptr) {
-                    const float4 b = *reinterpret_cast<const float4*>(&bias_s[nb - n0 + c4]);
-                    v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
+        for (int it = 0; it < STEPS; ++it) {
+            const int idx = it * 64 + lane, r = 32 / KG * kg + idx / PER_ROW, c = idx % PER_ROW * V;
+            const int m = mb + r, n = n0 + cb + c;
+            if (m >= M || n >= N) continue;
+            float v[V / 4][4];
+#pragma unroll
+            for (int h = 0; h < V / 4; ++h) {
+                const float4 t = *reinterpret_cast<const float4*>(&other[r * EPI_STRIDE + c + 4 * h]);
+                v[h][0] = t.x; v[h][1] = t.y; v[h][2] = t.z; v[h][3] = t.w;
+                if constexpr (KG > 1) {
+                    const float4 u = *reinterpret_cast<const float4*>(&second[r * EPI_STRIDE + c + 4 * h]);
+                    v[h][0] += u.x; v[h][1] += u.y; v[h][2] += u.z; v[h][3] += u.w;
                 }
-                if constexpr (MODE == EPI_THROUGH) through4(static_cast<float*>(C), static_cast<size_t>(m) * ldc + n, n, v, vec, n_left, kv);
-                else store4<MODE>(C, static_cast<size_t>(m) * ldc + n, v, vec, n_left);
-                if constexpr (MODE == EPI_STORE) if (kv.slots != nullptr && n >= kv.q_cols) {
-                    const int slot = kv.slots[m];
-                    if (slot >= 0) {
-                        // q_cols and kv_dim are multiples of 4: the four columns lie in one of the two parts
-                        const int c = n - kv.q_cols;
-                        bf16_t* dst = (c < kv.kv_dim ? kv.k_pages + c : kv.v_pages + (c - kv.kv_dim)) +
-                                      static_cast<size_t>(slot) * kv.kv_dim;
-                        if (n_left >= 4) {
-                            uint2 pk;
-                            pk.x = pack_bf16x2(v[0], v[1]);
-                            pk.y = pack_bf16x2(v[2], v[3]);
-                            *reinterpret_cast<uint2*>(dst) = pk;
-                        } else {
-                            for (int e = 0; e < n_left; ++e) dst[e] = float_to_bf16(v[e]);
-                        }
+                if constexpr (GATED && KG > 1) {
+                    // (the up map's columns stand behind the gate's)
+                    const float4 a = *reinterpret_cast<const float4*>(&other[r * EPI_STRIDE + EC + c + 4 * h]), b = *reinterpret_cast<const float4*>(&second[r * EPI_STRIDE + EC + c + 4 * h]);
+                    v[h][0] = gated_value(v[h][0], a.x + b.x, kv); v[h][1] = gated_value(v[h][1], a.y + b.y, kv);
+                    v[h][2] = gated_value(v[h][2], a.z + b.z, kv); v[h][3] = gated_value(v[h][3], a.w + b.w, kv);
+                }
+                if constexpr (!GATED) {
+                    const float4 b = *reinterpret_cast<const float4*>(&bias_s[cb + c + 4 * h]);
+                    v[h][0] += b.x; v[h][1] += b.y; v[h][2] += b.z; v[h][3] += b.w;
+                }
+            }
+            const size_t at = static_cast<size_t>(m) * ldc + n;
+            if constexpr (MODE == EPI_THROUGH) {
+                through4(static_cast<float*>(C), at, n, v[0], vec, min(4, N - n), kv);
+            } else if constexpr (MODE == EPI_ADD_RESIDUAL) {
+                if (vec && n + 4 <= N)
+                    *reinterpret_cast<float4*>(static_cast<float*>(C) + at) = make_float4(old[EARLY ? i : 0][it].x + v[0][0], old[EARLY ? i : 0][it].y + v[0][1], old[EARLY ? i : 0][it].z + v[0][2], old[EARLY ? i : 0][it].w + v[0][3]);
+                else store4<MODE>(C, at, v[0], vec, min(4, N - n));
+            } else if constexpr (MODE == EPI_STORE_F32) {
+                store4<MODE>(C, at, v[0], vec, min(4, N - n));
+            } else if (vec8 && n + 8 <= N) {
+                uint4 pk;
+                pk.x = pack_bf16x2(activated<MODE>(v[0][0]), activated<MODE>(v[0][1])); pk.y = pack_bf16x2(activated<MODE>(v[0][2]), activated<MODE>(v[0][3]));
+                pk.z = pack_bf16x2(activated<MODE>(v[1][0]), activated<MODE>(v[1][1])); pk.w = pack_bf16x2(activated<MODE>(v[1][2]), activated<MODE>(v[1][3]));
+                *reinterpret_cast<uint4*>(static_cast<bf16_t*>(C) + at) = pk;
+            } else {
+#pragma unroll
+                for (int h = 0; h < 2; ++h)
+                    if (n + 4 * h < N) store4<MODE>(C, at + 4 * h, v[h], vec, min(4, N - n - 4 * h));
+            }
+            if constexpr (MODE == EPI_STORE) if (kv.slots != nullptr && n + 7 >= kv.q_cols) {
+                const int slot = slot_s[mb - m0 + r];
+                const int col8 = n - kv.q_cols;
+                if (kv8 && n + 8 <= N) {
+                    bf16_t* dst = (col8 < kv.kv_dim ? kv.k_pages + col8 : kv.v_pages + (col8 - kv.kv_dim)) + static_cast<size_t>(max(slot, 0)) * kv.kv_dim;
+                    if (slot >= 0) *reinterpret_cast<uint4*>(dst) = make_uint4(pack_bf16x2(v[0][0], v[0][1]), pack_bf16x2(v[0][2], v[0][3]), pack_bf16x2(v[1][0], v[1][1]), pack_bf16x2(v[1][2], v[1][3]));
+                    continue;
+                }
+#pragma unroll
+                for (int h = 0; h < 2; ++h) {
+                    // q_cols and kv_dim are multiples of 4: four columns lie in one of the two parts
+                    const int col = n + 4 * h - kv.q_cols;
+                    if (slot < 0 || col < 0 || n + 4 * h >= N) continue;
+                    bf16_t* dst = (col < kv.kv_dim ? kv.k_pages + col : kv.v_pages + (col - kv.kv_dim)) + static_cast<size_t>(slot) * kv.kv_dim;
+                    if (n + 4 * h + 4 <= N) {
+                        *reinterpret_cast<uint2*>(dst) = make_uint2(pack_bf16x2(v[h][0], v[h][1]), pack_bf16x2(v[h][2], v[h][3]));
+                    } else {
+                        for (int e = 0; e < N - n - 4 * h; ++e) dst[e] = float_to_bf16(v[h][e]);
                     }
                 }
             }
@@ -411,19 +445,19 @@ static int split_among_xcds(int tiles_m, int tiles_n, int bm, int bn, int& xm, i
     return ((tiles_m + xm - 1) / xm) * ((tiles_n + xn - 1) / xn) * N_XCD;
 }
 
-template <int WM, int WN, int TM, int TN, int BKP, int DEPTH, int KG = 1>
+template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG = 1, bool HALVES = false>
 static void launch_tiled_gated(const bf16_t* a, int lda, const bf16_t* w, int ldw, void* C, int ldc, int M, int N, int K,
                                const GatedPair& pair, hipStream_t stream) {
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN / 2 - 1) / (BN / 2);
     int xm, xn;
     const dim3 grid(split_among_xcds(tiles_m, tiles_n, BM, BN, xm, xn)), block(WM * WN * KG * 64);
-#define TILED(E) gemm_bf16_mfma<WM, WN, TM, TN, BKP, DEPTH, E, EPI_GATED, KG><<<grid, block, 0, stream>>>(a, lda, w, ldw, nullptr, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, pair)
-    if (K % (BKP * KG) != 0) TILED(true); else TILED(false);
+#define TILED(E) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, E, EPI_GATED><<<grid, block, 0, stream>>>(a, lda, w, ldw, nullptr, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, pair)
+    if (K % BK != 0) TILED(true); else TILED(false);
 #undef TILED
 }
 
-template <int WM, int WN, int TM, int TN, int BKP, int DEPTH, int KG = 1>
+template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG = 1, bool HALVES = false>
 static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, const float* bias, void* C, int ldc,
                          int M, int N, int K, int mode, hipStream_t stream, KvScatter kv = KvScatter{},
                          const MllmStreamAdd* through = nullptr) {
@@ -431,8 +465,8 @@ static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, con
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     int xm, xn;
     const dim3 grid(split_among_xcds(tiles_m, tiles_n, BM, BN, xm, xn)), block(WM * WN * KG * 64);
-    const bool edge = K % (BKP * KG) != 0;      // rows and columns beyond the matrices need no other kernel, see EDGE
-#define TILED(E, MD) gemm_bf16_mfma<WM, WN, TM, TN, BKP, DEPTH, E, MD, KG><<<grid, block, 0, stream>>>(a, lda, w, ldw, bias, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, extra)
+    const bool edge = K % BK != 0;      // rows and columns beyond the matrices need no other kernel
+#define TILED(E, MD) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, E, MD><<<grid, block, 0, stream>>>(a, lda, w, ldw, bias, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, extra)
     if (mode == EPI_THROUGH) {
         const MllmStreamAdd extra = *through;
         if (edge) TILED(true, EPI_THROUGH); else TILED(false, EPI_THROUGH);
@@ -1297,6 +1331,51 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 }
 
 
+// Tile choice. A compute unit holds one workgroup at a time (its stages fill the LDS), so the workgroups of an XCD run in rounds of 32. A
+// product is priced in microseconds as the launch, a round's start and end, and its k tiles, which take longer the more units load
+// side by side. The numbers are fitted to 74 products of 96 to 8,000 rows, 768 to 6,400 columns and as many summed, each with rows that a
+// kernel before it wrote and weights that no cache of an XCD holds, as a step has them: what is chosen takes 0.8 % more than the
+// fastest of the tiles on average, where sums come in halves no more. (With rows and weights left in the caches 64x128 tiles beat
+// 64x96 of two groups on the feed-forward's second product, 16.9 to 16.3 us; in a step they take 25.7 us and 22.3.)
+struct TilePrice { int bm, bn; double launch, round, tile, load; };
+static const TilePrice plain_tiles[] = {{128, 256, 4.15, -0.04, 0.583, 0.320}, {128, 192, 2.98, 0.89, 0.478, 0.232}, {128, 128, 2.39, 1.06, 0.362, 0.172},
+                                        {64, 128, 1.57, 1.53, 0.290, 0.070},   {64, 64, 1.57, 1.55, 0.209, 0.051},   {64, 32, 3.80, -0.27, 0.138, 0.040}};
+static const TilePrice halved_tiles[] = {{128, 256, 7.77, -5.49, 0.639, 0.299}, {128, 192, 4.61, -2.20, 0.522, 0.212}, {128, 128, 4.71, -2.01, 0.384, 0.182},
+                                         {64, 128, 3.05, -0.29, 0.295, 0.085},  {64, 96, 2.08, 2.50, 0.215, 0.069},    {64, 64, 1.81, 1.69, 0.162, 0.071},
+                                         {64, 32, 1.12, 2.01, 0.118, 0.044}};
+static int cheapest_tile(const TilePrice* prices, int n, int M, int N, int K) {
+    int best = 0;
+    double best_price = 1e300;
+    for (int c = 0; c < n; ++c) {
+        const TilePrice& p = prices[c];
+        const int tiles_m = (M + p.bm - 1) / p.bm, tiles_n = (N + p.bn - 1) / p.bn;
+        int xm, xn;
+        const int per_xcd = split_among_xcds(tiles_m, tiles_n, p.bm, p.bn, xm, xn) / N_XCD, rounds = (per_xcd + 31) / 32;
+        const double k_tiles = (K + 63) / 64, blocks = static_cast<double>(tiles_m) * tiles_n;
+        const double price = p.launch + rounds * (p.round + p.tile * k_tiles) + p.load * k_tiles * blocks / 256.0;
+        if (price < best_price) { best_price = price; best = c; }
+    }
+    return best;
+}
+
+// Which products are summed in two halves (HALVES, or two groups of wavefronts): those that tiles of at most 128x128 suit by the count of
+// workgroups, where K is long, and the smallest. It is a rule of its own, apart from the tile: the tile may change with what is
+// measured, the order of the sums, and with it the last bit of every result, does not.
+static bool sums_in_halves(int M, int N, int K) {
+    struct Shape { int bm, bn; double efficiency; };
+    static const Shape shapes[] = {{128, 256, 1.05}, {128, 192, 1.0}, {128, 128, 0.9}, {64, 128, 0.7},
+                                   {64, 96, 0.65},   {64, 64, 0.55}, {64, 32, 0.4}};
+    int best = 0;
+    double best_cost = 1e300;
+    for (int c = 0; c < 7; ++c) {
+        if (c == 4 && N > 1024) continue;
+        const long blocks = static_cast<long>((M + shapes[c].bm - 1) / shapes[c].bm) * ((N + shapes[c].bn - 1) / shapes[c].bn);
+        const double cost = static_cast<double>((blocks + 255) / 256) * shapes[c].bm * shapes[c].bn / shapes[c].efficiency;
+        if (cost < best_cost) { best_cost = cost; best = c; }
+    }
+    return best == 6 || (K >= 2048 && (best == 2 || best == 4 || best == 5));
+}
+
 static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, const float* bias, void* C, int ldc,
                               int M, int N, int K, int mode, hipStream_t stream, KvScatter kv,
                               void* workspace = nullptr, size_t workspace_bytes = 0, const MllmStreamAdd* through = nullptr) {
@@ -1330,38 +1409,28 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
                                                                                 MergedA{}, 0, through, kv) == 0) {
         // few rows: weight-streaming kernel
     } else if (M <= 32) {
-        launch_tiled<1, 4, 1, 1, 64, 3>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through);
+        launch_tiled<1, 4, 1, 1, 64, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through);
     } else {
-        // Tile choice. The compute units run the workgroups in rounds of 256, and a workgroup's time
-        // grows with its tile's area, less so for large tiles (they move fewer bytes per flop). So
-        // each shape is priced as rounds x area / efficiency, the efficiencies fitted to measurements
-        // at 2048 rows on the products of GPT-2 small to XL, and the cheapest runs. Few workgroups
-        // (one round for every shape) thus take the smallest tiles, which spread over more units
-        // (64x32 where even 64x64 tiles leave most units idle: decode at 48 to 128 rows).
-        struct Shape { int bm, bn; double efficiency; };
-        static const Shape shapes[] = {{128, 256, 1.05}, {128, 192, 1.0}, {128, 128, 0.9}, {64, 128, 0.7},
-                                       {64, 96, 0.65},   {64, 64, 0.55}, {64, 32, 0.4}};
-        int best = 0;
-        double best_cost = 1e300;
-        for (int c = 0; c < 7; ++c) {
-            if (c == 4 && N > 1024) continue;       // 64x96 pays on narrow outputs only (measured: up to twice the time of 64x64 on wide ones)
-            const long blocks = static_cast<long>((M + shapes[c].bm - 1) / shapes[c].bm) * ((N + shapes[c].bn - 1) / shapes[c].bn);
-            const double cost = static_cast<double>((blocks + 255) / 256) * shapes[c].bm * shapes[c].bn / shapes[c].efficiency;
-            if (cost < best_cost) { best_cost = cost; best = c; }
-        }
-        // With a long K the smaller tiles' time goes to the barrier intervals of the k loop, and two
-        // groups of wavefronts per workgroup, each on half of a twice as wide k tile, halve their
-        // number (measured at K of 3072 to 6400: 9 to 17 % less time; at K of 768 to 1600: none).
-        const bool long_k = K >= 2048;
 #define TILE(...) launch_tiled<__VA_ARGS__>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through)
-        switch (best) {
-            case 0: TILE(2, 4, 2, 2, 64, 4); break;
-            case 1: TILE(4, 2, 1, 3, 64, 3); break;
-            case 2: if (long_k) TILE(2, 4, 2, 1, 64, 3, 2); else TILE(2, 4, 2, 1, 64, 3); break;
-            case 3: TILE(2, 4, 1, 1, 64, 4); break;
-            case 4: if (long_k) TILE(2, 3, 1, 1, 64, 5, 2); else TILE(2, 3, 1, 1, 64, 5); break;
-            case 5: if (long_k) TILE(2, 2, 1, 1, 64, 4, 2); else TILE(2, 2, 1, 1, 64, 4); break;
-            default: TILE(2, 1, 1, 1, 64, 4, 2); break;     // 64x32 (few workgroups in all): two wavefronts, always two groups
+        if (sums_in_halves(M, N, K)) {
+            switch (cheapest_tile(halved_tiles, 7, M, N, K)) {
+                case 0: TILE(2, 4, 2, 2, 64, 3, 1, true); break;
+                case 1: TILE(4, 2, 1, 3, 64, 3, 1, true); break;
+                case 2: TILE(4, 2, 1, 2, 64, 4, 1, true); break;
+                case 3: TILE(2, 4, 1, 1, 64, 6, 1, true); break;
+                case 4: TILE(2, 1, 1, 3, 128, 3, 2); break;
+                case 5: TILE(2, 2, 1, 1, 128, 4, 2); break;
+                default: TILE(2, 1, 1, 1, 128, 4, 2); break;
+            }
+        } else {
+            switch (cheapest_tile(plain_tiles, 6, M, N, K)) {
+                case 0: TILE(2, 4, 2, 2, 64, 3); break;
+                case 1: TILE(4, 2, 1, 3, 64, 3); break;
+                case 2: TILE(4, 2, 1, 2, 64, 4); break;
+                case 3: TILE(2, 2, 1, 2, 64, 4); break;
+                case 4: TILE(2, 2, 1, 1, 64, 6); break;
+                default: TILE(2, 1, 1, 1, 64, 6); break;
+            }
         }
 #undef TILE
     }
@@ -1489,7 +1558,8 @@ int mllm_gated_gemm_bf16(const void* A, int lda, const void* gate, const void* u
     if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) return -1;
     const bf16_t *a = static_cast<const bf16_t*>(A), *w = static_cast<const bf16_t*>(gate);
     const GatedPair pair{static_cast<const bf16_t*>(up), limit, alpha};
-    struct Shape { int bm, bn; double efficiency; };      // (priced as the single product's, the columns of both maps counted)
+    // (the columns of both maps counted; few tiles of 64x64 are summed in halves, a rule that stays as sums_in_halves does)
+    struct Shape { int bm, bn; double efficiency; };
     static const Shape shapes[] = {{128, 256, 1.05}, {128, 128, 0.9}, {64, 128, 0.7}, {64, 64, 0.55}};
     int best = 0;
     double best_cost = 1e300;
@@ -1498,12 +1568,14 @@ int mllm_gated_gemm_bf16(const void* A, int lda, const void* gate, const void* u
         const double cost = static_cast<double>((blocks + 255) / 256) * shapes[c].bm * shapes[c].bn / shapes[c].efficiency;
         if (cost < best_cost) { best_cost = cost; best = c; }
     }
+    static const TilePrice gated_tiles[] = {plain_tiles[0], plain_tiles[2], plain_tiles[3]};
+    if (best < 3) best = cheapest_tile(gated_tiles, 3, M, 2 * N, K);
 #define TILE(...) launch_tiled_gated<__VA_ARGS__>(a, lda, w, ldw, C, ldc, M, N, K, pair, stream)
     switch (best) {
-        case 0: TILE(2, 4, 2, 2, 64, 4); break;
-        case 1: TILE(4, 2, 1, 2, 64, 3); break;
+        case 0: TILE(2, 4, 2, 2, 64, 3); break;
+        case 1: TILE(4, 2, 1, 2, 64, 4); break;
         case 2: TILE(2, 2, 1, 2, 64, 4); break;
-        default: TILE(2, 1, 1, 2, 64, 4, 2); break;
+        default: TILE(2, 1, 1, 2, 128, 4, 2); break;
     }
 #undef TILE
     MLLM_LAUNCH_CHECK();
