@@ -164,6 +164,94 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
         epilogue<float>(mode, mine, bias ? bias[n] : 0.f, C, static_cast<size_t>(lane) * ldc + n);
 }
 
+// The same for narrow results (the output projection, the feed-forward's second product), where one column a wavefront leaves few
+// wavefronts and each waits for chunk after chunk of its column: two wavefronts share a column, 256 columns of K in turn, and
+// ask for all their weights of a pass of KP = 512 STEPS columns at once, behind the pass's activations, which lie in LDS whole. One
+// pass covers K up to 3,072; beyond, the next pass's weights are on their way while one is used. What the epilogue adds is asked for
+// first. Bound by the chain launch, activations, weights, sums: 8 x 768 x 768 and 8 x 768 x 3,072 in a decode step 4.1 and 6.0
+// us, together 17.1 with a column a wavefront.
+template <int ROWS, int STEPS>
+__global__ void __launch_bounds__(512)
+gemm_f32_narrow_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
+                       const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K, int mode) {
+    constexpr int COLS = 4, KP = 512 * STEPS, STAGED = ROWS * KP / 4 / 512;
+    static_assert(COLS * ROWS <= 64, "the first wavefront holds the outputs");
+    __shared__ __attribute__((aligned(16))) float a_s[ROWS][KP];
+    __shared__ float sums[2][COLS][ROWS];
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
+    const int column = wave % COLS, half = wave / COLS;
+    const float* wrow = W + static_cast<size_t>(min(blockIdx.x * COLS + column, static_cast<unsigned>(N - 1))) * ldw;   // (a surplus column repeats the last)
+    const int out_r = tid % ROWS, out_n = blockIdx.x * COLS + tid / ROWS;
+    const bool owns = tid < COLS * ROWS && out_r < M && out_n < N;
+    const size_t out_at = static_cast<size_t>(min(out_r, M - 1)) * ldc + min(out_n, N - 1);
+    float out_bias = 0.f, out_old = 0.f;
+    if (owns && bias != nullptr) out_bias = bias[out_n];
+    if (owns && mode == EPI_ADD_RESIDUAL) out_old = static_cast<const float*>(C)[out_at];
+    float4 v[STAGED], w[STEPS], next[STEPS];
+    auto fetch_rows = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < STAGED; ++u) {
+            const int idx = tid + 512 * u, r = idx / (KP / 4), k = k0 + idx % (KP / 4) * 4;
+            const float4 a = *reinterpret_cast<const float4*>(A + static_cast<size_t>(min(r, M - 1)) * lda + min(k, K - 4));
+            v[u] = r < M && k < K ? a : make_float4(0.f, 0.f, 0.f, 0.f);
+        }
+    };
+    auto fetch_weights = [&](float4 (&to)[STEPS], int k0) {        // (beyond K: the row's last four, against zeros)
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) to[s] = *reinterpret_cast<const float4*>(wrow + min(k0 + (2 * s + half) * 256 + 4 * lane, K - 4));
+    };
+    float acc[ROWS];
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
+    fetch_rows(0);
+    __builtin_amdgcn_sched_barrier(0);
+    fetch_weights(w, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (int k0 = 0; k0 < K; k0 += KP) {
+        if (k0 > 0) lds_barrier();             // the pass before has been read
+#pragma unroll
+        for (int u = 0; u < STAGED; ++u) {
+            const int idx = tid + 512 * u;
+            *reinterpret_cast<float4*>(&a_s[idx / (KP / 4)][idx % (KP / 4) * 4]) = v[u];
+        }
+        lds_barrier();
+        const bool more = k0 + KP < K;
+        if (more) {
+            fetch_rows(k0 + KP);
+            fetch_weights(next, k0 + KP);
+        }
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) {
+            const int q = (2 * s + half) * 256 + 4 * lane;
+            if (k0 + (2 * s + half) * 256 >= K) continue;
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {
+                const float4 a4 = *reinterpret_cast<const float4*>(&a_s[r][q]);
+                acc[r] = fmaf(a4.x, w[s].x, acc[r]);
+                acc[r] = fmaf(a4.y, w[s].y, acc[r]);
+                acc[r] = fmaf(a4.z, w[s].z, acc[r]);
+                acc[r] = fmaf(a4.w, w[s].w, acc[r]);
+            }
+        }
+        if (more) {
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s) w[s] = next[s];
+        }
+    }
+    float mine = 0.f;
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+        const float t = wave_sum(acc[r]);
+        if (lane == r) mine = t;
+    }
+    if (lane < ROWS) sums[half][column][lane] = mine;
+    lds_barrier();
+    if (!owns) return;
+    const float sum = sums[0][tid / ROWS][out_r] + sums[1][tid / ROWS][out_r];
+    if (mode == EPI_ADD_RESIDUAL) static_cast<float*>(C)[out_at] = out_old + (sum + out_bias);
+    else epilogue<float>(mode, sum, out_bias, C, out_at);
+}
+
 // More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). Four
 // wavefronts, two by two, of TM x TN tiles of 16 x 16 each share k tiles of 32 columns (a row's piece is one 128-byte line) in
 // LDS, double buffered with one barrier a tile; the loads of the two tiles behind the next are in flight in registers. KG such
@@ -390,9 +478,12 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
             if (M <= 8) gemm_f32_rows_kernel<8, 8><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
             else gemm_f32_rows_kernel<16, 8><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
         } else {
+            // (3,072 columns a pass take the LDS of a unit: while there is one workgroup a unit; 9 to 16 rows would take twice as much)
             const dim3 rows_grid((N + 3) / 4);
-            if (M <= 8) gemm_f32_rows_kernel<8, 4><<<rows_grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
-            else gemm_f32_rows_kernel<16, 4><<<rows_grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            if (M > 8) gemm_f32_rows_kernel<16, 4><<<rows_grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            else if (K <= 1024) gemm_f32_narrow_kernel<8, 2><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            else if (N <= 1024) gemm_f32_narrow_kernel<8, 6><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            else gemm_f32_narrow_kernel<8, 3><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
         }
         MLLM_LAUNCH_CHECK();
         return 0;

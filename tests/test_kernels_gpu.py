@@ -185,6 +185,24 @@ def test_linear_bf16_tile_choices(ops, M, N, K, epi):
     assert err <= (2e-5 + 2e-5 * math.sqrt(K) if f32_out else 4e-2), err
 
 
+@pytest.mark.parametrize("M,N", [(33, 40), (100, 768), (260, 1000), (520, 772), (1000, 1024), (1030, 3072), (2100, 2300), (2048, 6400)])
+@pytest.mark.parametrize("K", [8, 56, 64, 72, 136, 200, 328, 2048, 2056, 2120, 2184])
+def test_linear_bf16_stages_and_remainders(ops, M, N, K):
+    """Products on every tile, with fewer k tiles than stages and with 8 to 64 columns in the last: every element against the
+    sum in fp32 of the same bfloat16 values. Rounding to bfloat16 is 2^-9 of the result (2^-8 allowed), the sums' own order K^0.5 2^-24 of the terms."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = _rand((M, K), torch.bfloat16, g), _rand((N, K), torch.bfloat16, g, K ** -0.5)
+    bias = _rand((N,), torch.float32, g)
+    want = a.to(DEV).float() @ w.to(DEV).float().T + bias.to(DEV)
+    out = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ops.linear(a.to(DEV), w.to(DEV), bias.to(DEV), out)
+    assert bool(((out.float() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-4).all())
+    x = _rand((M, N), torch.float32, g).to(DEV)
+    got = x.clone()
+    ops.linear(a.to(DEV), w.to(DEV), bias.to(DEV), got, "add_residual")
+    assert bool(((got - (x + want)).abs() <= 1e-4).all())
+
+
 @pytest.mark.parametrize("M,H,Hkv,dh,K", [(2048, 12, 12, 64, 768),      # 128x192 tiles
                                           (300, 6, 2, 16, 96),         # 64x64 tiles, ragged, grouped heads
                                           (70, 3, 3, 48, 144),         # just above the few-row kernel
@@ -453,6 +471,21 @@ def test_linear_fp32_is_as_exact_on_tiles_as_for_few_rows(ops, K):
         ops.linear(a[m:m + 16], w, None, rows[m:m + 16], "store")
     assert not torch.equal(tiles, rows)
     assert (tiles.double() - want).norm() <= (rows.double() - want).norm()
+
+
+@pytest.mark.parametrize("M", [1, 5, 8])
+@pytest.mark.parametrize("N,K", [(3, 4), (70, 252), (70, 260), (768, 1020), (768, 1024), (1024, 1028), (1024, 3072), (1024, 3076), (1025, 1536), (1600, 1540), (1600, 6400)])
+@pytest.mark.parametrize("epi", ["store", "add_residual"])
+def test_linear_fp32_narrow_results(ops, M, N, K, epi):
+    """Up to 8 rows of narrow results: passes of 1,024, 1,536 and 3,072 columns of K, filled, missed and begun by four. A lane sums at
+    most 2 K / 128 + 48 terms in a chain, so the error is below that many halves of 2^-23 of the terms' absolute sum."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w, bias, x = _rand((M, K), torch.float32, g), _rand((N, K), torch.float32, g), _rand((N,), torch.float32, g), _rand((M, N), torch.float32, g)
+    want = a.double() @ w.double().T + bias.double() + (x.double() if epi == "add_residual" else 0)
+    bound = (K / 64 + 48) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T + 2.0)
+    out = x.to(DEV)
+    ops.linear(a.to(DEV), w.to(DEV), bias.to(DEV), out, epi)
+    assert bool(((out.cpu().double() - want).abs() <= bound).all())
 
 
 @pytest.mark.parametrize("N,K", [(16381, 64), (16385, 64), (16385, 68), (20001, 96), (32001, 128), (32001, 132), (16384, 96), (16384, 100), (20000, 16)])
