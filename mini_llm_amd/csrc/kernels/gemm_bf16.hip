@@ -1408,6 +1408,8 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
                                                                                 nullptr, 0.f, nullptr, stream, workspace, workspace_bytes,
                                                                                 MergedA{}, 0, through, kv) == 0) {
         // few rows: weight-streaming kernel
+    } else if (lda > 1 << 23 || ldw > 1 << 23) {
+        return -1;          // (a tile's rows are reached by 32-bit byte offsets)
     } else if (M <= 32) {
         launch_tiled<1, 4, 1, 1, 64, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through);
     } else {
@@ -1441,7 +1443,7 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
 extern "C" {
 
 // Returns 0, a HIP error code, or -1 when K or the row strides are not multiples of 8
-// elements or a base pointer is not 16-byte aligned.
+// elements, a base pointer is not 16-byte aligned, or rows of a product on tiles lie more than 2^23 elements apart.
 // `workspace` (optional; 4-byte aligned, zero when first handed over, never written by anyone else)
 // lets narrow products of few rows and a long K share a tile among several workgroups: 16 KB of
 // counters, then 1 KB per workgroup of such a launch (at most 256). Launches that use one
@@ -1555,7 +1557,7 @@ int mllm_gated_gemm_bf16(const void* A, int lda, const void* gate, const void* u
                          int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K % 8 != 0 || lda % 8 != 0 || ldw % 8 != 0) return -1;
-    if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) return -1;
+    if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) || lda > 1 << 23 || ldw > 1 << 23) return -1;
     const bf16_t *a = static_cast<const bf16_t*>(A), *w = static_cast<const bf16_t*>(gate);
     const GatedPair pair{static_cast<const bf16_t*>(up), limit, alpha};
     // (the columns of both maps counted; few tiles of 64x64 are summed in halves, a rule that stays as sums_in_halves does)
