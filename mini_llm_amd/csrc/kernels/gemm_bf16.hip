@@ -131,9 +131,11 @@ __device__ __forceinline__ void store4(void* C, size_t idx, const float (&v)[4],
 
 // One piece of a wavefront's loads straight into LDS: every lane's 16 bytes at base + offset go to lane-linear places from `lds` on. In
 // assembly, because a load into LDS that the compiler knows of makes it wait for all of them in front of the next LDS read:
-// whoever calls this waits (wait_loads) and passes a barrier before the bytes are read. It has no result register.
+// whoever calls this waits (wait_loads_and_meet) and passes a barrier before the bytes are read. It has no result register. The compiler sees no
+// instruction in here, so the wait state that gfx9 needs between a scalar write of m0 and a load into LDS (which would otherwise
+// go to the place of the load before it) stands here too; m0 is ours for the length of the block only.
 __device__ __forceinline__ void load_to_lds(const unsigned char* base, unsigned offset, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(offset), "s"(base) : "memory");
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(offset), "s"(base) : "m0", "memory");
 }
 // Waits until at most N of the wavefront's loads are under way (they end in their order) and its LDS reads are done, then for the others.
 template <int N>
