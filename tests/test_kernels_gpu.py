@@ -488,6 +488,27 @@ def test_linear_fp32_narrow_results(ops, M, N, K, epi):
     assert bool(((out.cpu().double() - want).abs() <= bound).all())
 
 
+@pytest.mark.parametrize("M", [1, 8])
+@pytest.mark.parametrize("N,K", [(70, 252), (70, 1000), (1024, 1028), (1024, 3076), (1025, 1540), (1600, 3076)])
+def test_linear_fp32_narrow_results_keep_infinite_weights(ops, M, N, K):
+    """K that ends within a piece of 256: lanes beyond it must not multiply the row's last weights by anything. An infinity there
+    meets an activation of 1 and gives an infinity of its sign, an infinite activation meets a weight of 1; other columns stay as they are."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = _rand((M, K), torch.float32, g), _rand((N, K), torch.float32, g)
+    a[:, -4:] = 1.0
+    clean = torch.empty(M, N, device=DEV)
+    ops.linear(a.to(DEV), w.to(DEV), None, clean)
+    w[1, -1], w[2, -4] = math.inf, -math.inf
+    out = torch.empty(M, N, device=DEV)
+    ops.linear(a.to(DEV), w.to(DEV), None, out)
+    assert bool((out[:, 1] == math.inf).all()) and bool((out[:, 2] == -math.inf).all())
+    assert torch.equal(out[:, 3:], clean[:, 3:]) and torch.equal(out[:, 0], clean[:, 0])
+    w[:, -4:] = 1.0
+    a[M - 1, -2] = math.inf
+    ops.linear(a.to(DEV), w.to(DEV), None, out)
+    assert bool((out[M - 1] == math.inf).all()) and bool(out[:M - 1].isfinite().all())
+
+
 @pytest.mark.parametrize("N,K", [(16381, 64), (16385, 64), (16385, 68), (20001, 96), (32001, 128), (32001, 132), (16384, 96), (16384, 100), (20000, 16)])
 @pytest.mark.parametrize("M", [64, 65, 130])
 def test_linear_fp32_wide_rows_of_short_sums(ops, M, N, K):
