@@ -240,10 +240,6 @@ static void check_scatter(const KvScatter& kv, int dtype, int64_t N, int epilogu
     if (N != kv.q_cols + 2 * kv_dim) fail("%s: %lld columns are not %d + 2 x %d", what, (long long)N, kv.q_cols, kv_dim);
 }
 
-// The many-row matrix-core kernel reaches the rows of a tile by 32-bit byte offsets (up to 256 rows apart);
-// up to 16 rows are the few-row kernel's.
-static bool rows_near(const Tensor2& a, const Tensor2& w) { return a.rows <= 16 || (a.stride <= 1 << 23 && w.stride <= 1 << 23); }
-
 void linear(const Tensor2& a, const Tensor2& w, const float* bias, const Tensor2& out, int epilogue,
             const KvScatter* kv, hipStream_t stream) {
     need_dtype(a, "a");
@@ -256,7 +252,7 @@ void linear(const Tensor2& a, const Tensor2& w, const float* bias, const Tensor2
         // do not take go through a product and a copy.
         const bool fits = kv->q_cols % 4 == 0 && kv_dim % 4 == 0 && K % 8 == 0 && a.stride % 8 == 0 && w.stride % 8 == 0 &&
                           aligned(a.data, 16) && aligned(w.data, 16);
-        if (a.dtype != BF16 || (M <= 64 && !fits) || !rows_near(a, w)) {
+        if (a.dtype != BF16 || (M <= 64 && !fits)) {
             linear(a, w, bias, out, epilogue, nullptr, stream);
             kv_append(out, kv->q_cols, kv->q_cols + kv_dim, kv->k_pages, kv->v_pages, kv->slots, stream);
             return;
@@ -268,7 +264,7 @@ void linear(const Tensor2& a, const Tensor2& w, const float* bias, const Tensor2
         rc = mllm_gemm_f32(static_cast<const float*>(a.data), static_cast<int>(a.stride), static_cast<const float*>(w.data),
                            static_cast<int>(w.stride), bias, out.data, static_cast<int>(out.stride), static_cast<int>(M),
                            static_cast<int>(N), static_cast<int>(K), epilogue, stream);
-    } else if (kv == nullptr && (!rows_near(a, w) || K % 8 != 0 || a.stride % 8 != 0 || w.stride % 8 != 0 || !aligned(a.data, 16) || !aligned(w.data, 16))) {
+    } else if (kv == nullptr && (K % 8 != 0 || a.stride % 8 != 0 || w.stride % 8 != 0 || !aligned(a.data, 16) || !aligned(w.data, 16))) {
         // sizes that the matrix-core kernels do not read (16 bytes at a time): the plain kernel, slow and general
         rc = mllm_gemm_bf16_plain(a.data, static_cast<int>(a.stride), w.data, static_cast<int>(w.stride), bias, out.data,
                                   static_cast<int>(out.stride), static_cast<int>(M), static_cast<int>(N), static_cast<int>(K), epilogue, stream);
@@ -294,7 +290,7 @@ void linear_stream_add(const Tensor2& a, const Tensor2& w, const float* bias, co
     check_stream_add(add, "linear_stream_add");
     const int64_t M = a.rows, K = a.cols;
     check_linear(M, K, a.dtype, w, add.x, ADD_RESIDUAL, "linear_stream_add");
-    if (tuning().through_products && a.dtype == BF16 && rows_near(a, w) && K % 8 == 0 && a.stride % 8 == 0 && w.stride % 8 == 0 && aligned(a.data, 16) && aligned(w.data, 16)) {
+    if (tuning().through_products && a.dtype == BF16 && K % 8 == 0 && a.stride % 8 == 0 && w.stride % 8 == 0 && aligned(a.data, 16) && aligned(w.data, 16)) {
         void* ws = M <= 256 ? gemm_workspace(stream) : nullptr;
         const MllmStreamAdd k{add.norm, add.next, add.copy.data, static_cast<int>(add.copy.stride)};
         const int rc = mllm_gemm_bf16_through(a.data, static_cast<int>(a.stride), w.data, static_cast<int>(w.stride), bias, static_cast<float*>(add.x.data),

@@ -137,13 +137,21 @@ __device__ __forceinline__ void store4(void* C, size_t idx, const float (&v)[4],
 __device__ __forceinline__ void load_to_lds(const unsigned char* base, unsigned offset, unsigned lds) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" :: "s"(lds), "v"(offset), "s"(base) : "m0", "memory");
 }
+__device__ __forceinline__ void load_to_lds(const unsigned char* base, size_t offset, unsigned lds) {         // (for offsets of any size)
+    asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" :: "s"(lds), "v"(base + offset) : "m0", "memory");
+}
 // Waits until at most N of the wavefront's loads are under way (they end in their order) and its LDS reads are done, then for the others.
 template <int N>
 __device__ __forceinline__ void wait_loads_and_meet() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
 
-template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG, bool HALVES, bool EDGE, int MODE>
+// How far apart (in elements) the rows of a matrix may lie for the 32-bit byte offsets from a tile's first row to the other 255 and a
+// k tile's pieces. Beyond it (FAR) a lane forms 64-bit addresses, which only one shape of tile for either order of sums does: rows over 16 MiB
+// apart have nothing else in common with what the prices know.
+#define NEAR_ROWS (1 << 23)
+
+template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG, bool HALVES, bool FAR, bool EDGE, int MODE>
 __global__ void __launch_bounds__(WM * WN * KG * 64)
 gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
                const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K,
@@ -195,20 +203,21 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
     // rows, one piece) fall on 16 different groups of banks; a lane asks for the piece whose place is its own.
     auto swizzle = [](int row) { return PIECES == 8 ? (row >> 1) & 7 : row & 15; };
     const unsigned char* base[LOADS];      // (uniform: a wavefront's load lies in one matrix)
-    unsigned offset[LOADS];
+    typedef typename std::conditional<FAR, size_t, unsigned>::type Offset;
+    Offset offset[LOADS];
 #pragma unroll
     for (int q = 0; q < LOADS; ++q) {
         const int first = (wid * LOADS + q) * ROWS_PER_LOAD, row = first + lane / PIECES;
         // (rows beyond the matrices: the last one; what is computed from it is never stored)
         if (first < BM) {
             base[q] = reinterpret_cast<const unsigned char*>(A + static_cast<size_t>(m0) * lda);
-            offset[q] = static_cast<unsigned>(min(row, M - 1 - m0)) * lda * 2;
+            offset[q] = static_cast<Offset>(min(row, M - 1 - m0)) * lda * 2;
         } else {
             const int w_row = row - BM, n = GATED ? w_row / 64 * 32 + w_row % 32 : w_row;
             const bf16_t* map = W;
             if constexpr (GATED) map = (first - BM) / 32 % 2 ? kv.up : W;
             base[q] = reinterpret_cast<const unsigned char*>(map + static_cast<size_t>(n0) * ldw);
-            offset[q] = static_cast<unsigned>(min(n, N - 1 - n0)) * ldw * 2;
+            offset[q] = static_cast<Offset>(min(n, N - 1 - n0)) * ldw * 2;
         }
         offset[q] += (lane % PIECES ^ swizzle(row)) * 16;
     }
@@ -216,7 +225,7 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
     const int nk = (K + BK - 1) / BK, rest = K - (nk - 1) * BK;      // k tiles; columns of the last
     auto fetch = [&](int q, int t, int stage) {                     // t: past the last tile, the last one again
         t = min(t, nk - 1);
-        unsigned at = offset[q];
+        Offset at = offset[q];
         if (EDGE && t == nk - 1) {
             // (pieces beyond K: the row's last one, against zeros)
             const int piece = (lane % PIECES ^ swizzle((wid * LOADS + q) * ROWS_PER_LOAD + lane / PIECES)) * 16;
@@ -447,19 +456,19 @@ static int split_among_xcds(int tiles_m, int tiles_n, int bm, int bn, int& xm, i
     return ((tiles_m + xm - 1) / xm) * ((tiles_n + xn - 1) / xn) * N_XCD;
 }
 
-template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG = 1, bool HALVES = false>
+template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG = 1, bool HALVES = false, bool FAR = false>
 static void launch_tiled_gated(const bf16_t* a, int lda, const bf16_t* w, int ldw, void* C, int ldc, int M, int N, int K,
                                const GatedPair& pair, hipStream_t stream) {
     constexpr int BM = WM * TM * 32, BN = WN * TN * 32;
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN / 2 - 1) / (BN / 2);
     int xm, xn;
     const dim3 grid(split_among_xcds(tiles_m, tiles_n, BM, BN, xm, xn)), block(WM * WN * KG * 64);
-#define TILED(E) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, E, EPI_GATED><<<grid, block, 0, stream>>>(a, lda, w, ldw, nullptr, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, pair)
-    if (K % BK != 0) TILED(true); else TILED(false);
+#define TILED(E) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, FAR, E, EPI_GATED><<<grid, block, 0, stream>>>(a, lda, w, ldw, nullptr, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, pair)
+    if (FAR || K % BK != 0) TILED(true); else if constexpr (!FAR) TILED(false);
 #undef TILED
 }
 
-template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG = 1, bool HALVES = false>
+template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG = 1, bool HALVES = false, bool FAR = false>
 static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, const float* bias, void* C, int ldc,
                          int M, int N, int K, int mode, hipStream_t stream, KvScatter kv = KvScatter{},
                          const MllmStreamAdd* through = nullptr) {
@@ -467,18 +476,18 @@ static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, con
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
     int xm, xn;
     const dim3 grid(split_among_xcds(tiles_m, tiles_n, BM, BN, xm, xn)), block(WM * WN * KG * 64);
-    const bool edge = K % BK != 0;      // rows and columns beyond the matrices need no other kernel
-#define TILED(E, MD) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, E, MD><<<grid, block, 0, stream>>>(a, lda, w, ldw, bias, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, extra)
+    const bool edge = FAR || K % BK != 0;      // rows and columns beyond the matrices need no other kernel
+#define TILED(E, MD) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, FAR, E, MD><<<grid, block, 0, stream>>>(a, lda, w, ldw, bias, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, extra)
     if (mode == EPI_THROUGH) {
         const MllmStreamAdd extra = *through;
-        if (edge) TILED(true, EPI_THROUGH); else TILED(false, EPI_THROUGH);
+        if (edge) TILED(true, EPI_THROUGH); else if constexpr (!FAR) TILED(false, EPI_THROUGH);
         return;
     }
     const KvScatter extra = kv;
-#define TILED_MODE(MD) case MD: if (edge) TILED(true, MD); else TILED(false, MD); break;
+#define TILED_MODE(MD) case MD: if (edge) TILED(true, MD); else if constexpr (!FAR) TILED(false, MD); break;
     switch (mode) {
         TILED_MODE(EPI_STORE) TILED_MODE(EPI_GELU_TANH) TILED_MODE(EPI_GELU_ERF) TILED_MODE(EPI_RELU2) TILED_MODE(EPI_ADD_RESIDUAL)
-        default: if (edge) TILED(true, EPI_STORE_F32); else TILED(false, EPI_STORE_F32); break;
+        default: if (edge) TILED(true, EPI_STORE_F32); else if constexpr (!FAR) TILED(false, EPI_STORE_F32); break;
     }
 #undef TILED_MODE
 #undef TILED
@@ -1410,13 +1419,14 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
                                                                                 nullptr, 0.f, nullptr, stream, workspace, workspace_bytes,
                                                                                 MergedA{}, 0, through, kv) == 0) {
         // few rows: weight-streaming kernel
-    } else if (lda > 1 << 23 || ldw > 1 << 23) {
-        return -1;          // (a tile's rows are reached by 32-bit byte offsets)
-    } else if (M <= 32) {
-        launch_tiled<1, 4, 1, 1, 64, 4>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through);
     } else {
 #define TILE(...) launch_tiled<__VA_ARGS__>(a, lda, w, ldw, bias, C, ldc, M, N, K, mode, stream, kv, through)
-        if (sums_in_halves(M, N, K)) {
+        const bool far = lda > NEAR_ROWS || ldw > NEAR_ROWS, halves = M > 32 && sums_in_halves(M, N, K);
+        if (far) {
+            if (halves) TILE(2, 2, 1, 1, 128, 4, 2, false, true); else TILE(2, 2, 1, 1, 64, 6, 1, false, true);
+        } else if (M <= 32) {
+            TILE(1, 4, 1, 1, 64, 4);
+        } else if (halves) {
             switch (cheapest_tile(halved_tiles, 7, M, N, K)) {
                 case 0: TILE(2, 4, 2, 2, 64, 3, 1, true); break;
                 case 1: TILE(4, 2, 1, 3, 64, 3, 1, true); break;
@@ -1445,7 +1455,7 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
 extern "C" {
 
 // Returns 0, a HIP error code, or -1 when K or the row strides are not multiples of 8
-// elements, a base pointer is not 16-byte aligned, or rows of a product on tiles lie more than 2^23 elements apart.
+// elements or a base pointer is not 16-byte aligned.
 // `workspace` (optional; 4-byte aligned, zero when first handed over, never written by anyone else)
 // lets narrow products of few rows and a long K share a tile among several workgroups: 16 KB of
 // counters, then 1 KB per workgroup of such a launch (at most 256). Launches that use one
@@ -1559,7 +1569,7 @@ int mllm_gated_gemm_bf16(const void* A, int lda, const void* gate, const void* u
                          int M, int N, int K, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
     if (K % 8 != 0 || lda % 8 != 0 || ldw % 8 != 0) return -1;
-    if (((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) || lda > 1 << 23 || ldw > 1 << 23) return -1;
+    if ((reinterpret_cast<uintptr_t>(A) | reinterpret_cast<uintptr_t>(gate) | reinterpret_cast<uintptr_t>(up)) & 15) return -1;
     const bf16_t *a = static_cast<const bf16_t*>(A), *w = static_cast<const bf16_t*>(gate);
     const GatedPair pair{static_cast<const bf16_t*>(up), limit, alpha};
     // (the columns of both maps counted; few tiles of 64x64 are summed in halves, a rule that stays as sums_in_halves does)
@@ -1573,13 +1583,15 @@ int mllm_gated_gemm_bf16(const void* A, int lda, const void* gate, const void* u
         if (cost < best_cost) { best_cost = cost; best = c; }
     }
     static const TilePrice gated_tiles[] = {plain_tiles[0], plain_tiles[2], plain_tiles[3]};
-    if (best < 3) best = cheapest_tile(gated_tiles, 3, M, 2 * N, K);
+    const bool far = lda > NEAR_ROWS || ldw > NEAR_ROWS;
+    if (best < 3) best = far ? 4 : cheapest_tile(gated_tiles, 3, M, 2 * N, K);
 #define TILE(...) launch_tiled_gated<__VA_ARGS__>(a, lda, w, ldw, C, ldc, M, N, K, pair, stream)
     switch (best) {
         case 0: TILE(2, 4, 2, 2, 64, 3); break;
         case 1: TILE(4, 2, 1, 2, 64, 4); break;
         case 2: TILE(2, 2, 1, 2, 64, 4); break;
-        default: TILE(2, 1, 1, 2, 128, 4, 2); break;
+        case 3: if (far) TILE(2, 1, 1, 2, 128, 4, 2, false, true); else TILE(2, 1, 1, 2, 128, 4, 2); break;
+        default: TILE(2, 2, 1, 2, 64, 4, 1, false, true); break;
     }
 #undef TILE
     MLLM_LAUNCH_CHECK();

@@ -203,6 +203,49 @@ def test_linear_bf16_stages_and_remainders(ops, M, N, K):
     assert bool(((got - (x + want)).abs() <= 1e-4).all())
 
 
+@pytest.mark.parametrize("M,N,K,far", [(17, 48, 200, "aw"),             # few rows
+                                       (2, 16404, 4096, "a"),           # of a width that the few-row kernel refuses
+                                       (300, 48, 200, "aw"), (300, 48, 2056, "aw"), (300, 48, 2048, "w"),     # sums in halves
+                                       (200, 4104, 200, "a"), (200, 4104, 2056, "a")])                        # and in one
+def test_linear_bf16_rows_far_apart(ops, M, N, K, far):
+    """Rows more than 2^23 elements apart, where a tile's 32-bit offsets end: every form of the product gives the bits it gives for
+    the same rows side by side."""
+    import ctypes
+    stride = (1 << 23) + 8
+    g = torch.Generator().manual_seed(M + N + K)
+
+    def apart(t):
+        out = torch.empty((t.shape[0] - 1) * stride + K, dtype=t.dtype, device=DEV).as_strided(t.shape, (stride, 1))
+        return out.copy_(t)
+
+    a, w, up = (_rand((n, K), torch.bfloat16, g, s).to(DEV) for n, s in ((M, 1), (N, K ** -0.5), (N, K ** -0.5)))
+    bias, x = _rand((N,), torch.float32, g).to(DEV), _rand((M, N), torch.float32, g).to(DEV)
+    a2, w2, up2 = apart(a) if "a" in far else a, apart(w) if "w" in far else w, apart(up) if "w" in far else up
+    for epilogue in ("store", "gelu_tanh", "gelu_erf", "add_residual", "store_f32"):
+        got = [x.clone() if epilogue in ("add_residual", "store_f32") else x.bfloat16() for _ in range(2)]
+        ops.linear(a, w, bias, got[0], epilogue)
+        ops.linear(a2, w2, bias, got[1], epilogue)
+        assert torch.equal(*got), epilogue
+    kv = N // 3 // 4 * 4
+    pages, got = [[torch.zeros(M, kv, dtype=torch.bfloat16, device=DEV) for _ in range(2)] for _ in range(2)], [x.bfloat16() for _ in range(2)]
+    slots = torch.randperm(M, generator=g).to(torch.int32).to(DEV)
+    ops.linear(a, w, bias, got[0], "store", kv_scatter=(slots, *pages[0], N - 2 * kv))
+    ops.linear(a2, w2, bias, got[1], "store", kv_scatter=(slots, *pages[1], N - 2 * kv))
+    assert torch.equal(*got) and all(torch.equal(*p) for p in zip(*pages))
+    streams, copies, rooms = [x.clone() for _ in range(2)], [x.bfloat16() for _ in range(2)], [torch.empty_like(x) for _ in range(2)]
+    ops.linear_stream_add(a, w, streams[0], bias, rooms[0], copy=copies[0])
+    ops.linear_stream_add(a2, w2, streams[1], bias, rooms[1], copy=copies[1])
+    assert torch.equal(*streams) and torch.equal(*copies)
+    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    fn = ops.engine_library().mllm_gated_gemm_bf16
+    fn.argtypes = [vp, i, vp, vp, i, f, f, vp, i, i, i, i, vp]
+    got = [torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=DEV) for _ in range(2)]
+    for out, (p, q, r) in zip(got, ((a, w, up), (a2, w2, up2))):
+        assert fn(p.data_ptr(), p.stride(0), q.data_ptr(), r.data_ptr(), q.stride(0), 7.0, 1.702, out.data_ptr(), N, M, N, K, None) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("M,H,Hkv,dh,K", [(2048, 12, 12, 64, 768),      # 128x192 tiles
                                           (300, 6, 2, 16, 96),         # 64x64 tiles, ragged, grouped heads
                                           (70, 3, 3, 48, 144),         # just above the few-row kernel
