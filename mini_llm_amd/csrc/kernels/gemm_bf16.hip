@@ -145,6 +145,14 @@ template <int N>
 __device__ __forceinline__ void wait_loads_and_meet() {
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" :: "n"(N) : "memory");
 }
+// The same for a number of k tiles that may stay under way, at most MOST (all wavefronts of a workgroup pass the same).
+template <int MOST, int LOADS>
+__device__ __forceinline__ void wait_tiles_and_meet(int under_way) {
+    if constexpr (MOST > 0) {
+        if (under_way < MOST) return wait_tiles_and_meet<MOST - 1, LOADS>(under_way);
+    }
+    wait_loads_and_meet<MOST * LOADS>();
+}
 
 // How far apart (in elements) the rows of a matrix may lie for the 32-bit byte offsets from a tile's first row to the other 255 and a
 // k tile's pieces. Beyond it (FAR) a lane forms 64-bit addresses, which only one shape of tile for either order of sums does: rows over 16 MiB
@@ -223,8 +231,7 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
     }
     const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem));
     const int nk = (K + BK - 1) / BK, rest = K - (nk - 1) * BK;      // k tiles; columns of the last
-    auto fetch = [&](int q, int t, int stage) {                     // t: past the last tile, the last one again
-        t = min(t, nk - 1);
+    auto fetch = [&](int q, int t, int stage) {
         Offset at = offset[q];
         if (EDGE && t == nk - 1) {
             // (pieces beyond K: the row's last one, against zeros)
@@ -257,9 +264,11 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
         for (int i = 0; i < TM; ++i) fetch_old(i);
     }
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
+    for (int s = 0; s < STAGES - 1; ++s) {
+        if (s >= nk) break;
 #pragma unroll
         for (int q = 0; q < LOADS; ++q) fetch(q, s, s);
+    }
 
     f32x16 acc[TM][TN], acc2[TM][TN];      // (acc2: only with HALVES)
 #pragma unroll
@@ -306,41 +315,61 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
     // of tile t + STAGES - 1 (into the stage that tile t - 1 left: all wavefronts had read it when they last met), the fragment
     // reads of the next k step and its MFMAs; the scheduling barriers keep that order. In front of the last step's MFMAs the
     // wavefronts wait for tile t + 1 and meet, and read its first fragments: met behind them instead, all wavefronts would stand at the
-    // barrier and then for these reads with idle matrix units (36.5 > 31.4 us at 2,048 x 2,304 x 3,072).
-    wait_loads_and_meet<(STAGES - 2) * LOADS>();
+    // barrier and then for these reads with idle matrix units (36.5 > 31.4 us at 2,048 x 2,304 x 3,072). The last STAGES - 1 tiles ask
+    // for nothing and wait for fewer and fewer loads. (Asking for the last tile again there, so that one loop did for all, cost short
+    // sums most: 2,048 x 2,048 x 512 12.0 > 8.9 us, 4,096 x 2,048 x 256 16.5 > 11.2, 8,192 x 3,072 x 192 34.6 > 24.4.)
+    wait_tiles_and_meet<STAGES - 2, LOADS>(nk - 1);
     read_frags(0, 0, 0);
     int stage_at = 0, fetch_stage = STAGES - 1;
-    auto tile = [&](int t, f32x16 (&sum)[TM][TN]) {
+    auto step = [&](auto fetches, int t, f32x16 (&sum)[TM][TN]) {
+        constexpr bool FETCHES = decltype(fetches)::value;
         const int next_at = stage_at == (STAGES - 1) * STAGE_BYTES ? 0 : stage_at + STAGE_BYTES;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
             for (int q = 0; q < LOADS; ++q)
-                if (q * KS / LOADS == ks) fetch(q, t + STAGES - 1, fetch_stage);
+                if (FETCHES && q * KS / LOADS == ks) fetch(q, t + STAGES - 1, fetch_stage);
             if (ks + 1 < KS) {
                 read_frags(stage_at, ks + 1, (ks + 1) & 1);
-            } else {
+            } else if (FETCHES) {
                 wait_loads_and_meet<(STAGES - 2) * LOADS>();
                 read_frags(next_at, 0, 0);
+            } else if (t + 1 < nk) {
+                wait_tiles_and_meet<STAGES - 3, LOADS>(nk - 2 - t);
+                read_frags(next_at, 0, 0);
             }
-            if (EDGE && t == nk - 1) zero_beyond(ks & 1, ks);
+            if (EDGE && !FETCHES && t == nk - 1) zero_beyond(ks & 1, ks);
             mma(ks & 1, sum);
             __builtin_amdgcn_sched_barrier(0);
         }
         stage_at = next_at;
         fetch_stage = fetch_stage == STAGES - 1 ? 0 : fetch_stage + 1;
     };
+    // (Loops of their own: a choice of both in one loop has every sum twice in registers, and moves them.)
+    const std::true_type asking;
+    const std::false_type done;
+    int t = 0;
     if constexpr (HALVES) {
-        for (int t = 0; t < nk; t += 2) {
-            tile(t, acc);
-            if (t + 1 < nk) tile(t + 1, acc2);
+        for (; t + STAGES < nk; t += 2) {
+            step(asking, t, acc);
+            step(asking, t + 1, acc2);
+        }
+        if (t + STAGES - 1 < nk) {
+            step(asking, t, acc);
+            step(done, t + 1, acc2);
+            t += 2;
+        }
+        for (; t < nk; t += 2) {
+            step(done, t, acc);
+            if (t + 1 < nk) step(done, t + 1, acc2);
         }
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) acc[i][j] += acc2[i][j];
     } else {
-        for (int t = 0; t < nk; ++t) tile(t, acc);
+        for (; t + STAGES - 1 < nk; ++t) step(asking, t, acc);
+        for (; t < nk; ++t) step(done, t, acc);
     }
     wait_loads_and_meet<0>();          // (nothing of the tiles is on its way or read any more)
     if (tid < BN) bias_s[tid] = bias_r;

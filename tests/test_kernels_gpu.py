@@ -203,6 +203,22 @@ def test_linear_bf16_stages_and_remainders(ops, M, N, K):
     assert bool(((got - (x + want)).abs() <= 1e-4).all())
 
 
+@pytest.mark.parametrize("M,N", [(300, 40), (520, 772), (1030, 3072), (2100, 2300)])
+def test_linear_bf16_of_no_columns(ops, M, N):
+    """A product on tiles that has no k tile asks for none: the bias alone, on every tile, and the old values stay."""
+    import ctypes
+    vp, i = ctypes.c_void_p, ctypes.c_int
+    fn = ops.engine_library().mllm_gemm_bf16
+    fn.argtypes = [vp, i, vp, i, vp, vp, i, i, i, i, i, vp, ctypes.c_size_t, vp]
+    g = torch.Generator().manual_seed(M + N)
+    bias, x = _rand((N,), torch.float32, g).to(DEV), _rand((M, N), torch.float32, g).to(DEV)
+    row = torch.zeros(64, dtype=torch.bfloat16, device=DEV)
+    for mode, out, want in ((0, torch.empty(M, N, dtype=torch.bfloat16, device=DEV), bias.bfloat16().expand(M, N)), (3, x.clone(), x + bias)):
+        assert fn(row.data_ptr(), 0, row.data_ptr(), 0, bias.data_ptr(), out.data_ptr(), N, M, N, 0, mode, None, 0, None) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(out, want), mode
+
+
 @pytest.mark.parametrize("M,N,K,far", [(17, 48, 200, "aw"),             # few rows
                                        (2, 16404, 4096, "a"),           # of a width that the few-row kernel refuses
                                        (300, 48, 200, "aw"), (300, 48, 2056, "aw"), (300, 48, 2048, "w"),     # sums in halves
