@@ -170,7 +170,8 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
 // pass covers K up to 3,072; beyond, the next pass's weights are on their way while one is used. What the epilogue adds is asked for
 // first. Bound by the chain launch, activations, weights, sums: 8 x 768 x 768 and 8 x 768 x 3,072 in a decode step 4.1 and 6.0
 // us, together 17.1 with a column a wavefront.
-template <int ROWS, int STEPS>
+// RAGGED: K is no multiple of 256, and what lies beyond it has to be left out (8 x 1,600 x 1,600 7.4 us, 7.2 if it were not).
+template <int ROWS, int STEPS, bool RAGGED>
 __global__ void __launch_bounds__(512)
 gemm_f32_narrow_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
                        const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K, int mode) {
@@ -219,9 +220,9 @@ gemm_f32_narrow_kernel(const float* __restrict__ A, int lda, const float* __rest
         if (more) {
             fetch_rows(k0 + KP);
             fetch_weights(next, k0 + KP);
-        } else if (K % 256 != 0) {
+        } else if constexpr (RAGGED) {
             // What lies beyond K is zero in both factors (0 x infinity is none). Neither where it is loaded nor a branch a lane in
-            // front of the products: the loads would wait for each other (8 x 768 x 3,072 11.7 us, 5.6 so).
+            // front of the products: the loads would wait for each other (8 x 1,600 x 1,600 18.2 us).
 #pragma unroll
             for (int s = 0; s < STEPS; ++s)
                 if (k0 + (2 * s + half) * 256 + 4 * lane >= K) w[s] = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -256,6 +257,13 @@ gemm_f32_narrow_kernel(const float* __restrict__ A, int lda, const float* __rest
     const float sum = sums[0][tid / ROWS][out_r] + sums[1][tid / ROWS][out_r];
     if (mode == EPI_ADD_RESIDUAL) static_cast<float*>(C)[out_at] = out_old + (sum + out_bias);
     else epilogue<float>(mode, sum, out_bias, C, out_at);
+}
+
+template <int ROWS, int STEPS>
+static void launch_f32_narrow(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
+    const dim3 grid((N + 3) / 4);
+    if (K % 256 != 0) gemm_f32_narrow_kernel<ROWS, STEPS, true><<<grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+    else gemm_f32_narrow_kernel<ROWS, STEPS, false><<<grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
 }
 
 // More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). Four
@@ -487,9 +495,9 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
             // (3,072 columns a pass take the LDS of a unit: while there is one workgroup a unit; 9 to 16 rows would take twice as much)
             const dim3 rows_grid((N + 3) / 4);
             if (M > 8) gemm_f32_rows_kernel<16, 4><<<rows_grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
-            else if (K <= 1024) gemm_f32_narrow_kernel<8, 2><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
-            else if (N <= 1024) gemm_f32_narrow_kernel<8, 6><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
-            else gemm_f32_narrow_kernel<8, 3><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            else if (K <= 1024) launch_f32_narrow<8, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else if (N <= 1024) launch_f32_narrow<8, 6>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else launch_f32_narrow<8, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
         }
         MLLM_LAUNCH_CHECK();
         return 0;
