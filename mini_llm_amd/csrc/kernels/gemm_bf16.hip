@@ -1377,6 +1377,9 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 // kernel before it wrote and weights that no cache of an XCD holds, as a step has them: what is chosen takes 0.8 % more than the
 // fastest of the tiles on average, where sums come in halves no more. (With rows and weights left in the caches 64x128 tiles beat
 // 64x96 of two groups on the feed-forward's second product, 16.9 to 16.3 us; in a step they take 25.7 us and 22.3.)
+// A K below the fitted ones is priced as their smallest, 768: for shorter sums the lines of the fit end in prices below zero (2,048 x 16,384
+// x 64 83 us on 64x32, 25 on 128x256), and the results to store suit the same tiles as a k loop does: over 624 products of 33 to 8,192 rows,
+// 64 to 50,257 columns and K of 32 to 512 0.6 % more than the fastest tile on average, 19 % at most.
 struct TilePrice { int bm, bn; double launch, round, tile, load; };
 static const TilePrice plain_tiles[] = {{128, 256, 4.15, -0.04, 0.583, 0.320}, {128, 192, 2.98, 0.89, 0.478, 0.232}, {128, 128, 2.39, 1.06, 0.362, 0.172},
                                         {64, 128, 1.57, 1.53, 0.290, 0.070},   {64, 64, 1.57, 1.55, 0.209, 0.051},   {64, 32, 3.80, -0.27, 0.138, 0.040}};
@@ -1391,7 +1394,7 @@ static int cheapest_tile(const TilePrice* prices, int n, int M, int N, int K) {
         const int tiles_m = (M + p.bm - 1) / p.bm, tiles_n = (N + p.bn - 1) / p.bn;
         int xm, xn;
         const int per_xcd = split_among_xcds(tiles_m, tiles_n, p.bm, p.bn, xm, xn) / N_XCD, rounds = (per_xcd + 31) / 32;
-        const double k_tiles = (K + 63) / 64, blocks = static_cast<double>(tiles_m) * tiles_n;
+        const double k_tiles = std::max(12, (K + 63) / 64), blocks = static_cast<double>(tiles_m) * tiles_n;
         const double price = p.launch + rounds * (p.round + p.tile * k_tiles) + p.load * k_tiles * blocks / 256.0;
         if (price < best_price) { best_price = price; best = c; }
     }

@@ -203,6 +203,23 @@ def test_linear_bf16_stages_and_remainders(ops, M, N, K):
     assert bool(((got - (x + want)).abs() <= 1e-4).all())
 
 
+@pytest.mark.parametrize("M,N", [(2048, 16384), (1024, 16384), (8192, 2048)])
+def test_linear_bf16_short_sums_are_not_slower(ops, M, N):
+    """The tile chosen for few columns of K suits them: products of 64 take no longer than those of 512 (half as long is usual; 1.4
+    times as long were those on tiles priced far outside what the prices know)."""
+    took = {}
+    for K in (64, 512):
+        a, w = (torch.randn(n, K, device=DEV).bfloat16() for n in (M, N))
+        out = torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        marks = [torch.cuda.Event(enable_timing=True) for _ in range(12)]
+        for m in marks:
+            ops.linear(a, w, None, out)
+            m.record()
+        torch.cuda.synchronize()
+        took[K] = sorted(x.elapsed_time(y) for x, y in zip(marks[2:], marks[3:]))[4]
+    assert took[64] <= took[512], took
+
+
 @pytest.mark.parametrize("M,N", [(300, 40), (520, 772), (1030, 3072), (2100, 2300)])
 def test_linear_bf16_of_no_columns(ops, M, N):
     """A product on tiles that has no k tile asks for none: the bias alone, on every tile, and the old values stay."""
