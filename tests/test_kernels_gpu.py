@@ -203,6 +203,41 @@ def test_linear_bf16_stages_and_remainders(ops, M, N, K):
     assert bool(((got - (x + want)).abs() <= 1e-4).all())
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 1001, 72), (100, 37, 200), (260, 1003, 776), (300, 70, 2048), (520, 771, 2056), (1030, 3001, 72), (2100, 2305, 200)])
+@pytest.mark.parametrize("start", [0, 1, 3])
+def test_linear_bf16_rows_that_start_anywhere(ops, M, N, K, start):
+    """16-bit results whose rows are no multiple of 8 bytes apart, or whose first element is not aligned, to the bit as in aligned rows (every
+    tile, every epilogue that stores 16 bits), and nothing beside them is written."""
+    import ctypes
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w, up = (_rand((n, K), torch.bfloat16, g, s).to(DEV) for n, s in ((M, 1), (N, K ** -0.5), (N, K ** -0.5)))
+    bias = _rand((N,), torch.float32, g).to(DEV)
+    stride, even = N + 2 + (N % 2 == 0), (N + 15) // 8 * 8
+    assert stride % 2 == 1
+
+    def rooms():
+        odd = torch.full((start + (M + 1) * stride,), 7.0, dtype=torch.bfloat16, device=DEV)[start:].view(M + 1, stride)
+        return torch.full((M, even), 7.0, dtype=torch.bfloat16, device=DEV), odd
+
+    def check(near, odd, what):
+        assert torch.equal(near[:, :N], odd[:M, :N]), what
+        assert bool((odd[:M, N:] == 7).all()) and bool((odd[M] == 7).all()), what
+
+    for epilogue in ("store", "gelu_tanh", "gelu_erf"):
+        near, odd = rooms()
+        ops.linear(a, w, bias, near[:, :N], epilogue)
+        ops.linear(a, w, bias, odd[:M, :N], epilogue)
+        check(near, odd, epilogue)
+    vp, i, f = ctypes.c_void_p, ctypes.c_int, ctypes.c_float
+    fn = ops.engine_library().mllm_gated_gemm_bf16
+    fn.argtypes = [vp, i, vp, vp, i, f, f, vp, i, i, i, i, vp]
+    near, odd = rooms()
+    for out, ld in ((near, even), (odd, stride)):
+        assert fn(a.data_ptr(), K, w.data_ptr(), up.data_ptr(), K, 7.0, 1.702, out.data_ptr(), ld, M, N, K, None) == 0
+    torch.cuda.synchronize()
+    check(near, odd, "gated")
+
+
 @pytest.mark.parametrize("M,N", [(2048, 16384), (1024, 16384), (8192, 2048)])
 def test_linear_bf16_short_sums_are_not_slower(ops, M, N):
     """The tile chosen for few columns of K suits them: products of 64 take no longer than those of 512 (half as long is usual; 1.4
