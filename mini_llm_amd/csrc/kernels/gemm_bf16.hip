@@ -2,8 +2,8 @@
 //   C[M,N] = A[M,K] * W[N,K]^T + bias, with the epilogues of common.h fused
 // (bias, GELU, residual add into the fp32 stream, fp32 store for logits).
 // Both operands are k-contiguous, so each lane feeds v_mfma_f32_32x32x16_bf16 with one
-// 16-byte LDS read per operand. Tiles are staged through LDS with the next tile's
-// global loads in flight during the current tile's MFMAs.
+// 16-byte LDS read per operand. Many rows: tiles of both matrices in stages of LDS, loaded
+// several k tiles ahead; few rows: the weights streamed once (each described below).
 //
 // It stands where the reference has its tiled SGEMM with fused store path
 // (/root/reference/src/kernels/gemm.cu:394-580, epilogue :534-564).
@@ -25,10 +25,11 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 // tile, each on half of a twice as wide k tile. The weight fragment is the MFMA's A operand, so a lane's accumulator registers hold 4
 // consecutive columns of one output row; the epilogue turns that, through LDS, into stores of whole rows.
 // Bound by the rate at which a compute unit takes tiles from its L2 and by what the matrix units wait around the barriers: at 2,048 x
-// 2,304 x 3,072 the products alone take 24.8 us, the loads alone 25.6, both 31.4. (With tiles loaded into registers and written to LDS from there,
-// at 78 bytes a clock, 40.3: 13 such instructions' time a k tile of 128x192. us, weights and rows cold, before / now: 2,048 x 2,304 x
-// 768 17.8 / 15.6 and x 3,072 x 768 18.2 / 16.6 in a step; alone 2,048 x 4,800 x 1,600 46.8 / 39.0, 2,048 x 6,400 x 1,600 58.4 / 48.0,
-// 2,048 x 1,600 x 6,400 60.0 / 45.4, 560 x 3,072 x 768 8.1 / 6.8, 256 x 3,072 x 768 6.5 / 5.2.)
+// 2,304 x 3,072 the products alone take 24.8 us, the loads alone 25.6, both 30.5. (With tiles loaded into registers and written to LDS from there,
+// at 78 bytes a clock, 37.5. us, so / now, alone with weights and rows that no cache holds: 2,048 x 2,304 x 768 14.9 / 12.7, 2,048 x 3,072
+// x 768 15.7 / 14.0, 2,048 x 4,800 x 1,600 42.1 / 36.5, 2,048 x 6,400 x 1,600 53.8 / 45.9, 560 x 3,072 x 768 7.9 / 7.3, 256 x 3,072 x 768 6.4 /
+// 6.2; in a step of 2,048 rows, where a kernel before wrote the rows, 18.3 / 15.4, 18.2 / 17.1, 52.9 / 40.3, 64.6 / 50.9. Long sums in
+// halves gain in a step only: 2,048 x 1,600 x 6,400 55.2 / 57.8 alone, 64.3 / 59.3 there.)
 // ---------------------------------------------------------------------------------------------
 // Optional second destination of a plain bf16 store: columns [q_cols, q_cols + kv_dim) of output row
 // m also go to row slots[m] of the key pages and the next kv_dim columns to the value pages (the
@@ -1391,7 +1392,8 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 }
 
 
-// Tile choice. A compute unit holds one workgroup at a time (its stages fill the LDS), so the workgroups of an XCD run in rounds of 32. A
+// Tile choice. A compute unit holds one workgroup at a time (its stages fill the LDS; of the six stages of plain 64x32 tiles it holds two, which their
+// fitted numbers contain), so the workgroups of an XCD run in rounds of 32. A
 // product is priced in microseconds as the launch, a round's start and end, and its k tiles, which take longer the more units load
 // side by side. The numbers are fitted to 74 products of 96 to 8,000 rows, 768 to 6,400 columns and as many summed, each with rows that a
 // kernel before it wrote and weights that no cache of an XCD holds, as a step has them: what is chosen takes 0.8 % more than the
@@ -1421,9 +1423,12 @@ static int cheapest_tile(const TilePrice* prices, int n, int M, int N, int K) {
     return best;
 }
 
-// Which products are summed in two halves (HALVES, or two groups of wavefronts): those that tiles of at most 128x128 suit by the count of
-// workgroups, where K is long, and the smallest. It is a rule of its own, apart from the tile: the tile may change with what is
-// measured, the order of the sums, and with it the last bit of every result, does not.
+// Which products are summed in two halves (HALVES, or two groups of wavefronts). A rule of sizes alone, apart from the tile: the tile may change with
+// what is measured, the order of the sums, and with it the last bit of every result, does not. Each of seven tile sizes is weighed as its
+// rounds of 256 workgroups times its area over its efficiency, and the lightest says: 64x32, which is any product of up to 256 such tiles,
+// halves; 64x64, 64x96 (results of up to 1,024 columns) and 128x128 halves from K = 2,048 on; the others never. (The efficiencies are
+// those of the kernel that the rule was made for and price nothing any more. What it costs: by the prices 4 % of 2,048 x 1,600 x 6,400;
+// few workgroups gain from halves, as two groups then share a tile's k loop.)
 static bool sums_in_halves(int M, int N, int K) {
     struct Shape { int bm, bn; double efficiency; };
     static const Shape shapes[] = {{128, 256, 1.05}, {128, 192, 1.0}, {128, 128, 0.9}, {64, 128, 0.7},
@@ -1451,8 +1456,11 @@ static int gemm_bf16_dispatch(const void* A, int lda, const void* W, int ldw, co
     // logits head) the weight-streaming kernel, always. In between both are priced, in microseconds,
     // by formulas fitted to measurements on the products of GPT-2 small to XL at 24 to 256 rows: the
     // weight-streaming kernel runs its 16-row by 16-column workgroups in rounds of 256 whose time
-    // grows with K (steeply beyond 3072, where a wavefront's share of K no longer fits its chunks);
-    // the tiled kernel's time is its k loop, a little more where K makes it take the checked loop.
+    // grows with K (steeply beyond 3072, where a wavefront's share of K no longer fits its chunks).
+    // The tiles' formula is that of tiles loaded through registers and stays, as the two kernels add in another order and the line
+    // between them is in every result's last bit. With today's tiles it still takes the faster kernel, within 5 %, for 108 of 120 products
+    // of 20 to 256 rows of those models. The others (us, taken / the other kernel, operands cold): 20 to 32 rows of 4,800 and 6,400 x 1,600
+    // 9.3 / 8.8 and 11.7 / 8.8, 40 and 48 of 2,304 x 768 5.5 / 4.6, 40 to 64 of 1,024 x 4,096 12.6 / 10.5, 96 and 128 of 768 x 768 5.1 / 4.5.
     const int col_tiles = (N + 15) / 16, row_blocks16 = (M + 15) / 16;
     auto streaming_is_faster = [&]() {
         const double rounds = static_cast<double>((static_cast<long>(col_tiles) * row_blocks16 + 255) / 256);
