@@ -271,6 +271,23 @@ def test_linear_bf16_of_no_columns(ops, M, N):
         assert torch.equal(out, want), mode
 
 
+@pytest.mark.parametrize("N,K,rows", [(1000, 2120, (260, 520, 1030, 1300, 2100)),      # sums in halves: 64x32, 64x64, 64x96, 64x128, 128x128
+                                      (1600, 2056, (260, 520, 1300, 2100)),            # and 128x192
+                                      (2304, 776, (260, 400, 800, 1700, 2600))])       # in one: 64x64 to 128x256
+@pytest.mark.parametrize("epi", ["store", "add_residual"])
+def test_linear_bf16_tiles_add_in_one_order(ops, N, K, rows, epi):
+    """Row counts that take different tiles, with sums of one kind: the rows they share have the same bits."""
+    g = torch.Generator().manual_seed(N + K)
+    a, w = _rand((max(rows), K), torch.bfloat16, g).to(DEV), _rand((N, K), torch.bfloat16, g, K ** -0.5).to(DEV)
+    bias, x = _rand((N,), torch.float32, g).to(DEV), _rand((max(rows), N), torch.float32, g).to(DEV)
+    first = None
+    for M in rows:
+        out = x[:M].clone() if epi == "add_residual" else torch.empty(M, N, dtype=torch.bfloat16, device=DEV)
+        ops.linear(a[:M], w, bias, out, epi)
+        first = out if first is None else first
+        assert torch.equal(out[:rows[0]], first), M
+
+
 @pytest.mark.parametrize("M,N,K,far", [(17, 48, 200, "aw"),             # few rows
                                        (2, 16404, 4096, "a"),           # of a width that the few-row kernel refuses
                                        (300, 48, 200, "aw"), (300, 48, 2056, "aw"), (300, 48, 2048, "w"),     # sums in halves
