@@ -58,8 +58,8 @@ LIBRARIES: Dict[str, dict] = {
     # plain C++ twins of the device operations: the oracle of the kernel tests (host only)
     "ref": {"kind": "cxx", "sources": ["ref/ref_ops.cc"], "headers": []},
     "elementwise": {"kind": "hip", "sources": ["kernels/elementwise.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
-    "gemm_f32": {"kind": "hip", "sources": ["kernels/gemm_f32.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
-    "gemm_bf16": {"kind": "hip", "sources": ["kernels/gemm_bf16.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
+    "gemm_f32": {"kind": "hip", "sources": ["kernels/gemm_f32.hip"], "headers": ["kernels/common.h", "kernels/lds_loads.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
+    "gemm_bf16": {"kind": "hip", "sources": ["kernels/gemm_bf16.hip"], "headers": ["kernels/common.h", "kernels/lds_loads.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "attention": {"kind": "hip", "sources": ["kernels/attention.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "attention_decode": {"kind": "hip", "sources": ["kernels/attention_decode.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "attention_prefill": {"kind": "hip", "sources": ["kernels/attention_prefill.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},

@@ -7,8 +7,10 @@
 // (/root/reference/src/kernels/gemm.cu:238-392: alpha*acc + beta*old + bias, optional GELU),
 // with the weight held as [N,K] (k contiguous) instead of [K,N].
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
+#include "lds_loads.h"
 
 #define F32_BM 64
 #define F32_BN 64
@@ -266,129 +268,225 @@ static void launch_f32_narrow(const float* A, int lda, const float* W, int ldw, 
     else gemm_f32_narrow_kernel<ROWS, STEPS, false><<<grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
 }
 
-// More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). Four
-// wavefronts, two by two, of TM x TN tiles of 16 x 16 each share k tiles of 32 columns (a row's piece is one 128-byte line) in
-// LDS, double buffered with one barrier a tile; the loads of the two tiles behind the next are in flight in registers. KG such
-// groups take the 32-column parts of a KG times as wide k tile and add their sums in LDS: for few tiles, where the chain of
-// k tiles (LDS write, barrier, read, products: 0.34 us) is what a workgroup waits for. A lane's 16-byte read holds the k
-// columns of four matrix instructions (lane group l / 16 takes columns 4 (l / 16) to + 3 of 16, the same for both operands);
-// rows are an odd number of 16-byte pieces apart (16 lanes on 16 different groups of banks). The weights are the
-// instruction's first operand, so that a lane ends up with four neighbouring columns of one row. Sixteen columns are summed on
-// their own before they join an output's sum, with tiles of 16 x 16 a wavefront 32 columns in eight sums: the error against 64 bits
-// (2-norm over 2-norm, normal values) is 1.5e-7 at K = 768 and 2.0e-7 at 3,072, with eight sums and four groups 8.8e-8 and 1.2e-7,
-// where one chain of FMAs had 5.0e-7 and 9.9e-7 and the kernel for few rows has 9.3e-8 and 1.4e-7. (Four sums of 16 columns, 9.6e-8
-// and 1.5e-7, were a little less exact than that kernel, which took up to 64 rows before; up to K = 256 the two are alike.)
-// Bound by the matrix cores where the tiles fill the chip evenly, else by the units that take one tile more or by that chain.
-// 2,048 x 3,072 x 768: 91 us (106 TFLOP/s of the 155 a loop of these instructions reaches; a kernel of vector FMAs on 64 x 64
-// tiles took 134); 2,048 x 768 x 3,072: 99 (209); 570 x 768 x 3,072: 40 (197); 64 x 768 x 3,072: 24 (the kernel for few
-// rows: 59). Needs K and the row strides in multiples of 4 floats, 16-byte aligned operands.
+// More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). WM x WN
+// wavefronts of TM x TN tiles of 16 x 16 each share k tiles of 32 columns (a row's piece is one 128-byte line) in STAGES stages of LDS,
+// filled by loads that write LDS without passing through registers, one barrier a tile. KG such groups take the 32-column parts of
+// a KG times as wide k tile and add their sums in LDS. A lane's 16-byte read holds the k columns of four matrix instructions (lane
+// group l / 16 takes columns 4 (l / 16) to + 3 of 16, the same for both operands). The weights are the instruction's first operand, so
+// that a lane ends up with four neighbouring columns of one row. While a step of 16 columns multiplies, the fragments of the next are
+// read (the scheduling barriers keep the reads in front: left alone, the compiler puts them behind the products and waits for them) and the
+// sums of the one before join the outputs'.
+//
+// How an output is summed decides its error: SUMS = 1 makes sums of 16 columns that join one after the other, 4 eight sums of four columns
+// a k tile that are added pairwise first; the 32-column parts of K go to PARTS x KG sums in turn, which are added at the end (which
+// of both the factors is does not change a bit). The error against 64 bits (2-norm over 2-norm, normal values, K = 768 and 3,072) is
+// 1.5e-7 and 2.4e-7 with one sum, 1.2e-7 and 2.0e-7 with two, 9.1e-8 and 1.2e-7 with four of eight sums; one chain of FMAs had 5.0e-7 and
+// 9.9e-7, the kernel for few rows has 9.3e-8 and 1.4e-7.
+//
+// Bound by the matrix cores (busy in 78 % of a unit's clocks at 2,048 x 3,072 x 768, where units idle for another 15 % of the
+// launch, at its start and while the last tiles run out) or, where tiles are few, by a workgroup's chain of k tiles. Weights from memory,
+// with loads that pass through registers before: 2,048 x 3,072 x 768 95 > 84 us (115 TFLOP/s of the 155 a loop of these instructions reaches),
+// 2,048 x 768 x 3,072 102 > 88, 560 x 768 x 3,072 44 > 39, 64 x 768 x 3,072 25.2 > 20.1, 64 x 50,257 x 768 80 > 68. Larger tiles
+// (128 x 128, 128 x 192) are no faster, so it is not the loads either. Needs K and the row strides in multiples of 4 floats,
+// 16-byte aligned operands.
 #define F32T_BK 32
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
-template <int TM, int TN, int KG>
-__global__ void __launch_bounds__(256 * KG)
+template <int WM, int WN, int TM, int TN, int KG, int PARTS, int STAGES, int SUMS, bool EDGE>
+__global__ void __launch_bounds__(WM * WN * KG * 64)
 gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, const float* __restrict__ bias,
                       void* __restrict__ C, int ldc, int M, int N, int K, int mode, int tiles_m, int tiles_n, int down) {
-    constexpr int BM = 32 * TM, BN = 32 * TN, ROWS = BM + BN, BK = F32T_BK * KG, STRIDE = BK + 4;
-    constexpr int SUMS = TM * TN == 1 ? 4 : 1;      // an output's 16 columns in so many sums
-    constexpr int THREADS = 256 * KG, PIECES = BK / 4, STEP = THREADS / PIECES, LOADS = ROWS / STEP;      // STEP: rows that all threads load at once
-    static_assert(STEP == 32 && (KG == 1 || KG == 2 || KG == 4) && (KG - 1) * 4 * TM * TN * 64 * 4 <= 2 * ROWS * STRIDE, "the groups' sums fit the tiles' LDS");
-    __shared__ __attribute__((aligned(16))) float tile_s[2][ROWS * STRIDE];      // rows of A, then rows of W
+    constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16, ROWS = BM + BN, BK = F32T_BK * KG, KS = F32T_BK / 16;
+    constexpr int LOADS = (ROWS / 8 + NW - 1) / NW; // of a wavefront and k tile: 8 rows of its group's 32 columns each (the last again where there are fewer)
+    constexpr int SLAB_BYTES = ROWS * F32T_BK * 4, STAGE_BYTES = SLAB_BYTES * KG;
+    static_assert(ROWS % 8 == 0 && BM % 8 == 0 && KS == 2 && STAGES >= 2 && (KG == 1 || KG == 2 || KG == 4), "whole loads, two fragment sets");
+    static_assert((KG - 1) * PARTS * NW * TM * TN * 64 * 16 <= STAGES * STAGE_BYTES, "the groups' sums fit the tiles' LDS");
+    __shared__ __attribute__((aligned(16))) unsigned char smem[STAGES * STAGE_BYTES];
     const int tid = threadIdx.x, lane = tid % 64;
-    const int kg = __builtin_amdgcn_readfirstlane(tid / 256), wave = __builtin_amdgcn_readfirstlane(tid / 64 % 4);
+    const int kg = __builtin_amdgcn_readfirstlane(tid / (64 * NW)), wave = __builtin_amdgcn_readfirstlane(tid / 64 % NW);
     // an XCD (workgroup id % 8) takes an even share of the tiles, neighbours in one direction: with `down` it walks down the
     // rows of A for a few columns of tiles, else along the rows of W for a few rows of tiles
     const int tiles = tiles_m * tiles_n, per = (tiles + 7) / 8, at = (blockIdx.x % 8) * per + blockIdx.x / 8;
     if (blockIdx.x / 8 >= per || at >= tiles) return;
     const int tm = down ? at % tiles_m : at / tiles_n, tn = down ? at / tiles_m : at % tiles_n;
     const int m0 = tm * BM, n0 = tn * BN;
-    // a thread's 16-byte pieces of a tile: rows beyond the matrix read the last one and are never stored
-    const float* src[LOADS];
-    const int piece = 4 * (tid % PIECES), row0 = tid / PIECES;
+
+    // A group's 32 columns of a k tile in LDS are its rows one behind the other (A's, then W's), as the loads leave them. 16-byte piece
+    // p of row r stands in place p ^ swizzle(r): the 16 lanes that an LDS read serves at a time (16 rows, one piece) fall on 16
+    // different groups of banks. A lane asks for the piece whose place is its own; rows beyond the matrices are the last one, never stored.
+    auto swizzle = [](int row) { return (row >> 1) & 7; };
+    const unsigned char* base[LOADS];
+    size_t offset[LOADS];
+    auto first_row = [&](int q) { return min((wave * LOADS + q) * 8, ROWS - 8); };
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) {
-        const int row = row0 + STEP * i;
-        src[i] = (STEP * i < BM ? A + static_cast<size_t>(min(m0 + row, M - 1)) * lda : W + static_cast<size_t>(min(n0 + row - BM, N - 1)) * ldw) + piece;
+    for (int q = 0; q < LOADS; ++q) {
+        const int first = first_row(q), row = first + lane / 8;
+        const bool of_a = first < BM;
+        base[q] = reinterpret_cast<const unsigned char*>(of_a ? A + static_cast<size_t>(m0) * lda : W + static_cast<size_t>(n0) * ldw);
+        offset[q] = static_cast<size_t>(of_a ? min(row, M - 1 - m0) : min(row - BM, N - 1 - n0)) * (of_a ? lda : ldw) * 4 + kg * 128 + (lane % 8 ^ swizzle(row)) * 16;
     }
-    float4 regs[2][LOADS];
-    auto fetch = [&](int set, int k0) {          // (columns beyond K: the row's last ones, zeroed when they are staged)
-        const int k = min(k0, K - 4 - piece);
-#pragma unroll
-        for (int i = 0; i < LOADS; ++i) regs[set][i] = *reinterpret_cast<const float4*>(src[i] + k);
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)smem)) + kg * SLAB_BYTES;
+    const int nk = (K + BK - 1) / BK, rest = K - (nk - 1) * BK;      // k tiles; columns of the last
+    auto fetch = [&](int q, int t, int stage) {
+        size_t from = offset[q];
+        if (EDGE && t == nk - 1) {         // (pieces beyond K: the row's last one, against zeros)
+            const int column = kg * 128 + (lane % 8 ^ swizzle(first_row(q) + lane / 8)) * 16;
+            from -= max(column - (rest * 4 - 16), 0);
+        }
+        load_to_lds(base[q] + static_cast<size_t>(t) * (BK * 4), from, lds0 + stage * STAGE_BYTES + first_row(q) * 128);
     };
-    auto stage = [&](int set, int buf, int k0) {
-        const bool ok = k0 + piece < K;
+    // lane l holds columns 4 (l / 16) to + 3 of row l % 16 of every 16 x 16 tile; what the epilogue adds there is asked for in front of the last tiles
+    const int wm = wave / WN, wn = wave % WN, row16 = lane % 16, quad = lane / 16;
+    const bool vec = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 && (bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 15) == 0);
 #pragma unroll
-        for (int i = 0; i < LOADS; ++i)
-            *reinterpret_cast<float4*>(&tile_s[buf][(row0 + STEP * i) * STRIDE + piece]) = ok ? regs[set][i] : make_float4(0.f, 0.f, 0.f, 0.f);
-    };
-    f32x4v acc[TM][TN];
+    for (int s = 0; s < STAGES - 1; ++s) {
+        if (s >= nk) break;
+#pragma unroll
+        for (int q = 0; q < LOADS; ++q) fetch(q, s, s);
+    }
+
+    const f32x4v zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4v acc[PARTS][TM][TN], sum[KS][SUMS][TM][TN], four[TM][TN], fa[KS][TM], fw[KS][TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i)
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = f32x4v{0.f, 0.f, 0.f, 0.f};
-    const int wm = wave / 2, wn = wave % 2, row16 = lane % 16, quad = lane / 16;
-    const int a_off = (wm * TM * 16 + row16) * STRIDE + F32T_BK * kg + 4 * quad, w_off = (BM + wn * TN * 16 + row16) * STRIDE + F32T_BK * kg + 4 * quad;
-    // TM x TN of 1: the 32 columns in eight sums of four that are added pairwise before they join; otherwise 16 columns in one sum each
-    auto multiply = [&](int buf) {
-        constexpr int KS = F32T_BK / 16;
-        f32x4v sum[SUMS == 4 ? KS : 1][SUMS][TM][TN];
+        for (int j = 0; j < TN; ++j) {
+            four[i][j] = zero;
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int at = SUMS == 4 ? ks : 0;
-            f32x4v fa[TM], fw[TN];
+            for (int p = 0; p < PARTS; ++p) acc[p][i][j] = zero;
 #pragma unroll
-            for (int i = 0; i < TM; ++i) fa[i] = *reinterpret_cast<const f32x4v*>(&tile_s[buf][a_off + i * 16 * STRIDE + ks * 16]);
-#pragma unroll
-            for (int j = 0; j < TN; ++j) fw[j] = *reinterpret_cast<const f32x4v*>(&tile_s[buf][w_off + j * 16 * STRIDE + ks * 16]);
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) {
-                        f32x4v& to = sum[at][e % SUMS][i][j];
-                        to = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[j][e], fa[i][e], e < SUMS ? f32x4v{0.f, 0.f, 0.f, 0.f} : to, 0, 0, 0);
-                    }
-            if constexpr (SUMS == 1) {
-#pragma unroll
-                for (int i = 0; i < TM; ++i)
-#pragma unroll
-                    for (int j = 0; j < TN; ++j) acc[i][j] += sum[0][0][i][j];
-            }
+            for (int e = 0; e < SUMS; ++e) sum[1][e][i][j] = zero;
         }
-        if constexpr (SUMS == 4) {
-            static_assert(KS == 2, "two times four sums");
-            auto four = [&](int ks) { return (sum[ks][0][0][0] + sum[ks][1][0][0]) + (sum[ks][2][0][0] + sum[ks][3][0][0]); };
-            acc[0][0] += four(0) + four(1);
-        }
-    };
-    const int nk = (K + BK - 1) / BK;
-    // tile t multiplies from buffer t % 2 while tile t + 1 is staged into the other one, whose readers (tile t - 1) passed the
-    // barrier before, and the loads of tile t + 3 go out into the registers that are free then (past the last tile: its own again)
-    fetch(0, 0);
-    fetch(1, min(1, nk - 1) * BK);
-    stage(0, 0, 0);
-    fetch(0, min(2, nk - 1) * BK);
-    lds_barrier();
-    for (int t = 0; t < nk; t += 2) {
-        stage(1, 1, (t + 1) * BK);
-        fetch(1, min(t + 3, nk - 1) * BK);
-        multiply(0);
-        lds_barrier();
-        if (t + 1 >= nk) break;
-        stage(0, 0, (t + 2) * BK);
-        fetch(0, min(t + 4, nk - 1) * BK);
-        multiply(1);
-        lds_barrier();
+    const int a_row = wm * TM * 16 + row16, w_row = BM + wn * TN * 16 + row16;       // (16 rows on the swizzle is the same)
+    int a_at[KS], w_at[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        a_at[ks] = kg * SLAB_BYTES + a_row * 128 + ((4 * ks + quad) ^ swizzle(a_row)) * 16;
+        w_at[ks] = kg * SLAB_BYTES + w_row * 128 + ((4 * ks + quad) ^ swizzle(w_row)) * 16;
     }
-    if constexpr (KG > 1) {          // the other groups leave their sums in LDS and go; group 0 adds them in their order
-        f32x4v* sums = reinterpret_cast<f32x4v*>(&tile_s[0][0]);
-        if (kg > 0) {
+    auto read_frags = [&](int stage_at, int ks) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i) fa[ks][i] = *reinterpret_cast<const f32x4v*>(smem + stage_at + a_at[ks] + i * 16 * 128);
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fw[ks][j] = *reinterpret_cast<const f32x4v*>(smem + stage_at + w_at[ks] + j * 16 * 128);
+    };
+    auto multiply = [&](int ks) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
 #pragma unroll
             for (int i = 0; i < TM; ++i)
 #pragma unroll
-                for (int j = 0; j < TN; ++j) sums[(((kg - 1) * 4 + wave) * TM * TN + i * TN + j) * 64 + lane] = acc[i][j];
+                for (int j = 0; j < TN; ++j) {
+                    f32x4v& to = sum[ks][e % SUMS][i][j];
+                    to = __builtin_amdgcn_mfma_f32_16x16x4f32(fw[ks][j][e], fa[ks][i][e], e < SUMS ? zero : to, 0, 0, 0);
+                }
+    };
+    // The sums of the step before join the outputs' while this step's are made. Eight sums of four columns (a k tile's, TM x TN of 1)
+    // are added pairwise first.
+    auto join = [&](int ks, f32x4v (&to)[TM][TN]) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                if constexpr (SUMS == 1) {
+                    to[i][j] += sum[1 - ks][0][i][j];
+                } else {
+                    const f32x4v t = (sum[1 - ks][0][i][j] + sum[1 - ks][1][i][j]) + (sum[1 - ks][2][i][j] + sum[1 - ks][3][i][j]);
+                    if (ks == 1) four[i][j] = t;
+                    else to[i][j] += four[i][j] + t;
+                }
+            }
+    };
+    // Tile t is in stage t % STAGES, the tiles up to t + STAGES - 2 are on their way, and tile t + STAGES - 1 is asked for into the
+    // stage that tile t - 1 left. The wavefronts wait for the next tile and meet in front of a tile's last products, and its first fragments
+    // are read there: neither stands alone.
+    wait_tiles_and_meet<STAGES - 2, LOADS>(nk - 1);
+    read_frags(0, 0);
+    int stage_at = 0, fetch_stage = STAGES - 1;
+    auto step = [&](auto fetches, int t, int part) {
+        constexpr bool FETCHES = decltype(fetches)::value;
+        const int next_at = stage_at == (STAGES - 1) * STAGE_BYTES ? 0 : stage_at + STAGE_BYTES;
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            if (FETCHES && ks == 0) {
+#pragma unroll
+                for (int q = 0; q < LOADS; ++q) fetch(q, t + STAGES - 1, fetch_stage);
+            }
+            if (ks + 1 < KS) {
+                read_frags(stage_at, ks + 1);
+            } else if (FETCHES) {
+                wait_loads_and_meet<(STAGES - 2) * LOADS>();
+                read_frags(next_at, 0);
+            } else if (t + 1 < nk) {
+                wait_tiles_and_meet<(STAGES > 2 ? STAGES - 3 : 0), LOADS>(nk - 2 - t);
+                read_frags(next_at, 0);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+            if (EDGE && !FETCHES && t == nk - 1 && kg * F32T_BK + 16 * ks + 4 * quad >= rest) {
+#pragma unroll
+                for (int i = 0; i < TM; ++i) fa[ks][i] = zero;
+#pragma unroll
+                for (int j = 0; j < TN; ++j) fw[ks][j] = zero;
+            }
+            multiply(ks);
+            join(ks, acc[ks == 1 ? part : (part + PARTS - 1) % PARTS]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        stage_at = next_at;
+        fetch_stage = fetch_stage == STAGES - 1 ? 0 : fetch_stage + 1;
+    };
+    const std::true_type asking;
+    const std::false_type done;
+    int t = 0;
+    if constexpr (PARTS == 2) {
+        for (; t + STAGES < nk; t += 2) {
+            step(asking, t, 0);
+            step(asking, t + 1, 1);
+        }
+    } else {
+        for (; t + STAGES - 1 < nk; ++t) step(asking, t, 0);
+    }
+    float4 add[TN], old[TM][TN];
+#pragma unroll
+    for (int j = 0; j < TN; ++j) {
+        const int n = n0 + (wn * TN + j) * 16 + 4 * quad;
+        add[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (vec && kg == 0 && bias != nullptr && n + 4 <= N) add[j] = *reinterpret_cast<const float4*>(bias + n);
+#pragma unroll
+        for (int i = 0; i < TM; ++i) {
+            const int m = m0 + (wm * TM + i) * 16 + row16;
+            old[i][j] = make_float4(0.f, 0.f, 0.f, 0.f);
+            if (vec && kg == 0 && mode == EPI_ADD_RESIDUAL && m < M && n + 4 <= N) old[i][j] = *reinterpret_cast<const float4*>(static_cast<const float*>(C) + static_cast<size_t>(m) * ldc + n);
+        }
+    }
+    if constexpr (PARTS == 2) {
+        if (t + STAGES - 1 < nk) {
+            step(asking, t, 0);
+            step(done, t + 1, 1);
+            t += 2;
+        }
+        for (; t < nk; t += 2) {
+            step(done, t, 0);
+            if (t + 1 < nk) step(done, t + 1, 1);
+        }
+    } else {
+        for (; t < nk; ++t) step(done, t, 0);
+    }
+    if (PARTS == 2 && nk % 2 == 0) join(0, acc[PARTS - 1]);
+    else join(0, acc[0]);
+    // The other groups leave their sums in LDS and go; group 0 adds them: parts 0 of the groups in their order, then parts 1; of four groups,
+    // two and two.
+    if constexpr (KG > 1) {
+        lds_barrier();               // (the tiles have been read; no load is under way)
+        f32x4v* sums = reinterpret_cast<f32x4v*>(smem);
+        auto place = [&](int g, int p, int i, int j) -> f32x4v& { return sums[((((g - 1) * PARTS + p) * NW + wave) * TM * TN + i * TN + j) * 64 + lane]; };
+        if (kg > 0) {
+#pragma unroll
+            for (int p = 0; p < PARTS; ++p)
+#pragma unroll
+                for (int i = 0; i < TM; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j) place(kg, p, i, j) = acc[p][i][j];
         }
         lds_barrier();
         if (kg > 0) return;
@@ -396,13 +494,16 @@ gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restr
         for (int i = 0; i < TM; ++i)
 #pragma unroll
             for (int j = 0; j < TN; ++j) {
-                auto other = [&](int g) { return sums[((g * 4 + wave) * TM * TN + i * TN + j) * 64 + lane]; };
-                if constexpr (KG == 4) acc[i][j] = (acc[i][j] + other(0)) + (other(1) + other(2));
-                else acc[i][j] += other(0);
+                if constexpr (KG == 4) acc[0][i][j] = (acc[0][i][j] + place(1, 0, i, j)) + (place(2, 0, i, j) + place(3, 0, i, j));
+                else if constexpr (PARTS == 2) acc[0][i][j] = (acc[0][i][j] + place(1, 0, i, j)) + (acc[1][i][j] + place(1, 1, i, j));
+                else acc[0][i][j] += place(1, 0, i, j);
             }
+    } else if constexpr (PARTS == 2) {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) acc[0][i][j] += acc[1][i][j];
     }
-    // lane l holds columns 4 (l / 16) to + 3 of row l % 16 of every 16 x 16 tile
-    const bool vec = ldc % 4 == 0 && (reinterpret_cast<uintptr_t>(C) & 15) == 0 && (bias == nullptr || (reinterpret_cast<uintptr_t>(bias) & 15) == 0);
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
         const int m = m0 + (wm * TM + i) * 16 + row16;
@@ -412,33 +513,29 @@ gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restr
             const int n = n0 + (wn * TN + j) * 16 + 4 * quad;
             float* out = static_cast<float*>(C) + static_cast<size_t>(m) * ldc + n;
             if (vec && n + 4 <= N) {
-                float v[4] = {acc[i][j][0], acc[i][j][1], acc[i][j][2], acc[i][j][3]}, o[4] = {0.f, 0.f, 0.f, 0.f};
-                if (bias != nullptr) {
-                    const float4 b = *reinterpret_cast<const float4*>(bias + n);
-                    v[0] += b.x; v[1] += b.y; v[2] += b.z; v[3] += b.w;
-                }
-                if (mode == EPI_ADD_RESIDUAL) {
-                    const float4 b = *reinterpret_cast<const float4*>(out);
-                    o[0] = b.x; o[1] = b.y; o[2] = b.z; o[3] = b.w;
-                }
+                const float v[4] = {acc[0][i][j][0] + add[j].x, acc[0][i][j][1] + add[j].y, acc[0][i][j][2] + add[j].z, acc[0][i][j][3] + add[j].w};
+                float o[4] = {old[i][j].x, old[i][j].y, old[i][j].z, old[i][j].w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e)
                     o[e] += mode == EPI_GELU_TANH ? gelu_tanh_precise(v[e]) : mode == EPI_GELU_ERF ? gelu_erf(v[e]) : mode == EPI_RELU2 ? relu2(v[e]) : v[e];
                 *reinterpret_cast<float4*>(out) = make_float4(o[0], o[1], o[2], o[3]);
             } else {
                 for (int e = 0; e < 4 && n + e < N; ++e)
-                    epilogue<float>(mode, acc[i][j][e], bias ? bias[n + e] : 0.f, C, static_cast<size_t>(m) * ldc + n + e);
+                    epilogue<float>(mode, acc[0][i][j][e], bias ? bias[n + e] : 0.f, C, static_cast<size_t>(m) * ldc + n + e);
             }
         }
     }
 }
 
-template <int TM, int TN, int KG>
+template <int WM, int WN, int TM, int TN, int KG, int PARTS, int STAGES, int SUMS>
 static void launch_f32_tiles(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int mode,
                              hipStream_t stream) {
-    const int tiles_m = (M + 32 * TM - 1) / (32 * TM), tiles_n = (N + 32 * TN - 1) / (32 * TN);
-    gemm_f32_tiles_kernel<TM, TN, KG><<<(tiles_m * tiles_n + 7) / 8 * 8, 256 * KG, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n,
-                                                                                             M > N ? 0 : 1);
+    const int tiles_m = (M + 16 * WM * TM - 1) / (16 * WM * TM), tiles_n = (N + 16 * WN * TN - 1) / (16 * WN * TN);
+    const dim3 grid((tiles_m * tiles_n + 7) / 8 * 8), block(64 * WM * WN * KG);
+    if (K % (F32T_BK * KG) != 0)
+        gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, true><<<grid, block, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n, M > N ? 0 : 1);
+    else
+        gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, false><<<grid, block, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n, M > N ? 0 : 1);
 }
 
 // bfloat16 operands of any K, strides and alignment (what the matrix-core kernels of gemm_bf16.hip refuse:
@@ -506,26 +603,27 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
     // vector FMAs, 2,048 x 50,257 x 64 346 / 239; 192 x 32,000 x 128 31.4 / 29.9 (at 192 columns 35.6 / 40.4), 192 x 16,384 x 64 13.8 / 13.4.
     const bool odd_wide = M > 64 && ldc % 4 != 0 && N >= 16384 && K <= (N >= 32000 ? 128 : N >= 20000 ? 96 : 64);
     if (quads && K > 0 && !odd_wide) {
-        // Tiles of 32 x 32 shared by four groups up to 64 rows (whose sums are as exact as the kernel's for few rows) and while
-        // there are at most two a compute unit (570 x 768 x 3,072: 40 us, with two groups 43, with tiles of 64 x 32 44).
-        // Otherwise the shape whose fullest compute unit does least: its tiles times their size times what 32 x 32 outputs
-        // take there at K = 768 (in tenths of a microsecond, measured at 2,048 rows). With two groups a sixth of that is there at
-        // any K, which shows up to 96 columns (130 x 50,304 x 96: 40 us with 32 x 32, 29 with 64 x 64; 65 x 50,304 x 256: 40.1, 41.5). Large tiles need several workgroups a unit
-        // to hide their barriers: 2,048 x 768 x 768 32 us with 64 x 32, 35 with 64 x 64 (384 tiles) and 64 x 96 (256).
+        // Two questions. How exactly a result is summed is a rule on its sizes alone: in four sums of eight (tiles of 32 x 32) up to
+        // 64 rows, whose result is then as exact as that of the kernel for few rows, while there are at most 512 such tiles, and where
+        // they were the fastest choice when tiles were loaded through registers (the price of the fullest compute unit: its tiles
+        // times what they took there at K = 768, in tenths of a microsecond; with two groups a sixth of that is there at any K);
+        // otherwise in two sums, or in one where that was.
         const auto tiles = [&](int tm, int tn) { return static_cast<long>((M + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
-        const auto cost = [&](int tm, int tn, int groups, long from, int each) {
-            const long n = tiles(tm, tn), k = K <= 96 ? K : 768;
-            return n < from ? (1L << 60) : ((n + 7) / 8 + 31) / 32 * tm * tn * each * (groups == 2 ? 5 * k + 768 : 6 * k);
-        };
-        if (M <= 64 || tiles(1, 1) <= 512) {
-            launch_f32_tiles<1, 1, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+        const auto fullest = [&](int tm, int tn) { return ((tiles(tm, tn) + 7) / 8 + 31) / 32; };
+        const long k = K <= 96 ? K : 768, two_groups = 5 * k + 768, one_group = 6 * k, never = 1L << 60;
+        const long c11 = fullest(1, 1) * 44 * two_groups, c21 = tiles(2, 1) < 256 ? never : fullest(2, 1) * 80 * two_groups;
+        const long c22 = std::min(tiles(2, 2) < 512 ? never : fullest(2, 2) * 144 * one_group, tiles(2, 3) < 512 ? never : fullest(2, 3) * 222 * one_group);
+        // Which tile then: four groups where a unit has one tile and a long chain of k tiles (128 x 1,600 x 6,400: 40.8 us, two groups of
+        // two parts 43.5; 560 x 768 x 768, two tiles a unit: 12.3, four groups 15.4); and of 64 x 32 in two sums, which is the fastest or within 3 %
+        // of it over 40 sizes, and of 128 x 64 in one the cheaper, by prices fitted to those sizes (microseconds: 2,048 x 3,072 x 768 91 and 84
+        // us, 1,812 x 768 x 2,048 60 and 79).
+        if (M <= 64 || tiles(1, 1) <= 512 || (c11 < c21 && c11 < c22)) {
+            if (tiles(1, 1) <= 256 && K >= 1536) launch_f32_tiles<2, 2, 1, 1, 4, 1, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else launch_f32_tiles<2, 2, 1, 1, 2, 2, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
         } else {
-            const long c11 = cost(1, 1, 2, 0, 44), c21 = cost(2, 1, 2, 256, 40), c22 = cost(2, 2, 1, 512, 36), c23 = cost(2, 3, 1, 512, 37);
-            const long least = std::min(std::min(c11, c21), std::min(c22, c23));
-            if (least == c22) launch_f32_tiles<2, 2, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
-            else if (least == c23) launch_f32_tiles<2, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
-            else if (least == c21) launch_f32_tiles<2, 1, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
-            else launch_f32_tiles<1, 1, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            const float small = 4.96f + fullest(2, 1) * (K * 0.00973f - 0.43f), large = 3.49f + fullest(4, 2) * (K * 0.03264f + 1.26f);
+            if (c22 <= c21 && large < small) launch_f32_tiles<4, 2, 2, 2, 1, 1, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+            else launch_f32_tiles<2, 2, 2, 1, 1, 2, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
         }
         MLLM_LAUNCH_CHECK();
         return 0;

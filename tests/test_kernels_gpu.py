@@ -588,6 +588,23 @@ def test_linear_fp32_tiles(ops, M, N, K, pad, epi):
     assert not torch.isfinite(out[M // 2, :N]).any() or epi == "gelu_tanh"
 
 
+@pytest.mark.parametrize("M,N,K0", [(33, 70, 0), (130, 96, 1536), (600, 1100, 0), (1812, 772, 0), (2049, 1540, 0)])
+@pytest.mark.parametrize("K", [4, 32, 36, 64, 100, 128, 132, 160, 192, 228])
+def test_linear_fp32_tiles_of_few_k_tiles(ops, M, N, K0, K):
+    """Every tile shape (32 x 32 with two and four groups, 64 x 32, 128 x 64) where the k tiles are fewer than the stages of LDS, odd and
+    even in number, with a last one that is full or not: the error is at most one rounding of 2^-24 a term of the terms'
+    absolute sum, and rows that lie apart are met."""
+    K += K0
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = _rand((M, K + 8), torch.float32, g).to(DEV), _rand((N, K + 4), torch.float32, g).to(DEV)
+    a[:, K:], w[:, K:] = math.inf, math.nan
+    bias, out = _rand((N,), torch.float32, g).to(DEV), torch.full((M, N + 4), 7.0, device=DEV)
+    ops.linear(a[:, :K], w[:, :K], bias, out[:, :N], "store")
+    a, w = a[:, :K].double(), w[:, :K].double()
+    assert ((out[:, :N].double() - (a @ w.T + bias.double())).abs() <= 2.0 ** -24 * (K + 2) * (a.abs() @ w.abs().T + bias.abs().double())).all()
+    assert (out[:, N:] == 7).all()
+
+
 @pytest.mark.parametrize("K", [768, 1600, 3072])
 def test_linear_fp32_is_as_exact_on_tiles_as_for_few_rows(ops, K):
     """64 rows run on tiles, 16 at a time on the kernel for few rows: the former's error against 64 bits is no larger."""
