@@ -60,12 +60,12 @@ LIBRARIES: Dict[str, dict] = {
     "elementwise": {"kind": "hip", "sources": ["kernels/elementwise.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "gemm_f32": {"kind": "hip", "sources": ["kernels/gemm_f32.hip"], "headers": ["kernels/common.h", "kernels/lds_loads.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "gemm_bf16": {"kind": "hip", "sources": ["kernels/gemm_bf16.hip"], "headers": ["kernels/common.h", "kernels/lds_loads.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
-    "attention": {"kind": "hip", "sources": ["kernels/attention.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
+    "attention": {"kind": "hip", "sources": ["kernels/attention.hip"], "headers": ["kernels/common.h", "kernels/query_tiles.h", "kernels/lds_loads.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "attention_decode": {"kind": "hip", "sources": ["kernels/attention_decode.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
-    "attention_prefill": {"kind": "hip", "sources": ["kernels/attention_prefill.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
+    "attention_prefill": {"kind": "hip", "sources": ["kernels/attention_prefill.hip"], "headers": ["kernels/common.h", "kernels/query_tiles.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "norm_gate": {"kind": "hip", "sources": ["kernels/norm_gate.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "ssm": {"kind": "hip", "sources": ["kernels/ssm.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
-    "latent_attention": {"kind": "hip", "sources": ["kernels/latent_attention.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
+    "latent_attention": {"kind": "hip", "sources": ["kernels/latent_attention.hip"], "headers": ["kernels/common.h", "kernels/query_tiles.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "scored_attention": {"kind": "hip", "sources": ["kernels/scored_attention.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "gated_recurrence": {"kind": "hip", "sources": ["kernels/gated_recurrence.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},
     "matrix_memory": {"kind": "hip", "sources": ["kernels/matrix_memory.hip"], "headers": ["kernels/common.h", "kernels/score_shape.h", "kernels/tanh_norm.h"]},

@@ -10,6 +10,8 @@
 // applied to 64 keys at a time. The reference's decode kernel adds 1e-6 to the
 // denominator (/root/reference/src/kernels/decode/paged_attention.cu:97); this does not.
 #include "common.h"
+#include "lds_loads.h"
+#include "query_tiles.h"
 
 #define ATT_WAVES 4
 #define ATT_MAX_ACC 4   // head_dim <= 64 * ATT_MAX_ACC
@@ -135,6 +137,39 @@ template <> __device__ __forceinline__ void store4f<bf16_t>(bf16_t* p, f32x4_t v
     *reinterpret_cast<uint2*>(p) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
 }
 
+// The end of a tiled kernel: the sink, the division by the sum, the gate and the store. The lane holds O^T[dims 16c + 4G + i] of the query
+// in row `row`, c < n_c.
+template <typename T, int DC, bool SHAPED>
+__device__ __forceinline__ void finish_tiled(f32x4_t (&o)[DC], int n_c, float m, float l, const MllmScoreShape& shape, const float* gate, int ldg,
+                                             int h, int head_dim, int row, int G, T* out, int out_stride) {
+    if (SHAPED && shape.sink != nullptr) {
+        // the sink: one more term of the denominator, exp(sink), without a value (the maximum is in base 2)
+        const float sk = shape.sink[h] * MLLM_LOG2E, m_new = fmaxf(m, sk);
+        const float a = (m == -INFINITY) ? 0.f : exp2_for<T>(m - m_new);
+        l = l * a + exp2_for<T>(sk - m_new);
+#pragma unroll
+        for (int c = 0; c < DC; ++c) o[c] *= a;
+    }
+    const float inv_l = 1.f / l;
+    const bool head_gate = SHAPED && gate != nullptr && shape.gate_per_head;
+    const float hg = head_gate ? 1.f / (1.f + expf(-gate[static_cast<size_t>(row) * ldg + h])) : 1.f;
+    T* op = out + static_cast<size_t>(row) * out_stride + h * head_dim + 4 * G;
+#pragma unroll
+    for (int c = 0; c < DC; ++c) {
+        if (c < n_c) {
+            f32x4_t r = o[c] * inv_l;
+            if (head_gate) {
+                r *= hg;
+            } else if (SHAPED && gate != nullptr) {
+                const float* gp = gate + static_cast<size_t>(row) * ldg + h * head_dim + 4 * G + 16 * c;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[i] *= 1.f / (1.f + expf(-gp[i]));
+            }
+            store4f<T>(op + 16 * c, r);
+        }
+    }
+}
+
 // DC: the most 16-dim chunks of a head (head_dim <= 16 DC); loops over chunks are unrolled to DC and
 // predicated, so that the register arrays are indexed by constants.
 // SHAPED: the scores are shaped before the softmax (score_shape.h), a chunked mask may stand in for the window, and
@@ -152,16 +187,8 @@ paged_attention_tiled(const T* __restrict__ q, int q_stride, int q_col, const T*
     float* Ks = tl_smem;                           // [TL_BK][ldk]
     float* Vt = tl_smem + TL_BK * ldk;             // [head_dim][TL_VSTRIDE]
 
-    // which sequence and which of its 64-query tiles (the heaviest causal tiles first)
-    int tile = gridDim.y - 1 - blockIdx.y, b = 0, q_begin = 0, q_len = 0;
-    for (; b < n_seqs; ++b) {
-        q_begin = cu_q[b];
-        q_len = cu_q[b + 1] - q_begin;
-        const int nt = (q_len + TL_BQ - 1) / TL_BQ;
-        if (tile < nt) break;
-        tile -= nt;
-    }
-    if (b >= n_seqs) return;                       // surplus workgroup; the whole workgroup leaves
+    const auto [b, tile, q_begin, q_len] = query_tile<TL_BQ>(cu_q, ctx_len, n_seqs, 1, blockIdx.y, gridDim.y);
+    if (b < 0) return;                             // surplus workgroup; the whole workgroup leaves
 
     const int h = blockIdx.x, hk = h / (n_heads / n_kv_heads);
     const int tid = threadIdx.x, lane = tid % 64, wave = tid / 64;
@@ -275,34 +302,179 @@ paged_attention_tiled(const T* __restrict__ q, int q_stride, int q_col, const T*
             }
         }
     }
-    if (!q_ok) return;
-    if (SHAPED && shape.sink != nullptr) {
-        // the sink: one more term of the denominator, exp(sink), without a value (the maximum is in base 2)
-        const float sk = shape.sink[blockIdx.x] * MLLM_LOG2E, m_new = fmaxf(m, sk);
-        const float a = (m == -INFINITY) ? 0.f : exp2_for<T>(m - m_new);
-        l = l * a + exp2_for<T>(sk - m_new);
-#pragma unroll
-        for (int c = 0; c < DC; ++c) o[c] *= a;
-    }
-    // lane holds O^T[dims 16c + 4G + i][its query]
-    const float inv_l = 1.f / l;
-    const bool head_gate = SHAPED && gate != nullptr && shape.gate_per_head;
-    const float hg = head_gate ? 1.f / (1.f + expf(-gate[static_cast<size_t>(q_begin + qi) * ldg + h])) : 1.f;
-    T* op = out + static_cast<size_t>(q_begin + qi) * out_stride + h * head_dim + 4 * G;
+    if (q_ok) finish_tiled<T, DC, SHAPED>(o, n_c, m, l, shape, gate, ldg, h, head_dim, q_begin + qi, G, out, out_stride);
+}
+
+// The same for 32-bit storage and heads of 64 or 128, which are most of what runs: key and value tiles go from the pages straight into LDS
+// (lds_loads.h), a tile ahead, the block table's entries lie in LDS, and a workgroup has eight wavefronts: two share 16 queries, take
+// half of every key tile each, and merge their states at the end, so that a tile's chain (wait, scores, softmax, values) is half as long
+// and there are four wavefronts a SIMD to fill the gaps. Keys and values stand row-major, 16-byte piece p of row r in place p ^ (r % 16):
+// the keys' 16-byte reads (16 rows, one piece) and the values' 4-byte reads (four rows, 16 columns) are free of bank conflicts.
+// Bound by the chain of a workgroup's key tiles where workgroups are few (2.5 us a tile, of which the matrix instructions are 1.7), by the
+// matrix cores for long prompts. 12 heads of 64, with the kernel above before: 8 x 256 tokens 30.7 > 20.7 us, 331 + 512 + 470 + 400
+// 43.6 > 30, 2 x 1,024 91 > 56, 8,000 988 > 892 (110 TFLOP/s of 155); 8 heads of 128, 4 x 512 76 > 45.
+// A place outside [k_lo, p_last] (not written yet, or given back by a window) loads the next key that is inside; its weight is 0.
+#define TD_TABLE 4096      // entries of a block table that fit LDS beside two stages of tiles, two workgroups a unit
+
+template <int DH, bool SHAPED>
+__global__ void __launch_bounds__(512)
+paged_attention_tiled_f32(const float* __restrict__ q, int q_stride, int q_col, const float* __restrict__ k_pages,
+                          const float* __restrict__ v_pages, int kv_dim, const int* __restrict__ block_tables, int max_blocks,
+                          const int* __restrict__ cu_q, const int* __restrict__ ctx_len, int n_seqs, int n_heads,
+                          int n_kv_heads, int page_size, float scale_log2e, int window,
+                          float* __restrict__ out, int out_stride, MllmScoreShape shape, const float* __restrict__ gate, int ldg) {
+    constexpr int DC = DH / 16, PIECES = DH / 4, KEYS_PER_LOAD = 64 / PIECES, LOADS = TL_BK / KEYS_PER_LOAD / 8;
+    constexpr int TILE_BYTES = TL_BK * DH * 4, STAGE_BYTES = 2 * TILE_BYTES;       // keys, then values
+    static_assert(LOADS * KEYS_PER_LOAD * 8 == TL_BK && PIECES % 16 == 0 && 4 * 64 * (DC * 4 + 2) * 4 <= 2 * STAGE_BYTES, "whole loads; the states fit");
+    extern __shared__ __attribute__((aligned(16))) unsigned char td_smem[];
+    int* table_s = reinterpret_cast<int*>(td_smem + 2 * STAGE_BYTES);
+
+    const auto [b, tile, q_begin, q_len] = query_tile<TL_BQ>(cu_q, ctx_len, n_seqs, 1, blockIdx.y, gridDim.y);
+    if (b < 0) return;                             // surplus workgroup; the whole workgroup leaves
+
+    const int h = blockIdx.x, hk = h / (n_heads / n_kv_heads);
+    const int tid = threadIdx.x, lane = tid % 64, wave = __builtin_amdgcn_readfirstlane(tid / 64), group = wave % 4, half = wave / 4;
+    const int G = lane / 16, c16 = lane % 16;
+    const int start = ctx_len[b] - q_len, q0 = tile * TL_BQ, qi = q0 + group * 16 + c16;
+    const bool q_ok = qi < q_len;
+    const int p = start + min(qi, q_len - 1);
+    const int p_first = start + q0, p_last = start + min(q0 + TL_BQ, q_len) - 1;
+    int k_lo = (window > 0 && p_first - window + 1 > 0) ? p_first - window + 1 : 0;
+    int my_lo = (window > 0 && p - window + 1 > 0) ? p - window + 1 : 0;
+    if (SHAPED && shape.chunk > 0) { k_lo = p_first - p_first % shape.chunk; my_lo = p - p % shape.chunk; }
+    const float r1 = SHAPED ? mllm_bias_r1(shape, h) : 0.f, r2 = (SHAPED && shape.r1) ? shape.r2[h] : 0.f;
+    const int kf = (SHAPED && window > 0) ? shape.keep_first : 0;
+    const int kt_first = k_lo / TL_BK, kt_last = p_last / TL_BK;
+    const int n_head = kf > 0 ? min((kf + TL_BK - 1) / TL_BK, kt_first) : 0;
+    const int vt_last = n_head + kt_last - kt_first;
+    const int wave_last = start + min(q0 + group * 16 + 15, q_len - 1);
+    int wave_lo = (window > 0 && wave_last - window + 1 > 0) ? wave_last - window + 1 : 0;      // the first key that all its queries see
+    if (SHAPED && shape.chunk > 0) wave_lo = wave_last - wave_last % shape.chunk;
+    auto tile_start = [&](int vt) { return (vt < n_head ? vt : vt - n_head + kt_first) * TL_BK; };
+    const int* table = block_tables + static_cast<size_t>(b) * max_blocks;
+    for (int i = tid; i <= p_last / page_size; i += 512) table_s[i] = table[i];
+
+    f32x4_t qf[DC], o[DC];
+    const float* qp = q + static_cast<size_t>(q_begin + min(qi, q_len - 1)) * q_stride + q_col + h * DH + 4 * G;
 #pragma unroll
     for (int c = 0; c < DC; ++c) {
-        if (c < n_c) {
-            f32x4_t r = o[c] * inv_l;
-            if (head_gate) {
-                r *= hg;
-            } else if (SHAPED && gate != nullptr) {
-                const float* gp = gate + static_cast<size_t>(q_begin + qi) * ldg + h * head_dim + 4 * G + 16 * c;
-#pragma unroll
-                for (int i = 0; i < 4; ++i) r[i] *= 1.f / (1.f + expf(-gp[i]));
-            }
-            store4f<T>(op + 16 * c, r);
-        }
+        o[c] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+        qf[c] = load4f<float>(qp + 16 * c) * scale_log2e;
     }
+    float m = -INFINITY, l = 0.f;
+    __syncthreads();                               // the table is in LDS
+
+    const unsigned lds0 = static_cast<unsigned>(reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) unsigned char*)td_smem));
+    const int page_shift = (page_size & (page_size - 1)) == 0 ? __ffs(page_size) - 1 : -1;
+    auto fetch = [&](int vt) {
+        const int k0 = tile_start(vt);
+#pragma unroll
+        for (int n = 0; n < LOADS; ++n) {
+            const int first = (wave * LOADS + n) * KEYS_PER_LOAD, key = first + lane / PIECES;
+            int j = min(k0 + key, p_last);
+            if (j < k_lo && j >= kf) j = k_lo;
+            const int block = page_shift >= 0 ? j >> page_shift : j / page_size;
+            const size_t row = static_cast<size_t>(table_s[block]) * page_size + (j - block * page_size);
+            const size_t at = (row * kv_dim + hk * DH) * 4 + (lane % PIECES ^ key % 16) * 16;
+            const unsigned to = lds0 + (vt & 1) * STAGE_BYTES + first * DH * 4;
+            load_to_lds(reinterpret_cast<const unsigned char*>(k_pages), at, to);
+            load_to_lds(reinterpret_cast<const unsigned char*>(v_pages), at, to + TILE_BYTES);
+        }
+    };
+    fetch(0);
+    for (int vt = 0; vt <= vt_last; ++vt) {
+        const int k0 = tile_start(vt);
+        wait_loads_and_meet<0>();                  // this tile has come, the one before it has been read
+        if (vt < vt_last) fetch(vt + 1);
+        if (k0 + 32 * half > wave_last) continue;  // nothing here for this wavefront's queries (it still keeps the barriers)
+        // S^T for 32 keys: lane holds keys k0 + 32 half + 16 g + 4 G + i, i = 0..3, of its query. All fragments are asked for in front
+        // of what uses them, the values' in front of the softmax (the scheduling barriers keep them there).
+        const unsigned char* keys = td_smem + (vt & 1) * STAGE_BYTES + 32 * half * DH * 4;
+        const unsigned char* values = keys + TILE_BYTES;
+        f32x4_t kr[DC][2], s[2] = {f32x4_t{0.f, 0.f, 0.f, 0.f}, f32x4_t{0.f, 0.f, 0.f, 0.f}};
+        float vr[2][4][DC];
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+#pragma unroll
+            for (int g = 0; g < 2; ++g) kr[c][g] = *reinterpret_cast<const f32x4_t*>(keys + (16 * g + c16) * DH * 4 + ((4 * c + G) ^ c16) * 16);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int c = 0; c < DC; ++c)
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+#pragma unroll
+                for (int g = 0; g < 2; ++g) s[g] = __builtin_amdgcn_mfma_f32_16x16x4f32(kr[c][g][j], qf[c][j], s[g], 0, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int c = 0; c < DC; ++c)
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+                    vr[g][i][c] = *reinterpret_cast<const float*>(values + (16 * g + 4 * G + i) * DH * 4 + ((4 * c + c16 / 4) ^ (4 * G + i)) * 16 + c16 % 4 * 4);
+        __builtin_amdgcn_sched_barrier(0);
+        if (SHAPED) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    s[g][i] = mllm_shaped_score<false>(s[g][i], shape, r1, r2, max(p - (k0 + 32 * half + 16 * g + 4 * G + i), 0)) * MLLM_LOG2E;
+        }
+        // (every query of the wavefront sees all 32 keys: nothing to mask)
+        const int first = k0 + 32 * half;
+        if (!(first + 31 <= start + q0 + group * 16 && first >= wave_lo)) {
+#pragma unroll
+            for (int g = 0; g < 2; ++g)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = first + 16 * g + 4 * G + i;
+                    s[g][i] = (j <= p && (j >= my_lo || j < kf)) ? s[g][i] : -INFINITY;
+                }
+        }
+        float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
+        const float m_new = fmaxf(m, rows_max(mx));
+        // (a query none of whose keys has come yet keeps m = -inf: all weights are zero against a finite number. Weights below the
+        // normal range are lost beside the maximum's 1, so the bare instruction does.)
+        const float against = fmaxf(m_new, -3.0e38f), alpha = fast_exp2(m - against);
+        float sum = 0.f;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                s[g][i] = fast_exp2(s[g][i] - against);
+                sum += s[g][i];
+            }
+        l = l * alpha + rows_sum(sum);
+        m = m_new;
+#pragma unroll
+        for (int c = 0; c < DC; ++c) o[c] *= alpha;
+#pragma unroll
+        for (int g = 0; g < 2; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < DC; ++c) o[c] = __builtin_amdgcn_mfma_f32_16x16x4f32(vr[g][i][c], s[g][i], o[c], 0, 0, 0);
+    }
+    // the second half's states pass through LDS (no load is under way; the tiles have been read)
+    lds_barrier();
+    float* states = reinterpret_cast<float*>(td_smem) + (group * 64 + lane) * 4;
+    constexpr int STATE_STEP = 4 * 64 * 4;
+    if (half == 1) {
+#pragma unroll
+        for (int c = 0; c < DC; ++c) *reinterpret_cast<f32x4_t*>(states + c * STATE_STEP) = o[c];
+        *reinterpret_cast<float2*>(states + DC * STATE_STEP - (group * 64 + lane) * 2) = make_float2(m, l);
+    }
+    lds_barrier();
+    if (half == 1 || !q_ok) return;
+    {
+        const float2 other = *reinterpret_cast<const float2*>(states + DC * STATE_STEP - (group * 64 + lane) * 2);
+        const float m_new = fmaxf(m, other.x);     // (a query sees itself: one of the two is finite)
+        const float a = fast_exp2(m - m_new), a2 = fast_exp2(other.x - m_new);
+        l = l * a + other.y * a2;
+        m = m_new;
+#pragma unroll
+        for (int c = 0; c < DC; ++c) o[c] = o[c] * a + *reinterpret_cast<const f32x4_t*>(states + c * STATE_STEP) * a2;
+    }
+    finish_tiled<float, DC, SHAPED>(o, DC, m, l, shape, gate, ldg, h, DH, q_begin + qi, G, out, out_stride);
 }
 
 extern "C" {
@@ -374,6 +546,31 @@ int mllm_paged_attention_tiled(const void* q, int q_stride, int q_col, const voi
             max_blocks, cu_q, ctx_len, n_seqs, n_heads, n_kv_heads, head_dim, page_size, sl2, window, (TYPE*)out,   \
             out_stride, sh, nullptr, 0);                                                                           \
     } while (0)
+#define TD_CASE(DH, SHAPED)                                                                                        \
+    do {                                                                                                           \
+        static bool lds_allowed = false;      /* more than 64 KB of LDS is asked for once */                       \
+        constexpr int tiles_bytes = 2 * 2 * TL_BK * DH * 4;                                                        \
+        if (!lds_allowed) {                                                                                        \
+            const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(paged_attention_tiled_f32<DH, SHAPED>), \
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, tiles_bytes + 4 * TD_TABLE); \
+            if (e != hipSuccess) return static_cast<int>(e);                                                       \
+            lds_allowed = true;                                                                                    \
+        }                                                                                                          \
+        paged_attention_tiled_f32<DH, SHAPED><<<grid, 512, tiles_bytes + 4 * max_blocks, stream>>>(                \
+            (const float*)q, q_stride, q_col, (const float*)k_pages, (const float*)v_pages, kv_dim, block_tables,  \
+            max_blocks, cu_q, ctx_len, n_seqs, n_heads, n_kv_heads, page_size, sl2, window, (float*)out,           \
+            out_stride, sh, shape ? gate : nullptr, ldg);                                                          \
+    } while (0)
+    if (dtype == MLLM_F32 && (head_dim == 64 || head_dim == 128) && max_blocks <= TD_TABLE) {
+        if (head_dim == 64) {
+            if (shape) TD_CASE(64, true); else TD_CASE(64, false);
+        } else {
+            if (shape) TD_CASE(128, true); else TD_CASE(128, false);
+        }
+        MLLM_LAUNCH_CHECK();
+        return 0;
+    }
+#undef TD_CASE
     const int dc = head_dim <= 64 ? 4 : head_dim <= 128 ? 8 : 16;
     if (dtype == MLLM_F32) {
         if (dc == 4) TL_CASE(float, 4); else if (dc == 8) TL_CASE(float, 8); else TL_CASE(float, 16);

@@ -946,6 +946,20 @@ def test_paged_attention_tiles_in_true_32_bit(ops, dtype, H, Hkv, dh, page, wind
     assert (out - ref).abs().max() <= _tol(dtype, 2)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("seqs", [[(5000, 70), (0, 300)],                               # one far in front of the other: their tiles' places are halved
+                                  [(4200, 130), (0, 1), (64, 64), (63, 65), (10, 129)],
+                                  [(i % 3 * 64, 1 + 37 * i % 140) for i in range(64)],   # a sequence a lane
+                                  [(0, 1 + i % 67) for i in range(65)]])                 # more of them
+@pytest.mark.parametrize("H,Hkv,dh", [(3, 1, 64), (2, 2, 128)])
+def test_paged_attention_gives_every_tile_away(ops, dtype, seqs, H, Hkv, dh):
+    """The order in which workgroups take the query tiles of several sequences, by how many keys they see: every row is written, once."""
+    g = torch.Generator().manual_seed(len(seqs) + dh)
+    out, ref = _attention_case(ops, dtype, H, Hkv, dh, 16, seqs, 0, g)
+    assert torch.isfinite(out).all()
+    assert (out - ref).abs().max() <= _tol(dtype, 2)
+
+
 @pytest.mark.parametrize("T", [1, 8, 16])
 @pytest.mark.parametrize("H,Hkv,dh,page,N", [(12, 12, 64, 16, 768), (25, 25, 64, 16, 1600), (3, 3, 32, 8, 96),
                                              (4, 2, 128, 16, 200), (16, 16, 64, 16, 1024)])

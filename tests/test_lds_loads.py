@@ -56,7 +56,7 @@ def test_the_check_sees_the_hazards():
     assert hazards(["v_readfirstlane_b32 s6, v0", "s_mov_b32 m0, s58", "s_nop 0", load]) == (1, [], [])
 
 
-@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_f32"])
+@pytest.mark.parametrize("name", ["gemm_bf16", "gemm_f32", "attention"])
 def test_loads_into_lds_wait_for_their_scalars(name, tmp_path):
     if not os.path.isfile(OBJDUMP):
         pytest.skip("no llvm-objdump on this machine")
