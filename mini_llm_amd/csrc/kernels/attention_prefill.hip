@@ -18,6 +18,7 @@
 // the reference reads its keys from the step's own qkv buffer (:99-111) and so cannot continue a
 // prompt from the cache.
 #include "common.h"
+#include "query_tiles.h"
 
 #include <type_traits>
 
@@ -45,7 +46,7 @@ union Frag8 {
 // MODE 0: plain softmax; 1: shaped scores; 2: shaped scores whose weights are sigmoid(score + bias of the head), every
 // visible key on its own: no running maximum, no sum, nothing to rescale, and the states of two wavefronts simply add.
 // The weights are fp32 until they are packed for the second product, as the softmax's are.
-template <int DH, int NW, int MODE = 0>
+template <int DH, int NW, int MODE, bool LONGEST_FIRST>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, (DH >= 128 && NW == 4) ? 1 : 2)))
 prefill_attention_kernel(const bf16_t* __restrict__ q, int q_stride, int q_col,
                          const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages, int kv_dim,
@@ -68,18 +69,9 @@ prefill_attention_kernel(const bf16_t* __restrict__ q, int q_stride, int q_col,
     __shared__ __attribute__((aligned(16))) bf16_t Vt2[2][DH * PF_VT_STRIDE];
     extern __shared__ int sm_table[];          // the sequence's block table (max_blocks entries)
 
-    // Which sequence and which of its 64-query tiles this workgroup has. Heads vary fastest and the
-    // tiles are handed out last-first: a causal tile's work grows with its position, so the long
-    // ones start in the first wave of workgroups and the short ones fill the tail.
-    int tile = gridDim.y - 1 - blockIdx.y, b = 0, q_begin = 0, q_len = 0;
-    for (; b < n_seqs; ++b) {
-        q_begin = cu_q[b];
-        q_len = cu_q[b + 1] - q_begin;
-        const int nt = (q_len + PF_BM - 1) / PF_BM;
-        if (tile < nt) break;
-        tile -= nt;
-    }
-    if (b >= n_seqs) return;               // surplus workgroup; the whole workgroup leaves
+    // Heads vary fastest.
+    const auto [b, tile, q_begin, q_len] = LONGEST_FIRST ? longest_tile<PF_BM>(cu_q, ctx_len, n_seqs, 1, blockIdx.y) : next_tile<PF_BM>(cu_q, n_seqs, 1, blockIdx.y, gridDim.y);
+    if (b < 0) return;                     // surplus workgroup; the whole workgroup leaves
 
     const int h = blockIdx.x, hk = h / (n_heads / n_kv_heads);
     const int tid = threadIdx.x, lane = tid % 64;
@@ -403,21 +395,25 @@ int mllm_prefill_attention_bf16(const void* q, int q_stride, int q_col, const vo
     const dim3 grid(n_heads, n_tiles_upper);
     const size_t table_bytes = static_cast<size_t>(max_blocks) * sizeof(int);
     const float sl2 = scale * 1.44269504088896340736f;
-#define PF_LAUNCH(D, W, S)                                                                                  \
+#define PF_LAUNCH_IN(D, W, S, L)                                                                                  \
     do {                                                                                                    \
         static bool lds_allowed = false;      /* static and dynamic LDS together pass 64 KB: asked for once */ \
         if (!lds_allowed) {                                                                                 \
-            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_attention_kernel<D, W, S>), \
+            hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(prefill_attention_kernel<D, W, S, L>), \
                                                hipFuncAttributeMaxDynamicSharedMemorySize,                  \
                                                PF_TABLE_LDS * static_cast<int>(sizeof(int)));               \
             if (e != hipSuccess) return static_cast<int>(e);                                                \
             lds_allowed = true;                                                                             \
         }                                                                                                   \
-        prefill_attention_kernel<D, W, S><<<grid, W * 64, table_bytes, stream>>>(                           \
+        prefill_attention_kernel<D, W, S, L><<<grid, W * 64, table_bytes, stream>>>(                           \
             (const bf16_t*)q, q_stride, q_col, (const bf16_t*)k_pages, (const bf16_t*)v_pages, kv_dim,      \
             block_tables, max_blocks, cu_q, ctx_len, n_seqs, n_heads, n_kv_heads, page_size, sl2, window,   \
             (bf16_t*)out, out_stride, sh, scale, gate, ldg);                                                \
     } while (0)
+    // The longest tiles of all sequences first, from four sequences on (next_tile and longest_tile; up to three the other order is
+    // the better one, or what finding the tile costs is more than it gives: 2 x 1,024 tokens 17.2 us against 17.4, 25 heads at 2 x 900 25.4, 27.5).
+    const bool longest_first = n_seqs >= 4 && n_seqs <= MLLM_WAVE;
+#define PF_LAUNCH(D, W, S) do { if (longest_first) PF_LAUNCH_IN(D, W, S, true); else PF_LAUNCH_IN(D, W, S, false); } while (0)
 #define PF_CASE(D, W, KEY)                                                                                  \
     case KEY: {                                                                                             \
         if (shape && shape->sigmoid) PF_LAUNCH(D, W, 2);                                                    \
@@ -437,6 +433,7 @@ int mllm_prefill_attention_bf16(const void* q, int q_stride, int q_col, const vo
     }
 #undef PF_CASE
 #undef PF_LAUNCH
+#undef PF_LAUNCH_IN
     MLLM_LAUNCH_CHECK();
     return 0;
 }

@@ -9,6 +9,7 @@
 #include <algorithm>
 
 #include "common.h"
+#include "query_tiles.h"
 
 namespace {
 
@@ -412,24 +413,15 @@ latent_prefill_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ 
     bf16_t* Vt = Ks + BN * KSTRIDE;                                  // [R][VSTRIDE]
     int* sm_table = reinterpret_cast<int*>(Vt + R * VSTRIDE);        // the sequence's block table
 
-    int tile = gridDim.x - 1 - blockIdx.x, b = 0, q_begin = 0, q_len = 0;
-    if (single_tokens) {
-        // every sequence brings one token: its tiles follow from the tile's index, without the walk over the
-        // sequences below, whose every step waits for a load
-        const int per = (H + 63) / 64;
-        b = tile / per;
-        tile -= b * per;
-        if (b < n_seqs) { q_begin = b; q_len = 1; }
+    QueryTile mine;
+    if (single_tokens) {       // (every sequence brings one token: its tiles follow from the tile's index)
+        const int per = (H + 63) / 64, at = gridDim.x - 1 - blockIdx.x;
+        mine = {at / per < n_seqs ? at / per : -1, at % per, at / per, 1};
     } else {
-        for (; b < n_seqs; ++b) {
-            q_begin = cu_q[b];
-            q_len = cu_q[b + 1] - q_begin;
-            const int nt = (q_len * H + 63) / 64;
-            if (tile < nt) break;
-            tile -= nt;
-        }
+        mine = query_tile<64>(cu_q, ctx_len, n_seqs, H, blockIdx.x, gridDim.x);
     }
-    if (b >= n_seqs) return;                       // surplus workgroup; the whole workgroup leaves
+    const auto [b, tile, q_begin, q_len] = mine;
+    if (b < 0) return;                             // surplus workgroup; the whole workgroup leaves
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64);
     const int G = lane / 16, c16 = lane % 16;
