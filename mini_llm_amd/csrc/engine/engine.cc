@@ -364,7 +364,7 @@ float* ModelRunner::run(const StepView& step) {
     return logits;
 }
 
-const float* ModelRunner::step(const std::vector<StepEntry>& entries, bool manage_cache, int* n_rows) {
+const float* ModelRunner::step(const std::vector<StepEntry>& entries, bool manage_cache, int* n_rows, float* into) {
     CacheManager& mgr = manager();
     std::vector<int64_t> fresh;
     if (manage_cache) {
@@ -404,6 +404,8 @@ const float* ModelRunner::step(const std::vector<StepEntry>& entries, bool manag
             HIP_OK(hipHostMalloc(reinterpret_cast<void**>(&host_logits_), host_logits_bytes_, hipHostMallocDefault));
         }
         HIP_OK(hipMemcpyAsync(host_logits_, logits, bytes, hipMemcpyDeviceToHost, stream_));
+        if (into != nullptr)
+            for (size_t at = 0; at < bytes; at += 4096) reinterpret_cast<volatile char*>(into)[at] = 0;
     }
     HIP_OK(hipStreamSynchronize(stream_));
     return logits != nullptr ? host_logits_ : nullptr;

@@ -349,7 +349,7 @@ int mllm_runner_step(void* runner, const long long* ids, const int* n_tokens, co
         if (total > cap_rows) fail("%lld rows of logits are wanted, the buffer holds %lld", total, cap_rows);
         int n = 0;
         ModelRunner* r = static_cast<ModelRunner*>(runner);
-        const float* host = r->step(entries, true, &n);
+        const float* host = r->step(entries, true, &n, logits);
         if (host != nullptr) std::memcpy(logits, host, static_cast<size_t>(n) * r->model().model.vocab_size() * sizeof(float));
         rows = n;
     });
