@@ -1220,8 +1220,17 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     int cols_per_wg = 16;
     const bool dealt_out = !MERGED && gated == nullptr && split_k && row_blocks == 1 && k_parts == 1 && tiles > 256 && tiles <= 512 &&
                            (LN_FUSED || M <= 8);
-    const bool two_tiles = dealt_out || gated != nullptr;      // (a gated pair: a tile of either map)
+    // The same behind the fused norm with 17 to 32 rows, 128 workgroups a row block: every workgroup normalises its 16 rows again, and more
+    // than 256 of them share compute units. One and two tiles a workgroup, 32 rows, us: 2,304 x 768 7.4 > 6.6, 3,072 x 1,024 10.9 > 7.3,
+    // 4,096 x 1,024 11.3 > 7.6, 3,600 x 1,600 14.7 > 9.2; two rounds of them pay only for a long K: 6,400 x 1,600 27.4 > 16.5, 5,120 x
+    // 1,280 17.5 > 14.7, but 4,112 x 768 10.0 / 11.7, 10,000 x 768 15.4 / 17.2.
+    const bool dealt_out_2 = gated == nullptr && split_k && LN_FUSED && row_blocks == 2 && tiles > 128 && (tiles <= 256 || K > 1024);
+    const bool two_tiles = dealt_out || dealt_out_2 || gated != nullptr;      // (a gated pair: a tile of either map)
     if (dealt_out) cols_per_wg = (N + 255) / 256;
+    if (dealt_out_2) {
+        const int rounds = (tiles + 255) / 256;      // of 128 workgroups a row block, two tiles each
+        cols_per_wg = (N + 128 * rounds - 1) / (128 * rounds);
+    }
     // Fewer than 256 tiles, one row block and a long K (the second product of the feed-forward):
     // narrower tiles, down to 4 columns, so that more compute units share the weights. (Short K, or
     // the fused norm: the kernel's time is latency, not bytes, and nothing is gained; measured.)

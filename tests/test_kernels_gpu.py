@@ -491,6 +491,25 @@ def test_linear_bf16_few_rows_long_k_shares_tiles(ops, M, N, K):
     assert torch.equal(x.cpu(), outs[0])
 
 
+@pytest.mark.parametrize("M", [17, 25, 32])
+@pytest.mark.parametrize("N,K", [(2048, 768), (2049, 768), (2304, 768), (2500, 1024), (4096, 768), (4097, 768), (4097, 1032), (6400, 1600)])
+@pytest.mark.parametrize("epi", ["store", "gelu_tanh"])
+def test_ln_linear_two_tiles_a_workgroup(ops, M, N, K, epi):
+    """17 to 32 rows behind the fused norm, where a workgroup has one tile of columns and where it has two, the second narrower: which rows
+    share a launch does not change a bit."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (_rand((M, K), torch.float32, g, std=2.0) + 0.3).to(DEV)
+    gamma, beta = (1 + 0.1 * _rand((K,), torch.float32, g)).to(DEV), (0.1 * _rand((K,), torch.float32, g)).to(DEV)
+    w, bias = _rand((N, K), torch.bfloat16, g, std=1.0 / math.sqrt(K)).to(DEV), (0.5 * _rand((N,), torch.float32, g)).to(DEV)
+    out, parts = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.ln_linear(x, gamma, beta, 1e-5, w, bias, out, epi)
+    for m in range(0, M, 16):
+        ops.ln_linear(x[m:m + 16], gamma, beta, 1e-5, w, bias, parts[m:m + 16], epi)
+    assert torch.equal(out, parts)
+    ref = plain_ops.ln_linear(x.cpu(), gamma.cpu(), beta.cpu(), 1e-5, w.cpu(), bias.cpu(), torch.empty(M, N, dtype=torch.float64), epi)
+    assert (out.cpu().double() - ref).abs().max().item() <= 4e-2
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(1, 2304, 768), (8, 3072, 768), (16, 320, 96), (5, 200, 1600), (17, 96, 64),
                                    (3, 64, 4096), (16, 6400, 1600), (9, 50257, 1024), (16, 3072, 1024), (33, 2304, 768),
