@@ -490,3 +490,37 @@ def test_scan_finds_chunks_among_many_portions(sizes, vdim, state):
     given = _scan_inputs(sizes, 1, vdim, state, seed=len(sizes))
     for got, want, size in zip(_scan(sizes, given), _scan_plain(sizes, given), _scan_plain(sizes, given, magnitudes=True)):
         assert ((got.double() - want).abs() <= 2.0 ** -24 * (state + 64 + 200) * size).all()
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("lens", [[1300], [1, 700, 2, 3, 597, 1], [1029, 250]])
+def test_convolution_of_many_tokens(taps, lens):
+    """From 2^21 inputs on a thread has four tokens: portions that begin and end within the four, and are shorter than they, have the bits that
+    every portion has alone, the carried rows in front of it and behind it too."""
+    import ctypes
+    import torch
+    from mini_llm_amd import build
+    f = build.load_library("ssm").mllm_conv_silu
+    C, T, B, dev, g = 1792, sum(lens), len(lens), "cuda:0", torch.Generator().manual_seed(taps)
+    x, w, bias = torch.randn(T, C + 8, generator=g).to(dev), torch.randn(C, taps, generator=g).to(dev), torch.randn(C, generator=g).to(dev)
+    state = torch.randn(B + 1, (taps - 1) * C + 4, generator=g).to(dev)
+    cu = [sum(lens[:i]) for i in range(B + 1)]
+
+    def run(rows, slots, seqs, state, out):
+        arrays = [torch.tensor(a, dtype=torch.int32, device=dev) for a in (seqs, [0] + [sum(1 for s in seqs if s <= b) for b in range(max(seqs) + 1)], slots)]
+        rc = f(*(ctypes.c_void_p(a.data_ptr()) if torch.is_tensor(a) else ctypes.c_int(a) for a in (rows, rows.stride(0), 8, C, w, bias, taps, *arrays, state)),
+               ctypes.c_size_t(state.stride(0)), ctypes.c_void_p(out.data_ptr()), *(ctypes.c_int(a) for a in (C, len(seqs), len(slots), 1)),
+               ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        assert rc == 0
+        torch.cuda.synchronize()
+
+    together, alone, s1, s2 = torch.zeros(T, C, device=dev), torch.zeros(T, C, device=dev), state.clone(), state.clone()
+    run(x, list(range(1, B + 1)), [b for b, n in enumerate(lens) for _ in range(n)], s1, together)
+    for b in range(B):
+        for t in range(cu[b], cu[b + 1], 1024):          # (cut, so that each call is below the line)
+            n = min(1024, cu[b + 1] - t)
+            run(x[t:t + n], [b + 1], [0] * n, s2, alone[t:t + n])
+    assert torch.equal(together, alone) and torch.equal(s1, s2)
+    first = torch.cat([s.reshape(taps - 1, C) for s in state[1:2, :(taps - 1) * C]] + [x[:lens[0], 8:]]).double()
+    y = sum(first[j:j + lens[0]] * w[:, j].double() for j in range(taps)) + bias.double()
+    assert (together[:lens[0]].double() - y * torch.sigmoid(y)).abs().max() <= 1e-5
