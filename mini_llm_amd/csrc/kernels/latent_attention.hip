@@ -170,7 +170,7 @@ union Frag8 {
 // (w_head_rows = N, w_head_cols = 0: every head has its own rows of w; w_head_rows = 0, w_head_cols = K: its own
 // columns). A workgroup takes 64 tokens, one head and 64 values of n; a wavefront 16 tokens: the weights are the
 // MFMA's A operand, so a lane ends up with four neighbouring n of one token. K is a multiple of 32; rows and head
-// offsets are 16-byte aligned. With `positions`, the workgroups of the first n tile also carry the `tail` columns
+// offsets are 16-byte aligned. With `positions`, the workgroups of a head also carry the `tail` columns
 // behind a head's K inputs over to behind its N outputs, the first rot_dims of them turned in pairs. With `gate` (fp32
 // rows of H columns) head h's result is multiplied by sigmoid(gate[t, h]). The inputs are bfloat16 or fp32 rows (TA),
 // which are rounded as they are loaded.
@@ -239,10 +239,11 @@ head_linear_mfma_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_
                 if (n + r < N) orow[n + r] = float_to_bf16(acc[ct][r] * g);
         }
     }
-    if (positions != nullptr && blockIdx.z == 0) {
-        // (pairs and plain columns in loops of their own: a wavefront that holds both would run the turn for a third of its lanes)
+    if (positions != nullptr) {
+        // (pairs and plain columns in loops of their own: a wavefront that holds both would run the turn for a third of its lanes; dealt out over
+        // the workgroups of all n tiles: done by those of the first alone they are what 2,048 tokens wait for)
         const int nt = min(64, n_tokens - t0), pairs = rot_dims / 2, plain = tail - rot_dims;
-        for (int i = threadIdx.x; i < nt * pairs; i += 256) {
+        for (int i = threadIdx.x + 256 * blockIdx.z; i < nt * pairs; i += 256 * gridDim.z) {
             const int tt = i / pairs, k = i % pairs;
             const TA* src = a + static_cast<size_t>(t0 + tt) * lda + static_cast<size_t>(h) * a_hs + K;
             bf16_t* dst = out + static_cast<size_t>(t0 + tt) * ldo + static_cast<size_t>(h) * out_hs + N;
@@ -252,7 +253,7 @@ head_linear_mfma_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_
             dst[first] = float_to_bf16(u);
             dst[second] = float_to_bf16(v);
         }
-        for (int i = threadIdx.x; i < nt * plain; i += 256) {
+        for (int i = threadIdx.x + 256 * blockIdx.z; i < nt * plain; i += 256 * gridDim.z) {
             const int tt = i / plain, c = rot_dims + i % plain;
             out[static_cast<size_t>(t0 + tt) * ldo + static_cast<size_t>(h) * out_hs + N + c] =
                 float_to_bf16(to_float(a[static_cast<size_t>(t0 + tt) * lda + static_cast<size_t>(h) * a_hs + K + c]));
