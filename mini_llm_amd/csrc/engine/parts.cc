@@ -126,7 +126,7 @@ const Tensor2& NormedInput::tensor(Arena& arena, hipStream_t s) {
 
 void NormedInput::linear(const Linear& lin, const Tensor2& out, int epilogue, const KvScatter* kv, Arena& arena,
                          hipStream_t s) {
-    if (have_) lin(h_, out, epilogue, kv, s);
+    if (have_ && (norm_ == nullptr || lin.weight.dtype == h_.dtype)) lin(h_, out, epilogue, kv, s);
     else norm_->linear(x_, lin, out, epilogue, nullptr, kv, arena, s);
 }
 
@@ -661,6 +661,8 @@ size_t DecoderModel::workspace_bytes(int tokens, int n_logits) const {
         if (l->wants_zeroed_rows()) { stream += one; break; }
     for (const auto& l : layers)
         if (l->wants_stream_copy()) { stream += one / 2 + 256; break; }
+    for (const auto& l : layers)
+        if (l->first_norm() != nullptr) { stream += one / 2 + 256; break; }
     for (const auto& st : stream_steps) {
         if (st->wants_embedding_output()) { stream += one; break; }
     }
@@ -695,6 +697,15 @@ void DecoderModel::forward(const StepView& step, const std::vector<CacheView>& c
         with_rows.step_copy = arena.tensor(BF16, step.n_tokens, hidden_size());
         break;
     }
+    // Where a block enters by a norm with statistics, the norm at the end of the block in front leaves it: 2,048 rows of 768 are read once
+    // less, 5.7 + 5.2 > 6.1 us a layer. (Few rows: a block's first product takes its norm inside, which costs no launch.)
+    Tensor2 first_normed;
+    for (const auto& l : layers) {
+        if (l->first_norm() == nullptr || step.n_tokens <= tuning().ln_fuse_max_rows) continue;
+        first_normed = arena.tensor(BF16, step.n_tokens, hidden_size());
+        break;
+    }
+    bool left = false;
     // What the block of call i (or a stream step) finds in its copy as it is entered, and what is there now. Whoever runs in front of a block
     // is told (StepView::leave) and leaves it if it can; otherwise it is made here.
     using Leave = StepView::Leave;
@@ -765,6 +776,14 @@ void DecoderModel::forward(const StepView& step, const std::vector<CacheView>& c
         if (enters.wanted && !have.same(enters)) make(enters);
         const Block& b = *layers[c.layer];
         with_rows.leave = c.after >= 0 ? wanted_by_step(c.after) : wanted_in_front(i + 1);
+        with_rows.entered = left ? first_normed : Tensor2();
+        left = false;
+        with_rows.next_norm = StepView::NextNorm();
+        if (first_normed.data != nullptr && c.after < 0 && i + 1 < order.size() && order[i + 1].before < 0) {
+            with_rows.next_norm.norm = layers[order[i + 1].layer]->first_norm();
+            with_rows.next_norm.into = first_normed;
+            with_rows.next_norm.left = &left;
+        }
         b.forward(x, with_rows, caches[c.cache], c.write, arena, s);
         // (a block that keeps a copy of the stream itself keeps it whether it is asked or not)
         const bool normed = with_rows.leave.norm.weight != nullptr;

@@ -80,6 +80,8 @@ private:
     size_t capacity_, used_ = 0, peak_ = 0;
 };
 
+class Norm;
+
 // The step's batch: sizes known to the host and device arrays (int32).
 struct StepView {
     int n_tokens = 0, n_seqs = 0, n_logits = 0, max_q_len = 0, max_ctx_len = 0, n_single = 0;
@@ -107,6 +109,14 @@ struct StepView {
         Tensor2 into;
         bool same(const Leave& o) const { return wanted == o.wanted && norm.weight == o.norm.weight && into.data == o.into.data; }
     } leave;
+    // Many rows between two blocks of which the one behind enters by a norm with statistics (Block::first_norm): the one in front
+    // may leave that norm of the stream in `into` and say so in *left (a host variable). The block behind finds it in `entered`.
+    struct NextNorm {
+        const Norm* norm = nullptr;
+        Tensor2 into;
+        bool* left = nullptr;
+    } next_norm;
+    Tensor2 entered;                   // the block's first norm of the stream, of the compute dtype, if the block in front left it
     int n_groups = 0;
     const int* const* block_tables = nullptr;   // per group [B, max_blocks[g]]
     const int* max_blocks = nullptr;            // per group
@@ -277,6 +287,7 @@ class NormedInput {
 public:
     NormedInput(const Norm& norm, const Tensor2& x) : norm_(&norm), x_(x) {}
     explicit NormedInput(const Tensor2& h) : norm_(nullptr), x_(h), h_(h), have_(true) {}     // normalised already
+    NormedInput(const Norm& norm, const Tensor2& x, const Tensor2& h) : norm_(&norm), x_(x), h_(h), have_(true) {}     // the same, where x is still there
     const Tensor2& tensor(Arena& arena, hipStream_t s);
     void linear(const Linear& lin, const Tensor2& out, int epilogue, const KvScatter* kv, Arena& arena, hipStream_t s);
     // the norm inside, where it is still to be taken and the kernels allow it (see Norm::linear_gated)
@@ -380,6 +391,8 @@ public:
     virtual bool entry_norm(MllmTanhNorm& n) const { (void)n; return false; }
     // true: the block leaves what StepView::leave asks for (the stream's norm, or the stream itself)
     virtual bool leaves_copy(bool normed) const { return wants_stream_copy() && !normed; }
+    // the norm through which forward() reads the stream, if it takes it ready as well (StepView::entered, bfloat16)
+    virtual const Norm* first_norm() const { return nullptr; }
     virtual void reserve(int max_seqs, hipStream_t s) const = 0;
     virtual void add_cost(StepCost&) const = 0;
 };

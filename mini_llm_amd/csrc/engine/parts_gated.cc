@@ -153,13 +153,14 @@ public:
         const size_t mark = arena.mark();
         Tensor2 y = result(set1);
         {
-            NormedInput h(*pre1_, x);
+            NormedInput h = step.entered.data != nullptr ? NormedInput(*pre1_, x, step.entered) : NormedInput(*pre1_, x);
             if (set1) mixer_->forward_set(h, step, cache, y, write, arena, s);
             else mixer_->forward(h, step, cache, y, write, arena, s);
         }
         arena.release(mark);
         const float* scale1 = static_cast<const float*>(scale1_.data);
-        const bool normed = h2.data != nullptr && post1_->add_scaled_then(y, scale1, mult_, x, !set1 && shared, *pre2_, h2, s);
+        const bool normed = h2.data != nullptr ? post1_->add_scaled_then(y, scale1, mult_, x, !set1 && shared, *pre2_, h2, s)
+                                               : !ff_ && leave_next(*post1_, y, scale1, x, !set1 && shared, step, s);
         if (!normed) post1_->add_scaled(y, scale1, mult_, x, !set1 && shared, s);
         StageTimes::get().mark("post_norm", s);
         if (ff_) {
@@ -170,7 +171,8 @@ public:
                 else ff_->forward(h, step, y, arena, s);
             }
             arena.release(mark);
-            post2_->add_scaled(y, static_cast<const float*>(scale2_.data), mult_, x, !set2 && shared, s);
+            const float* scale2 = static_cast<const float*>(scale2_.data);
+            if (!leave_next(*post2_, y, scale2, x, !set2 && shared, step, s)) post2_->add_scaled(y, scale2, mult_, x, !set2 && shared, s);
             StageTimes::get().mark("post_norm2", s);
         }
         arena.release(outer);
@@ -183,6 +185,7 @@ public:
     CacheNeed cache_need() const override { return mixer_->cache_need(); }
     bool wants_zeroed_rows() const override { return !pointwise_ && !(mixer_->sets_result() && (!ff_ || ff_->sets_result())); }
     bool wants_stream_copy() const override { return pointwise_ && dtype_ == BF16; }
+    const Norm* first_norm() const override { return !pointwise_ && dtype_ == BF16 ? pre1_.get() : nullptr; }
     bool entry_norm(MllmTanhNorm& n) const override { if (pointwise_) n = n_pre1_; return pointwise_; }
     bool leaves_copy(bool) const override { return wants_stream_copy(); }
     void reserve(int max_seqs, hipStream_t s) const override {
@@ -197,6 +200,14 @@ public:
     }
 
 private:
+    // The block's last norm, which adds y into the stream, with the next block's first in the same pass. Not asked for, or no such
+    // kernel: false, nothing was done.
+    bool leave_next(const Norm& last, const Tensor2& y, const float* scale, const Tensor2& x, bool clear, const StepView& step, hipStream_t s) const {
+        const StepView::NextNorm& next = step.next_norm;
+        if (next.norm == nullptr || !last.add_scaled_then(y, scale, mult_, x, clear, *next.norm, next.into, s)) return false;
+        *next.left = true;
+        return true;
+    }
     Tensor2 checked_scale(const Tensor2& t) {
         if (t.dtype != F32 || !t.contiguous() || t.rows * t.cols != size_) fail("a layer scale must be contiguous float32 [%d]", size_);
         return Tensor2(t.data, F32, 1, t.rows * t.cols);

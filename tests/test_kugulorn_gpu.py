@@ -87,6 +87,18 @@ def test_prompt_portions_on_the_matrix_cores(dirs, family, page):
     assert runner.check() == "" and runner.info()["n_requests"] == 0
 
 
+@pytest.mark.parametrize("name,page", [("TILED", 16), ("ODD", 4)])
+def test_norms_of_neighbouring_layers_join_from_33_rows(dirs, name, page):
+    """Up to 32 rows a layer's first products take their norm inside; from 33 on the norm behind the layer in front leaves it. Portions on
+    both sides of the line, and one that ends a request which began on the other side."""
+    cfg, d = getattr(kc, name), dirs(name)
+    reqs = kc.requests(cfg["vocab"], [31, 32, 33, 34, 65], seed=75)
+    for label, steps in (("whole", ru.trace_whole(reqs)), ("chunks", ru.trace_chunks(reqs, seed=3, sizes=(33, 32)))):
+        runner = _runner(d, "bfloat16", n_pages=ru.peak_tokens(steps) // page, page=page)
+        kc.check_against_plain(d, reqs, steps, ru.run_in_process(runner, steps), "bfloat16", cfg["vocab"], f"{name} {label}")
+        assert runner.check() == "" and runner.info()["n_requests"] == 0
+
+
 @pytest.mark.parametrize("family", ["whole", "mixed"])
 def test_widest_rows_on_the_matrix_cores(dirs, family):
     from mini_llm_amd.kernels import ops
