@@ -432,9 +432,9 @@ paged_attention_tiled_f32(const float* __restrict__ q, int q_stride, int q_col, 
         }
         float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
         const float m_new = fmaxf(m, rows_max(mx));
-        // (a query none of whose keys has come yet keeps m = -inf: all weights are zero against a finite number. Weights below the
+        // (a query none of whose scores so far is above -inf: all weights are zero against any finite number. Weights below the
         // normal range are lost beside the maximum's 1, so the bare instruction does.)
-        const float against = fmaxf(m_new, -3.0e38f), alpha = fast_exp2(m - against);
+        const float against = m_new == -INFINITY ? 0.f : m_new, alpha = fast_exp2(m - against);
         float sum = 0.f;
 #pragma unroll
         for (int g = 0; g < 2; ++g)
@@ -467,8 +467,8 @@ paged_attention_tiled_f32(const float* __restrict__ q, int q_stride, int q_col, 
     if (half == 1 || !q_ok) return;
     {
         const float2 other = *reinterpret_cast<const float2*>(states + DC * STATE_STEP - (group * 64 + lane) * 2);
-        const float m_new = fmaxf(m, other.x);     // (a query sees itself: one of the two is finite)
-        const float a = fast_exp2(m - m_new), a2 = fast_exp2(other.x - m_new);
+        const float m_new = fmaxf(m, other.x), against = m_new == -INFINITY ? 0.f : m_new;     // (all its scores -inf: nothing but a sink counts)
+        const float a = fast_exp2(m - against), a2 = fast_exp2(other.x - against);
         l = l * a + other.y * a2;
         m = m_new;
 #pragma unroll

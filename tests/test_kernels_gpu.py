@@ -729,8 +729,8 @@ def test_kv_append_reference_vector(ops, dtype):
     assert (kp.cpu()[untouched] == -1).all() and (vp.cpu()[untouched] == -1).all()
 
 
-def _attention_case(ops, dtype, H, Hkv, dh, page, seqs, window, gen, boost=None, n_single=0, q_col=8, shape=None, gated=False):
-    """seqs: list of (start, q_len). Builds pages in scrambled order, garbage elsewhere."""
+def _attention_case(ops, dtype, H, Hkv, dh, page, seqs, window, gen, boost=None, n_single=0, q_col=8, shape=None, gated=False, edit=None):
+    """seqs: list of (start, q_len). Builds pages in scrambled order, garbage elsewhere. `edit(b, q, k, v)` may change a sequence's rows."""
     B = len(seqs)
     ctx = [s + n for s, n in seqs]
     nblk = [-(-c // page) for c in ctx]
@@ -755,6 +755,8 @@ def _attention_case(ops, dtype, H, Hkv, dh, page, seqs, window, gen, boost=None,
             far = boost[0]
             k[far] = k[far] * 0 + (q[len(token_seq) + n - 1, q_col:q_col + H * dh].float().view(H, dh)[::H // Hkv]
                                    .reshape(-1) * boost[1]).to(dtype)
+        if edit is not None:
+            edit(b, q[len(token_seq):len(token_seq) + n, q_col:q_col + H * dh].view(n, H, dh), k.view(-1, Hkv, dh), v.view(-1, Hkv, dh))
         js = torch.arange(ctx[b])
         rows = tables[b].long()[js // page] * page + js % page
         kp[rows] = k
@@ -977,6 +979,35 @@ def test_paged_attention_gives_every_tile_away(ops, dtype, seqs, H, Hkv, dh):
     out, ref = _attention_case(ops, dtype, H, Hkv, dh, 16, seqs, 0, g)
     assert torch.isfinite(out).all()
     assert (out - ref).abs().max() <= _tol(dtype, 2)
+
+
+@pytest.mark.parametrize("H,Hkv,dh", [(3, 3, 32), (3, 1, 64), (2, 2, 128)])
+@pytest.mark.parametrize("window", [0, 1])
+def test_paged_attention_of_scores_at_the_lowest_end(ops, H, Hkv, dh, window):
+    """32-bit portions. Scores of -inf beside a sink: a query that sees no other key has the sink's weight alone, in either half of a
+    key tile, and gives 0. A score just above the lowest float, in base 2 too, is a score like any other."""
+    g = torch.Generator().manual_seed(dh + window)
+    seqs, at = [(0, 130), (0, 70), (60, 9)], [0, 5, 40, 64, 100]
+
+    def lowest(b, q, k, v):
+        if window == 0 and b == 1:                            # all that the sequence's queries see
+            k[..., 0], q[..., 0] = math.inf, -q[..., 0].abs() - 0.1
+        elif window == 1 and b == 0:                          # a query's own key
+            k[at, :, 0], q[at, :, 0] = math.inf, -q[at, :, 0].abs() - 0.1
+
+    out, ref = _attention_case(ops, torch.float32, H, Hkv, dh, 16, seqs, window, g, q_col=0, shape={"sink": torch.randn(H, generator=g)}, edit=lowest)
+    rows = [130 + i for i in range(70)] if window == 0 else at
+    assert (out[rows] == 0).all() and (ref[rows] == 0).all()
+    assert (out - ref).abs().max() <= _tol(torch.float32, 2)
+
+    def low(b, q, k, v):
+        if b == 0:
+            q[at, :], k[at, :] = 0.0, 0.0
+            q[at, :, 0], k[at, :, 0] = -16.0, 2.2e38 * math.sqrt(dh) / 16
+
+    if window == 1:
+        out, ref = _attention_case(ops, torch.float32, H, Hkv, dh, 16, seqs, window, g, edit=low)
+        assert (out - ref).abs().max() <= _tol(torch.float32, 2)
 
 
 @pytest.mark.parametrize("T", [1, 8, 16])
