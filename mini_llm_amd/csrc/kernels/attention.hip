@@ -313,7 +313,7 @@ paged_attention_tiled(const T* __restrict__ q, int q_stride, int q_col, const T*
 // Bound by the chain of a workgroup's key tiles where workgroups are few (2.5 us a tile, of which the matrix instructions are 1.7), by the
 // matrix cores for long prompts. 12 heads of 64, with the kernel above before: 8 x 256 tokens 30.7 > 20.7 us, 331 + 512 + 470 + 400
 // 43.6 > 30, 2 x 1,024 91 > 56, 8,000 988 > 892 (110 TFLOP/s of 155); 8 heads of 128, 4 x 512 76 > 45.
-// A place outside [k_lo, p_last] (not written yet, or given back by a window) loads the next key that is inside; its weight is 0.
+// A place outside [k_lo, p_last] (not written yet, or given back by a window) loads the next key that is inside; its weight is 0, its values are taken as 0.
 #define TD_TABLE 4096      // entries of a block table that fit LDS beside two stages of tiles, two workgroups a unit
 
 template <int DH, bool SHAPED>
@@ -429,6 +429,18 @@ paged_attention_tiled_f32(const float* __restrict__ q, int q_stride, int q_col, 
                     const int j = first + 16 * g + 4 * G + i;
                     s[g][i] = (j <= p && (j >= my_lo || j < kf)) ? s[g][i] : -INFINITY;
                 }
+            // (the places outside hold another key's values, which may be infinite: a weight of 0 does not take those away)
+            if (first + 31 > p_last || first < k_lo) {
+#pragma unroll
+                for (int g = 0; g < 2; ++g)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int j = first + 16 * g + 4 * G + i;
+                        const bool inside = j <= p_last && (j >= k_lo || j < kf);
+#pragma unroll
+                        for (int c = 0; c < DC; ++c) vr[g][i][c] = inside ? vr[g][i][c] : 0.f;
+                    }
+            }
         }
         float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
         const float m_new = fmaxf(m, rows_max(mx));

@@ -780,7 +780,7 @@ def _attention_case(ops, dtype, H, Hkv, dh, page, seqs, window, gen, boost=None,
     ref = torch.zeros(T, H * dh, dtype=torch.float64)
     plain_ops.paged_attention(q, q_col, H, Hkv, dh, kp, vp, page, tables, token_seq, positions, scale, window, ref,
                               shape=shape, gate=gate)
-    if shape is None and sum(c * n for c, (_, n) in zip(ctx, seqs)) * H * dh <= 2e8:
+    if shape is None and edit is None and sum(c * n for c, (_, n) in zip(ctx, seqs)) * H * dh <= 2e8:
         # the second oracle, the plain C++ twin, says the same
         twin = ref_ops.paged_attention(q, 8, H, Hkv, dh, kp, vp, page, tables, token_seq, positions, scale, window)
         assert (twin.double() - ref).abs().max() <= 2e-6
@@ -1008,6 +1008,25 @@ def test_paged_attention_of_scores_at_the_lowest_end(ops, H, Hkv, dh, window):
     if window == 1:
         out, ref = _attention_case(ops, torch.float32, H, Hkv, dh, 16, seqs, window, g, edit=low)
         assert (out - ref).abs().max() <= _tol(torch.float32, 2)
+
+
+@pytest.mark.parametrize("H,Hkv,dh", [(3, 3, 32), (3, 1, 64), (2, 2, 128)])
+@pytest.mark.parametrize("window,keep", [(0, 0), (8, 0), (8, 3), (40, 70)])
+def test_paged_attention_of_infinite_values_beside_empty_places(ops, H, Hkv, dh, window, keep):
+    """32-bit portions of one query (in a step with a longer one): an infinite value at the first and at the last key that it sees gives
+    an infinity. The places of a key tile in front of the first and behind the last have no values at all."""
+    g = torch.Generator().manual_seed(dh + window + keep)
+    seqs = [(0, 66), (0, 1), (31, 1), (70, 1), (127, 1), (300, 1)]
+    shape = {"keep_first": keep, "sink": torch.randn(H, generator=g)} if keep else None
+    for last in (True, False):
+        def infinite(b, q, k, v):
+            p = seqs[b][0]
+            if b > 0:
+                v[p if last or not window else max(0, p - window + 1)] = math.inf
+
+        out, ref = _attention_case(ops, torch.float32, H, Hkv, dh, 16, seqs, window, g, q_col=0, shape=shape, edit=infinite)
+        assert (out[66:] == math.inf).all() and (ref[66:] == math.inf).all()
+        assert (out[:66] - ref[:66]).abs().max() <= _tol(torch.float32, 2)
 
 
 @pytest.mark.parametrize("T", [1, 8, 16])
