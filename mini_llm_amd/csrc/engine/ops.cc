@@ -370,6 +370,15 @@ void linear_from_splits(const AttentionSplits& a, const Tensor2& w, const float*
     linear(merged, w, bias, out, epilogue, nullptr, stream);
 }
 
+// Where the norm inside the few-row product is worth it: not where that product wants two tiles of columns a workgroup and their LDS does
+// not fit (K over 2,016), so that it runs with one. Norm and product then are shorter (us, inside > apart): 17 rows 2,304 x 2,048 15.0 > 11.1, 32 rows
+// 4,096 x 2,048 16.4 > 12.8, 8 rows 6,144 x 2,048 13.4 > 11.4, 16 rows 8,192 x 2,024 18.4 > 16.0; at K = 2,016 8 rows 6,144 10.8 < 12.3, 32
+// rows 4,096 12.1 < 13.6.
+bool norm_inside_pays(int64_t rows, int64_t columns, int64_t k) {
+    const bool wants_two = rows <= 16 ? columns > 4096 && columns <= 8192 : rows <= 32 && columns > 2048;
+    return k <= 2016 || !wants_two;
+}
+
 void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float eps, const Tensor2& w,
                const float* bias, const Tensor2& out, int epilogue, const int* rows, void* tmp,
                const KvScatter* kv, hipStream_t stream) {
@@ -384,7 +393,7 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
     // again, and the norm and a product that writes the pages itself are shorter: a step of 17 tokens of GPT-2 XL takes 945 us so, 1,033 fused.)
     const bool kv_fits = kv == nullptr || (aligned(w.data, 16) && (M <= 16 || w.rows <= 4096));
     if (w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
-        (beta == nullptr || aligned(beta, 16)) && kv_fits) {
+        (beta == nullptr || aligned(beta, 16)) && kv_fits && (tmp == nullptr || norm_inside_pays(M, w.rows, K))) {
         int rc;
         if (kv != nullptr) {
             check_scatter(*kv, w.dtype, w.rows, epilogue, "ln_linear (key/value scatter)");

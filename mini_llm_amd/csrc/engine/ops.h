@@ -166,6 +166,8 @@ void linear(const Tensor2& a, const Tensor2& w, const float* bias, const Tensor2
 void linear_from_splits(const AttentionSplits& a, const Tensor2& w, const float* bias, const Tensor2& out,
                         int epilogue, void* tmp, hipStream_t stream);
 void merge_splits(const AttentionSplits& a, const Tensor2& out, hipStream_t stream);
+// Whether the norm inside the few-row product of these sizes is worth it (ln_linear, rms_linear; without room for normalised rows it runs all the same).
+bool norm_inside_pays(int64_t rows, int64_t columns, int64_t k);
 // out = epilogue(LayerNorm(x[rows]) w^T + bias), the norm fused into the product where the kernels allow;
 // `tmp` ([out.rows, K] in w's dtype) holds the normalised rows otherwise. `kv` as for linear.
 void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float eps, const Tensor2& w,

@@ -61,7 +61,7 @@ void rms_linear(const Tensor2& x, const float* weight, float eps, const Tensor2&
     if (out.dtype != (f32_out ? F32 : w.dtype)) fail("rms_linear: out must be %s", dtype_name(f32_out ? F32 : w.dtype));
     // (more rows than that: the norm is a kernel of its own, as for the LayerNorm product)
     if (w.dtype == BF16 && M <= tuning().ln_fuse_max_rows && K % 8 == 0 && w.stride % 8 == 0 && x.contiguous() &&
-        (reinterpret_cast<uintptr_t>(weight) & 15) == 0) {
+        (reinterpret_cast<uintptr_t>(weight) & 15) == 0 && (tmp == nullptr || norm_inside_pays(M, w.rows, K))) {
         const int rc = mllm_rms_gemm_bf16(static_cast<const float*>(x.data), i32(x.stride), rows, weight, eps, w.data, i32(w.stride), bias,
                                           out.data, i32(out.stride), i32(M), i32(w.rows), i32(K), epilogue, stream);
         if (rc == 0) return;

@@ -1215,16 +1215,24 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         nw = (tiles * row_blocks + 255) / 256;
         nw = nw < 4 ? 4 : (nw > 16 ? 16 : nw);
     }
+    // The LDS of a workgroup: the sums of its one or two tiles, the wavefronts' transposition regions (two k blocks at a time where the kernel
+    // stages two), behind the fused norm its 16 normalised rows and the norm's vectors. (Two tiles fit up to K = 2,016 there.)
+    const auto lds_bytes = [&](bool two) {
+        size_t bytes = split_k ? static_cast<size_t>(nw) * mt * (two ? 2 : 1) * 256 * sizeof(float) : 0;
+        bytes += static_cast<size_t>(nw) * (staged ? 2048 : LN_FUSED ? (two ? 8192 : 4096) : (two ? 6144 : 8192));
+        return LN_FUSED ? bytes + static_cast<size_t>(16) * mt * (K + 8) * sizeof(bf16_t) + static_cast<size_t>(2) * K * sizeof(float) : bytes;
+    };
+    const bool two_fit = lds_bytes(true) <= MAX_DYNAMIC_LDS;
     // More than 256 tiles (and one row block): two tiles per workgroup, the columns dealt out evenly
     // to 256 workgroups.
     int cols_per_wg = 16;
     const bool dealt_out = !MERGED && gated == nullptr && split_k && row_blocks == 1 && k_parts == 1 && tiles > 256 && tiles <= 512 &&
-                           (LN_FUSED || M <= 8);
+                           (LN_FUSED || M <= 8) && two_fit;
     // The same behind the fused norm with 17 to 32 rows, 128 workgroups a row block: every workgroup normalises its 16 rows again, and more
     // than 256 of them share compute units. One and two tiles a workgroup, 32 rows, us: 2,304 x 768 7.4 > 6.6, 3,072 x 1,024 10.9 > 7.3,
     // 4,096 x 1,024 11.3 > 7.6, 3,600 x 1,600 14.7 > 9.2; two rounds of them pay only for a long K: 6,400 x 1,600 27.4 > 16.5, 5,120 x
     // 1,280 17.5 > 14.7, but 4,112 x 768 10.0 / 11.7, 10,000 x 768 15.4 / 17.2.
-    const bool dealt_out_2 = gated == nullptr && split_k && LN_FUSED && row_blocks == 2 && tiles > 128 && (tiles <= 256 || K > 1024);
+    const bool dealt_out_2 = gated == nullptr && split_k && LN_FUSED && row_blocks == 2 && tiles > 128 && (tiles <= 256 || K > 1024) && two_fit;
     const bool two_tiles = dealt_out || dealt_out_2 || gated != nullptr;      // (a gated pair: a tile of either map)
     if (dealt_out) cols_per_wg = (N + 255) / 256;
     if (dealt_out_2) {
@@ -1238,9 +1246,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         cols_per_wg = std::min(16, std::max((N + 255) / 256, 4));
     const int col_blocks = split_k ? (N + cols_per_wg - 1) / cols_per_wg : (tiles + nw - 1) / nw;
     const dim3 grid((col_blocks + N_XCD - 1) / N_XCD * N_XCD * row_blocks, k_parts), block(nw * 64);
-    size_t smem = split_k ? static_cast<size_t>(nw) * mt * (two_tiles ? 2 : 1) * 256 * sizeof(float) : 0;
-    // the wavefronts' transposition regions (two k blocks at a time where the kernel stages two)
-    smem += static_cast<size_t>(nw) * (staged ? 2048 : LN_FUSED ? (two_tiles ? 8192 : 4096) : (two_tiles ? 6144 : 8192));
+    const size_t smem = lds_bytes(two_tiles);
     if (staged) {
         staged_bytes += smem;
 #define SKINNY_STAGED(MTV)                                                                             \
@@ -1263,7 +1269,6 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         return 0;
     }
     if (LN_FUSED) {
-        smem += static_cast<size_t>(16) * mt * (K + 8) * sizeof(bf16_t) + static_cast<size_t>(2) * K * sizeof(float);
         if (K > 2048 || (reinterpret_cast<uintptr_t>(A) & 15) || lda % 4 != 0 ||
             (reinterpret_cast<uintptr_t>(gamma) & 15) || (reinterpret_cast<uintptr_t>(beta) & 15))
             return -2;

@@ -510,6 +510,41 @@ def test_ln_linear_two_tiles_a_workgroup(ops, M, N, K, epi):
     assert (out.cpu().double() - ref).abs().max().item() <= 4e-2
 
 
+@pytest.mark.parametrize("M", [1, 16, 17, 32])
+@pytest.mark.parametrize("N", [2304, 4096, 4112, 8192])
+@pytest.mark.parametrize("K", [2008, 2016, 2024, 2048])
+@pytest.mark.parametrize("rms", [False, True])
+def test_norm_and_product_in_one_kernel_up_to_2048_columns(ops, M, N, K, rms):
+    """The kernel itself, without room for normalised rows: from K = 2,024 on two tiles of columns do not fit a workgroup's LDS, and it takes the
+    same sizes with one. Which rows share a launch does not change a bit. The op is as close to the reference on either way."""
+    import ctypes
+    from mini_llm_amd import build
+    lib = build.load_library("gemm_bf16")
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (_rand((M, K), torch.float32, g, std=2.0) + 0.3).to(DEV)
+    gamma, beta = (1 + 0.1 * _rand((K,), torch.float32, g)).to(DEV), (0.1 * _rand((K,), torch.float32, g)).to(DEV)
+    w, bias = _rand((N, K), torch.bfloat16, g, std=1.0 / math.sqrt(K)).to(DEV), (0.5 * _rand((N,), torch.float32, g)).to(DEV)
+
+    def run(m0, m1, out):
+        p, i = (lambda t: ctypes.c_void_p(t.data_ptr())), ctypes.c_int
+        f, norm = (lib.mllm_rms_gemm_bf16, [p(gamma)]) if rms else (lib.mllm_ln_gemm_bf16, [p(gamma), p(beta)])
+        assert f(p(x[m0:]), i(K), ctypes.c_void_p(0), *norm, ctypes.c_float(1e-5), p(w), i(K), p(bias), p(out[m0:]), i(N), i(m1 - m0), i(N), i(K), i(0),
+                 ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+
+    out, parts = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    run(0, M, out)
+    for m in range(M):
+        run(m, m + 1, parts)
+    assert torch.equal(out, parts)
+    x64 = x.double() - (0.0 if rms else x.double().mean(1, keepdim=True))
+    h = x64 / torch.sqrt((x64 * x64).mean(1, keepdim=True) + 1e-5) * gamma.double() + (0.0 if rms else beta.double())
+    want = h @ w.double().T + bias.double()
+    assert (out.double() - want).abs().max().item() <= 4e-2
+    if not rms:
+        ops.ln_linear(x, gamma, beta, 1e-5, w, bias, out, "store")
+        assert (out.double() - want).abs().max().item() <= 4e-2
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(1, 2304, 768), (8, 3072, 768), (16, 320, 96), (5, 200, 1600), (17, 96, 64),
                                    (3, 64, 4096), (16, 6400, 1600), (9, 50257, 1024), (16, 3072, 1024), (33, 2304, 768),
