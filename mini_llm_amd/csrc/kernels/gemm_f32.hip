@@ -538,6 +538,36 @@ static void launch_f32_tiles(const float* A, int lda, const float* W, int ldw, c
         gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, false><<<grid, block, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n, M > N ? 0 : 1);
 }
 
+// Which tiles: 32 x 32 with four groups, two groups of two parts or one group of two parts; 64 x 32 in two parts; 128 x 64 in one.
+enum TileShape { T32_FOUR, T32_TWO, T32_ONE, T64X32, T128X64 };
+
+// Two questions. How exactly a result is summed is a rule on its sizes alone: in four sums of eight (tiles of 32 x 32) up to
+// 64 rows, whose result is then as exact as that of the kernel for few rows, while there are at most 512 such tiles, and where
+// they were the fastest choice when tiles were loaded through registers (the price of the fullest compute unit: its tiles
+// times what they took there at K = 768, in tenths of a microsecond; with two groups a sixth of that is there at any K);
+// otherwise in two sums, or in one where that was.
+// Which tile then. Of 32 x 32: four groups where a unit has one tile and a long chain of k tiles (128 x 1,600 x 6,400: 40.8 us, two groups of
+// two parts 43.5; 560 x 768 x 768, two tiles a unit: 12.3, four groups 15.4); one group where there are many tiles of at most four k tiles, whose
+// eight wavefronts and three stages would be started for one round of loads (256 x 7,104 x 32 14.1 us with two groups, 7.9 with one, 512 x 3,328 x 100
+// 16.8 and 12.2; the eight-sums error is the same up to there, and 0.1 to 9 % larger than in four sums behind it).
+// Up to K = 48 64 x 32 and 128 x 64 make the same sums, and one of the latter costs what 3.3 of the former do
+// (2,560 x 44,096 x 24 228 us with 64 x 32, 174 with 128 x 64; 320 x 22,272 x 4 16.9 and 18.1).
+// Else of 64 x 32 in two sums, which is the fastest or within 3 % of it over 40 sizes from K = 256 on, and of 128 x 64 in one the cheaper, by prices
+// fitted to those sizes (microseconds: 2,048 x 3,072 x 768 91 and 84 us, 1,812 x 768 x 2,048 60 and 79; up to K of about 470 they say 64 x 32
+// for many tiles, which is the more exact and up to 12 % the slower: 4,096 x 4,096 x 256 90 and 80 us).
+static TileShape tile_shape(int M, int N, int K) {
+    const auto tiles = [&](int tm, int tn) { return static_cast<long>((M + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
+    const auto fullest = [&](int tm, int tn) { return ((tiles(tm, tn) + 7) / 8 + 31) / 32; };
+    const long k = K <= 96 ? K : 768, two_groups = 5 * k + 768, one_group = 6 * k, never = 1L << 60;
+    const long c11 = fullest(1, 1) * 44 * two_groups, c21 = tiles(2, 1) < 256 ? never : fullest(2, 1) * 80 * two_groups;
+    const long c22 = std::min(tiles(2, 2) < 512 ? never : fullest(2, 2) * 144 * one_group, tiles(2, 3) < 512 ? never : fullest(2, 3) * 222 * one_group);
+    if (M <= 64 || tiles(1, 1) <= 512) return tiles(1, 1) <= 256 && K >= 1536 ? T32_FOUR : T32_TWO;
+    if (c11 < c21 && c11 < c22) return K <= 128 ? T32_ONE : T32_TWO;
+    if (K <= 48) return 33 * fullest(4, 2) <= 10 * fullest(2, 1) ? T128X64 : T64X32;
+    const float small = 4.96f + fullest(2, 1) * (K * 0.00973f - 0.43f), large = 3.49f + fullest(4, 2) * (K * 0.03264f + 1.26f);
+    return c22 <= c21 && large < small ? T128X64 : T64X32;
+}
+
 // bfloat16 operands of any K, strides and alignment (what the matrix-core kernels of gemm_bf16.hip refuse:
 // they read 16 bytes at a time): one wavefront per output column and 8 rows, the lanes over k, sums in fp32.
 __global__ void __launch_bounds__(256)
@@ -574,6 +604,9 @@ int mllm_gemm_bf16_plain(const void* A, int lda, const void* W, int ldw, const f
     return 0;
 }
 
+// The tiles of a 32-bit product that runs on tiles (TileShape; for tests).
+int mllm_gemm_f32_tile_shape(int M, int N, int K) { return tile_shape(M, N, K); }
+
 int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc,
                   int M, int N, int K, int mode, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;
@@ -603,27 +636,12 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
     // vector FMAs, 2,048 x 50,257 x 64 346 / 239; 192 x 32,000 x 128 31.4 / 29.9 (at 192 columns 35.6 / 40.4), 192 x 16,384 x 64 13.8 / 13.4.
     const bool odd_wide = M > 64 && ldc % 4 != 0 && N >= 16384 && K <= (N >= 32000 ? 128 : N >= 20000 ? 96 : 64);
     if (quads && K > 0 && !odd_wide) {
-        // Two questions. How exactly a result is summed is a rule on its sizes alone: in four sums of eight (tiles of 32 x 32) up to
-        // 64 rows, whose result is then as exact as that of the kernel for few rows, while there are at most 512 such tiles, and where
-        // they were the fastest choice when tiles were loaded through registers (the price of the fullest compute unit: its tiles
-        // times what they took there at K = 768, in tenths of a microsecond; with two groups a sixth of that is there at any K);
-        // otherwise in two sums, or in one where that was.
-        const auto tiles = [&](int tm, int tn) { return static_cast<long>((M + 32 * tm - 1) / (32 * tm)) * ((N + 32 * tn - 1) / (32 * tn)); };
-        const auto fullest = [&](int tm, int tn) { return ((tiles(tm, tn) + 7) / 8 + 31) / 32; };
-        const long k = K <= 96 ? K : 768, two_groups = 5 * k + 768, one_group = 6 * k, never = 1L << 60;
-        const long c11 = fullest(1, 1) * 44 * two_groups, c21 = tiles(2, 1) < 256 ? never : fullest(2, 1) * 80 * two_groups;
-        const long c22 = std::min(tiles(2, 2) < 512 ? never : fullest(2, 2) * 144 * one_group, tiles(2, 3) < 512 ? never : fullest(2, 3) * 222 * one_group);
-        // Which tile then: four groups where a unit has one tile and a long chain of k tiles (128 x 1,600 x 6,400: 40.8 us, two groups of
-        // two parts 43.5; 560 x 768 x 768, two tiles a unit: 12.3, four groups 15.4); and of 64 x 32 in two sums, which is the fastest or within 3 %
-        // of it over 40 sizes, and of 128 x 64 in one the cheaper, by prices fitted to those sizes (microseconds: 2,048 x 3,072 x 768 91 and 84
-        // us, 1,812 x 768 x 2,048 60 and 79).
-        if (M <= 64 || tiles(1, 1) <= 512 || (c11 < c21 && c11 < c22)) {
-            if (tiles(1, 1) <= 256 && K >= 1536) launch_f32_tiles<2, 2, 1, 1, 4, 1, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
-            else launch_f32_tiles<2, 2, 1, 1, 2, 2, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
-        } else {
-            const float small = 4.96f + fullest(2, 1) * (K * 0.00973f - 0.43f), large = 3.49f + fullest(4, 2) * (K * 0.03264f + 1.26f);
-            if (c22 <= c21 && large < small) launch_f32_tiles<4, 2, 2, 2, 1, 1, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
-            else launch_f32_tiles<2, 2, 2, 1, 1, 2, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
+        switch (tile_shape(M, N, K)) {
+            case T32_FOUR: launch_f32_tiles<2, 2, 1, 1, 4, 1, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream); break;
+            case T32_TWO: launch_f32_tiles<2, 2, 1, 1, 2, 2, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream); break;
+            case T32_ONE: launch_f32_tiles<2, 2, 1, 1, 1, 2, 3, 4>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream); break;
+            case T64X32: launch_f32_tiles<2, 2, 2, 1, 1, 2, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream); break;
+            case T128X64: launch_f32_tiles<4, 2, 2, 2, 1, 1, 3, 1>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream); break;
         }
         MLLM_LAUNCH_CHECK();
         return 0;

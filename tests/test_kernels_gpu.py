@@ -659,6 +659,36 @@ def test_linear_fp32_tiles_of_few_k_tiles(ops, M, N, K0, K):
     assert (out[:, N:] == 7).all()
 
 
+TILES32 = ("32 x 32, four groups", "32 x 32, two groups", "32 x 32, one group", "64 x 32", "128 x 64")      # TileShape of gemm_f32.hip
+
+
+def _tiles32(M, N, K):
+    from mini_llm_amd import build
+    return TILES32[build.load_library("gemm_f32").mllm_gemm_f32_tile_shape(M, N, K)]
+
+
+@pytest.mark.parametrize("M,N,K,tiles,few,few_tiles", [
+    *[(600, 1100, k, "32 x 32, one group", 64, "32 x 32, two groups") for k in (4, 32, 36, 60, 64)],
+    *[(600, 1100, k, "32 x 32, one group", 0, "") for k in (68, 96, 100, 128)], (600, 1100, 132, "32 x 32, two groups", 0, ""),
+    *[(2049, 1540, k, "128 x 64", 1500, "64 x 32") for k in (4, 28, 32, 36, 48)], (2049, 1540, 52, "64 x 32", 1500, "64 x 32")])
+def test_linear_fp32_tiles_of_short_sums(ops, M, N, K, tiles, few, few_tiles):
+    """Short sums on the tiles that are the shorter way there: the same bits as on the others where the sums are the same (`few` of the rows
+    run on other tiles), and at most one rounding of 2^-24 a term of the terms' absolute sum everywhere."""
+    assert _tiles32(M, N, K) == tiles
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w, bias = _rand((M, K), torch.float32, g).to(DEV), _rand((N, K), torch.float32, g).to(DEV), _rand((N,), torch.float32, g).to(DEV)
+    out = torch.full((M, N + 4), 7.0, device=DEV)
+    ops.linear(a, w, bias, out[:, :N], "store")
+    assert (out[:, N:] == 7).all()
+    want, size = a.double() @ w.double().T + bias.double(), a.double().abs() @ w.double().abs().T + bias.double().abs()
+    assert ((out[:, :N].double() - want).abs() <= 2.0 ** -24 * (K + 2) * size).all()
+    if few:
+        assert _tiles32(few, N, K) == few_tiles
+        part = torch.empty(few, N, device=DEV)
+        ops.linear(a[:few], w, bias, part, "store")
+        assert torch.equal(part, out[:few, :N])
+
+
 @pytest.mark.parametrize("K", [768, 1600, 3072])
 def test_linear_fp32_is_as_exact_on_tiles_as_for_few_rows(ops, K):
     """64 rows run on tiles, 16 at a time on the kernel for few rows: the former's error against 64 bits is no larger."""
