@@ -311,8 +311,8 @@ paged_attention_tiled(const T* __restrict__ q, int q_stride, int q_col, const T*
 // and there are four wavefronts a SIMD to fill the gaps. Keys and values stand row-major, 16-byte piece p of row r in place p ^ (r % 16):
 // the keys' 16-byte reads (16 rows, one piece) and the values' 4-byte reads (four rows, 16 columns) are free of bank conflicts.
 // Bound by the chain of a workgroup's key tiles where workgroups are few (2.5 us a tile, of which the matrix instructions are 1.7), by the
-// matrix cores for long prompts. 12 heads of 64, with the kernel above before: 8 x 256 tokens 30.7 > 20.7 us, 331 + 512 + 470 + 400
-// 43.6 > 30, 2 x 1,024 91 > 56, 8,000 988 > 892 (110 TFLOP/s of 155); 8 heads of 128, 4 x 512 76 > 45.
+// matrix cores for long prompts. 12 heads of 64, with the kernel above before: 8 x 256 tokens 30.7 > 22.7 us, 331 + 512 + 470 + 400
+// 43.6 > 31, 2 x 1,024 91 > 60, 8,000 988 > 949 (104 TFLOP/s of 155); 8 heads of 128, 4 x 512 76 > 47.
 // A place outside [k_lo, p_last] (not written yet, or given back by a window) loads the next key that is inside; its weight is 0, its values are taken as 0.
 #define TD_TABLE 4096      // entries of a block table that fit LDS beside two stages of tiles, two workgroups a unit
 
@@ -444,15 +444,16 @@ paged_attention_tiled_f32(const float* __restrict__ q, int q_stride, int q_col, 
         }
         float mx = fmaxf(fmaxf(fmaxf(s[0][0], s[0][1]), fmaxf(s[0][2], s[0][3])), fmaxf(fmaxf(s[1][0], s[1][1]), fmaxf(s[1][2], s[1][3])));
         const float m_new = fmaxf(m, rows_max(mx));
-        // (a query none of whose scores so far is above -inf: all weights are zero against any finite number. Weights below the
-        // normal range are lost beside the maximum's 1, so the bare instruction does.)
-        const float against = m_new == -INFINITY ? 0.f : m_new, alpha = fast_exp2(m - against);
+        // (A query none of whose scores so far is above -inf: all weights are zero against any finite number. Weights below the normal range
+        // count as they do everywhere in 32 bits, 2^-130 of a value of 2^127 too; the bare instruction, which loses them, takes 4 to 5 % less:
+        // 8 x 256 tokens 21.6 us for 22.7, 8,000 901 for 949.)
+        const float against = m_new == -INFINITY ? 0.f : m_new, alpha = exp2_for<float>(m - against);
         float sum = 0.f;
 #pragma unroll
         for (int g = 0; g < 2; ++g)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                s[g][i] = fast_exp2(s[g][i] - against);
+                s[g][i] = exp2_for<float>(s[g][i] - against);
                 sum += s[g][i];
             }
         l = l * alpha + rows_sum(sum);
@@ -480,7 +481,7 @@ paged_attention_tiled_f32(const float* __restrict__ q, int q_stride, int q_col, 
     {
         const float2 other = *reinterpret_cast<const float2*>(states + DC * STATE_STEP - (group * 64 + lane) * 2);
         const float m_new = fmaxf(m, other.x), against = m_new == -INFINITY ? 0.f : m_new;     // (all its scores -inf: nothing but a sink counts)
-        const float a = fast_exp2(m - against), a2 = fast_exp2(other.x - against);
+        const float a = exp2_for<float>(m - against), a2 = exp2_for<float>(other.x - against);
         l = l * a + other.y * a2;
         m = m_new;
 #pragma unroll

@@ -1076,6 +1076,23 @@ def test_paged_attention_of_scores_at_the_lowest_end(ops, H, Hkv, dh, window):
 
 
 @pytest.mark.parametrize("H,Hkv,dh", [(3, 3, 32), (3, 1, 64), (2, 2, 128)])
+def test_paged_attention_keeps_weights_below_the_normal_range(ops, H, Hkv, dh):
+    """32-bit portions: a weight of 2^-130 against a value of 2^127, in either half of a key tile and in an earlier one than the highest score's.
+    The score of 130 has a rounding of some units of 2^-24 of itself, which the weight shows ln 2 times."""
+    g = torch.Generator().manual_seed(dh)
+    seqs, high = [(0, 130)] * 3, [1, 40, 70]
+
+    def far(b, q, k, v):
+        q[:], k[:], v[:] = 0.0, 0.0, 0.0
+        q[..., 0], k[high[b], :, 0], v[0] = 1.0, 130 * math.log(2) * math.sqrt(dh), 2.0 ** 127
+
+    out, ref = _attention_case(ops, torch.float32, H, Hkv, dh, 16, seqs, 0, g, q_col=0, edit=far)
+    for b, first in enumerate(high):
+        assert (ref[130 * b + first:130 * (b + 1)] - 0.125).abs().max() <= 1e-3
+    assert ((out - ref).abs() <= 130 * 8 * 2.0 ** -24 * ref.abs()).all()
+
+
+@pytest.mark.parametrize("H,Hkv,dh", [(3, 3, 32), (3, 1, 64), (2, 2, 128)])
 @pytest.mark.parametrize("window,keep", [(0, 0), (8, 0), (8, 3), (40, 70)])
 def test_paged_attention_of_infinite_values_beside_empty_places(ops, H, Hkv, dh, window, keep):
     """32-bit portions of one query (in a step with a longer one): an infinite value at the first and at the last key that it sees gives
