@@ -1048,10 +1048,11 @@ int mllm_conv_silu(const float* proj, int ld, int col0, int C, const float* w, c
     if (vec) {
         const long long total4 = total / 4;
         const int blocks4 = static_cast<int>((total4 + 255) / 256);
-        // (fewer threads than that have nothing to hide their longer way behind: 1,032 x 1,792 8.3 us either way, 2,048 x 768 6.4, four
-        // rows a thread 7.1)
+        // (Fewer threads than that have nothing to hide their longer way behind, the more of them the fewer times a row is read. Four taps: 1,032 x 1,792
+        // 8.3 us either way, 2,048 x 768 6.4, four rows a thread 7.1; three: 3,200 x 768 in portions of 65 10.7 and 11.1, 1,600 x 1,792 12.8 > 12.0; two:
+        // 1,200 x 1,792 8.8 and 9.4, 2,400 14.1 > 12.6.)
         constexpr int ROWS = 4;
-        if (!single && total4 >= 1 << 19 && taps >= 2 && taps <= 4) {
+        if (!single && total4 * taps >= 1 << 21 && taps >= 2 && taps <= 4) {
             const int blocks = static_cast<int>(((T + ROWS - 1) / ROWS * static_cast<long long>(C / 4) + 255) / 256);
 #define CSR(TAPS) case TAPS: conv_silu_rows_kernel<TAPS, ROWS><<<blocks, 256, 0, stream>>>(proj + col0, ld, C, w, bias, token_seq, cu_q, state_slots, state, \
                                                                                           slot_floats, out, ldo, T); break

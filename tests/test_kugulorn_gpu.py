@@ -505,9 +505,9 @@ def test_scan_finds_chunks_among_many_portions(sizes, vdim, state):
 
 
 @pytest.mark.parametrize("taps", [2, 3, 4])
-@pytest.mark.parametrize("lens", [[1300], [1, 700, 2, 3, 597, 1], [1029, 250]])
+@pytest.mark.parametrize("lens", [[1300], [1, 700, 2, 3, 597, 1], [1029, 250], [2400], [1, 1400, 2, 3, 1033, 1]])
 def test_convolution_of_many_tokens(taps, lens):
-    """From 2^21 inputs on a thread has four tokens: portions that begin and end within the four, and are shorter than they, have the bits that
+    """From 2^23 inputs times taps on a thread has four tokens: portions that begin and end within the four, and are shorter than they, have the bits that
     every portion has alone, the carried rows in front of it and behind it too."""
     import ctypes
     import torch
