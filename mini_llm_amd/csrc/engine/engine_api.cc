@@ -60,7 +60,7 @@ unsigned long long mllm_scratch_bytes(void) {
 }
 int mllm_release_scratch(hipStream_t stream) { return guarded([&] { release_scratch(stream); }); }
 // name: "decode_shape" (nsplit, waves; 0, 0 = automatic), "unmerged_shape", "merge_max_rows" (a), "ln_fuse_max_rows" (a), "long_context_splits" (a: 0 off, 1 on),
-// "latent_tiles", "scored_shared_kernels" (a: 0 off, 1 on), "halves_max_width" (a), "through_products" (a: 0 off, 1 on), "grouped_experts_rows" (a)
+// "latent_tiles", "scored_shared_kernels" (a: 0 off, 1 on), "halves_max_width" (a), "through_products", "joined_norms" (a: 0 off, 1 on), "grouped_experts_rows" (a)
 int mllm_set_tuning(const char* name, int a, int b) {
     return guarded([&] {
         Tuning& t = tuning();
@@ -74,6 +74,7 @@ int mllm_set_tuning(const char* name, int a, int b) {
         else if (n == "scored_shared_kernels") t.scored_shared_kernels = a;
         else if (n == "halves_max_width") t.halves_max_width = a;
         else if (n == "through_products") t.through_products = a;
+        else if (n == "joined_norms") t.joined_norms = a;
         else if (n == "grouped_experts_rows") t.grouped_experts_rows = a;
         else if (n == "reset_seen") t.seen = Tuning::Seen();
         else fail("unknown tuning value '%s'", name);
@@ -83,7 +84,7 @@ int mllm_set_tuning(const char* name, int a, int b) {
 // were split over), "merge_kernel_launches", "prefill_tile_launches" (the bfloat16 matrix-core kernel), "tiled_f32_launches" (the 32-bit one),
 // "generic_attention_launches", "latent_tile_launches" and "latent_token_launches" (latent attention on the matrix cores / one
 // workgroup per token), "through_products" (products that took their result into the stream themselves), "grouped_experts"
-// (feed-forwards of routed experts run as grouped products). -1: unknown name.
+// (feed-forwards of routed experts run as grouped products), "joined_norms" (blocks whose first norm the block in front left). -1: unknown name.
 long long mllm_get_seen(const char* name) {
     const Tuning::Seen& s = tuning().seen;
     const std::string n(name);
@@ -96,6 +97,7 @@ long long mllm_get_seen(const char* name) {
     if (n == "latent_token_launches") return s.latent_token_launches;
     if (n == "through_products") return s.through_products;
     if (n == "grouped_experts") return s.grouped_experts;
+    if (n == "joined_norms") return s.joined_norms;
     return -1;
 }
 

@@ -121,6 +121,7 @@ struct Tuning {
     int scored_shared_kernels = 1;                    // 1: attention with shaped scores may run on the kernels the plain attention runs on
     int grouped_experts_rows = 192;                   // tokens from which routed experts of which at most half are chosen run as grouped products (0: never)
     int through_products = 1;                         // 1: a product may take its result into the stream through norms itself
+    int joined_norms = 1;                             // 1: the norm at the end of a block may leave the first norm of the block behind (many rows)
     int halves_max_width = 1024;                      // stream widths up to which a block whose sub-layers read one stream runs the
                                                       // feed-forward's first products, with the norm inside, in front of the mixer
                                                       // (wider: every workgroup of a wide product redoing the norm costs more than the
@@ -131,6 +132,7 @@ struct Tuning {
         long long merge_kernel_launches = 0, prefill_tile_launches = 0, tiled_f32_launches = 0, generic_attention_launches = 0;
         long long latent_tile_launches = 0, latent_token_launches = 0;      // latent attention: matrix-core kernel, one workgroup per token
         long long through_products = 0, grouped_experts = 0;                // products that took their result into the stream; routed experts as grouped products
+        long long joined_norms = 0;                                         // blocks whose first norm the block in front left
     } seen;
 };
 Tuning& tuning();

@@ -701,7 +701,7 @@ void DecoderModel::forward(const StepView& step, const std::vector<CacheView>& c
     // less, 5.7 + 5.2 > 6.1 us a layer. (Few rows: a block's first product takes its norm inside, which costs no launch.)
     Tensor2 first_normed;
     for (const auto& l : layers) {
-        if (l->first_norm() == nullptr || step.n_tokens <= tuning().ln_fuse_max_rows) continue;
+        if (l->first_norm() == nullptr || step.n_tokens <= tuning().ln_fuse_max_rows || !tuning().joined_norms) continue;
         first_normed = arena.tensor(BF16, step.n_tokens, hidden_size());
         break;
     }

@@ -206,6 +206,7 @@ private:
         const StepView::NextNorm& next = step.next_norm;
         if (next.norm == nullptr || !last.add_scaled_then(y, scale, mult_, x, clear, *next.norm, next.into, s)) return false;
         *next.left = true;
+        tuning().seen.joined_norms += 1;
         return true;
     }
     Tensor2 checked_scale(const Tensor2& t) {

@@ -172,7 +172,8 @@ def scratch_bytes() -> int:
 
 def seen(name: str) -> int:
     """What the ops chose since ``reset_seen()``: "max_decode_splits", "merge_kernel_launches",
-    "prefill_tile_launches", "generic_attention_launches", "latent_tile_launches", "latent_token_launches"."""
+    "prefill_tile_launches", "tiled_f32_launches", "generic_attention_launches", "latent_tile_launches", "latent_token_launches",
+    "through_products", "grouped_experts", "joined_norms"."""
     v = engine_library().mllm_get_seen(name.encode())
     if v < 0:
         raise KernelError(f"unknown counter '{name}'")
@@ -197,6 +198,11 @@ def set_scored_shared_kernels(on: bool) -> None:
 def set_through_products(on: bool) -> None:
     """Whether a product may take its result into the stream through norms by itself (otherwise it passes through memory)."""
     _ok(engine_library().mllm_set_tuning(b"through_products", 1 if on else 0, 0))
+
+
+def set_joined_norms(on: bool) -> None:
+    """Whether the norm at the end of a block may leave the first norm of the block behind, for many rows (default: on)."""
+    _ok(engine_library().mllm_set_tuning(b"joined_norms", 1 if on else 0, 0))
 
 
 def set_grouped_experts_rows(rows: int) -> None:

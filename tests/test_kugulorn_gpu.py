@@ -99,6 +99,28 @@ def test_norms_of_neighbouring_layers_join_from_33_rows(dirs, name, page):
         assert runner.check() == "" and runner.info()["n_requests"] == 0
 
 
+@pytest.mark.parametrize("name,page", [("TILED", 16), ("ODD", 4)])
+def test_norms_of_neighbouring_layers_join_with_the_same_bits(dirs, name, page):
+    """The norm is left by the layer in front in steps of 33 and more rows and in no others, for every layer but the first, and the logits are those
+    of the two norms on their own."""
+    from mini_llm_amd.kernels import ops
+    cfg, d = getattr(kc, name), dirs(name)
+    got = []
+    try:
+        for on in (True, False):
+            ops.set_joined_norms(on)
+            runner = _runner(d, "bfloat16", n_pages=-(-65 // page), page=page)
+            got.append([])
+            for n in (31, 32, 33, 65):
+                ops.reset_seen()
+                steps = ru.trace_whole(kc.requests(cfg["vocab"], [n], seed=n))
+                got[-1].append(ru.run_in_process(runner, steps)[0])
+                assert ops.seen("joined_norms") == (len(cfg["layers"]) - 1 if on and n > 32 else 0)
+    finally:
+        ops.set_joined_norms(True)
+    assert all(np.isfinite(a).all() and np.array_equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("family", ["whole", "mixed"])
 def test_widest_rows_on_the_matrix_cores(dirs, family):
     from mini_llm_amd.kernels import ops
