@@ -611,17 +611,20 @@ def test_linear_fp32_few_rows(ops, M, N, K, pad):
         assert (out.cpu().double() - ref).abs().max().item() <= 3e-5
 
 
-@pytest.mark.parametrize("M,N,K,pad", [(17, 40, 4, 0), (33, 97, 100, 4), (64, 193, 772, 0),     # 32 x 32 tiles, four groups
-                                       (9, 16400, 36, 0),                                       # few rows of a wide head
-                                       (800, 700, 132, 8),                                      # 32 x 32, two groups
-                                       (1025, 800, 260, 0),                                     # 64 x 32, two groups
-                                       (2049, 2308, 20, 4), (1900, 1500, 292, 0)])              # 64 x 96 and 64 x 64
+@pytest.mark.parametrize("M,N,K,pad,tiles", [(17, 40, 4, 0, "32 x 32, two groups"), (33, 97, 100, 4, "32 x 32, two groups"), (64, 193, 772, 0, "32 x 32, two groups"),
+                                             (64, 193, 1540, 4, "32 x 32, four groups"),
+                                             (9, 16400, 36, 0, "32 x 32, two groups"),            # few rows of a wide head
+                                             (800, 700, 132, 8, "32 x 32, two groups"), (800, 700, 100, 8, "32 x 32, one group"),
+                                             (1025, 800, 260, 0, "64 x 32"), (1900, 1500, 292, 0, "64 x 32"),
+                                             (2049, 2308, 20, 4, "128 x 64"), (1812, 2050, 772, 4, "128 x 64"), (1813, 2050, 780, 0, "128 x 64"),
+                                             (1801, 3073, 804, 0, "128 x 64"), (2048, 3072, 768, 0, "128 x 64")])
 @pytest.mark.parametrize("epi", ["store", "gelu_tanh", "add_residual"])
-def test_linear_fp32_tiles(ops, M, N, K, pad, epi):
+def test_linear_fp32_tiles(ops, M, N, K, pad, tiles, epi):
     """Every tile shape of the 32-bit product at its edges (rows, columns and K that fill no tile, strides wider than the rows):
     an output's products pass through at most 16 roundings, one for each further 16 columns, and a few to join groups, bias and
     residual, so its error is at most that many units of 2^-24 of the sum of their magnitudes (GELU: at most 1.13 times as
     steep, and 8 units of its own result). A row of infinities leaves the others as they are."""
+    assert _tiles32(M, N, K) == tiles
     g = torch.Generator().manual_seed(M + K)
     a, w, b = _rand((M, K + pad), torch.float32, g), _rand((N, K + pad), torch.float32, g, 0.1), _rand((N,), torch.float32, g)
     a[M // 2] = float("inf")
@@ -645,8 +648,8 @@ def test_linear_fp32_tiles(ops, M, N, K, pad, epi):
 @pytest.mark.parametrize("M,N,K0", [(33, 70, 0), (130, 96, 1536), (600, 1100, 0), (1812, 772, 0), (2049, 1540, 0)])
 @pytest.mark.parametrize("K", [4, 32, 36, 64, 100, 128, 132, 160, 192, 228])
 def test_linear_fp32_tiles_of_few_k_tiles(ops, M, N, K0, K):
-    """Every tile shape (32 x 32 with two and four groups, 64 x 32, 128 x 64) where the k tiles are fewer than the stages of LDS, odd and
-    even in number, with a last one that is full or not: the error is at most one rounding of 2^-24 a term of the terms'
+    """Every tile shape with few k tiles, odd and even in number, with a last one that is full or not; all but 32 x 32 with four groups (which has
+    at least twelve) also with fewer of them than stages of LDS. The error is at most one rounding of 2^-24 a term of the terms'
     absolute sum, and rows that lie apart are met."""
     K += K0
     g = torch.Generator().manual_seed(M + N + K)
@@ -1039,11 +1042,52 @@ def test_paged_attention_tiles_in_true_32_bit(ops, dtype, H, Hkv, dh, page, wind
                                   [(0, 1 + i % 67) for i in range(65)]])                 # more of them
 @pytest.mark.parametrize("H,Hkv,dh", [(3, 1, 64), (2, 2, 128)])
 def test_paged_attention_gives_every_tile_away(ops, dtype, seqs, H, Hkv, dh):
-    """The order in which workgroups take the query tiles of several sequences, by how many keys they see: every row is written, once."""
+    """The order in which workgroups take the query tiles of several sequences, by how many keys they see: every row is written."""
     g = torch.Generator().manual_seed(len(seqs) + dh)
     out, ref = _attention_case(ops, dtype, H, Hkv, dh, 16, seqs, 0, g)
     assert torch.isfinite(out).all()
     assert (out - ref).abs().max() <= _tol(dtype, 2)
+
+
+@pytest.mark.parametrize("seqs", [[(0, 1)], [(5000, 70), (0, 300)], [(0, 300), (5000, 70)], [(4200, 130), (0, 1), (64, 64), (63, 65), (10, 129)],
+                                  [(0, 512)] * 4, [(i % 3 * 64, 1 + 37 * i % 140) for i in range(64)], [(i * 977 % 90000, i % 5 * 33) for i in range(64)],
+                                  [(0, 1 + i % 67) for i in range(65)]])
+@pytest.mark.parametrize("rows", [1, 5, 12])
+def test_every_query_tile_is_given_to_one_workgroup(seqs, rows):
+    """Each order gives every tile of 64 rows (a query has `rows`) to exactly one of the workgroups, the rest get none, and the order by length
+    begins with the pairs of tiles that see most."""
+    import ctypes
+    import toy  # noqa: F401  (registers the test-only library)
+    from mini_llm_amd import build
+    lib = build.load_library("lane_check")
+    cu = [sum(n for _, n in seqs[:b]) for b in range(len(seqs) + 1)]
+    want = {(b, t, cu[b], n) for b, (_, n) in enumerate(seqs) for t in range(-(-n * rows // 64))}
+    places = cu[-1] * rows // 64 + len(seqs)
+    on_dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (cu, [s + n for s, n in seqs])]
+    for order in (0, 1, 2) if len(seqs) <= 64 else (0, 1):
+        out = torch.full((places, 4), 77, dtype=torch.int32, device=DEV)
+        assert lib.mllm_query_tiles(*(ctypes.c_void_p(a.data_ptr()) for a in on_dev), len(seqs), rows, order, places, ctypes.c_void_p(out.data_ptr()),
+                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        got = [tuple(t) for t in out.cpu().tolist()]
+        given = [t for t in got if t[0] >= 0]
+        assert len(given) == len(want) and set(given) == want and all(t[0] == -1 for t in got if t not in want)
+        if order == 2:
+            sees = [(seqs[b][0] * rows // 64 + t) // 2 for b, t, _, _ in given]
+            assert sees == sorted(sees, reverse=True) and got[:len(given)] == given
+
+
+@pytest.mark.parametrize("H,Hkv,dh", [(2, 1, 64), (1, 1, 128)])
+@pytest.mark.parametrize("ctx", [4095, 4096, 4097])
+@pytest.mark.parametrize("shaped", [False, True])
+def test_paged_attention_of_the_longest_block_tables(ops, H, Hkv, dh, ctx, shaped):
+    """32-bit portions with pages of one token: a table of 4,096 entries is the longest that lies in LDS beside the tiles, one more runs on the
+    kernel that reads it from memory."""
+    g = torch.Generator().manual_seed(ctx + dh)
+    shape = {"sink": torch.randn(H, generator=g)} if shaped else None
+    ops.reset_seen()
+    out, ref = _attention_case(ops, torch.float32, H, Hkv, dh, 1, [(ctx - 70, 70), (0, 3), (ctx - 64, 64)], 0, g, q_col=0 if shaped else 8, shape=shape)
+    assert ops.seen("tiled_f32_launches") == 1
+    assert torch.isfinite(out).all() and (out - ref).abs().max() <= _tol(torch.float32, 2)
 
 
 @pytest.mark.parametrize("H,Hkv,dh", [(3, 3, 32), (3, 1, 64), (2, 2, 128)])

@@ -4,7 +4,7 @@ here if missing or stale; the build entry point compiles it beforehand):
 * the toy plugin (tests/native/toy_plugin.hip): toy parts and architectures that are registered with the
   engine from outside the package. ``plugin_path()`` is the built library, ``load()`` hands it to the
   engine of this process;
-* a kernel that exposes the lane exchanges of the kernels' common header (tests/native/lane_check.hip)."""
+* kernels that expose the lane exchanges of the kernels' common header and the orders of query tiles (tests/native/lane_check.hip)."""
 import os
 
 from mini_llm_amd import build
@@ -21,7 +21,7 @@ build.register_library("toy_plugin", {
 build.register_library("lane_check", {
     "kind": "hip",
     "sources": [os.path.join(HERE, "native", "lane_check.hip")],
-    "headers": [os.path.join(build.CSRC, "kernels", "common.h")],
+    "headers": [os.path.join(build.CSRC, "kernels", "common.h"), os.path.join(build.CSRC, "kernels", "query_tiles.h")],
     "out_dir": os.path.join(HERE, "native", "_lib"),
 })
 NATIVE = ("toy_plugin", "lane_check")
