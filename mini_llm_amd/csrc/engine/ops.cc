@@ -370,13 +370,15 @@ void linear_from_splits(const AttentionSplits& a, const Tensor2& w, const float*
     linear(merged, w, bias, out, epilogue, nullptr, stream);
 }
 
-// Where the norm inside the few-row product is worth it: not where that product wants two tiles of columns a workgroup and their LDS does
-// not fit (K over 2,016), so that it runs with one. Norm and product then are shorter (us, inside > apart): 17 rows 2,304 x 2,048 15.0 > 11.1, 32 rows
-// 4,096 x 2,048 16.4 > 12.8, 8 rows 6,144 x 2,048 13.4 > 11.4, 16 rows 8,192 x 2,024 18.4 > 16.0; at K = 2,016 8 rows 6,144 10.8 < 12.3, 32
-// rows 4,096 12.1 < 13.6.
+// Where the norm inside the few-row product is worth it. Up to 16 rows: not where that product wants two tiles of columns a workgroup and
+// their LDS does not fit (K over 2,016), so that it runs with one. Norm and product then are shorter (us, inside > apart): 8 rows 6,144 x 2,048
+// 13.4 > 11.4, 16 rows 8,192 x 2,024 18.4 > 16.0; at K = 2,016 8 rows 6,144 10.8 < 12.3.
+// 17 to 32 rows: inside, so that a row has the bits that it has alone, whoever shares its launch. Up to 4,096 columns that is the shorter way too up
+// to K = 2,016 (17 and 32 rows, 4,096 x 1,600 9.7 and 10.0 us, apart 10.8 and 11.7; K = 1,024 3 % longer); at K = 2,048 it costs 3.5 to 4 us (4,096 columns,
+// 32 rows: 16.4, apart 12.8), and above 4,096 columns, where the workgroups take two rounds, 4,352 x 1,024 16.3 and 17.3, apart 9.0 and 9.8, 5,120 x
+// 1,280 15.2 and 15.9, apart 12.4 and 13.5; 6,400 x 1,600 17.3 and 18.0, apart 16.5 and 18.3.
 bool norm_inside_pays(int64_t rows, int64_t columns, int64_t k) {
-    const bool wants_two = rows <= 16 ? columns > 4096 && columns <= 8192 : rows <= 32 && columns > 2048;
-    return k <= 2016 || !wants_two;
+    return k <= 2016 || rows > 16 || columns <= 4096 || columns > 8192;
 }
 
 void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float eps, const Tensor2& w,
@@ -389,8 +391,9 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
     // (More rows than that: the norm is a kernel of its own. Normalising in the tiled product while it stages
     // its rows was measured at 64 to 256 rows and lost: every workgroup of a row tile has to pull the tile's
     // fp32 rows through its own L1 for the statistics, 6.5 us at 64 rows of 768, more than the norm's kernel.)
-    // (Keys and values: 17 to 32 rows of more than 256 column tiles run in more than two rounds of workgroups, each normalising its rows
-    // again, and the norm and a product that writes the pages itself are shorter: a step of 17 tokens of GPT-2 XL takes 945 us so, 1,033 fused.)
+    // (Keys and values: 17 to 32 rows of more than 256 column tiles run in two rounds of workgroups, each normalising its rows again, and
+    // the norm and a product that writes the pages itself are shorter: 17 and 32 rows 4,224 x 1,408 16.4 and 17.2 us inside, 12.9 and 14.0 apart, 4,800 x
+    // 1,600 17.3 and 18.0, 13.8 and 15.2, 6,048 x 2,016 21.7 and 22.2, 16.5 and 18.7; 3,840 x 1,280 8.7 and 9.0, 10.0 and 10.9.)
     const bool kv_fits = kv == nullptr || (aligned(w.data, 16) && (M <= 16 || w.rows <= 4096));
     if (w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
         (beta == nullptr || aligned(beta, 16)) && kv_fits && (tmp == nullptr || norm_inside_pays(M, w.rows, K))) {

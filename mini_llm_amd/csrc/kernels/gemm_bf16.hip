@@ -1231,7 +1231,8 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     // The same behind the fused norm with 17 to 32 rows, 128 workgroups a row block: every workgroup normalises its 16 rows again, and more
     // than 256 of them share compute units. One and two tiles a workgroup, 32 rows, us: 2,304 x 768 7.4 > 6.6, 3,072 x 1,024 10.9 > 7.3,
     // 4,096 x 1,024 11.3 > 7.6, 3,600 x 1,600 14.7 > 9.2; two rounds of them pay only for a long K: 6,400 x 1,600 27.4 > 16.5, 5,120 x
-    // 1,280 17.5 > 14.7, but 4,112 x 768 10.0 / 11.7, 10,000 x 768 15.4 / 17.2.
+    // 1,280 17.5 > 14.7, but 4,112 x 768 10.0 / 11.7, 10,000 x 768 15.4 / 17.2. (Norm and product apart: see norm_inside_pays of
+    // the engine's ops.)
     const bool dealt_out_2 = gated == nullptr && split_k && LN_FUSED && row_blocks == 2 && tiles > 128 && (tiles <= 256 || K > 1024) && two_fit;
     const bool two_tiles = dealt_out || dealt_out_2 || gated != nullptr;      // (a gated pair: a tile of either map)
     if (dealt_out) cols_per_wg = (N + 255) / 256;

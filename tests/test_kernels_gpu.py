@@ -545,6 +545,21 @@ def test_norm_and_product_in_one_kernel_up_to_2048_columns(ops, M, N, K, rms):
         assert (out.double() - want).abs().max().item() <= 4e-2
 
 
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("N,K", [(2064, 2024), (2304, 2048), (4096, 2048), (8208, 2024)])
+def test_ln_linear_of_17_to_32_wide_rows_has_the_bits_of_16(ops, M, N, K):
+    """From K = 2,024 on the norm stays inside the product for 17 to 32 rows: a row has the bits that it has among up to 16."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (_rand((M, K), torch.float32, g, std=2.0) + 0.3).to(DEV)
+    gamma, beta = (1 + 0.1 * _rand((K,), torch.float32, g)).to(DEV), (0.1 * _rand((K,), torch.float32, g)).to(DEV)
+    w, bias = _rand((N, K), torch.bfloat16, g, std=1.0 / math.sqrt(K)).to(DEV), (0.5 * _rand((N,), torch.float32, g)).to(DEV)
+    out, parts = (torch.full((M, N), 7.0, dtype=torch.bfloat16, device=DEV) for _ in range(2))
+    ops.ln_linear(x, gamma, beta, 1e-5, w, bias, out, "store")
+    for m in range(0, M, 16):
+        ops.ln_linear(x[m:m + 16], gamma, beta, 1e-5, w, bias, parts[m:m + 16], "store")
+    assert torch.equal(out, parts)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("M,N,K", [(1, 2304, 768), (8, 3072, 768), (16, 320, 96), (5, 200, 1600), (17, 96, 64),
                                    (3, 64, 4096), (16, 6400, 1600), (9, 50257, 1024), (16, 3072, 1024), (33, 2304, 768),
