@@ -410,10 +410,8 @@ int mllm_prefill_attention_bf16(const void* q, int q_stride, int q_col, const vo
             block_tables, max_blocks, cu_q, ctx_len, n_seqs, n_heads, n_kv_heads, page_size, sl2, window,   \
             (bf16_t*)out, out_stride, sh, scale, gate, ldg);                                                \
     } while (0)
-    // The longest tiles of all sequences first, from four sequences on (next_tile and longest_tile; up to three the other order is
-    // the better one, or what finding the tile costs is more than it gives: 2 x 1,024 tokens 17.2 us against 17.4, 25 heads at 2 x 900 25.4, 27.5).
-    const bool longest_first = n_seqs >= 4 && n_seqs <= MLLM_WAVE;
-#define PF_LAUNCH(D, W, S) do { if (longest_first) PF_LAUNCH_IN(D, W, S, true); else PF_LAUNCH_IN(D, W, S, false); } while (0)
+    const bool longest = longest_first(n_seqs, 4, static_cast<long long>(n_heads) * n_tiles_upper);
+#define PF_LAUNCH(D, W, S) do { if (longest) PF_LAUNCH_IN(D, W, S, true); else PF_LAUNCH_IN(D, W, S, false); } while (0)
 #define PF_CASE(D, W, KEY)                                                                                  \
     case KEY: {                                                                                             \
         if (shape && shape->sigmoid) PF_LAUNCH(D, W, 2);                                                    \

@@ -58,8 +58,19 @@ __device__ __forceinline__ QueryTile longest_tile(const int* __restrict__ cu_q, 
     return {-1, 0, 0, 0};
 }
 
-// Either, where the kernel decides: the order costs 0.2 to 0.5 us to find, which a single sequence has no use for.
+// Whether the longest come first. With as many workgroups as compute units all start at once and the order is of no use, and finding it takes
+// 0.1 to 0.5 us longer than a walk over few sequences; a walk over many is the longer way. From eight sequences on, and below from `from` on where
+// a unit gets more than one workgroup. Longest first / in turn, us: bfloat16, 12 heads of 64, 8 portions of 37 to 177 tokens 7.3 / 7.7, 5 of 37 to 203
+// 7.4 / 7.0, 25 heads 4 x 512 22.2 / 26.8, 2 x 512 16.1 / 15.7 (from four there); 32-bit, 12 heads of 64, 2 x 1,024 66 / 80, 3 x 512
+// 33.2 / 35.5, 200 + 250 16.1 / 15.9; latent, 12 heads of 256 + 32, 2 x 1,024 59 / 61, 3 x 512 31.0 / 31.9, 200 + 250 16.9 / 16.3; 8 heads of 96, which run
+// on the kernel for any head, the same within 3 % in either.
+__host__ __device__ inline bool longest_first(int n_seqs, int from, long long workgroups) {
+    return n_seqs <= MLLM_WAVE && (n_seqs >= 8 || (n_seqs >= from && workgroups > 256));
+}
+
+// Either, where the kernel decides.
 template <int TILE>
 __device__ __forceinline__ QueryTile query_tile(const int* __restrict__ cu_q, const int* __restrict__ ctx_len, int n_seqs, int rows, int place, int places) {
-    return n_seqs > 1 && n_seqs <= MLLM_WAVE ? longest_tile<TILE>(cu_q, ctx_len, n_seqs, rows, place) : next_tile<TILE>(cu_q, n_seqs, rows, place, places);
+    return longest_first(n_seqs, 2, static_cast<long long>(gridDim.x) * gridDim.y) ? longest_tile<TILE>(cu_q, ctx_len, n_seqs, rows, place)
+                                                                                   : next_tile<TILE>(cu_q, n_seqs, rows, place, places);
 }

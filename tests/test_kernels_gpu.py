@@ -1091,6 +1091,26 @@ def test_every_query_tile_is_given_to_one_workgroup(seqs, rows):
             assert sees == sorted(sees, reverse=True) and got[:len(given)] == given
 
 
+@pytest.mark.parametrize("n_seqs,places,order", [(1, 300, 1), (2, 256, 1), (2, 257, 2), (7, 256, 1), (7, 257, 2), (8, 40, 2), (64, 300, 2), (65, 300, 1)])
+def test_query_tiles_are_ordered_where_it_pays(n_seqs, places, order):
+    """The longest tiles come first (order 2) from eight sequences on, and with two to seven where there are more workgroups than compute units; otherwise,
+    and with more than 64 sequences, a sequence's tiles come one after the other (order 1)."""
+    import ctypes
+    import toy  # noqa: F401  (registers the test-only library)
+    from mini_llm_amd import build
+    lib = build.load_library("lane_check")
+    lens = [70 + 10 * (b % 7) for b in range(n_seqs)]
+    cu, ctx = [sum(lens[:b]) for b in range(n_seqs + 1)], [n + 64 * (b % 3) for b, n in enumerate(lens)]
+    on_dev = [torch.tensor(a, dtype=torch.int32, device=DEV) for a in (cu, ctx)]
+    got = []
+    for o in (0, order):
+        out = torch.full((places, 4), 77, dtype=torch.int32, device=DEV)
+        assert lib.mllm_query_tiles(*(ctypes.c_void_p(a.data_ptr()) for a in on_dev), n_seqs, 1, o, places, ctypes.c_void_p(out.data_ptr()),
+                                    ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)) == 0
+        got.append(out.cpu())
+    assert torch.equal(*got)
+
+
 @pytest.mark.parametrize("H,Hkv,dh", [(2, 1, 64), (1, 1, 128)])
 @pytest.mark.parametrize("ctx", [4095, 4096, 4097])
 @pytest.mark.parametrize("shaped", [False, True])
