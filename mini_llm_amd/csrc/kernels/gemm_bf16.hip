@@ -549,6 +549,10 @@ static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, con
 // that would load 8 elements of a row loads those elements of every split's unnormalised output and
 // the splits' maxima and sums instead, and merges them in registers. The attention kernel then
 // needs no pass that waits for its last workgroup, and more workgroups stream the keys.
+// At up to 16 rows a launch is a chain of latencies, not a stream: of the 3.6 us that the norm and a 2,304 x 768 product took from their
+// first wavefront's start, 1.3 passed before the first row was asked for (an argument loaded from memory, integer divisions). With
+// what the first loads need in the preloaded arguments and an instance for every number of a lane's columns it takes 2.4 (back to back
+// 4.3 > 3.1 us at 1 row, 4.5 > 3.3 at 8; a token of GPT-2 small alone 0.344 > 0.317 ms, of eight 0.407 > 0.377).
 // ---------------------------------------------------------------------------------------------
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 
@@ -562,22 +566,23 @@ template <int MS> struct SplitStates {
 };
 
 template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false, int MS = MERGE_MAX_SPLITS,
-          bool ONE = false, bool GATED = false>
+          bool ONE = false, bool GATED = false, int NU = 8>
 __global__ void __launch_bounds__(ASRC == A_NORMED ? 512 : (ASRC == A_GLOBAL || ASRC == A_MERGED ? 768 : 1024))
-gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: what the first loads need
-                 const bf16_t* __restrict__ W, int ldw, int N, int K, int M, int col_blocks, int row_blocks,
-                 int cols_per_wg, int k_parts, const void* __restrict__ Ain, int lda, int mode,
-                 const float* __restrict__ bias,
+gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, and hold everything that the first loads need: an argument
+                 // behind them comes with a load of its own from memory that no cache holds (as does blockDim), 0.6 to 0.8 us
+                 // before which no row and no weight could be asked for.
+                 const bf16_t* __restrict__ W,
+                 // A_MERGED: the outputs of the attention's MS splits (layout: attention_decode.hip); otherwise A
+                 const void* __restrict__ Ain,
+                 // A_NORMED: scale and shift (GATED: the second map's weights). A_MERGED: the splits' maxima and sums, bias.
+                 // Otherwise bias and C.
+                 const void* __restrict__ p2, const void* __restrict__ p3,
+                 int ldw, unsigned columns, unsigned shape, int K_or_ldc,
+                 // A_MERGED: C; otherwise A's row stride and, in the upper half, C's
+                 void* __restrict__ C_or_strides,
                  // the rest is loaded by the kernel and needed later
-                 void* __restrict__ C, int ldc, const float* __restrict__ gamma, const float* __restrict__ beta,
-                 float eps, const int* __restrict__ rows, float* __restrict__ part_sums,
-                 int* __restrict__ part_counters,
-                 // A_MERGED: the states of the attention's MS splits (layout: attention_decode.hip),
-                 // heads per token and head size (K = heads x head size)
-                 const float* __restrict__ split_o = nullptr, const float* __restrict__ split_ml = nullptr,
-                 int a_heads = 1, int a_head_dim = 8,
-                 // A_NORMED: != 0: the norm does not centre (RMS norm: x / sqrt(mean(x^2) + eps) * gamma)
-                 int rms = 0,
+                 const float* __restrict__ late_bias, void* __restrict__ late_C, const int* __restrict__ late_rows, float eps,
+                 float* __restrict__ part_sums, int* __restrict__ part_counters,
                  // THROUGH (mode EPI_THROUGH): the norms the result passes and the copy it leaves; GATED: the second map and the
                  // activation; otherwise (plain store of a split-K kernel) the pages that its key and value columns go to as well
                  typename std::conditional<THROUGH, MllmStreamAdd, typename std::conditional<GATED, GatedPair, KvScatter>::type>::type add = {}) {
@@ -590,23 +595,42 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     static_assert(!GATED || (NT == 2 && ASRC == A_NORMED), "gated pairs: two tiles behind the norm");
     static_assert(NT == 1 || (MT == 1 && SPLIT_K), "column tiles per workgroup: split-K kernels of one row tile");
     constexpr int T = MT * NT;      // accumulators: row tiles (NT == 1) or column tiles (MT == 1)
+    constexpr int REDUCED = ASRC == A_NORMED ? 8 : 12;      // wavefronts whose sums meet, at most (SPLIT_K)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
     __shared__ int sm_last;
     constexpr bool LN_FUSED = ASRC == A_NORMED;
     constexpr bool IN_LDS = ASRC == A_NORMED || ASRC == A_STAGED;
     constexpr bool A_REGS = !IN_LDS;      // the rows of A travel through registers and the wavefront's LDS region
+    // (the word as few_row_shape packs it)
+    const int M = shape & 511, cols_per_wg = shape >> 9 & 63, k_parts = shape >> 15 & 15, mode = shape >> 19 & 15, row_blocks = ((M + 15) / 16 + MT - 1) / MT;
+    const int nw = ASRC == A_NORMED ? 8 : shape >> 23 & 31;
+    const bool rms = shape >> 28 & 1, scatters = shape >> 29 & 1, gathers = shape >> 30 & 1;
+    const int N = ASRC == A_MERGED ? columns & 0x3fff : columns;
+    const int a_head_dim = (columns >> 14 & 511) * 8, a_heads = columns >> 23;              // A_MERGED
+    const int K = ASRC == A_MERGED ? a_heads * a_head_dim : K_or_ldc;
+    const int lda = static_cast<int>(reinterpret_cast<uintptr_t>(C_or_strides));            // not A_MERGED
+    const float* gamma = static_cast<const float*>(p2);                                     // A_NORMED
+    const float* beta = GATED ? nullptr : static_cast<const float*>(p3);
+    const float* split_o = static_cast<const float*>(Ain);                                  // A_MERGED
+    const float* split_ml = static_cast<const float*>(p2);
+    const float* bias = ASRC == A_NORMED ? late_bias : static_cast<const float*>(ASRC == A_MERGED ? p3 : p2);
+    void* C = ASRC == A_NORMED ? late_C : ASRC == A_MERGED ? C_or_strides : const_cast<void*>(p3);
+    const int ldc = ASRC == A_MERGED ? K_or_ldc : static_cast<int>(reinterpret_cast<uintptr_t>(C_or_strides) >> 32);
     // The wavefront's index as a scalar: what depends on it alone (its k blocks, whether it has a
     // whole chunk, whether it owns outputs) then branches for real. Derived from threadIdx it would
     // count as divergent, both sides of every such condition would run one after the other under
     // masks, and loads pending from one side would be waited for on the other.
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
-    const int nw = blockDim.x / 64;
     const int row16 = lane % 16, kq = lane / 16;
     // workgroup id -> (column block, row block): the row blocks of one column block have ids that
     // agree modulo 8, i.e. run on one XCD
-    const int g = blockIdx.x;
-    const int cb = (g / (N_XCD * row_blocks)) * N_XCD + g % N_XCD, rb = (g / N_XCD) % row_blocks;
-    if (cb >= col_blocks) return;
+    int cb = blockIdx.x, rb = 0;
+    if (row_blocks > 1) {
+        const int g = blockIdx.x;
+        cb = (g / (N_XCD * row_blocks)) * N_XCD + g % N_XCD;
+        rb = (g / N_XCD) % row_blocks;
+    }
+    if (cb * (SPLIT_K ? cols_per_wg : nw * 16) >= N) return;
     const int m_base = rb * 16 * MT;
     const int n0 = SPLIT_K ? cb * cols_per_wg : (cb * nw + wave) * 16;
     // K is dealt out in blocks of 64 elements, one 128-byte line of a weight row. In the MFMAs
@@ -643,7 +667,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            if constexpr (GATED) wrow[t][j] = (t ? add.up : W) + static_cast<size_t>(min(n0 + lr + 8 * j, N - 1)) * ldw;
+            if constexpr (GATED) wrow[t][j] = (t ? static_cast<const bf16_t*>(p3) : W) + static_cast<size_t>(min(n0 + lr + 8 * j, N - 1)) * ldw;
             else wrow[t][j] = W + static_cast<size_t>(min(n0 + min(16 * t + lr + 8 * j, cols_per_wg - 1), N - 1)) * ldw;
         }
     // reads: this lane's MFMA row/column is row16; for MFMA step `half` it wants piece 2*kq + half
@@ -654,7 +678,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     for (int i = 0; i < T; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     // Split-K epilogue operands (thread tid < 256 owns output element tid of the 16x16 tile, in
-    // accumulator order): requested now so that their latency hides behind the product.
+    // accumulator order): requested with the first loads so that their latency hides behind the product.
     bool ep_ok[NT];
     size_t ep_idx[NT];
     int ep_col[NT], ep_slot = -1;
@@ -663,7 +687,8 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     float ep_alpha = 0.f, ep_alpha2 = 0.f;
 #pragma unroll
     for (int t = 0; t < NT; ++t) { ep_ok[t] = false; ep_idx[t] = 0; ep_col[t] = 0; ep_bias[t] = 0.f; ep_old[t] = 0.f; }
-    if (SPLIT_K && MT == 1 && wave < 4) {
+    auto epilogue_loads = [&]() {
+        if (!(SPLIT_K && MT == 1) || wave >= 4) return;
         // (loads without a per-lane condition: outputs beyond M or N read the last row or column)
         const int m = m_base + 4 * (lane / 16) + wave;
 #pragma unroll
@@ -684,9 +709,11 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
             if (add.norm.weight != nullptr) ep_alpha = add.norm.alpha[0];
             if (add.next.weight != nullptr) ep_alpha2 = add.next.alpha[0];
         } else if constexpr (!GATED) {
-            if (add.slots != nullptr) ep_slot = add.slots[min(m, M - 1)];
+            if (scatters) ep_slot = add.slots[min(m, M - 1)];
         }
-    }
+    };
+    // (behind the fused norm what they need comes late, and so do they: they are asked for behind the first loads there)
+    if (!LN_FUSED) epilogue_loads();
 
     // A wavefront takes its k blocks in chunks of H = U/2. All loads of a chunk are issued
     // together and without a condition inside (a load under a condition makes the compiler wait
@@ -716,7 +743,10 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     // A_MERGED: requests the splits' states for the 8 elements from k on of row `row` (all loads together; n_splits is MS),
     // and merges them later
     auto fetch_splits = [&](SplitStates<MS>& st, int row, int k) {
-        const int h = k / a_head_dim, e = k - h * a_head_dim;
+        // (k / head size in eighths, exact: both are small whole numbers, and half an eighth is further from the next
+        // quotient than the reciprocal's error)
+        const int h = static_cast<int>((static_cast<float>(k / 8) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(a_head_dim / 8)));
+        const int e = k - h * a_head_dim;
         const size_t pair = static_cast<size_t>(row) * a_heads + h;
 #pragma unroll
         for (int sidx = 0; sidx < MS; ++sidx) {
@@ -747,7 +777,13 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         for (int i = 0; i < 4; ++i) pk.w[i] = pack_bf16x2(o[2 * i] * inv, o[2 * i + 1] * inv);
         return pk.v;
     };
-    const int n_blocks = k_first < K ? (K - k_first + k_stride - 1) / k_stride : 0;   // of this wavefront
+    // blocks of this wavefront: those behind its first, divided by the wavefronts on the tile. (In floating point: of whole numbers up to
+    // 2^14 and at most 96 a half more lies further from the next quotient than the reciprocal errs; an integer division takes 40 instructions.)
+    int n_blocks = (K + 63) / 64;
+    if (SPLIT_K) {
+        const int takers = nw * k_parts, from = n_blocks - 1 - (part * nw + wave);
+        n_blocks = from < 0 ? 0 : 1 + __builtin_amdgcn_readfirstlane(static_cast<int>((static_cast<float>(from) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(takers))));
+    }
     const int n_chunks = n_blocks / H;
     struct Chunk {
         bf16x8 b[NT][U];
@@ -826,6 +862,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
             for (int half = 0; half < 2; ++half) {
                 const int k = k0 + i * k_stride + 16 * kq + 8 * half;
                 const int kc = min(k, K - 8);
+                const bool whole = k0 + i * k_stride + 64 <= K;       // (uniform over the wavefront)
 #pragma unroll
                 for (int mi = 0; mi < MT; ++mi) {
                     bf16x8 a;
@@ -833,7 +870,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
                     else a = af[i][half];
 #pragma unroll
                     for (int t = 0; t < NT; ++t) {
-                        const bf16x8 b = k < K ? bf[i][t][half] : zero;
+                        const bf16x8 b = whole || k < K ? bf[i][t][half] : zero;
                         acc[mi * NT + t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, acc[mi * NT + t], 0, 0, 0);
                     }
                 }
@@ -872,9 +909,12 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     int src_row[2] = {0, 0};
     if (LN_FUSED) {
 #pragma unroll
-        for (int j = 0; j < 2; ++j) {
-            const int m = min(m_base + wave + 8 * j, M - 1);      // 8 wavefronts, rows wave and wave + 8
-            src_row[j] = rows ? rows[m] : m;
+        for (int j = 0; j < 2; ++j) src_row[j] = min(m_base + wave + 8 * j, M - 1);      // 8 wavefronts, rows wave and wave + 8
+        if (gathers) {
+            src_row[0] = late_rows[src_row[0]];
+            src_row[1] = late_rows[src_row[1]];
+            // (waited for in here, not where the launches without a gather pass too)
+            asm volatile("" : "+s"(src_row[0]), "+s"(src_row[1]));
         }
     }
     Chunk c0, c1;
@@ -919,8 +959,11 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
     // The fused norm's operands are requested before the weights: loads return in the order of
     // their requests, so the norm (whose rows come from L2) can be computed while the weights are
     // still on their way from memory, which it could not if it had to wait for them first.
-    const int nq = K / 4, n_u = (nq + 63) / 64;       // float4 per row; per lane (uniform)
-    float4 gb_piece[2], v[2][8];
+    // (NU: float4 of a row per lane, so that nothing but the last is asked whether it exists: with 8 and a condition at each the
+    // kernel had 2,140 instructions, most of a short launch's time)
+    const int nq = K / 4;       // float4 per row
+    constexpr int GB_ROUNDS = NU > 4 ? 2 : 1;       // rounds of 512 threads over scale and shift
+    float4 gb_piece[GB_ROUNDS], v[2][NU];
     // whether this wavefront's two rows exist is uniform over it: rows beyond M are not read
     const bool row_ok[2] = {m_base + wave < M, m_base + wave + 8 < M};
     if (LN_FUSED) {
@@ -929,19 +972,17 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         const float4* b4 = reinterpret_cast<const float4*>(beta);
         // (the rows first: they come from L2, and their mean and variance need nothing else)
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            if (u < n_u) {
-                const int i = min(lane + 64 * u, nq - 1);
+        for (int j = 0; j < 2; ++j) {
+            if (!row_ok[j]) continue;
+            const float4* row = reinterpret_cast<const float4*>(x + static_cast<size_t>(src_row[j]) * lda);
 #pragma unroll
-                for (int j = 0; j < 2; ++j)
-                    if (row_ok[j]) v[j][u] = reinterpret_cast<const float4*>(x + static_cast<size_t>(src_row[j]) * lda)[i];
-            }
+            for (int u = 0; u < NU; ++u) v[j][u] = row[u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1)];
         }
         __builtin_amdgcn_sched_barrier(0);
         // scale and shift: 2 K / 4 pieces of 16 bytes over the workgroup's 512 threads (K <= 2048:
         // at most two each), shared through LDS instead of every wavefront loading all of both
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
+        for (int r = 0; r < GB_ROUNDS; ++r) {
             const int i = min(tid + 512 * r, 2 * nq - 1);
             const float4* src = i < nq ? g4 + i : (beta ? b4 + (i - nq) : g4);
             gb_piece[r] = *src;
@@ -949,21 +990,22 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         __builtin_amdgcn_sched_barrier(0);
     }
     first_loads();
+    if (LN_FUSED) epilogue_loads();
     if (ASRC == A_STAGED) {
         // the workgroup's rows of A, copied once into LDS for all its wavefronts
         // (four 16-byte pieces per thread requested together, then written)
         const int kv = K / 8, total = 16 * MT * kv;
-        for (int base = tid; base < total; base += 4 * blockDim.x) {
+        for (int base = tid; base < total; base += 4 * nw * 64) {
             bf16x8 v[4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int idx = min(base + j * static_cast<int>(blockDim.x), total - 1);
+                const int idx = min(base + j * nw * 64, total - 1);
                 const int m = idx / kv, c = idx - m * kv;
                 v[j] = *reinterpret_cast<const bf16x8*>(A + static_cast<size_t>(min(m_base + m, M - 1)) * lda + 8 * c);
             }
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int idx = base + j * static_cast<int>(blockDim.x);
+                const int idx = base + j * nw * 64;
                 const int m = idx / kv, c = idx - m * kv;
                 if (idx < total)
                     *reinterpret_cast<bf16x8*>(a_s + static_cast<size_t>(m) * a_stride + 8 * c) =
@@ -981,13 +1023,13 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
             if (!row_ok[j]) continue;
             float sum = 0.f;
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (u < n_u && lane + 64 * u < nq) sum += (v[j][u].x + v[j][u].y) + (v[j][u].z + v[j][u].w);
+            for (int u = 0; u < NU; ++u)
+                if (u < NU - 1 || lane + 64 * u < nq) sum += (v[j][u].x + v[j][u].y) + (v[j][u].z + v[j][u].w);
             mean[j] = rms ? 0.f : wave_sum(sum) / static_cast<float>(K);
             float q = 0.f;
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                if (u < n_u && lane + 64 * u < nq) {
+            for (int u = 0; u < NU; ++u) {
+                if (u < NU - 1 || lane + 64 * u < nq) {
                     const float a = v[j][u].x - mean[j], b = v[j][u].y - mean[j], c = v[j][u].z - mean[j], d = v[j][u].w - mean[j];
                     q += (a * a + b * b) + (c * c + d * d);
                 }
@@ -995,7 +1037,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
             inv[j] = 1.0f / sqrtf(wave_sum(q) / static_cast<float>(K) + eps);
         }
 #pragma unroll
-        for (int r = 0; r < 2; ++r) {
+        for (int r = 0; r < GB_ROUNDS; ++r) {
             const int i = tid + 512 * r;
             if (i < 2 * nq) gb_s[i] = (i >= nq && !beta) ? make_float4(0.f, 0.f, 0.f, 0.f) : gb_piece[r];
         }
@@ -1004,14 +1046,11 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         for (int j = 0; j < 2; ++j) {
             const int m = wave + 8 * j;
             bf16_t* dst = a_s + static_cast<size_t>(m) * a_stride;
-            if (!row_ok[j]) {
-                for (int i = lane; i < nq; i += 64) *reinterpret_cast<uint2*>(dst + 4 * i) = make_uint2(0, 0);
-                continue;
-            }
+            if (!row_ok[j]) continue;      // (what its place in LDS holds goes into its own row of the products alone, which is not stored)
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
+            for (int u = 0; u < NU; ++u) {
                 const int i = lane + 64 * u;
-                if (u < n_u && i < nq) {
+                if (u < NU - 1 || i < nq) {
                     const float4 g = gb_s[i], b = gb_s[nq + i];
                     uint2 pk;
                     pk.x = pack_bf16x2((v[j][u].x - mean[j]) * inv[j] * g.x + b.x, (v[j][u].y - mean[j]) * inv[j] * g.y + b.y);
@@ -1070,8 +1109,15 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
             vt[t] = 0.f;
-            if (tid < 256)
-                for (int w = 0; w < nw; ++w) vt[t] += red[(static_cast<size_t>(w) * NT + t) * 256 + tid];
+            if (wave < 4) {
+                // (all reads at once, then the sum in the order of the wavefronts)
+                float of_wave[REDUCED];
+#pragma unroll
+                for (int w = 0; w < REDUCED; ++w) of_wave[w] = red[(min(w, nw - 1) * NT + t) * 256 + tid];
+#pragma unroll
+                for (int w = 0; w < REDUCED; ++w)
+                    if (w < nw) vt[t] += of_wave[w];
+            }
         }
         float& v = vt[0];
         if (NT == 1 && k_parts > 1) {
@@ -1126,7 +1172,7 @@ gemm_bf16_skinny(// the first 16 dwords arrive in registers with the wavefront: 
         }
         return;
     }
-    for (int idx = tid; idx < MT * 256; idx += blockDim.x) {
+    for (int idx = tid; idx < MT * 256; idx += nw * 64) {
         const int i = idx / 256, r = (idx % 256) / 64, l = idx % 64;
         const int m = m_base + i * 16 + 4 * (l / 16) + r, nn = n0 + l % 16;
         if (m >= M || nn >= N) continue;
@@ -1142,6 +1188,13 @@ constexpr int SPLIT_COUNTERS = 4096;      // tiles that may be shared by several
 constexpr int SPLIT_MAX_PARTS = 8;
 constexpr int SPLIT_MIN_K_BLOCKS = 12;    // k blocks of 64 elements that every part keeps at least
 constexpr int SPLIT_FROM_K_BLOCKS = 80;   // shorter K: the fences cost more than the parallelism gains (measured)
+
+// What the few-row kernel is told in one word: rows of A (9 bits), columns a workgroup (6), parts of K (4), epilogue (4; one that does not
+// exist stores nothing), wavefronts (5), an RMS norm, page slots, gathered rows.
+static unsigned few_row_shape(int M, int cols_per_wg, int k_parts, int mode, int nw, bool rms, bool scatters, bool gathers) {
+    return static_cast<unsigned>(M) | cols_per_wg << 9 | k_parts << 15 | (mode < 0 || mode > 15 ? 15 : mode) << 19 | nw << 23 |
+           (rms ? 1u << 28 : 0u) | (scatters ? 1u << 29 : 0u) | (gathers ? 1u << 30 : 0u);
+}
 
 struct MergedA {        // A_MERGED: where the attention splits' states lie
     const float* split_o = nullptr;
@@ -1178,6 +1231,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         if (fit > 4) fit = 4;
         row_blocks = (mt + fit - 1) / fit;
         mt = (mt + row_blocks - 1) / row_blocks;
+        row_blocks = ((M + 15) / 16 + mt - 1) / mt;         // (as the kernel has it)
         staged_bytes = row16_bytes * mt;
     }
     int nw;
@@ -1246,6 +1300,11 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     if (split_k && !LN_FUSED && !MERGED && row_blocks == 1 && k_parts == 1 && tiles < 256 && k_blocks >= 48)
         cols_per_wg = std::min(16, std::max((N + 255) / 256, 4));
     const int col_blocks = split_k ? (N + cols_per_wg - 1) / cols_per_wg : (tiles + nw - 1) / nw;
+    // (what the words do not hold; K beyond 2^20: see the kernel's count of a wavefront's blocks)
+    if (M > 511 || K > 1 << 20 || (MERGED && (N > 0x3fff || merged.heads > 511 || merged.head_dim > 511 * 8))) return -2;
+    const unsigned shape = few_row_shape(M, cols_per_wg, k_parts, mode, nw, rms, kv.slots != nullptr, rows != nullptr);
+    const unsigned columns = MERGED ? N | merged.head_dim / 8 << 14 | static_cast<unsigned>(merged.heads) << 23 : N;
+    void* const strides = reinterpret_cast<void*>(static_cast<uintptr_t>(static_cast<unsigned>(lda)) | static_cast<uintptr_t>(static_cast<unsigned>(ldc)) << 32);
     const dim3 grid((col_blocks + N_XCD - 1) / N_XCD * N_XCD * row_blocks, k_parts), block(nw * 64);
     const size_t smem = lds_bytes(two_tiles);
     if (staged) {
@@ -1257,9 +1316,8 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
                                            hipFuncAttributeMaxDynamicSharedMemorySize,                 \
                                            static_cast<int>(staged_bytes));                            \
         if (e != hipSuccess) return static_cast<int>(e);                                               \
-        kernel<<<grid, block, staged_bytes, stream>>>(W, ldw, N, K, M, col_blocks, row_blocks, 16, 1, A, lda, mode, \
-                                                      bias, C, ldc, gamma, beta, eps, rows, nullptr, nullptr, \
-                                                      nullptr, nullptr, 1, 8, 0, KvScatter{});                    \
+        kernel<<<grid, block, staged_bytes, stream>>>(W, A, bias, C, ldw, columns, shape, K, strides, nullptr, nullptr, nullptr, 0.f, \
+                                                      nullptr, nullptr, KvScatter{});                  \
         break;                                                                                         \
     }
         switch (mt) {
@@ -1276,10 +1334,12 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     }
     if (smem > MAX_DYNAMIC_LDS) return -2;
     constexpr int ASRC = LN_FUSED ? A_NORMED : (MERGED ? A_MERGED : A_GLOBAL);
-#define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...) SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, false, __VA_ARGS__)
-#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, ...)                                  \
+    const void* p2 = LN_FUSED ? gamma : MERGED ? merged.split_ml : bias;
+    const void* p3 = LN_FUSED ? (gated != nullptr ? static_cast<const void*>(gated->up) : beta) : MERGED ? static_cast<const void*>(bias) : C;
+#define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...) SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, false, 8, __VA_ARGS__)
+#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, ...)                             \
     do {                                                                                               \
-        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED>;               \
+        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV>;          \
         static bool lds_allowed = false;      /* more than 64 KB of dynamic LDS has to be asked for once */ \
         if (!lds_allowed) {                                                                            \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                  \
@@ -1287,10 +1347,8 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
             if (e != hipSuccess) return static_cast<int>(e);                                           \
             lds_allowed = true;                                                                        \
         }                                                                                              \
-        kernel<<<grid, block, smem, stream>>>(W, ldw, N, K, M, col_blocks, row_blocks, cols_per_wg, k_parts, A, lda, \
-                                              mode, bias, C, ldc, gamma, beta, eps, rows, part_sums,      \
-                                              part_counters, merged.split_o, merged.split_ml,             \
-                                              merged.heads, merged.head_dim, rms, __VA_ARGS__);        \
+        kernel<<<grid, block, smem, stream>>>(W, MERGED ? merged.split_o : A, p2, p3, ldw, columns, shape, MERGED ? ldc : K, \
+                                              MERGED ? C : strides, bias, C, rows, eps, part_sums, part_counters, __VA_ARGS__); \
     } while (0)
 #define SKINNY_LAUNCH(SPLIT, UV, A2, NTV, ONE)                                                         \
     do {                                                                                               \
@@ -1338,24 +1396,26 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
                 default: SKINNY_MERGED(4); break;
             }
 #undef SKINNY_MERGED
-        } else if (gated != nullptr) {
-#define SKINNY_GATED(UV, ONE) SKINNY_ANY(true, UV, false, 2, false, MERGE_MAX_SPLITS, ONE, true, *gated)
-            if constexpr (LN_FUSED) {
-                if (per_wave <= 1) SKINNY_GATED(2, true);
-                else if (per_wave <= 2) SKINNY_GATED(4, true);
-                else SKINNY_GATED(4, false);
+        } else if constexpr (LN_FUSED) {
+            // (an instance for every count of a lane's float4s; two of them make one k block a wavefront. Two tiles take half the
+            // blocks per chunk.)
+#define SKINNY_NORMED(NUV)                                                                                                      \
+    case NUV: {                                                                                                                 \
+        constexpr int BLOCKS = (NUV + 1) / 2, U1 = BLOCKS > 3 ? 6 : 2 * BLOCKS, U2 = BLOCKS > 2 ? 4 : 2 * BLOCKS;                   \
+        if (gated != nullptr) SKINNY_ANY(true, U2, false, 2, false, MERGE_MAX_SPLITS, BLOCKS <= U2 / 2, true, NUV, *gated);         \
+        else if (two_tiles) SKINNY_ANY(true, U2, false, 2, false, MERGE_MAX_SPLITS, BLOCKS <= U2 / 2, false, NUV, kv);              \
+        else SKINNY_ANY(true, U1, false, 1, false, MERGE_MAX_SPLITS, BLOCKS <= U1 / 2, false, NUV, kv);                             \
+        break;                                                                                                                  \
+    }
+            switch ((K + 255) / 256) {
+                SKINNY_NORMED(1) SKINNY_NORMED(2) SKINNY_NORMED(3) SKINNY_NORMED(4)
+                SKINNY_NORMED(5) SKINNY_NORMED(6) SKINNY_NORMED(7) SKINNY_NORMED(8)
+                default: return -2;
             }
-#undef SKINNY_GATED
+#undef SKINNY_NORMED
         } else if (two_tiles) {
             // (two tiles per chunk slot: half the blocks per chunk)
-            if (per_wave <= 1 || !LN_FUSED) SKINNY_CHUNKS(2, false, 2);
-            else SKINNY_CHUNKS(4, false, 2);
-        } else if (LN_FUSED) {
-            switch (std::min(per_wave, 3)) {
-                case 1: SKINNY_LAUNCH(true, 2, false, 1, true); break;
-                case 2: SKINNY_LAUNCH(true, 4, false, 1, true); break;
-                default: SKINNY_CHUNKS(6, false, 1); break;
-            }
+            SKINNY_CHUNKS(2, false, 2);
         } else if (M <= 8) {
             switch (std::min(per_wave, 4)) {
                 case 1: SKINNY_LAUNCH(true, 2, false, 1, true); break;

@@ -594,6 +594,13 @@ def test_ln_linear(ops, dtype, M, N, K, epi):
     assert (out2.cpu().double() - ref).abs().max().item() <= tol
 
 
+@pytest.mark.parametrize("K", [k for n in range(1, 9) for k in (256 * n - 8, 256 * n, 256 * n + 8)][:-1])
+@pytest.mark.parametrize("M,N", [(1, 48), (9, 4104)])
+def test_ln_linear_at_every_number_of_columns_a_lane(ops, M, N, K):
+    """The product behind the norm has an instance for every 256 columns of K: around each, with one tile a workgroup and with two."""
+    test_ln_linear(ops, torch.bfloat16, M, N, K, "store")
+
+
 def test_linear_fp32_is_true_fp32(ops):
     """Values that bf16 or tf32 inputs would destroy: 1 + 2^-20 differs from 1 only in true fp32."""
     K = 64
