@@ -566,7 +566,7 @@ template <int MS> struct SplitStates {
 };
 
 template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false, int MS = MERGE_MAX_SPLITS,
-          bool ONE = false, bool GATED = false, int NU = 8>
+          bool ONE = false, bool GATED = false, int NU = 8, int WC = 16>
 __global__ void __launch_bounds__(ASRC == A_NORMED ? 512 : (ASRC == A_GLOBAL || ASRC == A_MERGED ? 768 : 1024))
 gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, and hold everything that the first loads need: an argument
                  // behind them comes with a load of its own from memory that no cache holds (as does blockDim), 0.6 to 0.8 us
@@ -659,8 +659,12 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     // swizzle of the row (the row modulo 8, its lowest bit flipped for rows 8..15), so that slot s
     // of row r, written to LDS lane-linearly, holds piece s ^ swizzle(r): then the 16 lanes of an
     // operand read (rows 0..15, one piece number) fall on 16 different 16-byte bank groups.
+    // WC: the columns that a workgroup has, at most: two loads cover 16 of a k block, one 8, and one 4 of two blocks. (768 x 3,072 on 192
+    // workgroups of 4 columns: of what two loads asked for three quarters were the last column again, and a compute unit takes 64 bytes a
+    // clock: 3.9 > 3.3 us from the first wavefront's start at 1 and 8 rows, with rows beyond M not asked for either.)
     const int lr = lane / 8;
     const int piece[2] = {(lane % 8) ^ lr, (lane % 8) ^ lr ^ 1};
+    static_assert(WC == 16 || (SPLIT_K && NT == 1 && U % 4 == 0 && U >= 4), "narrow column tiles: whole pairs of k blocks");
     // (columns beyond the workgroup's or the matrix's: the last valid one, never stored)
     const bf16_t* wrow[NT][2];
 #pragma unroll
@@ -670,6 +674,8 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             if constexpr (GATED) wrow[t][j] = (t ? static_cast<const bf16_t*>(p3) : W) + static_cast<size_t>(min(n0 + lr + 8 * j, N - 1)) * ldw;
             else wrow[t][j] = W + static_cast<size_t>(min(n0 + min(16 * t + lr + 8 * j, cols_per_wg - 1), N - 1)) * ldw;
         }
+    const bf16_t* wrow4 = W + static_cast<size_t>(min(n0 + min(lr % 4, cols_per_wg - 1), N - 1)) * ldw;     // (WC == 4)
+    const int piece4 = (lane % 8) ^ (lr % 4);
     // reads: this lane's MFMA row/column is row16; for MFMA step `half` it wants piece 2*kq + half
     const int rd_swz = row16 < 8 ? row16 : ((row16 - 8) ^ 1);
 
@@ -740,6 +746,8 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             arow[j] = A + static_cast<size_t>(arow_idx[j]) * lda;
         }
     }
+    // (lanes of rows beyond M ask for nothing: what they multiply reaches only outputs that are not stored)
+    const bool row_exists[2] = {m_base + lr < M, m_base + lr + 8 < M};
     // A_MERGED: requests the splits' states for the 8 elements from k on of row `row` (all loads together; n_splits is MS),
     // and merges them later
     auto fetch_splits = [&](SplitStates<MS>& st, int row, int k) {
@@ -748,10 +756,17 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
         const int h = static_cast<int>((static_cast<float>(k / 8) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(a_head_dim / 8)));
         const int e = k - h * a_head_dim;
         const size_t pair = static_cast<size_t>(row) * a_heads + h;
+        typedef float f32x4_of_8 __attribute__((ext_vector_type(4), aligned(8)));
+#pragma unroll
+        for (int sidx = 0; sidx + 1 < MS; sidx += 2) {
+            const f32x4_of_8 two = *reinterpret_cast<const f32x4_of_8*>(split_ml + (pair * MS + sidx) * 2);
+            st.ml[sidx] = make_float2(two.x, two.y);
+            st.ml[sidx + 1] = make_float2(two.z, two.w);
+        }
+        if constexpr (MS % 2 == 1) st.ml[MS - 1] = *reinterpret_cast<const float2*>(split_ml + (pair * MS + MS - 1) * 2);
 #pragma unroll
         for (int sidx = 0; sidx < MS; ++sidx) {
             const size_t slot = pair * MS + sidx;
-            st.ml[sidx] = *reinterpret_cast<const float2*>(split_ml + slot * 2);
             const float4* src = reinterpret_cast<const float4*>(split_o + slot * a_head_dim + e);
             st.o[sidx][0] = src[0];
             st.o[sidx][1] = src[1];
@@ -786,7 +801,7 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     }
     const int n_chunks = n_blocks / H;
     struct Chunk {
-        bf16x8 b[NT][U];
+        bf16x8 b[NT][U * WC / 16];
         bf16x8 a[A_REGS ? (A_TWO ? U : U / 2) : 1];
     };
     // (A_MERGED) the states requested for a chunk's blocks, rows 0..7 and 8..15
@@ -795,7 +810,7 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
         if (ASRC != A_MERGED) return;
 #pragma unroll
         for (int j = 0; j < (A_TWO ? 2 : 1); ++j)
-            if (j == 0 || a_two) fetch_splits(pending[h][j], arow_idx[j], min(k0 + 8 * piece[j], K - 8));
+            if ((j == 0 || a_two) && row_exists[j]) fetch_splits(pending[h][j], arow_idx[j], min(k0 + 8 * piece[j], K - 8));
     };
     auto merge_block_splits = [&](Chunk& c, int h) {
         if (ASRC != A_MERGED) return;
@@ -803,23 +818,37 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
         for (int j = 0; j < (A_TWO ? 2 : 1); ++j)
             if (j == 0 || a_two) c.a[A_TWO ? 2 * h + j : h] = merge_splits(pending[h][j]);
     };
-    auto load_steps = [&](Chunk& c, int u0, int k0) {      // the k block at k0 (rows 0..7, rows 8..15) into slots u0, u0+1
+    // Weights that one workgroup alone reads (one row block: at most 8 rows, or the fused norm's 16) and the wide product's (the logits
+    // head, as large as all the layers') are requested with streaming loads: read once a step, they would only displace what is read
+    // again (activations, scale and shift vectors, biases) from the caches. With several row blocks the later ones find the weights
+    // in L2 and plain loads are kept.
+    auto load_piece = [&](const bf16_t* from) -> bf16x8 {
+        constexpr bool STREAM = ASRC != A_GLOBAL || !A_TWO;
+        const bf16x8* src = reinterpret_cast<const bf16x8*>(from);
+        return STREAM ? __builtin_nontemporal_load(src) : *src;
+    };
+    auto load_steps = [&](Chunk& c, int u0, int k0) {      // weights of the k block at k0 (columns 0..7, columns 8..15) into slots u0, u0+1
+#pragma unroll
+        for (int j = 0; j < (WC == 16 ? 2 : WC / 8); ++j) {
+            const int k = min(k0 + 8 * piece[j], K - 8);
+#pragma unroll
+            for (int t = 0; t < NT; ++t) c.b[t][WC == 16 ? u0 + j : u0 / 2] = load_piece(wrow[t][j] + k);
+        }
+    };
+    auto load_rows = [&](Chunk& c, int count, auto k_of) {      // rows of A for the first `count` blocks of a chunk, block h at k_of(h)
+        if (ASRC != A_GLOBAL) return;       // (A_MERGED: the splits' states were requested before and are merged after the weights)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
-            const int k = min(k0 + 8 * piece[j], K - 8);
-            // Weights that one workgroup alone reads (one row block: at most 8 rows, or the fused
-            // norm's 16) and the wide product's (the logits head, as large as all the layers') are
-            // requested with streaming loads: read once a step, they would only displace what is
-            // read again (activations, scale and shift vectors, biases) from the caches. With
-            // several row blocks the later ones find the weights in L2 and plain loads are kept.
-            constexpr bool STREAM = ASRC != A_GLOBAL || !A_TWO;
+            if ((j == 1 && !a_two) || !row_exists[j]) continue;
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {
-                const bf16x8* src = reinterpret_cast<const bf16x8*>(wrow[t][j] + k);
-                c.b[t][u0 + j] = STREAM ? __builtin_nontemporal_load(src) : *src;
-            }
-            if (ASRC == A_GLOBAL && (j == 0 || a_two)) c.a[A_TWO ? u0 + j : u0 / 2] = *reinterpret_cast<const bf16x8*>(arow[j] + k);
-            // (A_MERGED: the splits' states were requested before the weights and are merged after them)
+            for (int h = 0; h < H; ++h)
+                if (h < count) c.a[A_TWO ? 2 * h + j : h] = *reinterpret_cast<const bf16x8*>(arow[j] + min(k_of(h) + 8 * piece[j], K - 8));
+        }
+    };
+    auto load_pairs = [&](Chunk& c, auto k_of) {           // (WC == 4) weights of all blocks of a chunk, two to a load
+        if constexpr (WC == 4) {
+#pragma unroll
+            for (int i = 0; i < U / 4; ++i) c.b[0][i] = load_piece(wrow4 + min((lane < 32 ? k_of(2 * i) : k_of(2 * i + 1)) + 8 * piece4, K - 8));
         }
     };
     auto wave_lds_order = [&]() {       // orders the wavefront's own LDS writes and reads (no instruction)
@@ -840,10 +869,11 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             }
 #pragma unroll
             for (int t = 0; t < NT; ++t) {
-                stage_w[(i * NT + t) * 128 + lane] = c.b[t][u0 + 2 * i];
-                stage_w[(i * NT + t) * 128 + 64 + lane] = c.b[t][u0 + 2 * i + 1];
+                if (WC > 4) stage_w[(i * NT + t) * 128 + lane] = c.b[t][WC == 16 ? u0 + 2 * i : u0 / 2 + i];
+                if (WC == 16) stage_w[(i * NT + t) * 128 + 64 + lane] = c.b[t][u0 + 2 * i + 1];
             }
         }
+        if (WC == 4) stage_w[(lane / 32) * 128 + lane % 32] = c.b[0][u0 / 4];       // (both blocks of the pair, columns 0..3)
         wave_lds_order();
         bf16x8 af[CNT][2], bf[CNT][NT][2];
 #pragma unroll
@@ -893,8 +923,12 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             for (int h = 0; h < H; ++h) fetch_block_splits(h, k_first + (chunk * H + h) * k_stride);
             __builtin_amdgcn_sched_barrier(0);
         }
+        auto k_of = [&](int h) { return k_first + (chunk * H + h) * k_stride; };
+        load_rows(c, H, k_of);
+        if (WC == 4) load_pairs(c, k_of);
+        else
 #pragma unroll
-        for (int h = 0; h < H; ++h) load_steps(c, 2 * h, k_first + (chunk * H + h) * k_stride);
+            for (int h = 0; h < H; ++h) load_steps(c, 2 * h, k_of(h));
         // the instruction scheduler must not sink these loads towards their uses: they are issued
         // here to be in flight together
         __builtin_amdgcn_sched_barrier(0);
@@ -926,9 +960,13 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
                 if (h < left) fetch_block_splits(h, k_first + (first + h) * k_stride);
             __builtin_amdgcn_sched_barrier(0);
         }
+        auto k_of = [&](int h) { return k_first + min(first + h, n_blocks - 1) * k_stride; };
+        load_rows(c1, left, k_of);
+        if (WC == 4) load_pairs(c1, k_of);
+        else
 #pragma unroll
-        for (int h = 0; h < H - 1; ++h)
-            if (h < left) load_steps(c1, 2 * h, k_first + (first + h) * k_stride);
+            for (int h = 0; h < H - 1; ++h)
+                if (h < left) load_steps(c1, 2 * h, k_of(h));
         __builtin_amdgcn_sched_barrier(0);
         if (ASRC == A_MERGED) {
 #pragma unroll
@@ -948,8 +986,12 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             for (int h = 0; h < H; ++h) fetch_block_splits(h, k_first + min(h, last_block) * k_stride);
             __builtin_amdgcn_sched_barrier(0);
         }
+        auto k_of = [&](int h) { return k_first + min(h, last_block) * k_stride; };
+        load_rows(c0, H, k_of);
+        if (WC == 4) load_pairs(c0, k_of);
+        else
 #pragma unroll
-        for (int h = 0; h < H; ++h) load_steps(c0, 2 * h, k_first + min(h, last_block) * k_stride);
+            for (int h = 0; h < H; ++h) load_steps(c0, 2 * h, k_of(h));
         __builtin_amdgcn_sched_barrier(0);
         if (ASRC == A_MERGED) {
 #pragma unroll
@@ -1084,6 +1126,10 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
         if (left > 0) load_left();
         mma_some(c1, left, k_first + first * k_stride);
     }
+    // (Arguments that the kernel loads itself stay where they are put until here: registers taken up again earlier are waited for, with the
+    // loads into them still in flight, in front of the first rows and weights.)
+    if constexpr (!THROUGH && !GATED) asm volatile("" ::"s"(add.slots), "s"(add.k_pages), "s"(add.v_pages), "s"(add.q_cols), "s"(add.kv_dim));
+    asm volatile("" ::"s"(late_bias), "s"(late_C), "s"(part_sums), "s"(part_counters));
     // accumulator layout of the 16x16 tile: register r of lane l holds row 4*(l/16) + r, column l%16
     if (!SPLIT_K) {
         if (!n_ok) return;
@@ -1336,10 +1382,10 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     constexpr int ASRC = LN_FUSED ? A_NORMED : (MERGED ? A_MERGED : A_GLOBAL);
     const void* p2 = LN_FUSED ? gamma : MERGED ? merged.split_ml : bias;
     const void* p3 = LN_FUSED ? (gated != nullptr ? static_cast<const void*>(gated->up) : beta) : MERGED ? static_cast<const void*>(bias) : C;
-#define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...) SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, false, 8, __VA_ARGS__)
-#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, ...)                             \
+#define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...) SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, false, 8, 16, __VA_ARGS__)
+#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, ...)                        \
     do {                                                                                               \
-        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV>;          \
+        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV>;     \
         static bool lds_allowed = false;      /* more than 64 KB of dynamic LDS has to be asked for once */ \
         if (!lds_allowed) {                                                                            \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                  \
@@ -1362,6 +1408,15 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     do {                                                                                               \
         if (per_wave <= UV / 2) SKINNY_LAUNCH(true, UV, A2, NTV, true);                                \
         else SKINNY_LAUNCH(true, UV, A2, NTV, false);                                                  \
+    } while (0)
+// the same with narrow column tiles: chunks of four blocks
+#define SKINNY_NARROW(WCV)                                                                              \
+    do {                                                                                               \
+        if (through != nullptr) {                                                                      \
+            if (per_wave <= 4) SKINNY_ANY(true, 8, false, 1, true, MERGE_MAX_SPLITS, true, false, 8, WCV, *through); \
+            else SKINNY_ANY(true, 8, false, 1, true, MERGE_MAX_SPLITS, false, false, 8, WCV, *through); \
+        } else if (per_wave <= 4) SKINNY_ANY(true, 8, false, 1, false, MERGE_MAX_SPLITS, true, false, 8, WCV, kv); \
+        else SKINNY_ANY(true, 8, false, 1, false, MERGE_MAX_SPLITS, false, false, 8, WCV, kv);          \
     } while (0)
     if (split_k) {
         // a chunk holds all k blocks of a wavefront when they are at most 3 (4 without the fused
@@ -1402,9 +1457,9 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 #define SKINNY_NORMED(NUV)                                                                                                      \
     case NUV: {                                                                                                                 \
         constexpr int BLOCKS = (NUV + 1) / 2, U1 = BLOCKS > 3 ? 6 : 2 * BLOCKS, U2 = BLOCKS > 2 ? 4 : 2 * BLOCKS;                   \
-        if (gated != nullptr) SKINNY_ANY(true, U2, false, 2, false, MERGE_MAX_SPLITS, BLOCKS <= U2 / 2, true, NUV, *gated);         \
-        else if (two_tiles) SKINNY_ANY(true, U2, false, 2, false, MERGE_MAX_SPLITS, BLOCKS <= U2 / 2, false, NUV, kv);              \
-        else SKINNY_ANY(true, U1, false, 1, false, MERGE_MAX_SPLITS, BLOCKS <= U1 / 2, false, NUV, kv);                             \
+        if (gated != nullptr) SKINNY_ANY(true, U2, false, 2, false, MERGE_MAX_SPLITS, BLOCKS <= U2 / 2, true, NUV, 16, *gated);         \
+        else if (two_tiles) SKINNY_ANY(true, U2, false, 2, false, MERGE_MAX_SPLITS, BLOCKS <= U2 / 2, false, NUV, 16, kv);              \
+        else SKINNY_ANY(true, U1, false, 1, false, MERGE_MAX_SPLITS, BLOCKS <= U1 / 2, false, NUV, 16, kv);                             \
         break;                                                                                                                  \
     }
             switch ((K + 255) / 256) {
@@ -1421,7 +1476,13 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
                 case 1: SKINNY_LAUNCH(true, 2, false, 1, true); break;
                 case 2: SKINNY_LAUNCH(true, 4, false, 1, true); break;
                 case 3: SKINNY_LAUNCH(true, 6, false, 1, true); break;
-                default: SKINNY_CHUNKS(8, false, 1); break;
+                default:
+                    if constexpr (ASRC == A_GLOBAL) {
+                        if (cols_per_wg <= 4) { SKINNY_NARROW(4); break; }
+                        if (cols_per_wg <= 8) { SKINNY_NARROW(8); break; }
+                    }
+                    SKINNY_CHUNKS(8, false, 1);
+                    break;
             }
         } else {
             switch (std::min(per_wave, 3)) {
@@ -1435,6 +1496,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         // staging them in LDS is faster than every workgroup normalising them again
         return -2;
     }
+#undef SKINNY_NARROW
 #undef SKINNY_CHUNKS
 #undef SKINNY_LAUNCH
 #undef SKINNY_KERNEL

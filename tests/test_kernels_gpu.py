@@ -491,6 +491,29 @@ def test_linear_bf16_few_rows_long_k_shares_tiles(ops, M, N, K):
     assert torch.equal(x.cpu(), outs[0])
 
 
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N", [12, 767, 1030, 1500, 2040, 2050])          # 4, 4, 5, 6, 8 and 9 columns a workgroup
+@pytest.mark.parametrize("K", [3016, 3072, 3080, 4104, 5000])             # 48 to 79 k blocks: one chunk a wavefront, a second one with 1 to 3 left
+def test_linear_bf16_few_rows_of_narrow_tiles(ops, M, N, K):
+    """Products with a long K whose columns are dealt out in fewer than 16 a workgroup: each result next to the plain one, and a row has the
+    same bits alone, among others, and among so many that another kernel of the same sums takes them."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a = _rand((9, K), torch.bfloat16, g)
+    w = _rand((N, K), torch.bfloat16, g, std=1.0 / math.sqrt(K))
+    bias = 0.5 * _rand((N,), torch.float32, g)
+    x0 = _rand((9, N), torch.float32, g)
+    outs = []
+    for rows in (M, 9):
+        x = x0[:rows].clone().to(DEV)
+        ops.linear(a[:rows].to(DEV), w.to(DEV), bias.to(DEV), x, "add_residual")
+        outs.append(x.cpu())
+    assert torch.equal(outs[0], outs[1][:M])
+    want = x0[:M].double() + a[:M].double() @ w.double().T + bias.double()
+    # fp32 sums: at most one rounding of 2^-24 for every eighth of the terms and of their magnitude, and a few for bias and residual
+    bound = 2.0 ** -24 * (K / 8 + 8) * (a[:M].double().abs() @ w.double().abs().T + x0[:M].double().abs() + bias.double().abs())
+    assert ((outs[0].double() - want).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("M", [17, 25, 32])
 @pytest.mark.parametrize("N,K", [(2048, 768), (2049, 768), (2304, 768), (2500, 1024), (4096, 768), (4097, 768), (4097, 1032), (6400, 1600)])
 @pytest.mark.parametrize("epi", ["store", "gelu_tanh"])
