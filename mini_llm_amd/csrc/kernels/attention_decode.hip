@@ -79,13 +79,8 @@ __device__ __forceinline__ void lane_halves(float first, float second, float& lo
     }
 }
 
-// Keys of a split, rounded up (in floating point below 2^20 keys: a half is further from the next quotient by up to 64 splits than the
-// reciprocal errs; an integer division takes 40 instructions).
-__device__ __forceinline__ int keys_per_split(int n_keys, int nsplit) {
-    if (nsplit == 1) return n_keys;
-    if (n_keys >= 1 << 20 || nsplit > 64) return (n_keys + nsplit - 1) / nsplit;
-    return n_keys <= 0 ? 0 : 1 + __builtin_amdgcn_readfirstlane(static_cast<int>((static_cast<float>(n_keys - 1) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(nsplit))));
-}
+// Keys of a split, rounded up.
+__device__ __forceinline__ int keys_per_split(int n_keys, int nsplit) { return nsplit == 1 ? n_keys : n_keys <= 0 ? 0 : 1 + uniform_quotient(n_keys - 1, nsplit); }
 
 // SHAPED: the scores are shaped before the softmax and a chunked mask may stand in for the window (score_shape.h);
 // the queries then come times the scale alone, and the shaped score goes to base 2 afterwards.

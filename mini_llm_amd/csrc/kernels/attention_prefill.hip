@@ -48,10 +48,12 @@ union Frag8 {
 // The weights are fp32 until they are packed for the second product, as the softmax's are.
 template <int DH, int NW, int MODE, bool LONGEST_FIRST>
 __global__ void __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(1, (DH >= 128 && NW == 4) ? 1 : 2)))
-prefill_attention_kernel(const bf16_t* __restrict__ q, int q_stride, int q_col,
-                         const bf16_t* __restrict__ k_pages, const bf16_t* __restrict__ v_pages, int kv_dim,
-                         const int* __restrict__ block_tables, int max_blocks,
-                         const int* __restrict__ cu_q, const int* __restrict__ ctx_len, int n_seqs,
+prefill_attention_kernel(// the first 14 dwords arrive in registers with the wavefront: what its tile, its queries and its table are found with
+                         const int* __restrict__ cu_q, const int* __restrict__ ctx_len, const int* __restrict__ block_tables,
+                         const bf16_t* __restrict__ q, int n_seqs, int places, int max_blocks, int q_stride,
+                         const bf16_t* __restrict__ k_pages,
+                         // the rest is loaded by the kernel
+                         const bf16_t* __restrict__ v_pages, int kv_dim,
                          int n_heads, int n_kv_heads, int page_size, float scale_log2e, int window,
                          bf16_t* __restrict__ out, int out_stride, MllmScoreShape shape, float scale,
                          const float* __restrict__ gate, int ldg) {
@@ -70,17 +72,27 @@ prefill_attention_kernel(const bf16_t* __restrict__ q, int q_stride, int q_col,
     extern __shared__ int sm_table[];          // the sequence's block table (max_blocks entries)
 
     // Heads vary fastest.
-    const auto [b, tile, q_begin, q_len] = LONGEST_FIRST ? longest_tile<PF_BM>(cu_q, ctx_len, n_seqs, 1, blockIdx.y) : next_tile<PF_BM>(cu_q, n_seqs, 1, blockIdx.y, gridDim.y);
+    const auto [b, tile, q_begin, q_len] = LONGEST_FIRST ? longest_tile<PF_BM>(cu_q, ctx_len, n_seqs, 1, blockIdx.y) : next_tile<PF_BM>(cu_q, n_seqs, 1, blockIdx.y, places);
     if (b < 0) return;                     // surplus workgroup; the whole workgroup leaves
 
-    const int h = blockIdx.x, hk = h / (n_heads / n_kv_heads);
+    const int h = blockIdx.x;
     const int tid = threadIdx.x, lane = tid % 64;
     const int wave = __builtin_amdgcn_readfirstlane(tid / 64) % 4;      // which 16 queries
     const int kh = __builtin_amdgcn_readfirstlane(tid / 64) / 4;        // which part of every key tile
     const int G = lane / 16, c16 = lane % 16;
-    const int start = ctx_len[b] - q_len;                 // position of the step's first query
+    // The sequence's block table goes to LDS first: the gathers below then depend on an LDS read, not on a global load that would have to be
+    // waited for in front of every key load. Its whole row (the host passes at most PF_TABLE_LDS blocks, and rows are filled to their
+    // end), so that neither it nor the queries wait for the context's length: one memory latency less in front of the first keys.
+    const int* gtable = block_tables + static_cast<size_t>(b) * max_blocks;
     const int q0 = tile * PF_BM;
     const int qi = q0 + wave * 16 + c16;                  // this lane's query within the step's rows
+    const int entry = gtable[min(tid, max_blocks - 1)];
+    Frag8 qf[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)      // a lane beyond the last query takes that query again; its scores are masked
+        qf[ks].q = *reinterpret_cast<const uint4*>(q + static_cast<size_t>(q_begin + min(qi, q_len - 1)) * q_stride + h * DH + 32 * ks + 8 * G);
+    const int start = ctx_len[b] - q_len;                 // position of the step's first query
+    const int hk = n_heads == n_kv_heads ? h : small_quotient(h, small_quotient(n_heads, n_kv_heads));
     const bool q_ok = qi < q_len;
     const int p = start + qi;                             // its position
     const int p_first = start + q0;
@@ -100,23 +112,14 @@ prefill_attention_kernel(const bf16_t* __restrict__ q, int q_stride, int q_col,
     auto tile_of = [&](int vt) { return vt < n_head ? vt : vt - n_head + kt_first; };
     // (shaped scores are in base 2 already when they meet the exponent)
     const float sl = SHAPED ? 1.f : scale_log2e;
-    // The sequence's block table goes to LDS first: the gathers below then depend on an LDS read,
-    // not on a global load that would have to be waited for in front of every key load.
-    // (The host passes page sizes that are powers of two and tables of at most PF_TABLE_LDS blocks.)
-    const int* gtable = block_tables + static_cast<size_t>(b) * max_blocks;
-    const int shift = __ffs(page_size) - 1;
+    const int shift = __ffs(page_size) - 1;       // (page sizes are powers of two)
     const int n_blocks_needed = (p_last >> shift) + 1;
-    for (int i = tid; i < n_blocks_needed; i += NTH) sm_table[i] = gtable[i];
-    __syncthreads();
+    if (tid < max_blocks) sm_table[tid] = entry;
+    for (int i = tid + NTH; i < n_blocks_needed; i += NTH) sm_table[i] = gtable[i];
+    lds_barrier();        // (the queries stay in flight)
     auto page_row = [&](int j) -> size_t {
         return (static_cast<size_t>(sm_table[j >> shift]) << shift) + (j & (page_size - 1));
     };
-
-    Frag8 qf[KS];
-#pragma unroll
-    for (int ks = 0; ks < KS; ++ks)      // a lane beyond the last query takes that query again; its scores are masked
-        qf[ks].q = *reinterpret_cast<const uint4*>(q + static_cast<size_t>(q_begin + min(qi, q_len - 1)) * q_stride +
-                                                   q_col + h * DH + 32 * ks + 8 * G);
 
     float m = -INFINITY, l = 0.f;
     f32x4 o[DT];
@@ -406,8 +409,8 @@ int mllm_prefill_attention_bf16(const void* q, int q_stride, int q_col, const vo
             lds_allowed = true;                                                                             \
         }                                                                                                   \
         prefill_attention_kernel<D, W, S, L><<<grid, W * 64, table_bytes, stream>>>(                           \
-            (const bf16_t*)q, q_stride, q_col, (const bf16_t*)k_pages, (const bf16_t*)v_pages, kv_dim,      \
-            block_tables, max_blocks, cu_q, ctx_len, n_seqs, n_heads, n_kv_heads, page_size, sl2, window,   \
+            cu_q, ctx_len, block_tables, (const bf16_t*)q + q_col, n_seqs, n_tiles_upper, max_blocks, q_stride, (const bf16_t*)k_pages, \
+            (const bf16_t*)v_pages, kv_dim, n_heads, n_kv_heads, page_size, sl2, window,                    \
             (bf16_t*)out, out_stride, sh, scale, gate, ldg);                                                \
     } while (0)
     const bool longest = longest_first(n_seqs, 4, static_cast<long long>(n_heads) * n_tiles_upper);

@@ -138,14 +138,18 @@ __device__ __forceinline__ void store4(void* C, size_t idx, const float (&v)[4],
 
 template <int WM, int WN, int TM, int TN, int BK, int STAGES, int KG, bool HALVES, bool FAR, bool EDGE, int MODE>
 __global__ void __launch_bounds__(WM * WN * KG * 64)
-gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__ W, int ldw,
-               const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K,
-               int tiles_m, int tiles_n, int xm, int xn, typename TiledExtra<MODE>::type kv) {
+gemm_bf16_mfma(// The first 14 dwords arrive in registers with the wavefront: all that the first tiles' loads need. (K, the tile counts and their split
+               // among the XCDs lay behind them and came from memory, 0.7 us in front of the first load.)
+               const bf16_t* __restrict__ A, const bf16_t* __restrict__ W,
+               const void* __restrict__ bias_or_up,        // (EPI_GATED: the second map)
+               int lda, int ldw, int M, int N, int K, int xm_bits,
+               void* __restrict__ C, int ldc, typename TiledExtra<MODE>::type kv) {
     // EPI_GATED: of a wavefront's TN column sub-tiles the even ones are the gate's and the odd ones the same 32 columns of the up
     // map, so that both values of an output lie in one register of one lane; N and the tile's columns count outputs.
     constexpr bool GATED = MODE == EPI_GATED, F32_OUT = MODE == EPI_ADD_RESIDUAL || MODE == EPI_STORE_F32 || MODE == EPI_THROUGH;
     static_assert(!GATED || TN % 2 == 0, "a wavefront holds whole pairs of sub-tiles");
     constexpr int PAIR = GATED ? 2 : 1;
+    const float* bias = GATED ? nullptr : static_cast<const float*>(bias_or_up);
     // KG groups of WM x WN wavefronts share the tile: group g multiplies the g-th part of every k tile; their sums meet in LDS.
     constexpr int NW = WM * WN * KG, BM = WM * TM * 32, BN = WN * TN * 32, ROWS = BM + BN;
     constexpr int ROW_BYTES = BK * 2, PIECES = BK / 8;         // 16-byte pieces of a row of the k tile
@@ -178,8 +182,11 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
     // tiles of one XCD (workgroup id % 8) form one compact rectangle of the output: the rows of A
     // and W it needs then fit in its L2 instead of every XCD streaming both matrices.
     const int xcd = blockIdx.x % N_XCD, local = blockIdx.x / N_XCD;
-    const int rect_m = (tiles_m + xm - 1) / xm, rect_n = (tiles_n + xn - 1) / xn;
-    const int tm = (xcd / xn) * rect_m + local / rect_n, tn = (xcd % xn) * rect_n + local % rect_n;
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN / PAIR - 1) / (BN / PAIR);
+    const int xn_bits = 3 - xm_bits;           // (8 XCDs)
+    const int rect_m = (tiles_m + (1 << xm_bits) - 1) >> xm_bits, rect_n = (tiles_n + (1 << xn_bits) - 1) >> xn_bits;
+    const int down = uniform_quotient(local, rect_n);
+    const int tm = (xcd >> xn_bits) * rect_m + down, tn = (xcd & ((1 << xn_bits) - 1)) * rect_n + local - down * rect_n;
     if (local >= rect_m * rect_n || tm >= tiles_m || tn >= tiles_n) return;      // padding of the grid
     const int m0 = tm * BM, n0 = tn * (BN / PAIR);
 
@@ -200,7 +207,7 @@ gemm_bf16_mfma(const bf16_t* __restrict__ A, int lda, const bf16_t* __restrict__
         } else {
             const int w_row = row - BM, n = GATED ? w_row / 64 * 32 + w_row % 32 : w_row;
             const bf16_t* map = W;
-            if constexpr (GATED) map = (first - BM) / 32 % 2 ? kv.up : W;
+            if constexpr (GATED) map = (first - BM) / 32 % 2 ? static_cast<const bf16_t*>(bias_or_up) : W;
             base[q] = reinterpret_cast<const unsigned char*>(map + static_cast<size_t>(n0) * ldw);
             offset[q] = static_cast<Offset>(min(n, N - 1 - n0)) * ldw * 2;
         }
@@ -489,7 +496,7 @@ static void launch_tiled_gated(const bf16_t* a, int lda, const bf16_t* w, int ld
     const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN / 2 - 1) / (BN / 2);
     int xm, xn;
     const dim3 grid(split_among_xcds(tiles_m, tiles_n, BM, BN, xm, xn)), block(WM * WN * KG * 64);
-#define TILED(E) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, FAR, E, EPI_GATED><<<grid, block, 0, stream>>>(a, lda, w, ldw, nullptr, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, pair)
+#define TILED(E) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, FAR, E, EPI_GATED><<<grid, block, 0, stream>>>(a, w, pair.up, lda, ldw, M, N, K, __builtin_ctz(xm), C, ldc, pair)
     if (FAR || K % BK != 0) TILED(true); else if constexpr (!FAR) TILED(false);
 #undef TILED
 }
@@ -503,7 +510,7 @@ static void launch_tiled(const bf16_t* a, int lda, const bf16_t* w, int ldw, con
     int xm, xn;
     const dim3 grid(split_among_xcds(tiles_m, tiles_n, BM, BN, xm, xn)), block(WM * WN * KG * 64);
     const bool edge = FAR || K % BK != 0;      // rows and columns beyond the matrices need no other kernel
-#define TILED(E, MD) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, FAR, E, MD><<<grid, block, 0, stream>>>(a, lda, w, ldw, bias, C, ldc, M, N, K, tiles_m, tiles_n, xm, xn, extra)
+#define TILED(E, MD) gemm_bf16_mfma<WM, WN, TM, TN, BK, STAGES, KG, HALVES, FAR, E, MD><<<grid, block, 0, stream>>>(a, w, bias, lda, ldw, M, N, K, __builtin_ctz(xm), C, ldc, extra)
     if (mode == EPI_THROUGH) {
         const MllmStreamAdd extra = *through;
         if (edge) TILED(true, EPI_THROUGH); else if constexpr (!FAR) TILED(false, EPI_THROUGH);
@@ -792,12 +799,11 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
         for (int i = 0; i < 4; ++i) pk.w[i] = pack_bf16x2(o[2 * i] * inv, o[2 * i + 1] * inv);
         return pk.v;
     };
-    // blocks of this wavefront: those behind its first, divided by the wavefronts on the tile. (In floating point: of whole numbers up to
-    // 2^14 and at most 96 a half more lies further from the next quotient than the reciprocal errs; an integer division takes 40 instructions.)
+    // blocks of this wavefront: those behind its first, divided by the wavefronts on the tile
     int n_blocks = (K + 63) / 64;
     if (SPLIT_K) {
-        const int takers = nw * k_parts, from = n_blocks - 1 - (part * nw + wave);
-        n_blocks = from < 0 ? 0 : 1 + __builtin_amdgcn_readfirstlane(static_cast<int>((static_cast<float>(from) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(takers))));
+        const int from = n_blocks - 1 - (part * nw + wave);
+        n_blocks = from < 0 ? 0 : 1 + small_quotient(from, nw * k_parts);
     }
     const int n_chunks = n_blocks / H;
     struct Chunk {

@@ -1094,6 +1094,18 @@ def test_paged_attention_gives_every_tile_away(ops, dtype, seqs, H, Hkv, dh):
     assert (out - ref).abs().max() <= _tol(dtype, 2)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("dh", [16, 32, 64, 128, 256])
+@pytest.mark.parametrize("waves", [1, 2, 3, 4, 5, 8, 9, 12, 13, 16])
+@pytest.mark.parametrize("nsplit", [1, 3])
+def test_decode_attention_merges_every_number_of_wavefronts(ops, monkeypatch, dtype, dh, waves, nsplit):
+    """The states of lane groups, wavefronts and splits, with wavefronts that have keys and some that have none."""
+    g = torch.Generator().manual_seed(waves * 3 + dh)
+    monkeypatch.setattr(ops, "DECODE_SHAPE_OVERRIDE", (nsplit, waves))
+    out, ref = _attention_case(ops, dtype, 6, 2, dh, 16, [(0, 1), (40, 1), (700, 1), (1500, 1)], 0, g)
+    assert (out - ref).abs().max() <= _tol(dtype, 2)
+
+
 @pytest.mark.parametrize("seqs", [[(0, 1)], [(5000, 70), (0, 300)], [(0, 300), (5000, 70)], [(4200, 130), (0, 1), (64, 64), (63, 65), (10, 129)],
                                   [(0, 512)] * 4, [(i % 3 * 64, 1 + 37 * i % 140) for i in range(64)], [(i * 977 % 90000, i % 5 * 33) for i in range(64)],
                                   [(0, 1 + i % 67) for i in range(65)]])
