@@ -10,8 +10,9 @@
 // sampled on the device and the host has not read yet; ids[t] is not read then. With `copy` the row is stored there once
 // more in bfloat16, behind the norm `next` if it has a weight.
 // ---------------------------------------------------------------------------
+#define EMBED_THREADS 256
 template <typename T>
-__global__ void embed_kernel(const int* __restrict__ ids, const int* __restrict__ pos,
+__global__ void __launch_bounds__(EMBED_THREADS) embed_kernel(const int* __restrict__ ids, const int* __restrict__ pos,
                              const T* __restrict__ wte, const T* __restrict__ wpe,
                              float* __restrict__ x, int D, const int* __restrict__ src,
                              const int* __restrict__ prev, int n_prev, float scale, bf16_t* __restrict__ copy, MllmTanhNorm next) {
@@ -25,13 +26,13 @@ __global__ void embed_kernel(const int* __restrict__ ids, const int* __restrict_
     float* xr = x + static_cast<size_t>(t) * D;
     if (wpe != nullptr) {
         const T* pe = wpe + static_cast<size_t>(pos[t]) * D;
-        for (int d = threadIdx.x; d < D; d += blockDim.x) {
+        for (int d = threadIdx.x; d < D; d += EMBED_THREADS) {
             const float v = to_float(te[d]) * scale + to_float(pe[d]);
             xr[d] = v;
             if (copy) copy[static_cast<size_t>(t) * D + d] = float_to_bf16(next.weight != nullptr ? fast_tanh(next.alpha[0] * v) * next.weight[d] + next.bias[d] : v);
         }
     } else {
-        for (int d = threadIdx.x; d < D; d += blockDim.x) {
+        for (int d = threadIdx.x; d < D; d += EMBED_THREADS) {
             const float v = to_float(te[d]) * scale;
             xr[d] = v;
             if (copy) copy[static_cast<size_t>(t) * D + d] = float_to_bf16(next.weight != nullptr ? fast_tanh(next.alpha[0] * v) * next.weight[d] + next.bias[d] : v);
@@ -113,7 +114,8 @@ __global__ void layernorm_kernel(const float* __restrict__ x, const int* __restr
 
 // Same norm, one wavefront per row (WAVES rows per workgroup), the row in registers as float4:
 // for D % 4 == 0 and D <= 2048. Fewer, fatter workgroups and 16-byte accesses.
-template <typename OutT, int WAVES>
+// NU: float4 of a row per lane, so that nothing but the last is asked whether it exists.
+template <typename OutT, int WAVES, int NU>
 __global__ void __launch_bounds__(64 * WAVES)
 layernorm_wave_kernel(const float* __restrict__ x, const int* __restrict__ rows,
                       const float* __restrict__ gamma, const float* __restrict__ beta,
@@ -125,32 +127,33 @@ layernorm_wave_kernel(const float* __restrict__ x, const int* __restrict__ rows,
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MLLM_WAVE), lane = threadIdx.x % MLLM_WAVE;
     const int r = blockIdx.x * WAVES + wave;
     if (r >= n) return;
-    const int src = rows ? rows[r] : r;
+    int src = r;
+    if (rows != nullptr) {
+        src = rows[r];
+        asm volatile("" : "+s"(src));       // waited for in here, not where the launches without a gather pass too
+    }
     const float4* xr = reinterpret_cast<const float4*>(x + static_cast<size_t>(src) * D);
     const float4* g4 = reinterpret_cast<const float4*>(gamma);
     const float4* b4 = reinterpret_cast<const float4*>(beta ? beta : gamma);
-    const int nq = D / 4, n_u = (nq + 63) / 64;
-    float4 v[8], gg[8], bb[8];
+    const int nq = D / 4;
+    float4 v[NU], gg[NU], bb[NU];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u) v[u] = xr[min(lane + 64 * u, nq - 1)];
+    for (int u = 0; u < NU; ++u) v[u] = xr[u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        if (u < n_u) {
-            const int i = min(lane + 64 * u, nq - 1);
-            gg[u] = g4[i];
-            bb[u] = b4[i];
-        }
+    for (int u = 0; u < NU; ++u) {
+        const int i = u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1);
+        gg[u] = g4[i];
+        bb[u] = b4[i];
     }
     float s = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u && lane + 64 * u < nq) s += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+    for (int u = 0; u < NU; ++u)
+        if (u < NU - 1 || lane + 64 * u < nq) s += (v[u].x + v[u].y) + (v[u].z + v[u].w);
     const float mean = wave_sum(s) / static_cast<float>(D);
     float q = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
-        if (u < n_u && lane + 64 * u < nq) {
+    for (int u = 0; u < NU; ++u) {
+        if (u < NU - 1 || lane + 64 * u < nq) {
             const float a = v[u].x - mean, b = v[u].y - mean, c = v[u].z - mean, d = v[u].w - mean;
             q += (a * a + b * b) + (c * c + d * d);
         }
@@ -158,9 +161,9 @@ layernorm_wave_kernel(const float* __restrict__ x, const int* __restrict__ rows,
     const float inv = 1.0f / sqrtf(wave_sum(q) / static_cast<float>(D) + eps);
     OutT* yr = y + static_cast<size_t>(r) * D;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < NU; ++u) {
         const int i = lane + 64 * u;
-        if (u < n_u && i < nq) {
+        if (u < NU - 1 || i < nq) {
             const float4 g = gg[u];
             const float4 b = beta ? bb[u] : make_float4(0.f, 0.f, 0.f, 0.f);
             const float o0 = (v[u].x - mean) * inv * g.x + b.x, o1 = (v[u].y - mean) * inv * g.y + b.y;
@@ -271,9 +274,9 @@ int mllm_embed(const int* ids, const int* pos, const void* wte, const void* wpe,
     if (T <= 0) return 0;
     bf16_t* copy = static_cast<bf16_t*>(copy_bf16);
     if (dtype == MLLM_F32)
-        embed_kernel<float><<<T, 256, 0, stream>>>(ids, pos, (const float*)wte, (const float*)wpe, x, D, src, prev, n_prev, scale, copy, next);
+        embed_kernel<float><<<T, EMBED_THREADS, 0, stream>>>(ids, pos, (const float*)wte, (const float*)wpe, x, D, src, prev, n_prev, scale, copy, next);
     else
-        embed_kernel<bf16_t><<<T, 256, 0, stream>>>(ids, pos, (const bf16_t*)wte, (const bf16_t*)wpe, x, D, src, prev, n_prev, scale, copy, next);
+        embed_kernel<bf16_t><<<T, EMBED_THREADS, 0, stream>>>(ids, pos, (const bf16_t*)wte, (const bf16_t*)wpe, x, D, src, prev, n_prev, scale, copy, next);
     MLLM_LAUNCH_CHECK();
     return 0;
 }
@@ -316,19 +319,15 @@ int mllm_layernorm(const float* x, const int* rows, const float* gamma, const fl
     if (D % 4 == 0 && D <= 2048 && aligned) {
         // Workgroups start at a limited rate (about 200 a microsecond over the chip): many rows go eight to a
         // workgroup instead of four (2,048 rows of 768: 6.9 us with 512 workgroups of four)
-        if (n >= 512) {
-            const int blocks = (n + 7) / 8;
-            if (out_dtype == MLLM_F32)
-                layernorm_wave_kernel<float, 8><<<blocks, 512, 0, stream>>>(x, rows, gamma, beta, (float*)y, n, D, eps);
-            else
-                layernorm_wave_kernel<bf16_t, 8><<<blocks, 512, 0, stream>>>(x, rows, gamma, beta, (bf16_t*)y, n, D, eps);
-        } else {
-            const int blocks = (n + 3) / 4;
-            if (out_dtype == MLLM_F32)
-                layernorm_wave_kernel<float, 4><<<blocks, 256, 0, stream>>>(x, rows, gamma, beta, (float*)y, n, D, eps);
-            else
-                layernorm_wave_kernel<bf16_t, 4><<<blocks, 256, 0, stream>>>(x, rows, gamma, beta, (bf16_t*)y, n, D, eps);
-        }
+#define LN_LAUNCH(OUT, WAVES, NU) layernorm_wave_kernel<OUT, WAVES, NU><<<(n + WAVES - 1) / WAVES, 64 * WAVES, 0, stream>>>(x, rows, gamma, beta, (OUT*)y, n, D, eps)
+#define LN_CASE(NU)                                                                                     \
+    case NU:                                                                                            \
+        if (n >= 512) { if (out_dtype == MLLM_F32) LN_LAUNCH(float, 8, NU); else LN_LAUNCH(bf16_t, 8, NU); } \
+        else if (out_dtype == MLLM_F32) LN_LAUNCH(float, 4, NU); else LN_LAUNCH(bf16_t, 4, NU);        \
+        break;
+        switch ((D + 255) / 256) { LN_CASE(1) LN_CASE(2) LN_CASE(3) LN_CASE(4) LN_CASE(5) LN_CASE(6) LN_CASE(7) LN_CASE(8) }
+#undef LN_CASE
+#undef LN_LAUNCH
         MLLM_LAUNCH_CHECK();
         return 0;
     }

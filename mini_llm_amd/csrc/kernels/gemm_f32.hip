@@ -95,13 +95,15 @@ gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ 
 
 template <int ROWS, int WAVES>
 __global__ void __launch_bounds__(64 * WAVES)
-gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-                     const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K, int mode) {
+gemm_f32_rows_kernel(// (the first 14 dwords arrive in registers with the wavefront, the rest comes from memory, 0.6 to 0.8 us later)
+                     const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias, void* __restrict__ C,
+                     int lda, int ldw, int ldc, int M, int N, int K, int mode) {
     __shared__ __attribute__((aligned(16))) float a_s[ROWS][F32R_KC];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid / 64), lane = tid % 64;
     const int n = blockIdx.x * WAVES + wave;
     const float* wrow = W + static_cast<size_t>(min(n, N - 1)) * ldw;       // a surplus wavefront repeats the last column
     constexpr int STAGED = (ROWS * (F32R_KC / 4) + 64 * WAVES - 1) / (64 * WAVES);   // 16-byte steps of a chunk a thread stages
+    static_assert(WAVES % 2 == 0 && F32R_KC == 512, "two wavefronts a staged row");
     float acc[ROWS];
 #pragma unroll
     for (int r = 0; r < ROWS; ++r) acc[r] = 0.f;
@@ -110,17 +112,21 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
     // A chunk is at most two 16-byte steps per lane (the second from a clamped address; its product is
     // left out where it is past the chunk).
     const int q0 = lane, q1 = lane + 64;
-    float4 w0, w1, v[STAGED];
+    typedef float f4 __attribute__((ext_vector_type(4)));        // (float4s that are set under a condition would go through scratch memory)
+    float4 w0, w1;
+    f4 v[STAGED];
+    // (a chunk's rows lie 128 steps apart, so that no step is found by a division; a row belongs to whole wavefronts, and rows beyond M
+    // are neither read nor set: what stands in their place counts in no result that is stored)
+    constexpr int PASS_ROWS = 64 * WAVES / 128;
+    const int my_q = tid % 128, first_r = wave / 2;
     auto fetch = [&](int kc0) {
         const int quads = min(F32R_KC, K - kc0) / 4;
         w0 = *reinterpret_cast<const float4*>(wrow + kc0 + 4 * min(q0, quads - 1));
         w1 = *reinterpret_cast<const float4*>(wrow + kc0 + 4 * min(q1, quads - 1));
 #pragma unroll
         for (int u = 0; u < STAGED; ++u) {
-            const int idx = tid + 64 * WAVES * u, r = idx / quads, q = idx % quads;
-            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (idx < ROWS * quads && r < M)
-                v[u] = *reinterpret_cast<const float4*>(A + static_cast<size_t>(r) * lda + kc0 + 4 * q);
+            const int r = first_r + u * PASS_ROWS;
+            if (r < M) v[u] = *reinterpret_cast<const f4*>(A + static_cast<size_t>(r) * lda + kc0 + 4 * min(my_q, quads - 1));
         }
     };
     fetch(0);
@@ -130,8 +136,8 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
         __syncthreads();          // the chunk before has been read
 #pragma unroll
         for (int u = 0; u < STAGED; ++u) {
-            const int idx = tid + 64 * WAVES * u, r = idx / quads, q = idx % quads;
-            if (idx < ROWS * quads) *reinterpret_cast<float4*>(&a_s[r][4 * q]) = v[u];
+            const int r = first_r + u * PASS_ROWS;
+            if (r < M) *reinterpret_cast<f4*>(&a_s[r][4 * my_q]) = v[u];
         }
         if (kc0 + F32R_KC < K) fetch(kc0 + F32R_KC);
         __syncthreads();
@@ -175,8 +181,10 @@ gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restri
 // RAGGED: K is no multiple of 256, and what lies beyond it has to be left out (8 x 1,600 x 1,600 7.4 us, 7.2 if it were not).
 template <int ROWS, int STEPS, bool RAGGED>
 __global__ void __launch_bounds__(512)
-gemm_f32_narrow_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
-                       const float* __restrict__ bias, void* __restrict__ C, int ldc, int M, int N, int K, int mode) {
+gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers; rows in the lower half of the last, the epilogue in the upper)
+                       const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias, void* __restrict__ C,
+                       int lda, int ldw, int ldc, int N, int K, int M_mode) {
+    const int M = M_mode & 0xffff, mode = M_mode >> 16;
     constexpr int COLS = 4, KP = 512 * STEPS, STAGED = ROWS * KP / 4 / 512;
     static_assert(COLS * ROWS <= 64, "the first wavefront holds the outputs");
     __shared__ __attribute__((aligned(16))) float a_s[ROWS][KP];
@@ -264,8 +272,8 @@ gemm_f32_narrow_kernel(const float* __restrict__ A, int lda, const float* __rest
 template <int ROWS, int STEPS>
 static void launch_f32_narrow(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
     const dim3 grid((N + 3) / 4);
-    if (K % 256 != 0) gemm_f32_narrow_kernel<ROWS, STEPS, true><<<grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
-    else gemm_f32_narrow_kernel<ROWS, STEPS, false><<<grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+    if (K % 256 != 0) gemm_f32_narrow_kernel<ROWS, STEPS, true><<<grid, 512, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, N, K, M | mode << 16);
+    else gemm_f32_narrow_kernel<ROWS, STEPS, false><<<grid, 512, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, N, K, M | mode << 16);
 }
 
 // More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). WM x WN
@@ -294,8 +302,9 @@ typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 template <int WM, int WN, int TM, int TN, int KG, int PARTS, int STAGES, int SUMS, bool EDGE>
 __global__ void __launch_bounds__(WM * WN * KG * 64)
-gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw, const float* __restrict__ bias,
-                      void* __restrict__ C, int ldc, int M, int N, int K, int mode, int tiles_m, int tiles_n, int down) {
+gemm_f32_tiles_kernel(// (all that the first tiles' loads need is among the 14 dwords that arrive in registers)
+                      const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias, void* __restrict__ C,
+                      int lda, int ldw, int M, int N, int K, int ldc, int mode) {
     constexpr int NW = WM * WN, BM = WM * TM * 16, BN = WN * TN * 16, ROWS = BM + BN, BK = F32T_BK * KG, KS = F32T_BK / 16;
     constexpr int LOADS = (ROWS / 8 + NW - 1) / NW; // of a wavefront and k tile: 8 rows of its group's 32 columns each (the last again where there are fewer)
     constexpr int SLAB_BYTES = ROWS * F32T_BK * 4, STAGE_BYTES = SLAB_BYTES * KG;
@@ -306,9 +315,12 @@ gemm_f32_tiles_kernel(const float* __restrict__ A, int lda, const float* __restr
     const int kg = __builtin_amdgcn_readfirstlane(tid / (64 * NW)), wave = __builtin_amdgcn_readfirstlane(tid / 64 % NW);
     // an XCD (workgroup id % 8) takes an even share of the tiles, neighbours in one direction: with `down` it walks down the
     // rows of A for a few columns of tiles, else along the rows of W for a few rows of tiles
+    const int tiles_m = (M + BM - 1) / BM, tiles_n = (N + BN - 1) / BN;
+    const bool down = M <= N;
     const int tiles = tiles_m * tiles_n, per = (tiles + 7) / 8, at = (blockIdx.x % 8) * per + blockIdx.x / 8;
-    if (blockIdx.x / 8 >= per || at >= tiles) return;
-    const int tm = down ? at % tiles_m : at / tiles_n, tn = down ? at / tiles_m : at % tiles_n;
+    if (static_cast<int>(blockIdx.x / 8) >= per || at >= tiles) return;
+    const int side = down ? tiles_m : tiles_n, over = uniform_quotient(at, side), within = at - over * side;
+    const int tm = down ? within : over, tn = down ? over : within;
     const int m0 = tm * BM, n0 = tn * BN;
 
     // A group's 32 columns of a k tile in LDS are its rows one behind the other (A's, then W's), as the loads leave them. 16-byte piece
@@ -533,9 +545,9 @@ static void launch_f32_tiles(const float* A, int lda, const float* W, int ldw, c
     const int tiles_m = (M + 16 * WM * TM - 1) / (16 * WM * TM), tiles_n = (N + 16 * WN * TN - 1) / (16 * WN * TN);
     const dim3 grid((tiles_m * tiles_n + 7) / 8 * 8), block(64 * WM * WN * KG);
     if (K % (F32T_BK * KG) != 0)
-        gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, true><<<grid, block, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n, M > N ? 0 : 1);
+        gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, true><<<grid, block, 0, stream>>>(A, W, bias, C, lda, ldw, M, N, K, ldc, mode);
     else
-        gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, false><<<grid, block, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, tiles_m, tiles_n, M > N ? 0 : 1);
+        gemm_f32_tiles_kernel<WM, WN, TM, TN, KG, PARTS, STAGES, SUMS, false><<<grid, block, 0, stream>>>(A, W, bias, C, lda, ldw, M, N, K, ldc, mode);
 }
 
 // Which tiles: 32 x 32 with four groups, two groups of two parts or one group of two parts; 64 x 32 in two parts; 128 x 64 in one.
@@ -619,12 +631,12 @@ int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float*
         // 50,257 columns 54 us against 45).
         if (N >= 2048) {
             const dim3 rows_grid((N + 7) / 8);
-            if (M <= 8) gemm_f32_rows_kernel<8, 8><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
-            else gemm_f32_rows_kernel<16, 8><<<rows_grid, 512, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            if (M <= 8) gemm_f32_rows_kernel<8, 8><<<rows_grid, 512, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, M, N, K, mode);
+            else gemm_f32_rows_kernel<16, 8><<<rows_grid, 512, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, M, N, K, mode);
         } else {
             // (3,072 columns a pass take the LDS of a unit: while there is one workgroup a unit; 9 to 16 rows would take twice as much)
             const dim3 rows_grid((N + 3) / 4);
-            if (M > 8) gemm_f32_rows_kernel<16, 4><<<rows_grid, 256, 0, stream>>>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode);
+            if (M > 8) gemm_f32_rows_kernel<16, 4><<<rows_grid, 256, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, M, N, K, mode);
             else if (K <= 1024) launch_f32_narrow<8, 2>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
             else if (N <= 1024) launch_f32_narrow<8, 6>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
             else launch_f32_narrow<8, 3>(A, lda, W, ldw, bias, C, ldc, M, N, K, mode, stream);
