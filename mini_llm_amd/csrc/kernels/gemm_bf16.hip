@@ -573,7 +573,7 @@ template <int MS> struct SplitStates {
 };
 
 template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false, int MS = MERGE_MAX_SPLITS,
-          bool ONE = false, bool GATED = false, int NU = 8, int WC = 16>
+          bool ONE = false, bool GATED = false, int NU = 8, int WC = 16, int KP = 1>
 __global__ void __launch_bounds__(ASRC == A_NORMED ? 512 : (ASRC == A_GLOBAL || ASRC == A_MERGED ? 768 : 1024))
 gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, and hold everything that the first loads need: an argument
                  // behind them comes with a load of its own from memory that no cache holds (as does blockDim), 0.6 to 0.8 us
@@ -601,6 +601,9 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     // GATED: the two tiles are the same 16 columns of the gate's map and of the up map, and one value leaves for both.
     static_assert(!GATED || (NT == 2 && ASRC == A_NORMED), "gated pairs: two tiles behind the norm");
     static_assert(NT == 1 || (MT == 1 && SPLIT_K), "column tiles per workgroup: split-K kernels of one row tile");
+    // KP == 2: the two parts of K that two workgroups would take, one behind the other in every wavefront, with sums of their own that
+    // are added at the end as the workgroups' would be: the same bits without the exchange through memory (the launcher's k_parts).
+    static_assert(KP == 1 || (KP == 2 && ONE && SPLIT_K && MT == 1 && NT == 1 && ASRC == A_GLOBAL), "parts of K in one workgroup: kernels of one chunk");
     constexpr int T = MT * NT;      // accumulators: row tiles (NT == 1) or column tiles (MT == 1)
     constexpr int REDUCED = ASRC == A_NORMED ? 8 : 12;      // wavefronts whose sums meet, at most (SPLIT_K)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -647,7 +650,7 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     const int part = SPLIT_K ? blockIdx.y : 0;
     const int k_first = SPLIT_K ? (part * nw + wave) * 64 : 0;      // first k block of this wavefront
     const int k_stride = SPLIT_K ? nw * k_parts * 64 : 64;         // distance between its k blocks
-    const size_t red_bytes = SPLIT_K ? static_cast<size_t>(nw) * T * 256 * sizeof(float) : 0;
+    const size_t red_bytes = SPLIT_K ? static_cast<size_t>(nw) * T * KP * 256 * sizeof(float) : 0;
     // per wavefront: SB k blocks at a time change lanes through LDS, each NT weight tiles (+ the A block)
     constexpr int SB = (ASRC == A_STAGED || (A_REGS && NT > 1) || U < 4) ? 1 : 2;
     constexpr int STAGE_BYTES = SB * (NT * 2048 + (A_REGS ? 2048 : 0));
@@ -986,19 +989,28 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     // norm that follows registers that count as pending on one side of the branch, and it would
     // wait for the weights.)
     const int last_block = n_blocks > 0 ? n_blocks - 1 : 0;
+    int n_second = 0, k_second = 0;             // (KP == 2: this wavefront's blocks of the second part)
+    if (KP == 2) {
+        const int from = (K + 63) / 64 - 1 - (nw + wave);
+        n_second = from < 0 ? 0 : 1 + small_quotient(from, nw * KP);
+        k_second = (nw + wave) * 64;
+    }
     auto first_loads = [&]() {
         if (ASRC == A_MERGED) {
 #pragma unroll
             for (int h = 0; h < H; ++h) fetch_block_splits(h, k_first + min(h, last_block) * k_stride);
             __builtin_amdgcn_sched_barrier(0);
         }
-        auto k_of = [&](int h) { return k_first + min(h, last_block) * k_stride; };
-        load_rows(c0, H, k_of);
-        if (WC == 4) load_pairs(c0, k_of);
-        else
+        auto ask = [&](Chunk& c, auto k_of) {
+            load_rows(c, H, k_of);
+            if (WC == 4) load_pairs(c, k_of);
+            else
 #pragma unroll
-            for (int h = 0; h < H; ++h) load_steps(c0, 2 * h, k_of(h));
-        __builtin_amdgcn_sched_barrier(0);
+                for (int h = 0; h < H; ++h) load_steps(c, 2 * h, k_of(h));
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        ask(c0, [&](int h) { return k_first + min(h, last_block) * k_stride; });
+        if (KP == 2) ask(c1, [&](int h) { return k_second + min(h, max(n_second - 1, 0)) * k_stride; });
         if (ASRC == A_MERGED) {
 #pragma unroll
             for (int h = 0; h < H; ++h) merge_block_splits(c0, h);
@@ -1113,7 +1125,13 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     // ONE: the launcher knows that a chunk holds all of a wavefront's blocks, and a second one takes no registers. (With it the
     // kernels of four blocks a wavefront, and those that merge splits, kept 76 to 1,220 bytes a lane in scratch memory.)
     constexpr bool SINGLE = ONE || ASRC == A_MERGED;
-    if (n_chunks == 0) {
+    f32x4 of_first = {0.f, 0.f, 0.f, 0.f};      // (KP == 2: the first part's sums)
+    if constexpr (KP == 2) {
+        mma_some(c0, n_blocks, k_first);
+        of_first = acc[0];
+        acc[0] = f32x4{0.f, 0.f, 0.f, 0.f};
+        mma_some(c1, n_second, k_second);
+    } else if (n_chunks == 0) {
         mma_some(c0, n_blocks, k_first);
     } else if (SINGLE || n_chunks == 1) {
         mma_chunk(c0, 0);
@@ -1152,7 +1170,10 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
 #pragma unroll
     for (int i = 0; i < T; ++i)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) red[(static_cast<size_t>(wave) * T + i) * 256 + r * 64 + lane] = acc[i][r];
+        for (int r = 0; r < 4; ++r) red[(static_cast<size_t>(wave) * T * KP + i) * 256 + r * 64 + lane] = KP == 2 ? of_first[r] : acc[i][r];
+    if (KP == 2)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[(wave * KP + 1) * 256 + r * 64 + lane] = acc[0][r];
     __syncthreads();
     if (MT == 1) {
         // one output per tile and thread (the first 256); its bias and old residual value were
@@ -1162,17 +1183,24 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
         for (int t = 0; t < NT; ++t) {
             vt[t] = 0.f;
             if (wave < 4) {
-                // (all reads at once, then the sum in the order of the wavefronts)
-                float of_wave[REDUCED];
+                // (all reads at once, then the sum in the order of the wavefronts; parts one by one)
+                float of_wave[KP][REDUCED];
 #pragma unroll
-                for (int w = 0; w < REDUCED; ++w) of_wave[w] = red[(min(w, nw - 1) * NT + t) * 256 + tid];
+                for (int p = 0; p < KP; ++p)
 #pragma unroll
-                for (int w = 0; w < REDUCED; ++w)
-                    if (w < nw) vt[t] += of_wave[w];
+                    for (int w = 0; w < REDUCED; ++w) of_wave[p][w] = red[(min(w, nw - 1) * NT * KP + t + p) * 256 + tid];
+#pragma unroll
+                for (int p = 0; p < KP; ++p) {
+                    float sum = 0.f;
+#pragma unroll
+                    for (int w = 0; w < REDUCED; ++w)
+                        if (w < nw) sum += of_wave[p][w];
+                    vt[t] = p == 0 ? sum : vt[t] + sum;
+                }
             }
         }
         float& v = vt[0];
-        if (NT == 1 && k_parts > 1) {
+        if (NT == 1 && KP == 1 && k_parts > 1) {
             // The parts of a tile meet in the workspace. Stores and loads of it are at device scope
             // (workgroups of one tile may run on different XCDs, whose L2 caches do not see each
             // other's lines); one thread's fences order them around the counter (a fence in every
@@ -1304,6 +1332,10 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
             k_parts = 1;
         k_blocks = (k_blocks + k_parts - 1) / k_parts;      // per workgroup from here on
     }
+    // Two parts and at most 8 rows: one workgroup takes both, and the columns are dealt out to 256 workgroups (5 to 8 each) instead. What
+    // it saves is the exchange of the parts' sums (stores, fences, a counter: about 2 us). 1,600 x 6,400 7.9 > 6.5 us at 1 row, 8.7 > 7.5 at
+    // 8 (a chunk of five blocks with the exchange as it was: 7.6 and 8.4).
+    const bool parts_inside = k_parts == 2 && M <= 8 && (N + 255) / 256 <= 8 && (k_blocks + 11) / 12 <= 6;
     int* part_counters = static_cast<int*>(workspace);
     float* part_sums = reinterpret_cast<float*>(static_cast<char*>(workspace) + SPLIT_COUNTERS * sizeof(int));
     if (split_k) {
@@ -1349,7 +1381,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     // Fewer than 256 tiles, one row block and a long K (the second product of the feed-forward):
     // narrower tiles, down to 4 columns, so that more compute units share the weights. (Short K, or
     // the fused norm: the kernel's time is latency, not bytes, and nothing is gained; measured.)
-    if (split_k && !LN_FUSED && !MERGED && row_blocks == 1 && k_parts == 1 && tiles < 256 && k_blocks >= 48)
+    if (split_k && !LN_FUSED && !MERGED && row_blocks == 1 && (k_parts == 1 || parts_inside) && tiles < 256 && k_blocks >= (parts_inside ? 0 : 48))
         cols_per_wg = std::min(16, std::max((N + 255) / 256, 4));
     const int col_blocks = split_k ? (N + cols_per_wg - 1) / cols_per_wg : (tiles + nw - 1) / nw;
     // (what the words do not hold; K beyond 2^20: see the kernel's count of a wavefront's blocks)
@@ -1357,8 +1389,8 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     const unsigned shape = few_row_shape(M, cols_per_wg, k_parts, mode, nw, rms, kv.slots != nullptr, rows != nullptr);
     const unsigned columns = MERGED ? N | merged.head_dim / 8 << 14 | static_cast<unsigned>(merged.heads) << 23 : N;
     void* const strides = reinterpret_cast<void*>(static_cast<uintptr_t>(static_cast<unsigned>(lda)) | static_cast<uintptr_t>(static_cast<unsigned>(ldc)) << 32);
-    const dim3 grid((col_blocks + N_XCD - 1) / N_XCD * N_XCD * row_blocks, k_parts), block(nw * 64);
-    const size_t smem = lds_bytes(two_tiles);
+    const dim3 grid((col_blocks + N_XCD - 1) / N_XCD * N_XCD * row_blocks, parts_inside ? 1 : k_parts), block(nw * 64);
+    const size_t smem = lds_bytes(two_tiles) + (parts_inside ? static_cast<size_t>(nw) * 256 * sizeof(float) : 0);
     if (staged) {
         staged_bytes += smem;
 #define SKINNY_STAGED(MTV)                                                                             \
@@ -1389,9 +1421,10 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     const void* p2 = LN_FUSED ? gamma : MERGED ? merged.split_ml : bias;
     const void* p3 = LN_FUSED ? (gated != nullptr ? static_cast<const void*>(gated->up) : beta) : MERGED ? static_cast<const void*>(bias) : C;
 #define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...) SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, false, 8, 16, __VA_ARGS__)
-#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, ...)                        \
+#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, ...) SKINNY_PARTS(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, 1, __VA_ARGS__)
+#define SKINNY_PARTS(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, KPV, ...)                 \
     do {                                                                                               \
-        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV>;     \
+        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, KPV>; \
         static bool lds_allowed = false;      /* more than 64 KB of dynamic LDS has to be asked for once */ \
         if (!lds_allowed) {                                                                            \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                  \
@@ -1422,6 +1455,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
             if (per_wave <= 4) SKINNY_ANY(true, 8, false, 1, true, MERGE_MAX_SPLITS, true, false, 8, WCV, *through); \
             else SKINNY_ANY(true, 8, false, 1, true, MERGE_MAX_SPLITS, false, false, 8, WCV, *through); \
         } else if (per_wave <= 4) SKINNY_ANY(true, 8, false, 1, false, MERGE_MAX_SPLITS, true, false, 8, WCV, kv); \
+        else if (per_wave <= 6) SKINNY_ANY(true, 12, false, 1, false, MERGE_MAX_SPLITS, true, false, 8, WCV, kv); \
         else SKINNY_ANY(true, 8, false, 1, false, MERGE_MAX_SPLITS, false, false, 8, WCV, kv);          \
     } while (0)
     if (split_k) {
@@ -1484,6 +1518,16 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
                 case 3: SKINNY_LAUNCH(true, 6, false, 1, true); break;
                 default:
                     if constexpr (ASRC == A_GLOBAL) {
+                        if (parts_inside) {
+#define SKINNY_INSIDE(UV)                                                                              \
+    do {                                                                                               \
+        if (through != nullptr) SKINNY_PARTS(true, UV, false, 1, true, MERGE_MAX_SPLITS, true, false, 8, 8, 2, *through); \
+        else SKINNY_PARTS(true, UV, false, 1, false, MERGE_MAX_SPLITS, true, false, 8, 8, 2, kv);       \
+    } while (0)
+                            if (per_wave <= 4) SKINNY_INSIDE(8); else SKINNY_INSIDE(12);
+#undef SKINNY_INSIDE
+                            break;
+                        }
                         if (cols_per_wg <= 4) { SKINNY_NARROW(4); break; }
                         if (cols_per_wg <= 8) { SKINNY_NARROW(8); break; }
                     }
@@ -1507,6 +1551,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 #undef SKINNY_LAUNCH
 #undef SKINNY_KERNEL
 #undef SKINNY_ANY
+#undef SKINNY_PARTS
     return 0;
 }
 

@@ -514,6 +514,13 @@ def test_linear_bf16_few_rows_of_narrow_tiles(ops, M, N, K):
     assert ((outs[0].double() - want).abs() <= bound).all()
 
 
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N,K", [(1361, 5128), (1600, 6400), (2048, 5120), (2040, 7000), (1500, 9216), (1500, 9224)])
+def test_linear_bf16_few_rows_with_both_parts_of_k_inside(ops, M, N, K):
+    """Long sums in two parts: up to 8 rows one workgroup has both (a chunk of 4 to 6 blocks of K each), from 9 on two share a tile. The same bits."""
+    test_linear_bf16_few_rows_of_narrow_tiles(ops, M, N, K)
+
+
 @pytest.mark.parametrize("M", [17, 25, 32])
 @pytest.mark.parametrize("N,K", [(2048, 768), (2049, 768), (2304, 768), (2500, 1024), (4096, 768), (4097, 768), (4097, 1032), (6400, 1600)])
 @pytest.mark.parametrize("epi", ["store", "gelu_tanh"])
