@@ -364,6 +364,12 @@ void linear_from_splits(const AttentionSplits& a, const Tensor2& w, const float*
         if (rc == 0) return;
         if (rc != -2) check(rc, "linear (merging attention splits)");
     }
+    if (a.dtype == F32 && w.stride % 4 == 0 && aligned(w.data, 16)) {
+        const int rc = mllm_gemm_f32_merged(a.ws, a.ml(), a.nsplit, a.n_heads, a.head_dim, static_cast<const float*>(w.data), static_cast<int>(w.stride),
+                                            bias, out.data, static_cast<int>(out.stride), static_cast<int>(M), static_cast<int>(w.rows), epilogue, stream);
+        if (rc == 0) return;
+        if (rc != -2) check(rc, "linear (merging attention splits)");
+    }
     if (tmp == nullptr) fail("linear (merging attention splits): these sizes need a buffer for the merged rows");
     Tensor2 merged(tmp, a.dtype, M, K);
     merge_splits(a, merged, stream);
@@ -435,9 +441,9 @@ static void decode_launch_shape(int pairs, int max_ctx_len, int keys_per_wave, b
         if (t.unmerged_nsplit > 0) { *nsplit = t.unmerged_nsplit; *waves = t.unmerged_waves; return; }
         const int n = std::max(1, std::min({4, 256 / std::max(pairs, 1), max_ctx_len / 128}));
         if (n > 1) {
-            const int keys = (max_ctx_len + n - 1) / n;
+            const int keys = (max_ctx_len + n - 1) / n, each = bf16 ? 64 : keys_per_wave;
             *nsplit = n;
-            *waves = std::max(2, std::min(12, (keys + 63) / 64));
+            *waves = std::max(2, std::min(12, (keys + each - 1) / each));
             return;
         }
     }
@@ -582,8 +588,10 @@ bool paged_attention(const AttentionArgs& a, AttentionSplits* splits, hipStream_
     }
     if (decode) {
         const int pairs = T * a.n_heads;
-        bool unmerged = a.may_split && splits != nullptr && a.q.dtype == BF16 && T <= tuning().merge_max_rows &&
-                        a.head_dim % 8 == 0 && tuning().decode_nsplit == 0;
+        // (32 bits: where the product that follows merges, up to 8 rows of 3,072 columns)
+        bool unmerged = a.may_split && splits != nullptr && tuning().decode_nsplit == 0 &&
+                        (a.q.dtype == BF16 ? T <= tuning().merge_max_rows && a.head_dim % 8 == 0
+                                           : T <= std::min(8, tuning().merge_max_rows) && a.head_dim % 4 == 0 && a.n_heads * a.head_dim <= 3072);
         int nsplit = 1, waves = 12;
         bool merge_kernel = false;
         decode_launch_shape(pairs, a.max_ctx_len, 512 / lpk, a.q.dtype == BF16, unmerged, &nsplit, &waves, &merge_kernel);      // (8 rows a lane group: the kernel's UNR)

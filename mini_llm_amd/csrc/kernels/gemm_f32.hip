@@ -176,15 +176,25 @@ gemm_f32_rows_kernel(// (the first 14 dwords arrive in registers with the wavefr
 // wavefronts and each waits for chunk after chunk of its column: two wavefronts share a column, 256 columns of K in turn, and
 // ask for all their weights of a pass of KP = 512 STEPS columns at once, behind the pass's activations, which lie in LDS whole. One
 // pass covers K up to 3,072; beyond, the next pass's weights are on their way while one is used. What the epilogue adds is asked for
-// first. Bound by the chain launch, activations, weights, sums: 8 x 768 x 768 and 8 x 768 x 3,072 in a decode step 4.1 and 6.0
-// us, together 17.1 with a column a wavefront.
+// first. Bound by the chain launch, activations, weights, sums: 8 x 768 x 768 and 8 x 768 x 3,072 in a decode step 4.1 and 5.4
+// us, together 17.1 with a column a wavefront, and 4.9 for the former with two splits of attention merged in it.
 // RAGGED: K is no multiple of 256, and what lies beyond it has to be left out (8 x 1,600 x 1,600 7.4 us, 7.2 if it were not).
-template <int ROWS, int STEPS, bool RAGGED>
+// MS > 0: A is the output of split decode attention, the states of MS splits of every (token, head) pair as attention_decode.hip leaves them
+// (partial_out), merged while the rows are staged: weights over the full range of 32 bits, as the attention's own.
+template <int ROWS, int STEPS, bool RAGGED, int MS>
 __global__ void __launch_bounds__(512)
-gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers; rows in the lower half of the last, the epilogue in the upper)
+gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers)
                        const float* __restrict__ A, const float* __restrict__ W, const float* __restrict__ bias, void* __restrict__ C,
-                       int lda, int ldw, int ldc, int N, int K, int M_mode) {
-    const int M = M_mode & 0xffff, mode = M_mode >> 16;
+                       // columns and, in the upper half, columns summed; MS > 0: the splits' maxima and sums
+                       const void* __restrict__ sizes_or_ml,
+                       // MS > 0: head size and heads, 16 bits each, for the row stride
+                       int lda, int ldw, int ldc,
+                       unsigned form /* rows (4 bits), epilogue (4), MS > 0: columns */) {
+    const int M = form & 15, mode = form >> 4 & 15;
+    const int head_dim = lda & 0xffff, heads = static_cast<unsigned>(lda) >> 16;
+    const int N = MS > 0 ? form >> 8 : static_cast<int>(reinterpret_cast<uintptr_t>(sizes_or_ml));
+    const int K = MS > 0 ? heads * head_dim : static_cast<int>(reinterpret_cast<uintptr_t>(sizes_or_ml) >> 32);
+    const float* split_ml = static_cast<const float*>(sizes_or_ml);
     constexpr int COLS = 4, KP = 512 * STEPS, STAGED = ROWS * KP / 4 / 512;
     static_assert(COLS * ROWS <= 64, "the first wavefront holds the outputs");
     __shared__ __attribute__((aligned(16))) float a_s[ROWS][KP];
@@ -203,7 +213,32 @@ gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers; rows in the l
 #pragma unroll
         for (int u = 0; u < STAGED; ++u) {
             const int idx = tid + 512 * u, r = idx / (KP / 4), k = k0 + idx % (KP / 4) * 4;
-            const float4 a = *reinterpret_cast<const float4*>(A + static_cast<size_t>(min(r, M - 1)) * lda + min(k, K - 4));
+            float4 a = make_float4(0.f, 0.f, 0.f, 0.f);
+            if constexpr (MS == 0) {
+                a = *reinterpret_cast<const float4*>(A + static_cast<size_t>(min(r, M - 1)) * lda + min(k, K - 4));
+            } else if (r < M) {        // (uniform over a wavefront: a row is a quarter of a pass or more)
+                // (k / head size in quarters, as small_quotient but lane by lane)
+                const int kc = min(k, K - 4), h = static_cast<int>((static_cast<float>(kc / 4) + 0.5f) * __builtin_amdgcn_rcpf(static_cast<float>(head_dim / 4)));
+                const size_t pair = static_cast<size_t>(r) * heads + h;
+                float2 ml[MS];
+                float4 o[MS];
+#pragma unroll
+                for (int s = 0; s < MS; ++s) {
+                    ml[s] = *reinterpret_cast<const float2*>(split_ml + (pair * MS + s) * 2);
+                    o[s] = *reinterpret_cast<const float4*>(A + (pair * MS + s) * head_dim + (kc - h * head_dim));
+                }
+                float mx = ml[0].x, l = 0.f;
+#pragma unroll
+                for (int s = 1; s < MS; ++s) mx = fmaxf(mx, ml[s].x);
+#pragma unroll
+                for (int s = 0; s < MS; ++s) {
+                    const float weight = exp2f(ml[s].x - mx);
+                    l = fmaf(weight, ml[s].y, l);
+                    a.x = fmaf(weight, o[s].x, a.x); a.y = fmaf(weight, o[s].y, a.y); a.z = fmaf(weight, o[s].z, a.z); a.w = fmaf(weight, o[s].w, a.w);
+                }
+                const float inv = 1.0f / l;
+                a = make_float4(a.x * inv, a.y * inv, a.z * inv, a.w * inv);
+            }
             v[u] = r < M && k < K ? a : make_float4(0.f, 0.f, 0.f, 0.f);
         }
     };
@@ -272,8 +307,18 @@ gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers; rows in the l
 template <int ROWS, int STEPS>
 static void launch_f32_narrow(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
     const dim3 grid((N + 3) / 4);
-    if (K % 256 != 0) gemm_f32_narrow_kernel<ROWS, STEPS, true><<<grid, 512, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, N, K, M | mode << 16);
-    else gemm_f32_narrow_kernel<ROWS, STEPS, false><<<grid, 512, 0, stream>>>(A, W, bias, C, lda, ldw, ldc, N, K, M | mode << 16);
+    const void* sizes = reinterpret_cast<const void*>(static_cast<uintptr_t>(static_cast<unsigned>(N)) | static_cast<uintptr_t>(static_cast<unsigned>(K)) << 32);
+    const unsigned form = M | (mode < 0 || mode > 15 ? 15 : mode) << 4;
+    if (K % 256 != 0) gemm_f32_narrow_kernel<ROWS, STEPS, true, 0><<<grid, 512, 0, stream>>>(A, W, bias, C, sizes, lda, ldw, ldc, form);
+    else gemm_f32_narrow_kernel<ROWS, STEPS, false, 0><<<grid, 512, 0, stream>>>(A, W, bias, C, sizes, lda, ldw, ldc, form);
+}
+template <int STEPS, int MS>
+static void launch_f32_narrow_merged(const float* split_o, const float* split_ml, int heads, int head_dim, const float* W, int ldw, const float* bias, void* C,
+                                     int ldc, int M, int N, int mode, hipStream_t stream) {
+    const dim3 grid((N + 3) / 4);
+    const unsigned form = M | mode << 4 | static_cast<unsigned>(N) << 8;
+    if (heads * head_dim % 256 != 0) gemm_f32_narrow_kernel<8, STEPS, true, MS><<<grid, 512, 0, stream>>>(split_o, W, bias, C, split_ml, head_dim | heads << 16, ldw, ldc, form);
+    else gemm_f32_narrow_kernel<8, STEPS, false, MS><<<grid, 512, 0, stream>>>(split_o, W, bias, C, split_ml, head_dim | heads << 16, ldw, ldc, form);
 }
 
 // More than a few rows, on the fp32 matrix cores (v_mfma_f32_16x16x4_f32, 256 operations a clock and compute unit). WM x WN
@@ -612,6 +657,24 @@ int mllm_gemm_bf16_plain(const void* A, int lda, const void* W, int ldw, const f
     const dim3 grid((N + 3) / 4, std::min((M + 7) / 8, 256));
     gemm_bf16_plain_kernel<<<grid, 256, 0, stream>>>(static_cast<const bf16_t*>(A), lda, static_cast<const bf16_t*>(W), ldw, bias, C, ldc,
                                                      M, N, K, mode);
+    MLLM_LAUNCH_CHECK();
+    return 0;
+}
+
+// The product whose A is the output of split decode attention, merged from the splits' states while it is staged: see mllm_gemm_bf16_merged.
+// Up to 8 rows, 2 to 4 splits, results of fewer than 2,048 columns, heads of a multiple of 4 columns, up to 3,072 in all. -1: misaligned
+// operands, -2: sizes the kernel does not take.
+int mllm_gemm_f32_merged(const float* split_o, const float* split_ml, int n_splits, int n_heads, int head_dim, const float* W, int ldw, const float* bias,
+                         void* C, int ldc, int M, int N, int mode, hipStream_t stream) {
+    const int K = n_heads * head_dim;
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 8 || n_splits < 2 || n_splits > 4 || N >= 2048 || K > 3072 || head_dim % 4 != 0 || mode < 0 || mode > 15 || n_heads > 0xffff) return -2;
+    if (ldw % 4 != 0 || ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(split_o)) & 15) || (reinterpret_cast<uintptr_t>(split_ml) & 7)) return -1;
+#define MERGED(STEPS, MS) launch_f32_narrow_merged<STEPS, MS>(split_o, split_ml, n_heads, head_dim, W, ldw, bias, C, ldc, M, N, mode, stream)
+#define MERGED_SPLITS(STEPS) do { if (n_splits == 2) MERGED(STEPS, 2); else if (n_splits == 3) MERGED(STEPS, 3); else MERGED(STEPS, 4); } while (0)
+    if (K <= 1024) MERGED_SPLITS(2); else MERGED_SPLITS(3);
+#undef MERGED_SPLITS
+#undef MERGED
     MLLM_LAUNCH_CHECK();
     return 0;
 }

@@ -1307,6 +1307,43 @@ def test_decode_attention_splits_merged_by_the_next_product(ops, T, H, Hkv, dh, 
         assert (y.cpu().double() - ref_y).abs().max() <= 3e-2
 
 
+@pytest.mark.parametrize("T", [1, 3, 8])
+@pytest.mark.parametrize("H,dh,N", [(12, 64, 768), (25, 64, 1600), (6, 16, 96), (5, 128, 200), (24, 128, 2047), (12, 64, 2048)])
+@pytest.mark.parametrize("shape", [(2, 4), (3, 2), (4, 12), None])
+def test_decode_attention_splits_merged_by_the_32_bit_product(ops, T, H, dh, N, shape):
+    """The same in 32 bits: the product merges while it stages its rows, and a merge of its own stands in front of products that do not."""
+    g = torch.Generator().manual_seed(T * 31 + H + dh)
+    page, D = 16, H * dh
+    ctx = [1, 700, 130, 2, 64, 65, 300, 17][:T] if T > 1 else [700]
+    nblk = [-(-c // page) for c in ctx]
+    perm = torch.randperm(sum(nblk) + 2, generator=g).tolist()
+    kp, vp = (torch.full((len(perm) * page, D), float("nan")) for _ in range(2))
+    tables, slots = torch.zeros(T, max(nblk), dtype=torch.int32), torch.zeros(T, dtype=torch.int32)
+    qkv = _rand((T, 3 * D), torch.float32, g)
+    for b in range(T):
+        tables[b, :nblk[b]] = torch.tensor([perm.pop() for _ in range(nblk[b])])
+        js = torch.arange(ctx[b] - 1)
+        rows = tables[b].long()[js // page] * page + js % page
+        kp[rows], vp[rows] = _rand((ctx[b] - 1, D), torch.float32, g), _rand((ctx[b] - 1, D), torch.float32, g)
+        slots[b] = int(tables[b, (ctx[b] - 1) // page]) * page + (ctx[b] - 1) % page
+    token_seq, positions = torch.arange(T, dtype=torch.int32), torch.tensor([c - 1 for c in ctx], dtype=torch.int32)
+    w, bias, x0 = _rand((N, D), torch.float32, g, std=1.0 / math.sqrt(D)), 0.5 * _rand((N,), torch.float32, g), _rand((T, N), torch.float32, g)
+    att = torch.zeros(T, D, dtype=torch.float64)
+    plain_ops.paged_attention(qkv, 0, H, H, dh, kp.clone(), vp.clone(), page, tables, token_seq, positions, dh ** -0.5, 0, att, append=(D, 2 * D, slots))
+    ref = plain_ops.linear(att, w.double(), bias, x0.double().clone(), "add_residual")
+    ops.DECODE_UNMERGED_SHAPE = shape
+    try:
+        a = ops.paged_attention(qkv.to(DEV), 0, H, H, dh, kp.to(DEV), vp.to(DEV), page, tables.to(DEV), token_seq.to(DEV), positions.to(DEV), dh ** -0.5, 0,
+                                torch.empty(T, D, device=DEV), max_q_len=1, max_ctx_len=max(ctx), append=(D, 2 * D, slots.to(DEV)), may_split=True)
+    finally:
+        ops.DECODE_UNMERGED_SHAPE = None
+    assert isinstance(a, ops.AttentionSplits) == (shape is not None or T * H <= 128) and (shape is None or a.nsplit == shape[0])
+    x = x0.clone().to(DEV)
+    ops.linear(a, w.to(DEV), bias.to(DEV), x, "add_residual")
+    # (a score's rounding, 2^-24 of its terms' sum, moves its weight by as much; then fp32 sums)
+    assert (x.cpu().double() - ref).abs().max() <= 3e-5
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("H,Hkv,dh,page,window", [(12, 12, 64, 16, 0), (3, 3, 32, 8, 0), (4, 1, 128, 16, 40), (4, 4, 16, 4, 0)])
 def test_paged_attention_single_tokens_before_portions(ops, dtype, H, Hkv, dh, page, window):
