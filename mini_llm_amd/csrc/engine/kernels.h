@@ -28,6 +28,8 @@ int mllm_kv_append(const void* src, int src_stride, int k_col, int v_col, void* 
 // gemm_f32.hip, gemm_bf16.hip
 int mllm_gemm_f32_merged(const float* split_o, const float* split_ml, int n_splits, int n_heads, int head_dim, const float* W, int ldw, const float* bias,
                          void* C, int ldc, int M, int N, int mode, hipStream_t stream);
+int mllm_norm_gemm_f32(const float* x, int ldx, const float* gamma, const float* beta, float eps, int rms, const float* W, int ldw, const float* bias,
+                       void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream);
 int mllm_gemm_f32(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc,
                   int M, int N, int K, int mode, hipStream_t stream);
 int mllm_gemm_bf16_plain(const void* A, int lda, const void* W, int ldw, const float* bias, void* C, int ldc,

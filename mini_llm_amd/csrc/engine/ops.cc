@@ -418,6 +418,14 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
         if (rc == 0) return;
         if (rc != -2) check(rc, "ln_linear");
     }
+    // 32 bits: up to 8 rows of wide products (the others sum in another order, or take the rows in other shares)
+    if (w.dtype == F32 && rows == nullptr && kv == nullptr && M <= tuning().ln_fuse_max_rows && x.contiguous()) {
+        const int rc = mllm_norm_gemm_f32(static_cast<const float*>(x.data), static_cast<int>(x.stride), gamma, beta, eps, 0, static_cast<const float*>(w.data),
+                                          static_cast<int>(w.stride), bias, out.data, static_cast<int>(out.stride), static_cast<int>(M),
+                                          static_cast<int>(w.rows), static_cast<int>(K), epilogue, stream);
+        if (rc == 0) return;
+        if (rc != -2) check(rc, "ln_linear");
+    }
     if (tmp == nullptr) fail("ln_linear: these sizes need a buffer for the normalised rows");
     Tensor2 h(tmp, w.dtype, M, K);
     layernorm(x, gamma, beta, eps, h, rows, stream);

@@ -67,6 +67,12 @@ void rms_linear(const Tensor2& x, const float* weight, float eps, const Tensor2&
         if (rc == 0) return;
         if (rc != -2) check(rc, "rms_linear");
     }
+    if (w.dtype == F32 && rows == nullptr && M <= tuning().ln_fuse_max_rows && x.contiguous()) {      // (see ln_linear)
+        const int rc = mllm_norm_gemm_f32(static_cast<const float*>(x.data), i32(x.stride), weight, nullptr, eps, 1, static_cast<const float*>(w.data),
+                                          i32(w.stride), bias, out.data, i32(out.stride), i32(M), i32(w.rows), i32(K), epilogue, stream);
+        if (rc == 0) return;
+        if (rc != -2) check(rc, "rms_linear");
+    }
     if (tmp == nullptr) fail("rms_linear: these sizes need a buffer for the normalised rows");
     Tensor2 h(tmp, w.dtype, M, K);
     rmsnorm(x, weight, eps, 1, nullptr, h, rows, stream);

@@ -304,6 +304,101 @@ gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers)
     else epilogue<float>(mode, sum, out_bias, C, out_at);
 }
 
+// The norm in front of a product of up to 8 rows, inside it: wavefront w normalises row w (K <= 2,048: a row lives in registers, NU float4
+// a lane) into LDS while the weights of its CPW columns, all of them, are on their way; then every wavefront sums its columns as the few-row
+// kernel does, in the same order, so that the result has the bits of norm and product apart. Every workgroup normalises the rows again,
+// which costs it the rows and the norm's vectors from L2 (30 KB at K = 768) but no launch. RMS: the norm does not centre.
+// Bound by its chain: launch, rows, norm, products, sums. At 8 rows of K = 768: 5.7 us for 2,304
+// columns and 6.2 for 3,072, where the few-row kernel alone takes 6.2 and 6.5 behind a norm of 2.2 and a launch's gap of 1.2 (4.4 and 3.8 at one row).
+template <int NU, int CPW, int ROWS>
+__global__ void __launch_bounds__(512)
+gemm_f32_normed_kernel(// (the 14 dwords that arrive in registers; K in the lower 12 bits of the last, rows (4), epilogue (4), the kind of norm)
+                       const float* __restrict__ x, const float* __restrict__ W, const float* __restrict__ gamma, const float* __restrict__ beta,
+                       const float* __restrict__ bias, int ldx, int ldw, int N, unsigned form,
+                       void* __restrict__ C, int ldc, float eps) {
+    static_assert(CPW * ROWS <= 64, "a lane an output");
+    __shared__ float4 a_s[ROWS][NU * 64];
+    const int K = form & 0xfff, M = form >> 12 & 15, mode = form >> 16 & 15;
+    const bool rms = form >> 20 & 1;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), lane = threadIdx.x % 64, nq = K / 4;
+    const int n0 = (blockIdx.x * 8 + wave) * CPW;
+    auto quad = [&](int u) { return u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1); };
+    typedef float f4 __attribute__((ext_vector_type(4)));
+    f4 v[NU], gg[NU], bb[NU], w[CPW][NU];
+    const bool has_row = wave < M;
+    if (has_row) {
+        const f4* row = reinterpret_cast<const f4*>(x + static_cast<size_t>(wave) * ldx);
+        const f4 *g4 = reinterpret_cast<const f4*>(gamma), *b4 = reinterpret_cast<const f4*>(beta != nullptr ? beta : gamma);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) v[u] = row[quad(u)];
+#pragma unroll
+        for (int u = 0; u < NU; ++u) { gg[u] = g4[quad(u)]; bb[u] = b4[quad(u)]; }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) {
+        const f4* wrow = reinterpret_cast<const f4*>(W + static_cast<size_t>(min(n0 + c, N - 1)) * ldw);       // (a surplus column repeats the last)
+#pragma unroll
+        for (int u = 0; u < NU; ++u) w[c][u] = __builtin_nontemporal_load(wrow + quad(u));
+    }
+    const int out_r = lane % ROWS, out_n = n0 + lane / ROWS;
+    const float out_bias = bias != nullptr ? bias[min(out_n, N - 1)] : 0.f;
+    __builtin_amdgcn_sched_barrier(0);
+    if (has_row) {
+        float s = 0.f;
+#pragma unroll
+        for (int u = 0; u < NU; ++u)
+            if (u < NU - 1 || lane + 64 * u < nq) s += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+        const float mean = rms ? 0.f : wave_sum(s) / static_cast<float>(K);
+        float q = 0.f;
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            if (u < NU - 1 || lane + 64 * u < nq) {
+                const float a = v[u].x - mean, b = v[u].y - mean, c = v[u].z - mean, d = v[u].w - mean;
+                q += (a * a + b * b) + (c * c + d * d);
+            }
+        }
+        const float inv = 1.0f / sqrtf(wave_sum(q) / static_cast<float>(K) + eps);
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            const f4 g = gg[u], b = beta != nullptr ? bb[u] : f4{0.f, 0.f, 0.f, 0.f};
+            a_s[wave][lane + 64 * u] = make_float4((v[u].x - mean) * inv * g.x + b.x, (v[u].y - mean) * inv * g.y + b.y,
+                                                   (v[u].z - mean) * inv * g.z + b.z, (v[u].w - mean) * inv * g.w + b.w);
+        }
+    }
+    lds_barrier();
+    float acc[CPW][ROWS];
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) acc[c][r] = 0.f;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+        if (u < NU - 1 || lane + 64 * u < nq) {
+#pragma unroll
+            for (int r = 0; r < ROWS; ++r) {        // (rows beyond M: what stands there counts in no result that is stored)
+                const float4 a4 = a_s[r][lane + 64 * u];
+#pragma unroll
+                for (int c = 0; c < CPW; ++c) {
+                    acc[c][r] = fmaf(a4.x, w[c][u].x, acc[c][r]);
+                    acc[c][r] = fmaf(a4.y, w[c][u].y, acc[c][r]);
+                    acc[c][r] = fmaf(a4.z, w[c][u].z, acc[c][r]);
+                    acc[c][r] = fmaf(a4.w, w[c][u].w, acc[c][r]);
+                }
+            }
+        }
+    }
+    float mine = 0.f;
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+        for (int r = 0; r < ROWS; ++r) {
+            const float t = wave_sum(acc[c][r]);
+            if (lane == c * ROWS + r) mine = t;
+        }
+    if (lane < CPW * ROWS && out_r < M && out_n < N) epilogue<float>(mode, mine, out_bias, C, static_cast<size_t>(out_r) * ldc + out_n);
+}
+
 template <int ROWS, int STEPS>
 static void launch_f32_narrow(const float* A, int lda, const float* W, int ldw, const float* bias, void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
     const dim3 grid((N + 3) / 4);
@@ -675,6 +770,34 @@ int mllm_gemm_f32_merged(const float* split_o, const float* split_ml, int n_spli
     if (K <= 1024) MERGED_SPLITS(2); else MERGED_SPLITS(3);
 #undef MERGED_SPLITS
 #undef MERGED
+    MLLM_LAUNCH_CHECK();
+    return 0;
+}
+
+// The norm of the fp32 rows x [M, K] (a LayerNorm, or with rms != 0 an RMS norm) inside the product of up to 8 of them: C = epilogue(norm(x) W^T + bias).
+// -2: sizes the kernel does not take (more rows, K over 2,048 or no multiple of 4, operands that are not 16-byte aligned, or fewer columns than
+// the few-row kernel has in this order of sums); norm and product apart are right for those.
+int mllm_norm_gemm_f32(const float* x, int ldx, const float* gamma, const float* beta, float eps, int rms, const float* W, int ldw, const float* bias,
+                       void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
+    if (M <= 0 || N <= 0) return 0;
+    if (M > 8 || N < 2048 || K < 4 || K > 2048 || K % 4 != 0 || ldx % 4 != 0 || ldw % 4 != 0 || mode < 0 || mode > 15 || gamma == nullptr ||
+        ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(gamma) | reinterpret_cast<uintptr_t>(beta)) & 15) != 0)
+        return -2;
+    const unsigned form = K | M << 12 | mode << 16 | (rms ? 1u << 20 : 0u);
+    // (two columns a wavefront where one would take more than two rounds of workgroups)
+    const bool two = N > 4096;
+    const dim3 grid(two ? (N + 15) / 16 : (N + 7) / 8);
+#define NORMED(NU, CPW, ROWS) gemm_f32_normed_kernel<NU, CPW, ROWS><<<grid, 512, 0, stream>>>(x, W, gamma, beta, bias, ldx, ldw, N, form, C, ldc, eps)
+#define NORMED_CASE(NU)                                                                                   \
+    case NU:                                                                                            \
+        if (M <= 2) { if (two) NORMED(NU, 2, 2); else NORMED(NU, 1, 2); }                               \
+        else if (two) NORMED(NU, 2, 8); else NORMED(NU, 1, 8);                                          \
+        break;
+    switch ((K + 255) / 256) {
+        NORMED_CASE(1) NORMED_CASE(2) NORMED_CASE(3) NORMED_CASE(4) NORMED_CASE(5) NORMED_CASE(6) NORMED_CASE(7) NORMED_CASE(8)
+    }
+#undef NORMED_CASE
+#undef NORMED
     MLLM_LAUNCH_CHECK();
     return 0;
 }

@@ -631,6 +631,28 @@ def test_ln_linear_at_every_number_of_columns_a_lane(ops, M, N, K):
     test_ln_linear(ops, torch.bfloat16, M, N, K, "store")
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
+@pytest.mark.parametrize("N,K", [(2048, 4), (2050, 252), (2304, 256), (2048, 260), (2304, 768), (3072, 768), (4096, 1024), (4097, 772), (4800, 1600),
+                                 (6400, 1600), (2056, 2044), (4104, 2048)])
+@pytest.mark.parametrize("epi", ["store", "gelu_tanh"])
+def test_ln_linear_fp32_inside_has_the_bits_of_norm_and_product(ops, monkeypatch, M, N, K, epi):
+    """The 32-bit norm inside the few-row product, around every 256 columns a lane's share grows by: the bits of norm and product apart."""
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (_rand((M, K), torch.float32, g, std=2.0) + 0.3).to(DEV)
+    gamma, beta = (1 + 0.1 * _rand((K,), torch.float32, g)).to(DEV), (0.1 * _rand((K,), torch.float32, g)).to(DEV)
+    w, bias = _rand((N, K), torch.float32, g, std=1.0 / math.sqrt(K)).to(DEV), (0.5 * _rand((N,), torch.float32, g)).to(DEV)
+    inside, apart = (torch.full((M, N), 7.0, device=DEV) for _ in range(2))
+    for b, c in ((beta, bias), (None, None)):
+        ops.ln_linear(x, gamma, b, 1e-5, w, c, inside, epi)
+        with monkeypatch.context() as m:
+            m.setattr(ops, "LN_FUSE_MAX_ROWS", 0)
+            ops.ln_linear(x, gamma, b, 1e-5, w, c, apart, epi)
+        assert torch.equal(inside, apart)
+    h = plain_ops.layernorm(x.cpu(), gamma.cpu(), None, 1e-5, torch.empty(M, K, dtype=torch.float64))
+    ref = plain_ops.linear(h, w.cpu().double(), None, torch.zeros(M, N, dtype=torch.float64), epi)
+    assert (inside.cpu().double() - ref).abs().max().item() <= 3e-5
+
+
 def test_linear_fp32_is_true_fp32(ops):
     """Values that bf16 or tf32 inputs would destroy: 1 + 2^-20 differs from 1 only in true fp32."""
     K = 64
