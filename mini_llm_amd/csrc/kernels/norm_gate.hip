@@ -257,66 +257,78 @@ rmsnorm_add_many_kernel(const float* __restrict__ y, size_t y_stride, const floa
 // first use (a load under a condition waits for all loads in flight, and a row of 768 then costs eight round trips).
 // `parts` > 1: the input is the sum of that many arrays `part_stride` floats apart (partial results of a kernel
 // that splits a sum over workgroups), added in the order of their index.
-template <typename OutT, int WAVES, bool SHARES = false>
+// NU: float4 of a part per lane, so that none but the last is asked whether it exists. The arguments stand in the order in which they
+// are needed (the first 14 words are in registers when a wavefront starts); with one group there is nothing to divide. A chain of latencies
+// at few rows, memory at many: 8 gated rows of 1,536 4.6 > 4.0 us, 2,048 8.7 > 7.9.
+template <typename OutT, int WAVES, int NU, bool SHARES = false>
 __global__ void __launch_bounds__(64 * WAVES)
-rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, const int* __restrict__ rows, const float* __restrict__ w,
-                   const float* __restrict__ gate, int ldg, OutT* __restrict__ y, int ldy, int n, int D, int groups,
-                   float eps, int parts, size_t part_stride) {
+rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, int n, const int* __restrict__ rows, const float* __restrict__ gate, int ldg, int D,
+                   const float* __restrict__ w, int groups, float eps, OutT* __restrict__ y, int ldy, int parts, size_t part_stride) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MLLM_WAVE), lane = threadIdx.x % MLLM_WAVE;
-    const long long pair = static_cast<long long>(blockIdx.x) * WAVES + wave;
-    if (pair >= static_cast<long long>(n) * groups) return;
-    const int r = static_cast<int>(pair / groups), g = static_cast<int>(pair % groups), Dg = D / groups;
-    const int src = rows ? rows[r] : r;
+    int r, g = 0, Dg = D;
+    if (groups == 1) {
+        r = blockIdx.x * WAVES + wave;
+        if (r >= n) return;
+    } else {
+        const long long pair = static_cast<long long>(blockIdx.x) * WAVES + wave;
+        if (pair >= static_cast<long long>(n) * groups) return;
+        r = static_cast<int>(pair / groups);
+        g = static_cast<int>(pair - static_cast<long long>(r) * groups);
+        Dg = D / groups;
+    }
+    int src = r;
+    if (rows != nullptr) {
+        src = rows[r];
+        asm volatile("" : "+s"(src));       // waited for in here, not where the launches without a gather pass too
+    }
     const float4* xr = reinterpret_cast<const float4*>(x + static_cast<size_t>(src) * ldx + g * Dg);
-    const float4* gr = reinterpret_cast<const float4*>(gate ? gate + static_cast<size_t>(src) * ldg + g * Dg : x);
+    const float4* gr = reinterpret_cast<const float4*>(gate ? gate + static_cast<size_t>(src) * ldg + g * Dg : x + g * Dg);
     const float4* wr = reinterpret_cast<const float4*>(w + g * Dg);
-    const int nq = Dg / 4, n_u = (nq + 63) / 64;
-    float4 v[8], gg[8], ww[8];
+    const int nq = Dg / 4;
+    float4 v[NU], gg[NU], ww[NU];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u) v[u] = xr[min(lane + 64 * u, nq - 1)];
+    for (int u = 0; u < NU; ++u) v[u] = xr[u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1)];
     if (SHARES) {
         // up to four shares (the launcher sends more to the plain kernel): all of them requested before the first
         // is added, a share beyond `parts` read from the last one and not added
-        float4 sh[3][8];
+        float4 sh[3][NU];
 #pragma unroll
         for (int part = 1; part < 4; ++part) {
             const float4* xp = reinterpret_cast<const float4*>(reinterpret_cast<const float*>(xr) + min(part, parts - 1) * part_stride);
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (u < n_u) sh[part - 1][u] = xp[min(lane + 64 * u, nq - 1)];
+            for (int u = 0; u < NU; ++u) sh[part - 1][u] = xp[u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1)];
         }
 #pragma unroll
         for (int part = 1; part < 4; ++part)
 #pragma unroll
-            for (int u = 0; u < 8; ++u)
-                if (u < n_u && part < parts) {
+            for (int u = 0; u < NU; ++u)
+                if (part < parts) {
                     v[u].x += sh[part - 1][u].x; v[u].y += sh[part - 1][u].y; v[u].z += sh[part - 1][u].z; v[u].w += sh[part - 1][u].w;
                 }
     }
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u) {
-            const int i = min(lane + 64 * u, nq - 1);
-            gg[u] = gr[i];
-            ww[u] = wr[i];
+    for (int u = 0; u < NU; ++u) {
+        const int i = u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1);
+        gg[u] = gr[i];
+        ww[u] = wr[i];
+    }
+    if (gate) {
+#pragma unroll
+        for (int u = 0; u < NU; ++u) {
+            v[u].x *= gg[u].x * sigmoid_precise(gg[u].x); v[u].y *= gg[u].y * sigmoid_precise(gg[u].y);
+            v[u].z *= gg[u].z * sigmoid_precise(gg[u].z); v[u].w *= gg[u].w * sigmoid_precise(gg[u].w);
         }
+    }
     float ss = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u) {
-            if (gate) {
-                v[u].x *= gg[u].x * sigmoid_precise(gg[u].x); v[u].y *= gg[u].y * sigmoid_precise(gg[u].y);
-                v[u].z *= gg[u].z * sigmoid_precise(gg[u].z); v[u].w *= gg[u].w * sigmoid_precise(gg[u].w);
-            }
-            if (lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
-        }
+    for (int u = 0; u < NU; ++u)
+        if (u < NU - 1 || lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
     const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(Dg) + eps);
     OutT* yr = y + static_cast<size_t>(r) * ldy + g * Dg;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < NU; ++u) {
         const int i = lane + 64 * u;
-        if (u < n_u && i < nq) {
+        if (u < NU - 1 || i < nq) {
             const float o0 = v[u].x * inv * ww[u].x, o1 = v[u].y * inv * ww[u].y, o2 = v[u].z * inv * ww[u].z, o3 = v[u].w * inv * ww[u].w;
             if (sizeof(OutT) == 2) {
                 uint2 pk;
@@ -333,11 +345,11 @@ rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, const int* __restrict__
 // NEXT: `copy` receives the new row behind the RMS norm that stands in front of the next sub-layer (next_w, next_eps) instead of
 // the row itself: the row is in registers, and a norm kernel of its own would read it again. Bound by memory: y and x once, x and
 // the copy written.
-template <int WAVES, bool CENTER, bool NEXT = false>
+// Arguments and NU as above (8 rows of 768 2.53 > 2.41 us, 2,048 with the next norm 6.15 > 6.00); `extra` is beta (CENTER) or next_w (NEXT).
+template <int WAVES, int NU, bool CENTER, bool NEXT = false>
 __global__ void __launch_bounds__(64 * WAVES)
-rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const float* __restrict__ beta, const float* __restrict__ scale,
-                       float mult, float eps, float* __restrict__ x, int n, int D, int clear, bf16_t* __restrict__ copy,
-                       const float* __restrict__ next_w = nullptr, float next_eps = 0.f) {
+rmsnorm_add_vec_kernel(float* __restrict__ y, int n, int D, float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ scale,
+                       const float* __restrict__ extra, float mult, float eps, bf16_t* __restrict__ copy, int clear, float next_eps) {
     static_assert(!(CENTER && NEXT), "the next norm stands behind RMS norms");
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MLLM_WAVE), lane = threadIdx.x % MLLM_WAVE;
     const int r = blockIdx.x * WAVES + wave;
@@ -346,46 +358,41 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const
     float4* xr = reinterpret_cast<float4*>(x + static_cast<size_t>(r) * D);
     const float4* wr = reinterpret_cast<const float4*>(w);
     const float4* sr = reinterpret_cast<const float4*>(scale ? scale : w);
-    const float4* br = reinterpret_cast<const float4*>(CENTER && beta ? beta : w);
-    const int nq = D / 4, n_u = (nq + 63) / 64;
-    const float4* next_r = reinterpret_cast<const float4*>(next_w);
-    float4 v[8], xx[8], ww[8], sc[8], bb[8];
+    const float4* br = reinterpret_cast<const float4*>(extra ? extra : w);
+    const int nq = D / 4;
+    float4 v[NU], xx[NU], ww[NU], sc[NU], bb[NU];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u) v[u] = yr[min(lane + 64 * u, nq - 1)];
+    for (int u = 0; u < NU; ++u) v[u] = yr[u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1)];
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u) {
-            const int i = min(lane + 64 * u, nq - 1);
-            xx[u] = xr[i];
-            ww[u] = wr[i];
-            sc[u] = sr[i];
-            if (CENTER) bb[u] = br[i];
-            if (NEXT) bb[u] = next_r[i];
-        }
+    for (int u = 0; u < NU; ++u) {
+        const int i = u < NU - 1 ? lane + 64 * u : min(lane + 64 * u, nq - 1);
+        xx[u] = xr[i];
+        ww[u] = wr[i];
+        sc[u] = sr[i];
+        if (CENTER || NEXT) bb[u] = br[i];
+    }
     if (CENTER) {
         float sum = 0.f;
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (u < n_u && lane + 64 * u < nq) sum += (v[u].x + v[u].y) + (v[u].z + v[u].w);
+        for (int u = 0; u < NU; ++u)
+            if (u < NU - 1 || lane + 64 * u < nq) sum += (v[u].x + v[u].y) + (v[u].z + v[u].w);
         const float mean = wave_sum(sum) / static_cast<float>(D);
 #pragma unroll
-        for (int u = 0; u < 8; ++u)
-            if (u < n_u) { v[u].x -= mean; v[u].y -= mean; v[u].z -= mean; v[u].w -= mean; }
+        for (int u = 0; u < NU; ++u) { v[u].x -= mean; v[u].y -= mean; v[u].z -= mean; v[u].w -= mean; }
     }
     float ss = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u)
-        if (u < n_u && lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
+    for (int u = 0; u < NU; ++u)
+        if (u < NU - 1 || lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
     const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(D) + eps);
     float next_ss = 0.f;
 #pragma unroll
-    for (int u = 0; u < 8; ++u) {
+    for (int u = 0; u < NU; ++u) {
         const int i = lane + 64 * u;
-        if (u < n_u && i < nq) {
+        if (u < NU - 1 || i < nq) {
             const float4 s4 = scale ? make_float4(sc[u].x * mult, sc[u].y * mult, sc[u].z * mult, sc[u].w * mult) : make_float4(mult, mult, mult, mult);
             float4 o = make_float4(v[u].x * inv * ww[u].x, v[u].y * inv * ww[u].y, v[u].z * inv * ww[u].z, v[u].w * inv * ww[u].w);
-            if (CENTER && beta) { o.x += bb[u].x; o.y += bb[u].y; o.z += bb[u].z; o.w += bb[u].w; }
+            if (CENTER && extra) { o.x += bb[u].x; o.y += bb[u].y; o.z += bb[u].z; o.w += bb[u].w; }
             const float4 now = make_float4(xx[u].x + s4.x * o.x, xx[u].y + s4.y * o.y, xx[u].z + s4.z * o.z, xx[u].w + s4.w * o.w);
             xr[i] = now;
             if (NEXT) {
@@ -403,9 +410,9 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, const float* __restrict__ w, const
     if (NEXT) {
         const float next_inv = 1.0f / sqrtf(wave_sum(next_ss) / static_cast<float>(D) + next_eps);
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
+        for (int u = 0; u < NU; ++u) {
             const int i = lane + 64 * u;
-            if (u < n_u && i < nq) {
+            if (u < NU - 1 || i < nq) {
                 uint2 pk;
                 pk.x = pack_bf16x2(xx[u].x * next_inv * bb[u].x, xx[u].y * next_inv * bb[u].y);
                 pk.y = pack_bf16x2(xx[u].z * next_inv * bb[u].z, xx[u].w * next_inv * bb[u].w);
@@ -434,6 +441,20 @@ __global__ void fill_zero_kernel(float4* __restrict__ p, size_t n4) {
         p[i] = make_float4(0.f, 0.f, 0.f, 0.f);
 }
 
+// (many rows go eight to a workgroup: workgroups start at a limited rate)
+template <bool CENTER, bool NEXT>
+void norm_add_vec(float* y, const float* w, const float* scale, const float* extra, float mult, float eps, float* x, int n, int D, int clear,
+                  bf16_t* copy, float next_eps, hipStream_t stream) {
+#define NORM_ADD(WAVES, NU) \
+    rmsnorm_add_vec_kernel<WAVES, NU, CENTER, NEXT><<<(n + WAVES - 1) / WAVES, 64 * WAVES, 0, stream>>>(y, n, D, x, w, scale, extra, mult, eps, copy, clear, next_eps)
+#define NORM_ADD_CASE(NU) case NU: if (n >= 512) NORM_ADD(8, NU); else NORM_ADD(4, NU); break;
+    switch ((D + 255) / 256) {
+        NORM_ADD_CASE(1) NORM_ADD_CASE(2) NORM_ADD_CASE(3) NORM_ADD_CASE(4) NORM_ADD_CASE(5) NORM_ADD_CASE(6) NORM_ADD_CASE(7) NORM_ADD_CASE(8)
+    }
+#undef NORM_ADD_CASE
+#undef NORM_ADD
+}
+
 }  // namespace
 
 extern "C" {
@@ -452,12 +473,19 @@ int mllm_rmsnorm(const float* x, int ldx, const int* rows, const float* w, const
                      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(gate) |
                        reinterpret_cast<uintptr_t>(y)) & 15) == 0;
     // (workgroups start at a limited rate: many rows go eight to a workgroup)
-#define RMS(KERNEL, TYPE, WAVES)                                                                                        \
-    KERNEL<TYPE, WAVES><<<static_cast<int>((pairs + WAVES - 1) / WAVES), 64 * WAVES, 0, stream>>>(                      \
+#define RMS(TYPE, WAVES)                                                                                                \
+    rmsnorm_kernel<TYPE, WAVES><<<static_cast<int>((pairs + WAVES - 1) / WAVES), 64 * WAVES, 0, stream>>>(              \
         x, ldx, rows, w, gate, ldg, static_cast<TYPE*>(y), ldy, n, D, groups, eps, parts, part_stride)
-#define RMS_SHARES(TYPE)                                                                                                \
-    rmsnorm_vec_kernel<TYPE, 4, true><<<static_cast<int>((pairs + 3) / 4), 256, 0, stream>>>(                           \
-        x, ldx, rows, w, gate, ldg, static_cast<TYPE*>(y), ldy, n, D, groups, eps, parts, part_stride)
+#define RMS_VEC_NU(TYPE, WAVES, NU, SHARES)                                                                             \
+    rmsnorm_vec_kernel<TYPE, WAVES, NU, SHARES><<<static_cast<int>((pairs + WAVES - 1) / WAVES), 64 * WAVES, 0, stream>>>( \
+        x, ldx, n, rows, gate, ldg, D, w, groups, eps, static_cast<TYPE*>(y), ldy, parts, part_stride)
+#define RMS_VEC(TYPE, WAVES, SHARES)                                                                                    \
+    switch ((Dg + 255) / 256) {                                                                                         \
+        case 1: RMS_VEC_NU(TYPE, WAVES, 1, SHARES); break; case 2: RMS_VEC_NU(TYPE, WAVES, 2, SHARES); break;           \
+        case 3: RMS_VEC_NU(TYPE, WAVES, 3, SHARES); break; case 4: RMS_VEC_NU(TYPE, WAVES, 4, SHARES); break;           \
+        case 5: RMS_VEC_NU(TYPE, WAVES, 5, SHARES); break; case 6: RMS_VEC_NU(TYPE, WAVES, 6, SHARES); break;           \
+        case 7: RMS_VEC_NU(TYPE, WAVES, 7, SHARES); break; default: RMS_VEC_NU(TYPE, WAVES, 8, SHARES); break;          \
+    }
     if (vec && groups > 1 && rows == nullptr && gate == nullptr && (Dg == 16 || Dg == 32 || Dg == 64 || Dg == 128)) {
         // many short groups: several of them a wavefront
         const int per_wg = 4 * (64 / (Dg / 4));
@@ -470,15 +498,16 @@ int mllm_rmsnorm(const float* x, int ldx, const int* rows, const float* w, const
 #undef RSG_T
 #undef RSG
     } else if (vec && parts > 1) {
-        if (out_dtype == MLLM_F32) RMS_SHARES(float); else RMS_SHARES(bf16_t);
+        if (out_dtype == MLLM_F32) { RMS_VEC(float, 4, true) } else { RMS_VEC(bf16_t, 4, true) }
     } else if (vec) {
-        if (out_dtype == MLLM_F32) { if (pairs >= 512) RMS(rmsnorm_vec_kernel, float, 8); else RMS(rmsnorm_vec_kernel, float, 4); }
-        else { if (pairs >= 512) RMS(rmsnorm_vec_kernel, bf16_t, 8); else RMS(rmsnorm_vec_kernel, bf16_t, 4); }
+        if (out_dtype == MLLM_F32) { if (pairs >= 512) { RMS_VEC(float, 8, false) } else { RMS_VEC(float, 4, false) } }
+        else { if (pairs >= 512) { RMS_VEC(bf16_t, 8, false) } else { RMS_VEC(bf16_t, 4, false) } }
     } else {
-        if (out_dtype == MLLM_F32) RMS(rmsnorm_kernel, float, 4); else RMS(rmsnorm_kernel, bf16_t, 4);
+        if (out_dtype == MLLM_F32) RMS(float, 4); else RMS(bf16_t, 4);
     }
 #undef RMS
-#undef RMS_SHARES
+#undef RMS_VEC
+#undef RMS_VEC_NU
     MLLM_LAUNCH_CHECK();
     return 0;
 }
@@ -518,15 +547,14 @@ int mllm_norm_add(float* y, const float* w, const float* beta, const float* scal
     const bool vec = D % 4 == 0 && D <= 2048 &&
                      ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(scale) |
                        reinterpret_cast<uintptr_t>(beta) | reinterpret_cast<uintptr_t>(copy) | reinterpret_cast<uintptr_t>(y)) & 15) == 0;
-#define NORM_ADD(KERNEL, WAVES)                                                                                                             \
-    do {                                                                                                                                    \
-        if (center) KERNEL<WAVES, true><<<(n + WAVES - 1) / WAVES, 64 * WAVES, 0, stream>>>(y, w, beta, scale, mult, eps, x, n, D, clear, copy); \
-        else KERNEL<WAVES, false><<<(n + WAVES - 1) / WAVES, 64 * WAVES, 0, stream>>>(y, w, beta, scale, mult, eps, x, n, D, clear, copy);   \
-    } while (0)
-    if (vec && n >= 512) NORM_ADD(rmsnorm_add_vec_kernel, 8);
-    else if (vec) NORM_ADD(rmsnorm_add_vec_kernel, 4);
-    else NORM_ADD(rmsnorm_add_kernel, 4);
-#undef NORM_ADD
+    if (vec) {
+        if (center) norm_add_vec<true, false>(y, w, scale, beta, mult, eps, x, n, D, clear, copy, 0.f, stream);
+        else norm_add_vec<false, false>(y, w, scale, nullptr, mult, eps, x, n, D, clear, copy, 0.f, stream);
+    } else if (center) {
+        rmsnorm_add_kernel<4, true><<<(n + 3) / 4, 256, 0, stream>>>(y, w, beta, scale, mult, eps, x, n, D, clear, copy);
+    } else {
+        rmsnorm_add_kernel<4, false><<<(n + 3) / 4, 256, 0, stream>>>(y, w, beta, scale, mult, eps, x, n, D, clear, copy);
+    }
     MLLM_LAUNCH_CHECK();
     return 0;
 }
@@ -540,8 +568,7 @@ int mllm_rmsnorm_add_norm(float* y, const float* w, const float* scale, float mu
     if (D % 4 != 0 || D > 2048 || ((reinterpret_cast<uintptr_t>(x) | reinterpret_cast<uintptr_t>(w) | reinterpret_cast<uintptr_t>(scale) |
                                     reinterpret_cast<uintptr_t>(next_w) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(y)) & 15) != 0)
         return -2;
-    if (n >= 512) rmsnorm_add_vec_kernel<8, false, true><<<(n + 7) / 8, 512, 0, stream>>>(y, w, nullptr, scale, mult, eps, x, n, D, clear, out, next_w, next_eps);
-    else rmsnorm_add_vec_kernel<4, false, true><<<(n + 3) / 4, 256, 0, stream>>>(y, w, nullptr, scale, mult, eps, x, n, D, clear, out, next_w, next_eps);
+    norm_add_vec<false, true>(y, w, scale, next_w, mult, eps, x, n, D, clear, out, next_eps, stream);
     MLLM_LAUNCH_CHECK();
     return 0;
 }
