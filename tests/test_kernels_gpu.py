@@ -1619,3 +1619,45 @@ def test_sample_frequencies_follow_softmax(ops):
     freq = torch.bincount(out.cpu().long(), minlength=4).double() / 4096
     p = torch.softmax(logits[0].double() / 0.8, 0)
     assert (freq - p).abs().max() < 4 * math.sqrt(0.25 / 4096)
+
+
+def _entry(library, name, *args):
+    """A kernel library's C entry point on the null stream; tensors go in as their addresses, doubles and floats by their ctypes."""
+    import ctypes
+    from mini_llm_amd import build
+    f = getattr(build.load_library(library), name)
+    conv = [ctypes.c_void_p(a.data_ptr()) if isinstance(a, torch.Tensor) else ctypes.c_void_p(None) if a is None else
+            ctypes.c_int(a) if isinstance(a, int) else a for a in args]
+    torch.cuda.synchronize()
+    rc = f(*conv)
+    torch.cuda.synchronize()
+    return rc
+
+
+@pytest.mark.parametrize("C,taps", [(4, 2), (252, 4), (256, 3), (260, 8), (1792, 4), (1028, 5)])
+@pytest.mark.parametrize("T", [1, 8])
+def test_conv_of_one_token_a_sequence(T, C, taps):
+    """Around a workgroup's 256 channels: results, the carried rows moved up by one, and a sequence without a slot left alone."""
+    import ctypes
+    g = torch.Generator().manual_seed(C + taps + T)
+    ld, slot_floats = C + 8, (taps - 1) * C + 12
+    x, w, bias = _rand((T, ld), torch.float32, g), _rand((C, taps), torch.float32, g), _rand((C,), torch.float32, g)
+    state = _rand((T + 1, slot_floats), torch.float32, g)
+    slots = torch.randperm(T + 1, generator=g)[:T].int()
+    if T > 1:
+        slots[2] = -1
+    seq, cu = torch.arange(T, dtype=torch.int32), torch.arange(T + 1, dtype=torch.int32)
+    out, dev_state = torch.full((T, C), 7.0, device=DEV), state.clone().to(DEV)
+    assert _entry("ssm", "mllm_conv_silu", x.to(DEV), ld, 4, C, w.to(DEV), bias.to(DEV), taps, seq.to(DEV), cu.to(DEV), slots.to(DEV), dev_state,
+                  ctypes.c_size_t(slot_floats), out, C, T, T, 1, None) == 0
+    want, after = torch.full((T, C), 7.0, dtype=torch.float64), state.clone()
+    for t in range(T):
+        if slots[t] < 0:
+            continue
+        rows = torch.cat([state[slots[t], :(taps - 1) * C].view(taps - 1, C), x[t:t + 1, 4:4 + C]])
+        v = bias.double() + (w.double().T * rows.double()).sum(0)
+        want[t] = v * torch.sigmoid(v)
+        after[slots[t], :(taps - 1) * C] = rows[1:].reshape(-1)
+    assert torch.equal(dev_state.cpu(), after)
+    # a rounding of 2^-24 for each of up to nine terms of up to about 16, and the exponential's
+    assert (out.cpu().double() - want).abs().max() <= 9 * 16 * 2.0 ** -23
