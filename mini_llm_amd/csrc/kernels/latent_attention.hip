@@ -25,28 +25,46 @@ __device__ __forceinline__ void turn_pair(float u, float v, int pos, int i, doub
     b = v * c + u * s;
 }
 
-// One wavefront per token:
+// Two wavefronts per token:
 //   cq[t]  = rmsnorm(dq[t]) * wq                                      (the query latent, activation dtype; dq may be null)
 //   page row slots[t] = [ c = rmsnorm(dkv[t, :R]) * wkv | turned dkv[t, R:R+Dr] ]   (if dkv is given and slot >= 0)
 // The first rot_dims of the Dr columns are turned in pairs, the rest pass unchanged. The mean of c's squares runs over
 // Rn <= R columns (a latent widened with zero columns: the columns behind Rn are zero).
+// A chain of latencies at a few tokens: nothing waits for an argument or for the slot before it asks for the rows (the first 14 words of the
+// arguments are in registers when a wavefront starts), and a second wavefront turns the key part, whose angles in double are as long as the
+// norms. 8 tokens of 384 and 256 + 32 columns 3.8 > 2.9 us.
 template <typename T>
-__global__ void __launch_bounds__(64)
-latent_prepare_kernel(const float* __restrict__ dq, int ld_dq, int Rq, const float* __restrict__ wq, T* __restrict__ cq,
-                      int ld_cq, const float* __restrict__ dkv, int ld_dkv, int R, int Dr, const float* __restrict__ wkv,
-                      T* __restrict__ pages, T* __restrict__ vt_pages, int page_size, const int* __restrict__ slots,
-                      const int* __restrict__ positions, float eps, double log2_base, int rot_dims, int Rn, int half) {
-    const int t = blockIdx.x, lane = threadIdx.x;
+__global__ void __launch_bounds__(128)
+latent_prepare_kernel(const float* __restrict__ dq, int ld_dq, int Rq, const float* __restrict__ wq, const float* __restrict__ dkv, int ld_dkv,
+                      int R, const float* __restrict__ wkv, const int* __restrict__ slots, const int* __restrict__ positions, int Dr, int rot_dims,
+                      double log2_base, T* __restrict__ cq, int ld_cq, T* __restrict__ pages, T* __restrict__ vt_pages, int page_size, float eps,
+                      int Rn, int half) {
+    const int t = blockIdx.x, lane = threadIdx.x % 64;
+    const bool fed = dkv != nullptr;
+    const int slot = fed ? slots[t] : -1;
+    if (threadIdx.x >= 64) {
+        const int pos = fed && positions != nullptr ? positions[t] : 0;          // (asked for beside the slot)
+        if (slot < 0) return;
+        const float* row = dkv + static_cast<size_t>(t) * ld_dkv + R;
+        T* o = pages + static_cast<size_t>(slot) * (R + Dr) + R;
+        for (int i = lane; i < rot_dims / 2; i += 64) {
+            float a, b;
+            const int u = pair_first(i, half), v = pair_second(i, half, rot_dims);
+            turn_pair(row[u], row[v], pos, i, log2_base, rot_dims, a, b);
+            o[u] = from_float<T>(a);
+            o[v] = from_float<T>(b);
+        }
+        for (int i = rot_dims + lane; i < Dr; i += 64) o[i] = from_float<T>(row[i]);
+        return;
+    }
     // Up to 8 values a lane of each latent are requested up front, without conditions (a loop of unknown length
     // would wait for every load before it asks for the next); longer latents read the rest in a loop.
-    const int slot = dkv ? slots[t] : -1;
-    const bool fill = dkv != nullptr && slot >= 0;
-    if (dq == nullptr && !fill) return;
     // (no latent to fill, or none of the query's: the loads below repeat the other's)
     const float* qrow = dq ? dq + static_cast<size_t>(t) * ld_dq : dkv + static_cast<size_t>(t) * ld_dkv;
-    const float* row = fill ? dkv + static_cast<size_t>(t) * ld_dkv : qrow;
-    const int Rk = fill ? R : Rq;
+    const float* row = fed ? dkv + static_cast<size_t>(t) * ld_dkv : qrow;
+    const int Rk = fed ? R : Rq;
     if (dq == nullptr) { Rq = R; wq = wkv; }
+    const float* wk = fed ? wkv : wq;
     float qv[8], kv[8], qw[8], kw[8];
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
@@ -54,7 +72,7 @@ latent_prepare_kernel(const float* __restrict__ dq, int ld_dq, int Rq, const flo
         qv[u] = qrow[iq];
         qw[u] = wq[iq];
         kv[u] = row[ik];
-        kw[u] = fill ? wkv[ik] : 0.f;
+        kw[u] = wk[ik];
     }
     if (dq != nullptr) {
         float ss = 0.f;
@@ -67,7 +85,7 @@ latent_prepare_kernel(const float* __restrict__ dq, int ld_dq, int Rq, const flo
         for (int u = 0; u < 8; ++u) if (lane + 64 * u < Rq) o[lane + 64 * u] = from_float<T>(qv[u] * inv * qw[u]);
         for (int i = lane + 512; i < Rq; i += 64) o[i] = from_float<T>(qrow[i] * inv * wq[i]);
     }
-    if (!fill) return;
+    if (slot < 0) return;
     T* o = pages + static_cast<size_t>(slot) * (R + Dr);
     float ss = 0.f;
 #pragma unroll
@@ -76,7 +94,11 @@ latent_prepare_kernel(const float* __restrict__ dq, int ld_dq, int Rq, const flo
     const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(Rn) + eps);
     // (vt_pages, optional: the latent once more, transposed page by page, [page][R][page_size], which is the
     // operand shape of the matrix-core kernel's second product)
-    T* vt = vt_pages ? vt_pages + static_cast<size_t>(slot / page_size) * page_size * R + slot % page_size : nullptr;
+    T* vt = nullptr;
+    if (vt_pages) {
+        const int first = uniform_quotient(slot, page_size) * page_size;          // the page's first slot
+        vt = vt_pages + static_cast<size_t>(first) * R + (slot - first);
+    }
 #pragma unroll
     for (int u = 0; u < 8; ++u) {
         const int i = lane + 64 * u;
@@ -91,15 +113,6 @@ latent_prepare_kernel(const float* __restrict__ dq, int ld_dq, int Rq, const flo
         o[i] = c;
         if (vt) vt[static_cast<size_t>(i) * page_size] = c;
     }
-    const int pos = positions[t];
-    for (int i = lane; i < rot_dims / 2; i += 64) {
-        float a, b;
-        const int u = R + pair_first(i, half), v = R + pair_second(i, half, rot_dims);
-        turn_pair(row[u], row[v], pos, i, log2_base, rot_dims, a, b);
-        o[u] = from_float<T>(a);
-        o[v] = from_float<T>(b);
-    }
-    for (int i = rot_dims + lane; i < Dr; i += 64) o[R + i] = from_float<T>(row[R + i]);
 }
 
 // Queries into the latent space. q rows: per head [Dn plain | Dr to be turned]; w_ukt [R, H * Dn] is the key
@@ -616,7 +629,9 @@ latent_prefill_kernel(const bf16_t* __restrict__ qa, const bf16_t* __restrict__ 
 
 // The splits' states of a row merged: o = sum_s 2^(m_s - M) o_s / sum_s 2^(m_s - M) l_s. One wavefront per row
 // (up to 64 splits: lane s weighs split s; the weights pass through LDS; the outputs are added in the order of
-// the splits, four columns a lane at a time, every load issued before the first use).
+// the splits, four columns a lane at a time). The first NB * 4 splits' columns are asked for beside the splits' maxima and sums: one trip to
+// memory instead of two and one more for every few splits (96 rows of 10 to 14 splits of 256 columns 3.8 > 3.2 us).
+template <int NB>
 __global__ void __launch_bounds__(256)
 latent_merge_kernel(const float* __restrict__ partials, int n_rows, int nsplit, int R, bf16_t* __restrict__ o_lat) {
     __shared__ float weights[4][64];
@@ -624,8 +639,17 @@ latent_merge_kernel(const float* __restrict__ partials, int n_rows, int nsplit, 
     const int row = blockIdx.x * 4 + wave;
     if (row >= n_rows) return;
     const float* st = partials + static_cast<size_t>(row) * nsplit * (R + 2);
-    const float* mine = st + static_cast<size_t>(min(lane, nsplit - 1)) * (R + 2);
-    const float m = lane < nsplit ? mine[0] : -INFINITY, l = lane < nsplit ? mine[1] : 0.f;
+    const float2 ml = *reinterpret_cast<const float2*>(st + static_cast<size_t>(min(lane, nsplit - 1)) * (R + 2));
+    // (R + 2 is even and a column's number a multiple of 4: the columns of a state are 8-byte aligned)
+    float2 a[4 * NB], b[4 * NB];
+    const int mine = min(4 * lane, R - 4);
+#pragma unroll
+    for (int sp = 0; sp < 4 * NB; ++sp) {
+        const float* cols = st + static_cast<size_t>(min(sp, nsplit - 1)) * (R + 2) + 2 + mine;
+        a[sp] = *reinterpret_cast<const float2*>(cols);
+        b[sp] = *reinterpret_cast<const float2*>(cols + 2);
+    }
+    const float m = lane < nsplit ? ml.x : -INFINITY, l = lane < nsplit ? ml.y : 0.f;
     const float M = wave_max(m);
     const float wgt = fast_exp2(m - M);
     const float inv = 1.0f / wave_sum(wgt * l);
@@ -633,18 +657,34 @@ latent_merge_kernel(const float* __restrict__ partials, int n_rows, int nsplit, 
     wave_lds_sync();
     for (int c = 4 * lane; c < R; c += 256) {
         float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
-        for (int sp = 0; sp < nsplit; ++sp) {
-            // (R + 2 is even and c a multiple of 4: the columns of a state are 8-byte aligned)
-            const float2 a = *reinterpret_cast<const float2*>(st + static_cast<size_t>(sp) * (R + 2) + 2 + c);
-            const float2 b = *reinterpret_cast<const float2*>(st + static_cast<size_t>(sp) * (R + 2) + 4 + c);
+        int sp = 0;
+        if (c < 256) {
+#pragma unroll
+            for (int k = 0; k < 4 * NB; ++k)
+                if (k < nsplit) {
+                    const float ws = weights[wave][k];
+                    acc.x += ws * a[k].x; acc.y += ws * a[k].y; acc.z += ws * b[k].x; acc.w += ws * b[k].y;
+                }
+            sp = 4 * NB;
+        }
+        for (; sp < nsplit; ++sp) {
+            const float2 x = *reinterpret_cast<const float2*>(st + static_cast<size_t>(sp) * (R + 2) + 2 + c);
+            const float2 y = *reinterpret_cast<const float2*>(st + static_cast<size_t>(sp) * (R + 2) + 4 + c);
             const float ws = weights[wave][sp];
-            acc.x += ws * a.x; acc.y += ws * a.y; acc.z += ws * b.x; acc.w += ws * b.y;
+            acc.x += ws * x.x; acc.y += ws * x.y; acc.z += ws * y.x; acc.w += ws * y.y;
         }
         uint2 pk;
         pk.x = pack_bf16x2(acc.x, acc.y);
         pk.y = pack_bf16x2(acc.z, acc.w);
         *reinterpret_cast<uint2*>(o_lat + static_cast<size_t>(row) * R + c) = pk;
     }
+}
+void latent_merge(const float* partials, int n_rows, int nsplit, int R, bf16_t* o_lat, hipStream_t stream) {
+    const int blocks = (n_rows + 3) / 4;
+    if (nsplit <= 4) latent_merge_kernel<1><<<blocks, 256, 0, stream>>>(partials, n_rows, nsplit, R, o_lat);
+    else if (nsplit <= 8) latent_merge_kernel<2><<<blocks, 256, 0, stream>>>(partials, n_rows, nsplit, R, o_lat);
+    else if (nsplit <= 12) latent_merge_kernel<3><<<blocks, 256, 0, stream>>>(partials, n_rows, nsplit, R, o_lat);
+    else latent_merge_kernel<4><<<blocks, 256, 0, stream>>>(partials, n_rows, nsplit, R, o_lat);
 }
 
 constexpr int MAX_LDS = 160 * 1024;
@@ -665,13 +705,11 @@ int mllm_latent_prepare(const float* dq, int ld_dq, int Rq, const float* wq, voi
     if (rot_dims < 0 || rot_dims % 2 != 0 || rot_dims > Dr || !(base > 0) || (vt_pages != nullptr && page_size < 1)) return -1;
     const double l2 = log2(base);
     if (dtype == MLLM_F32)
-        latent_prepare_kernel<float><<<T, 64, 0, stream>>>(dq, ld_dq, Rq, wq, static_cast<float*>(cq), ld_cq, dkv, ld_dkv, R, Dr, wkv,
-                                                           static_cast<float*>(pages), static_cast<float*>(vt_pages), page_size, slots, positions,
-                                                           eps, l2, rot_dims, Rn, half_split);
+        latent_prepare_kernel<float><<<T, 128, 0, stream>>>(dq, ld_dq, Rq, wq, dkv, ld_dkv, R, wkv, slots, positions, Dr, rot_dims, l2,
+            static_cast<float*>(cq), ld_cq, static_cast<float*>(pages), static_cast<float*>(vt_pages), page_size, eps, Rn, half_split);
     else
-        latent_prepare_kernel<bf16_t><<<T, 64, 0, stream>>>(dq, ld_dq, Rq, wq, static_cast<bf16_t*>(cq), ld_cq, dkv, ld_dkv, R, Dr, wkv,
-                                                            static_cast<bf16_t*>(pages), static_cast<bf16_t*>(vt_pages), page_size, slots, positions,
-                                                            eps, l2, rot_dims, Rn, half_split);
+        latent_prepare_kernel<bf16_t><<<T, 128, 0, stream>>>(dq, ld_dq, Rq, wq, dkv, ld_dkv, R, wkv, slots, positions, Dr, rot_dims, l2,
+            static_cast<bf16_t*>(cq), ld_cq, static_cast<bf16_t*>(pages), static_cast<bf16_t*>(vt_pages), page_size, eps, Rn, half_split);
     MLLM_LAUNCH_CHECK();
     return 0;
 }
@@ -797,8 +835,7 @@ int mllm_latent_attention_tiles(const void* qa, const void* k_pages, const void*
             nsplit, partials, single_tokens);                                                                        \
         MLLM_LAUNCH_CHECK();                                                                                         \
         if (nsplit > 1) {                                                                                            \
-            latent_merge_kernel<<<(n_rows + 3) / 4, 256, 0, stream>>>(partials, n_rows, nsplit, R,                   \
-                                                                     static_cast<bf16_t*>(o_lat));                  \
+            latent_merge(partials, n_rows, nsplit, R, static_cast<bf16_t*>(o_lat), stream);                          \
             MLLM_LAUNCH_CHECK();                                                                                     \
         }                                                                                                            \
         return 0;                                                                                                    \

@@ -1661,3 +1661,27 @@ def test_conv_of_one_token_a_sequence(T, C, taps):
     assert torch.equal(dev_state.cpu(), after)
     # a rounding of 2^-24 for each of up to nine terms of up to about 16, and the exponential's
     assert (out.cpu().double() - want).abs().max() <= 9 * 16 * 2.0 ** -23
+
+
+@pytest.mark.parametrize("R,Dr", [(64, 32), (256, 32), (512, 32)])
+@pytest.mark.parametrize("nsplit", [2, 4, 5, 8, 9, 12, 13, 16, 17, 20])
+def test_latent_attention_merges_every_number_of_splits(R, Dr, nsplit):
+    """The splits' states merged, around every four splits whose columns are asked for together, next to the same kernel without splits."""
+    import ctypes
+    g = torch.Generator().manual_seed(R + nsplit)
+    H, page, ctx, B = 5, 16, 64 * 20 + 7, 2
+    E, n_pages = R + Dr, -(-ctx // page)
+    qa = (_rand((B * H, E), torch.bfloat16, g)).to(DEV)
+    pages = _rand((B * n_pages, page, E), torch.bfloat16, g)
+    vt = pages[..., :R].transpose(1, 2).contiguous().to(DEV)
+    tables = torch.randperm(B * n_pages, generator=g).int().view(B, n_pages).to(DEV)
+    cu, lens = torch.arange(B + 1, dtype=torch.int32, device=DEV), torch.tensor([ctx, 3 * 64], dtype=torch.int32, device=DEV)
+    outs = []
+    for n in (1, nsplit):
+        out = torch.full((B * H, R), float("nan"), dtype=torch.bfloat16, device=DEV)
+        part = torch.full((B * H * n * (R + 2),), float("nan"), device=DEV)
+        assert _entry("latent_attention", "mllm_latent_attention_tiles", qa, pages.to(DEV), vt, tables, n_pages, cu, lens, B, B, H, R, Dr, page,
+                      ctypes.c_float(E ** -0.5), 0, out, B * H, n, part, 1, None) == 0
+        outs.append(out.cpu().double())
+    # weights are 16-bit operands of the second product: each split's maximum moves their rounding (2^-9 of each, at most 2^-8 of values of up to about 4)
+    assert (outs[0] - outs[1]).abs().max() <= 2.0 ** -6
