@@ -17,10 +17,15 @@ namespace {
 // are 2i and 2i + 1 (interleaved), or i and i + dims / 2 (half != 0).
 __device__ __forceinline__ int pair_first(int i, int half) { return half ? i : 2 * i; }
 __device__ __forceinline__ int pair_second(int i, int half, int dims) { return half ? i + dims / 2 : 2 * i + 1; }
-__device__ __forceinline__ void turn_pair(float u, float v, int pos, int i, double log2_base, int dims, float& a, float& b) {
+__device__ __forceinline__ void turn_of(int pos, int i, double log2_base, int dims, float& c, float& s) {
     const double f = exp2(-2.0 * static_cast<double>(i) / static_cast<double>(dims) * log2_base);
     const double angle = static_cast<double>(pos) * f;
-    const float c = static_cast<float>(cos(angle)), s = static_cast<float>(sin(angle));
+    c = static_cast<float>(cos(angle));
+    s = static_cast<float>(sin(angle));
+}
+__device__ __forceinline__ void turn_pair(float u, float v, int pos, int i, double log2_base, int dims, float& a, float& b) {
+    float c, s;
+    turn_of(pos, i, log2_base, dims, c, s);
     a = u * c - v * s;
     b = v * c + u * s;
 }
@@ -178,11 +183,11 @@ union Frag8 {
     uint32_t w[4];
 };
 
-// One small product per head on the matrix cores (bfloat16, fp32 sums), operands straight from memory:
+// One small product per head on the matrix cores (bfloat16, fp32 sums):
 //   out[t, h*out_hs + n] = sum_k a[t, h*a_hs + k] * w[(h*w_head_rows + n) * ldw + h*w_head_cols + k],  n < N, k < K
 // (w_head_rows = N, w_head_cols = 0: every head has its own rows of w; w_head_rows = 0, w_head_cols = K: its own
 // columns). A workgroup takes 64 tokens, one head and 64 values of n; a wavefront 16 tokens: the weights are the
-// MFMA's A operand, so a lane ends up with four neighbouring n of one token. K is a multiple of 32; rows and head
+// MFMA's A operand, so a lane ends up with four neighbouring n of one token. K is a multiple of 32 UN NCH; rows and head
 // offsets are 16-byte aligned. With `positions`, the workgroups of a head also carry the `tail` columns
 // behind a head's K inputs over to behind its N outputs, the first rot_dims of them turned in pairs. With `gate` (fp32
 // rows of H columns) head h's result is multiplied by sigmoid(gate[t, h]). The inputs are bfloat16 or fp32 rows (TA),
@@ -192,47 +197,70 @@ __device__ __forceinline__ u32x4 operand8(const float* p) {
     const float4 x = *reinterpret_cast<const float4*>(p), y = *reinterpret_cast<const float4*>(p + 4);
     return u32x4{pack_bf16x2(x.x, x.y), pack_bf16x2(x.z, x.w), pack_bf16x2(y.x, y.y), pack_bf16x2(y.z, y.w)};
 }
-// UN steps of the inner loop ask for their operands together (K is a multiple of 32 UN): one step at a time waits a round
-// trip to memory each.
-template <typename TA, int UN>
+// Both matrices pass through LDS in NCH chunks of 32 UN columns, asked for together, 16 bytes a lane and whole lines an instruction (rows in LDS
+// are an odd number of 16-byte pieces apart). Loaded in operand shape straight from memory, every wavefront asked for all the weights, 16 rows
+// an instruction: 40 KB a wavefront where a workgroup now takes 16 or 64 KB, at half the rate. An angle is worked out in double once
+// for up to four heads, a wavefront a workgroup having its share of them: once a head they were half of the kernel's instructions.
+// Bound by what it writes or reads. 2,048 tokens of 12 heads: 64 > 256 columns and 32 turned ones 13.0 > 8.1 us, 256 > 64 11.7 > 6.0.
+template <typename TA, int UN, int NCH>
 __global__ void __launch_bounds__(256)
 head_linear_mfma_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_t* __restrict__ w, int ldw, int w_head_rows,
-                        int w_head_cols, bf16_t* __restrict__ out, int ldo, int out_hs, int n_tokens, int N, int K,
-                        const int* __restrict__ positions, int tail, int rot_dims, double log2_base, int half,
-                        const float* __restrict__ gate, int ldg) {
+                        int w_head_cols, int n_tokens, int N, int K, const float* __restrict__ gate, bf16_t* __restrict__ out, int ldo, int out_hs,
+                        int ldg, int H, const int* __restrict__ positions, int tail, int rot_dims, double log2_base, int half) {
+    constexpr int KC = 32 * UN, ROW = KC + 8, PIECES = 4 * UN;          // columns of a chunk, elements between rows in LDS, 16-byte pieces of a row
+    __shared__ __attribute__((aligned(16))) bf16_t stage_s[2][64][ROW];
+    static_assert(sizeof(stage_s) >= 4 * 16 * 72 * sizeof(bf16_t), "the results pass through the same place");
     const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
     const int G = lane / 16, c16 = lane % 16;
     const int h = blockIdx.y, t0 = blockIdx.x * 64, n_base = blockIdx.z * 64;
-    const int tok = min(t0 + 16 * wave + c16, n_tokens - 1);
-    const TA* arow = a + static_cast<size_t>(tok) * lda + static_cast<size_t>(h) * a_hs + 8 * G;
-    const bf16_t* wbase = w + static_cast<size_t>(h) * w_head_rows * ldw + static_cast<size_t>(h) * w_head_cols + 8 * G;
-    const bf16_t* wrow[4];
-#pragma unroll
-    for (int ct = 0; ct < 4; ++ct) wrow[ct] = wbase + static_cast<size_t>(min(n_base + 16 * ct + c16, N - 1)) * ldw;
+    const TA* abase = a + static_cast<size_t>(t0) * lda + static_cast<size_t>(h) * a_hs;
+    const bf16_t* wbase = w + (static_cast<size_t>(h) * w_head_rows + n_base) * ldw + static_cast<size_t>(h) * w_head_cols;
+    const int last_t = n_tokens - 1 - t0, last_n = N - 1 - n_base;
     f32x4 acc[4];
 #pragma unroll
     for (int ct = 0; ct < 4; ++ct) acc[ct] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (int k0 = 0; k0 < K; k0 += 32 * UN) {
-        Frag8 af[UN], wf[UN][4];
+    for (int k0 = 0; k0 < K; k0 += KC * NCH) {
+        u32x4 aq[NCH][UN], wq[NCH][UN];
 #pragma unroll
-        for (int u = 0; u < UN; ++u) {
-            af[u].q = operand8(arow + k0 + 32 * u);
+        for (int c = 0; c < NCH; ++c)
 #pragma unroll
-            for (int ct = 0; ct < 4; ++ct) wf[u][ct].q = *reinterpret_cast<const u32x4*>(wrow[ct] + k0 + 32 * u);
+            for (int u = 0; u < UN; ++u) {
+                const int e = threadIdx.x + 256 * u, row = e / PIECES, col = k0 + KC * c + 8 * (e % PIECES);
+                aq[c][u] = operand8(abase + static_cast<size_t>(min(row, last_t)) * lda + col);
+                wq[c][u] = operand8(wbase + static_cast<size_t>(min(row, last_n)) * ldw + col);
+            }
+#pragma unroll
+        for (int c = 0; c < NCH; ++c) {
+            if (c > 0 || k0 > 0) lds_barrier();          // the chunk before has been read
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                const int e = threadIdx.x + 256 * u;
+                *reinterpret_cast<u32x4*>(&stage_s[0][e / PIECES][8 * (e % PIECES)]) = aq[c][u];
+                *reinterpret_cast<u32x4*>(&stage_s[1][e / PIECES][8 * (e % PIECES)]) = wq[c][u];
+            }
+            lds_barrier();
+#pragma unroll
+            for (int u = 0; u < UN; ++u) {
+                Frag8 af;
+                af.q = *reinterpret_cast<const u32x4*>(&stage_s[0][16 * wave + c16][32 * u + 8 * G]);
+#pragma unroll
+                for (int ct = 0; ct < 4; ++ct) {
+                    Frag8 wf;
+                    wf.q = *reinterpret_cast<const u32x4*>(&stage_s[1][16 * ct + c16][32 * u + 8 * G]);
+                    acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf.v, af.v, acc[ct], 0, 0, 0);
+                }
+            }
         }
-        __builtin_amdgcn_sched_barrier(0);              // (left alone the compiler moves each load to its use)
-#pragma unroll
-        for (int u = 0; u < UN; ++u)
-#pragma unroll
-            for (int ct = 0; ct < 4; ++ct) acc[ct] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u][ct].v, af[u].v, acc[ct], 0, 0, 0);
     }
+    const int tok = min(t0 + 16 * wave + c16, n_tokens - 1);
     const float g = gate != nullptr ? 1.f / (1.f + expf(-gate[static_cast<size_t>(tok) * ldg + h])) : 1.f;
     if (n_base + 64 <= N && ((ldo | out_hs) & 7) == 0 && (reinterpret_cast<uintptr_t>(out) & 15) == 0) {
-        // a whole tile: through LDS (this wavefront's own), so that a store instruction covers eight rows of 128 bytes
-        __shared__ __attribute__((aligned(16))) bf16_t tile_s[4][16][72];
+        // a whole tile: through LDS (this wavefront's own part), so that a store instruction covers eight rows of 128 bytes
+        lds_barrier();
+        bf16_t (*tile_s)[72] = reinterpret_cast<bf16_t (*)[72]>(&stage_s[0][0][0]) + 16 * wave;
 #pragma unroll
         for (int ct = 0; ct < 4; ++ct)
-            *reinterpret_cast<uint2*>(&tile_s[wave][c16][16 * ct + 4 * G]) =
+            *reinterpret_cast<uint2*>(&tile_s[c16][16 * ct + 4 * G]) =
                 make_uint2(pack_bf16x2(acc[ct][0] * g, acc[ct][1] * g), pack_bf16x2(acc[ct][2] * g, acc[ct][3] * g));
         wave_lds_sync();
 #pragma unroll
@@ -240,7 +268,7 @@ head_linear_mfma_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_
             const int r = 8 * u + lane / 8, t = t0 + 16 * wave + r;
             if (t < n_tokens)
                 *reinterpret_cast<u32x4*>(out + static_cast<size_t>(t) * ldo + static_cast<size_t>(h) * out_hs + n_base + 8 * (lane % 8)) =
-                    *reinterpret_cast<const u32x4*>(&tile_s[wave][r][8 * (lane % 8)]);
+                    *reinterpret_cast<const u32x4*>(&tile_s[r][8 * (lane % 8)]);
         }
     } else if (t0 + 16 * wave + c16 < n_tokens) {
         bf16_t* orow = out + static_cast<size_t>(tok) * ldo + static_cast<size_t>(h) * out_hs;
@@ -253,18 +281,29 @@ head_linear_mfma_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_
         }
     }
     if (positions != nullptr) {
-        // (pairs and plain columns in loops of their own: a wavefront that holds both would run the turn for a third of its lanes; dealt out over
-        // the workgroups of all n tiles: done by those of the first alone they are what 2,048 tokens wait for)
+        // (pairs and plain columns in loops of their own: a wavefront that holds both would run the turn for a third of its lanes. The tile's pairs are
+        // dealt out, 64 at a time, over the workgroups of four heads and all their n tiles, which turn them for the four.)
         const int nt = min(64, n_tokens - t0), pairs = rot_dims / 2, plain = tail - rot_dims;
-        for (int i = threadIdx.x + 256 * blockIdx.z; i < nt * pairs; i += 256 * gridDim.z) {
+        const int h0 = h & ~3, heads = min(4, H - h0), shares = heads * gridDim.z, share = blockIdx.z * heads + (h - h0);
+        for (int i = 64 * (share + shares * wave) + lane; i < nt * pairs; i += 256 * shares) {
             const int tt = i / pairs, k = i % pairs;
-            const TA* src = a + static_cast<size_t>(t0 + tt) * lda + static_cast<size_t>(h) * a_hs + K;
-            bf16_t* dst = out + static_cast<size_t>(t0 + tt) * ldo + static_cast<size_t>(h) * out_hs + N;
-            float u, v;
             const int first = pair_first(k, half), second = pair_second(k, half, rot_dims);
-            turn_pair(to_float(src[first]), to_float(src[second]), positions[t0 + tt], k, log2_base, rot_dims, u, v);
-            dst[first] = float_to_bf16(u);
-            dst[second] = float_to_bf16(v);
+            const TA* src = a + static_cast<size_t>(t0 + tt) * lda + static_cast<size_t>(h0) * a_hs + K;
+            bf16_t* dst = out + static_cast<size_t>(t0 + tt) * ldo + static_cast<size_t>(h0) * out_hs + N;
+            float us[4], vs[4], c, s;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const TA* from = src + static_cast<size_t>(min(j, heads - 1)) * a_hs;
+                us[j] = to_float(from[first]);
+                vs[j] = to_float(from[second]);
+            }
+            turn_of(positions[t0 + tt], k, log2_base, rot_dims, c, s);
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
+                if (j < heads) {
+                    dst[static_cast<size_t>(j) * out_hs + first] = float_to_bf16(us[j] * c - vs[j] * s);
+                    dst[static_cast<size_t>(j) * out_hs + second] = float_to_bf16(vs[j] * c + us[j] * s);
+                }
         }
         for (int i = threadIdx.x + 256 * blockIdx.z; i < nt * plain; i += 256 * gridDim.z) {
             const int tt = i / plain, c = rot_dims + i % plain;
@@ -272,6 +311,84 @@ head_linear_mfma_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_
                 float_to_bf16(to_float(a[static_cast<size_t>(t0 + tt) * lda + static_cast<size_t>(h) * a_hs + K + c]));
         }
     }
+}
+
+// The same with turned columns for up to 16 tokens (the same sums): these columns are a workgroup's of their own, beside the others instead of
+// behind them, and a wavefront takes 16 of the workgroup's 64 columns, with operands straight from memory. Bound by the chain of a load, an angle
+// and a store. 8 tokens of 12 heads, 64 > 256 columns and 32 turned ones 4.5 > 3.0 us in a step.
+template <typename TA, int UN>
+__global__ void __launch_bounds__(256)
+head_linear_few_kernel(const TA* __restrict__ a, int lda, int a_hs, const bf16_t* __restrict__ w, int ldw, int w_head_rows,
+                       int w_head_cols, int n_tokens, int N, int K, bf16_t* __restrict__ out, int ldo, int out_hs, const int* __restrict__ positions,
+                        int tail, int rot_dims, double log2_base, int half) {
+    const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+    const int h = blockIdx.y, n_base = blockIdx.z * 64;
+    if (n_base >= N) {                   // the last of a head
+        const int pairs = rot_dims / 2, plain = tail - rot_dims;
+        for (int i = threadIdx.x; i < n_tokens * pairs; i += 256) {
+            const int t = i / pairs, k = i % pairs;
+            const TA* src = a + static_cast<size_t>(t) * lda + static_cast<size_t>(h) * a_hs + K;
+            bf16_t* dst = out + static_cast<size_t>(t) * ldo + static_cast<size_t>(h) * out_hs + N;
+            const int first = pair_first(k, half), second = pair_second(k, half, rot_dims);
+            float u, v;
+            turn_pair(to_float(src[first]), to_float(src[second]), positions[t], k, log2_base, rot_dims, u, v);
+            dst[first] = float_to_bf16(u);
+            dst[second] = float_to_bf16(v);
+        }
+        for (int i = threadIdx.x; i < n_tokens * plain; i += 256) {
+            const int t = i / plain, c = rot_dims + i % plain;
+            out[static_cast<size_t>(t) * ldo + static_cast<size_t>(h) * out_hs + N + c] =
+                float_to_bf16(to_float(a[static_cast<size_t>(t) * lda + static_cast<size_t>(h) * a_hs + K + c]));
+        }
+        return;
+    }
+    if (n_base + 16 * wave >= N) return;
+    const int G = lane / 16, c16 = lane % 16, tok = min(c16, n_tokens - 1), col = min(n_base + 16 * wave + c16, N - 1);
+    const TA* arow = a + static_cast<size_t>(tok) * lda + static_cast<size_t>(h) * a_hs + 8 * G;
+    const bf16_t* wrow = w + static_cast<size_t>(h) * w_head_rows * ldw + static_cast<size_t>(h) * w_head_cols + static_cast<size_t>(col) * ldw + 8 * G;
+    f32x4 acc{0.f, 0.f, 0.f, 0.f};
+    for (int k0 = 0; k0 < K; k0 += 32 * UN) {
+        Frag8 af[UN], wf[UN];
+#pragma unroll
+        for (int u = 0; u < UN; ++u) {
+            wf[u].q = *reinterpret_cast<const u32x4*>(wrow + k0 + 32 * u);
+            af[u].q = operand8(arow + k0 + 32 * u);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < UN; ++u) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[u].v, af[u].v, acc, 0, 0, 0);
+    }
+    if (c16 >= n_tokens) return;
+    const int n = n_base + 16 * wave + 4 * G;                  // acc[r] is output n + r of this lane's token
+    bf16_t* orow = out + static_cast<size_t>(c16) * ldo + static_cast<size_t>(h) * out_hs;
+    if (n + 4 <= N && ((ldo | out_hs) & 3) == 0 && (reinterpret_cast<uintptr_t>(out) & 7) == 0) {
+        *reinterpret_cast<uint2*>(orow + n) = make_uint2(pack_bf16x2(acc[0], acc[1]), pack_bf16x2(acc[2], acc[3]));
+    } else {
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (n + r < N) orow[n + r] = float_to_bf16(acc[r]);
+    }
+}
+// 16 tokens are one tile of the matrix instruction; the kernel for few takes no second one (16 tokens 2.7 us there, 17 here 3.9). Products without
+// turned columns have nothing to gain from it: 256 > 64 of 8 tokens 3.96 us there, 4.04 here, in a step.
+template <typename TA>
+void head_linear(const TA* a, int lda, int a_hs, const bf16_t* w, int ldw, int w_head_rows, int w_head_cols, bf16_t* out, int ldo, int out_hs,
+                 int n_tokens, int H, int N, int K, const int* positions, int tail, int rot_dims, double log2_base, int half, const float* gate,
+                 int ldg, hipStream_t stream) {
+    const int tiles = (N + 63) / 64;
+    if (n_tokens <= 16 && positions != nullptr) {
+#define FEW(UN)                                                                                                                            \
+    head_linear_few_kernel<TA, UN><<<dim3(1, H, tiles + 1), 256, 0, stream>>>(                                                             \
+        a, lda, a_hs, w, ldw, w_head_rows, w_head_cols, n_tokens, N, K, out, ldo, out_hs, positions, tail, rot_dims, log2_base, half)
+        if (K % 128 == 0) FEW(4); else if (K % 64 == 0) FEW(2); else FEW(1);
+#undef FEW
+        return;
+    }
+#define MANY(UN, NCH)                                                                                                                      \
+    head_linear_mfma_kernel<TA, UN, NCH><<<dim3((n_tokens + 63) / 64, H, tiles), 256, 0, stream>>>(                                        \
+        a, lda, a_hs, w, ldw, w_head_rows, w_head_cols, n_tokens, N, K, gate, out, ldo, out_hs, ldg, H, positions, tail, rot_dims, log2_base, half)
+    if (K % 256 == 0) MANY(4, 2); else if (K % 128 == 0) MANY(4, 1); else if (K % 64 == 0) MANY(2, 1); else MANY(1, 1);
+#undef MANY
 }
 
 // Attention of one token's heads over its sequence's page rows. One workgroup per (token, group of up to HG
@@ -725,13 +842,12 @@ int mllm_latent_absorb(const void* q, int ldq, const void* w_uk, int ldw, void* 
     const double l2 = log2(base);
     const auto aligned16 = [](const void* ptr) { return (reinterpret_cast<uintptr_t>(ptr) & 15) == 0; };
     if (dtype == MLLM_BF16 && Dn % 32 == 0 && ldq % 8 == 0 && (Dn + Dr) % 8 == 0 && ldw % 8 == 0 && aligned16(q) && aligned16(w_uk)) {
-#define ABSORB_MFMA(TQ, UN)                                                                                                            \
-    head_linear_mfma_kernel<TQ, UN><<<dim3((T + 63) / 64, H, (R + 63) / 64), 256, 0, stream>>>(                                               \
-        static_cast<const TQ*>(q), ldq, Dn + Dr, static_cast<const bf16_t*>(w_uk), ldw, 0, Dn, static_cast<bf16_t*>(qa), ldqa, R + Dr, T, R, \
-        Dn, positions, Dr, rot_dims, l2, half_split, nullptr, 0)
-        if (q_dtype == MLLM_F32) { if (Dn % 64 == 0) ABSORB_MFMA(float, 2); else ABSORB_MFMA(float, 1); }
-        else { if (Dn % 64 == 0) ABSORB_MFMA(bf16_t, 2); else ABSORB_MFMA(bf16_t, 1); }
-#undef ABSORB_MFMA
+        if (q_dtype == MLLM_F32)
+            head_linear(static_cast<const float*>(q), ldq, Dn + Dr, static_cast<const bf16_t*>(w_uk), ldw, 0, Dn, static_cast<bf16_t*>(qa), ldqa, R + Dr, T, H, R,
+                        Dn, positions, Dr, rot_dims, l2, half_split, nullptr, 0, stream);
+        else
+            head_linear(static_cast<const bf16_t*>(q), ldq, Dn + Dr, static_cast<const bf16_t*>(w_uk), ldw, 0, Dn, static_cast<bf16_t*>(qa), ldqa, R + Dr, T, H, R,
+                        Dn, positions, Dr, rot_dims, l2, half_split, nullptr, 0, stream);
         MLLM_LAUNCH_CHECK();
         return 0;
     }
@@ -851,12 +967,8 @@ int mllm_latent_expand(const void* o_lat, int ldo, const void* w_uv, int ldw, vo
     if (T <= 0) return 0;
     if (dtype == MLLM_BF16 && R % 32 == 0 && ldo % 8 == 0 && ldw % 8 == 0 && (reinterpret_cast<uintptr_t>(o_lat) & 15) == 0 &&
         (reinterpret_cast<uintptr_t>(w_uv) & 15) == 0) {
-#define EXPAND_MFMA(UN)                                                                                                                  \
-    head_linear_mfma_kernel<bf16_t, UN><<<dim3((T + 63) / 64, H, (Dv + 63) / 64), 256, 0, stream>>>(                                        \
-        static_cast<const bf16_t*>(o_lat), ldo, R, static_cast<const bf16_t*>(w_uv), ldw, Dv, 0, static_cast<bf16_t*>(out), ldout, Dv, T, Dv, R, \
-        nullptr, 0, 0, 0.0, 0, gate, ldg)
-        if (R % 128 == 0) EXPAND_MFMA(4); else if (R % 64 == 0) EXPAND_MFMA(2); else EXPAND_MFMA(1);
-#undef EXPAND_MFMA
+        head_linear(static_cast<const bf16_t*>(o_lat), ldo, R, static_cast<const bf16_t*>(w_uv), ldw, Dv, 0, static_cast<bf16_t*>(out), ldout, Dv, T, H, Dv, R,
+                    static_cast<const int*>(nullptr), 0, 0, 0.0, 0, gate, ldg, stream);
         MLLM_LAUNCH_CHECK();
         return 0;
     }

@@ -1634,6 +1634,49 @@ def _entry(library, name, *args):
     return rc
 
 
+@pytest.mark.parametrize("T", [1, 15, 16, 17, 63, 64, 65, 130])
+@pytest.mark.parametrize("H,Dn,Dr,R,Dv,rot,half", [(12, 64, 32, 256, 64, 32, 0), (5, 32, 16, 128, 96, 8, 1), (1, 96, 32, 512, 40, 32, 0), (7, 128, 64, 96, 128, 64, 1),
+                                                   (6, 64, 0, 100, 72, 0, 0)])
+@pytest.mark.parametrize("wide", [False, True])          # queries in 32 bits, results behind a gate
+def test_latent_products_per_head(T, H, Dn, Dr, R, Dv, rot, half, wide):
+    """Queries into the latent space and results out of it: up to 16 tokens (a kernel of their own) and more, heads that are no multiple of 4,
+    output columns that are no multiple of 64, and the turned columns next to their angles in double."""
+    import ctypes
+    g = torch.Generator().manual_seed(T + R + H)
+    E, q_dtype = R + Dr, torch.float32 if wide else torch.bfloat16
+    q, w = _rand((T, H * (Dn + Dr)), q_dtype, g), _rand((R, H * Dn), torch.bfloat16, g, std=Dn ** -0.5)
+    pos = torch.randint(0, 8000, (T,), generator=g, dtype=torch.int32)
+    qa = torch.full((T, H * E), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert _entry("latent_attention", "mllm_latent_absorb", q.to(DEV), H * (Dn + Dr), w.to(DEV), H * Dn, qa, H * E, pos.to(DEV), T, H, Dn, Dr, R,
+                  ctypes.c_double(1e4), rot, 1, None, 0 if wide else 1, half) == 0
+    rows = q.view(T, H, Dn + Dr).double()
+    plain = rows[..., :Dn].bfloat16().double()
+    want = torch.einsum("thd,rhd->thr", plain, w.view(R, H, Dn).double())
+    size = torch.einsum("thd,rhd->thr", plain.abs(), w.view(R, H, Dn).double().abs())
+    tail = rows[..., Dn:].clone()
+    i = torch.arange(rot // 2)
+    a, b = (i, i + rot // 2) if half else (2 * i, 2 * i + 1)
+    if rot:
+        angle = pos.double()[:, None, None] * 1e4 ** (-2.0 * i.double() / rot)
+        tail[..., a], tail[..., b] = (rows[..., Dn + a] * angle.cos() - rows[..., Dn + b] * angle.sin(), rows[..., Dn + b] * angle.cos() + rows[..., Dn + a] * angle.sin())
+    got = qa.cpu().view(T, H, E).double()
+    # one rounding to 8 bits of mantissa, 32-bit sums before it
+    assert ((got[..., :R] - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -22 * size).all()
+    assert ((got[..., R:] - tail).abs() <= 2.0 ** -8 * tail.abs() + 2.0 ** -20).all()
+    if R % 32:
+        return
+    o, wv = _rand((T, H * R), torch.bfloat16, g), _rand((H * Dv, R), torch.bfloat16, g, std=R ** -0.5)
+    gate = _rand((T, H), torch.float32, g) if wide else None
+    out = torch.full((T, H * Dv), float("nan"), dtype=torch.bfloat16, device=DEV)
+    assert _entry("latent_attention", "mllm_latent_expand", o.to(DEV), H * R, wv.to(DEV), R, out, H * Dv, T, H, Dv, R, 1, None,
+                  gate.to(DEV) if wide else None, H if wide else 0) == 0
+    want = torch.einsum("thr,hvr->thv", o.view(T, H, R).double(), wv.view(H, Dv, R).double())
+    size = torch.einsum("thr,hvr->thv", o.view(T, H, R).double().abs(), wv.view(H, Dv, R).double().abs())
+    if wide:
+        want, size = want * torch.sigmoid(gate.double())[..., None], size * torch.sigmoid(gate.double())[..., None]
+    assert ((out.cpu().view(T, H, Dv).double() - want).abs() <= 2.0 ** -8 * want.abs() + 2.0 ** -21 * size).all()
+
+
 @pytest.mark.parametrize("C,taps", [(4, 2), (252, 4), (256, 3), (260, 8), (1792, 4), (1028, 5)])
 @pytest.mark.parametrize("T", [1, 8])
 def test_conv_of_one_token_a_sequence(T, C, taps):
