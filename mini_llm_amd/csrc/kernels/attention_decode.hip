@@ -109,7 +109,7 @@ decode_attention_kernel(// the first 14 dwords arrive in registers with the wave
     // (the words as launch_decode packs them)
     const int n_heads = heads & 0xffff, n_kv_heads = heads >> 16;
     const int max_blocks = form & 0x1fff, shift = form >> 13 & 31, n_waves = form >> 18 & 31;
-    const bool windowed = form >> 23 & 1, append = form >> 24 & 1, one_each = form >> 25 & 1;
+    const bool windowed = form >> 23 & 1, append = !SHAPED && (form >> 24 & 1), one_each = form >> 25 & 1;      // (shaped scores: the pages hold every key)
 
     // workgroups: (head, split, token)
     const int h = blockIdx.x, split = blockIdx.y, t = blockIdx.z;
@@ -219,14 +219,18 @@ decode_attention_kernel(// the first 14 dwords arrive in registers with the wave
             j[u] = key_at(min(j0 + u * group_keys + g, ke_pages - 1));
             block[u] = sm_table[(j[u] >> shift) - first_blk];
         }
-        __builtin_amdgcn_sched_barrier(0);      // (the table's entries together, then the loads together: left alone the compiler
-#pragma unroll                                  // widens the first keys, and waits for them, between the others' requests)
+        // (The table's entries together, then the loads together: left alone the compiler widens the first keys, and waits for them, between
+        // the others' requests. Shaped scores, and heads that fill a wavefront with one key, have the work for that wait: 16 heads of 128 in 32
+        // bits, one token of 4,096 keys 26.8 us so and 24.8 without, 8 heads of 256 2 % without.)
+        constexpr bool ALL_AT_ONCE = !SHAPED && KPW > 1;
+        if (ALL_AT_ONCE) __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
         for (int u = 0; u < UNR; ++u) {
             const uint64_t at = static_cast<uint64_t>((static_cast<uint32_t>(block[u]) << shift) + (j[u] & mask)) * static_cast<uint32_t>(kv_dim);
             kraw[u] = load_stream16(k_col_pages + at);
             vraw[u] = load_stream16(v_col_pages + at);
         }
-        __builtin_amdgcn_sched_barrier(0);
+        if (ALL_AT_ONCE) __builtin_amdgcn_sched_barrier(0);
         float dot[UNR];
         float mx = NEG;
 #pragma unroll
@@ -338,6 +342,16 @@ decode_attention_kernel(// the first 14 dwords arrive in registers with the wave
         const float2 ml = sm_ml[min(lane, n_waves - 1)];
         const int at = (lane * EW) % DH;
         float wm[DEC_MAX_WAVES] = {}, wl[DEC_MAX_WAVES] = {}, wo[DEC_MAX_WAVES][EW] = {};
+        auto join = [&](int x, int y) {        // state y into state x
+            const float mn = fmaxf(wm[x], wm[y]), a = exp2_for<T>(wm[x] - mn), b2 = exp2_for<T>(wm[y] - mn);
+            wl[x] = fmaf(wl[x], a, wl[y] * b2);
+#pragma unroll
+            for (int e = 0; e < EW; ++e) wo[x][e] = fmaf(wo[y][e], b2, wo[x][e] * a);
+            wm[x] = mn;
+        };
+        // (four elements of 16 wavefronts and more: each four are joined before the next are read, which then needs a quarter of the
+        // registers; 8 heads of 256 and 40 keys 6.3 > 6.1 us in 32 bits. The order is the same.)
+        constexpr bool JOIN_AT_ONCE = EW >= 4;
 #pragma unroll
         for (int w0 = 0; w0 < DEC_MAX_WAVES; w0 += 4) {
             if (w0 >= n_waves) continue;
@@ -348,17 +362,15 @@ decode_attention_kernel(// the first 14 dwords arrive in registers with the wave
                 wm[w] = row_lane(ml.x, w);
                 wl[w] = row_lane(ml.y, w);
             }
+            if (JOIN_AT_ONCE)
+#pragma unroll
+                for (int y = w0; y < w0 + 4; ++y)
+                    if (y >= KPW && y < n_waves) join(y % KPW, y);
         }
-        auto join = [&](int x, int y) {        // state y into state x
-            const float mn = fmaxf(wm[x], wm[y]), a = exp2_for<T>(wm[x] - mn), b2 = exp2_for<T>(wm[y] - mn);
-            wl[x] = fmaf(wl[x], a, wl[y] * b2);
+        if (!JOIN_AT_ONCE)
 #pragma unroll
-            for (int e = 0; e < EW; ++e) wo[x][e] = fmaf(wo[y][e], b2, wo[x][e] * a);
-            wm[x] = mn;
-        };
-#pragma unroll
-        for (int y = KPW; y < DEC_MAX_WAVES; ++y)
-            if (y < n_waves) join(y % KPW, y);
+            for (int y = KPW; y < DEC_MAX_WAVES; ++y)
+                if (y < n_waves) join(y % KPW, y);
 #pragma unroll
         for (int d = 1; d < KPW && d < DEC_MAX_WAVES; d <<= 1)
 #pragma unroll
@@ -547,7 +559,7 @@ long mllm_decode_attention_ws_floats(int n_q, int n_heads, int head_dim, int nsp
 // must be a power of two in [2, 64], page_size a power of two, and max_blocks at most 4096. `counters` holds n_q*n_heads ints that are zero before the
 // first launch (the kernel leaves them zero). With `slots` (n_q rows of the page pools, < 0: none) the
 // tokens' own keys/values are taken from columns k_col/v_col of q and written to the pages by this
-// kernel; without, they must be in the pages already.
+// kernel; without, they must be in the pages already, as they must for shaped scores (-1 otherwise).
 // partial_out != 0: nothing is written to `out`; the workspace holds, for pair = token * n_heads + head
 // and split s, the unnormalised output at ws[(pair * nsplit + s) * head_dim ..] and (maximum in base 2,
 // sum) at ws[n_q * n_heads * nsplit * head_dim + (pair * nsplit + s) * 2 ..]; a split without keys has
@@ -573,6 +585,8 @@ int mllm_decode_attention(const void* q, int q_stride, int q_col, const void* k_
     if (gate != nullptr && (shape == nullptr || partial_out)) return -1;
     // (weights that are not normalised leave no sum for another kernel to divide by)
     if (shape && shape->sigmoid && partial_out) return -1;
+    // (the kernels of shaped scores read every key from the pages)
+    if (shape && slots != nullptr) return -1;
     // (tokens are the grid's third dimension, which takes 65,535)
     for (int t0 = 0; t0 < n_q; t0 += 65535) {
         const dim3 grid(n_heads, nsplit, std::min(n_q - t0, 65535));
