@@ -573,7 +573,7 @@ template <int MS> struct SplitStates {
 };
 
 template <int MT, int ASRC, bool SPLIT_K, int U, bool A_TWO = true, int NT = 1, bool THROUGH = false, int MS = MERGE_MAX_SPLITS,
-          bool ONE = false, bool GATED = false, int NU = 8, int WC = 16, int KP = 1>
+          bool ONE = false, bool GATED = false, int NU = 8, int WC = 16, int KP = 1, bool IN_TURN = false>
 __global__ void __launch_bounds__(ASRC == A_NORMED ? 512 : (ASRC == A_GLOBAL || ASRC == A_MERGED ? 768 : 1024))
 gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, and hold everything that the first loads need: an argument
                  // behind them comes with a load of its own from memory that no cache holds (as does blockDim), 0.6 to 0.8 us
@@ -604,6 +604,10 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
     // KP == 2: the two parts of K that two workgroups would take, one behind the other in every wavefront, with sums of their own that
     // are added at the end as the workgroups' would be: the same bits without the exchange through memory (the launcher's k_parts).
     static_assert(KP == 1 || (KP == 2 && ONE && SPLIT_K && MT == 1 && NT == 1 && ASRC == A_GLOBAL), "parts of K in one workgroup: kernels of one chunk");
+    // IN_TURN: the rows of A are asked for block by block beside the weights, else all of a chunk's in front of them. What comes first is used
+    // first: with a few blocks the rows, which come from L2 and are short behind weights; over a longer stretch of K the blocks,
+    // whose weights the products then need not wait for (see the launcher).
+    static_assert(!IN_TURN || (ASRC == A_GLOBAL && NT == 1 && WC == 16), "rows in turn: whole column tiles");
     constexpr int T = MT * NT;      // accumulators: row tiles (NT == 1) or column tiles (MT == 1)
     constexpr int REDUCED = ASRC == A_NORMED ? 8 : 12;      // wavefronts whose sums meet, at most (SPLIT_K)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
@@ -756,8 +760,11 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             arow[j] = A + static_cast<size_t>(arow_idx[j]) * lda;
         }
     }
-    // (lanes of rows beyond M ask for nothing: what they multiply reaches only outputs that are not stored)
-    const bool row_exists[2] = {m_base + lr < M, m_base + lr + 8 < M};
+    // (Lanes of rows beyond M ask for nothing: what they multiply reaches only outputs that are not stored. Where rows stand in turn with
+    // weights, or splits are merged, for more than 8 rows they ask for the last row again: under a condition those kernels kept up to
+    // 70 registers more in scratch memory, 5 heads of 256, 12 rows of four splits 25.0 us against 22.9.)
+    constexpr bool EVERY_ROW = A_TWO && (IN_TURN || ASRC == A_MERGED);
+    const bool row_exists[2] = {EVERY_ROW || m_base + lr < M, EVERY_ROW || m_base + lr + 8 < M};
     // A_MERGED: requests the splits' states for the 8 elements from k on of row `row` (all loads together; n_splits is MS),
     // and merges them later
     auto fetch_splits = [&](SplitStates<MS>& st, int row, int k) {
@@ -842,10 +849,11 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             const int k = min(k0 + 8 * piece[j], K - 8);
 #pragma unroll
             for (int t = 0; t < NT; ++t) c.b[t][WC == 16 ? u0 + j : u0 / 2] = load_piece(wrow[t][j] + k);
+            if (IN_TURN && (j == 0 || a_two) && row_exists[j]) c.a[A_TWO ? u0 + j : u0 / 2] = *reinterpret_cast<const bf16x8*>(arow[j] + k);
         }
     };
     auto load_rows = [&](Chunk& c, int count, auto k_of) {      // rows of A for the first `count` blocks of a chunk, block h at k_of(h)
-        if (ASRC != A_GLOBAL) return;       // (A_MERGED: the splits' states were requested before and are merged after the weights)
+        if (ASRC != A_GLOBAL || IN_TURN) return;       // (A_MERGED: the splits' states were requested before and are merged after the weights)
 #pragma unroll
         for (int j = 0; j < 2; ++j) {
             if ((j == 1 && !a_two) || !row_exists[j]) continue;
@@ -901,7 +909,8 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
             for (int half = 0; half < 2; ++half) {
                 const int k = k0 + i * k_stride + 16 * kq + 8 * half;
                 const int kc = min(k, K - 8);
-                const bool whole = k0 + i * k_stride + 64 <= K;       // (uniform over the wavefront)
+                // (uniform over the wavefront; where the rows are in registers too, a branch costs them more than the comparison)
+                const bool whole = IN_LDS && k0 + i * k_stride + 64 <= K;
 #pragma unroll
                 for (int mi = 0; mi < MT; ++mi) {
                     bf16x8 a;
@@ -1332,7 +1341,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
             k_parts = 1;
         k_blocks = (k_blocks + k_parts - 1) / k_parts;      // per workgroup from here on
     }
-    // Two parts and at most 8 rows: one workgroup takes both, and the columns are dealt out to 256 workgroups (5 to 8 each) instead. What
+    // Two parts and at most 8 rows: one workgroup takes both, and the columns are dealt out to 256 workgroups (6 to 8 each) instead. What
     // it saves is the exchange of the parts' sums (stores, fences, a counter: about 2 us). 1,600 x 6,400 7.9 > 6.5 us at 1 row, 8.7 > 7.5 at
     // 8 (a chunk of five blocks with the exchange as it was: 7.6 and 8.4).
     const bool parts_inside = k_parts == 2 && M <= 8 && (N + 255) / 256 <= 8 && (k_blocks + 11) / 12 <= 6;
@@ -1421,10 +1430,10 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
     const void* p2 = LN_FUSED ? gamma : MERGED ? merged.split_ml : bias;
     const void* p3 = LN_FUSED ? (gated != nullptr ? static_cast<const void*>(gated->up) : beta) : MERGED ? static_cast<const void*>(bias) : C;
 #define SKINNY_KERNEL(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, ...) SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, false, 8, 16, __VA_ARGS__)
-#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, ...) SKINNY_PARTS(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, 1, __VA_ARGS__)
-#define SKINNY_PARTS(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, KPV, ...)                 \
+#define SKINNY_ANY(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, ...) SKINNY_PARTS(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, 1, false, __VA_ARGS__)
+#define SKINNY_PARTS(SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, KPV, TURN, ...)           \
     do {                                                                                               \
-        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, KPV>; \
+        auto kernel = gemm_bf16_skinny<1, ASRC, SPLIT, UV, A2, NTV, THROUGH, MSV, ONE, GATED, NUV, WCV, KPV, TURN>; \
         static bool lds_allowed = false;      /* more than 64 KB of dynamic LDS has to be asked for once */ \
         if (!lds_allowed) {                                                                            \
             hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),                  \
@@ -1435,18 +1444,19 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
         kernel<<<grid, block, smem, stream>>>(W, MERGED ? merged.split_o : A, p2, p3, ldw, columns, shape, MERGED ? ldc : K, \
                                               MERGED ? C : strides, bias, C, rows, eps, part_sums, part_counters, __VA_ARGS__); \
     } while (0)
-#define SKINNY_LAUNCH(SPLIT, UV, A2, NTV, ONE)                                                         \
+#define SKINNY_TURNED(SPLIT, UV, A2, NTV, ONE, TURN)                                                   \
     do {                                                                                               \
         if constexpr (ASRC == A_GLOBAL) {                                                              \
-            if (through != nullptr) { SKINNY_KERNEL(SPLIT, UV, A2, NTV, true, MERGE_MAX_SPLITS, ONE, *through); break; } \
+            if (through != nullptr) { SKINNY_PARTS(SPLIT, UV, A2, NTV, true, MERGE_MAX_SPLITS, ONE, false, 8, 16, 1, TURN, *through); break; } \
         }                                                                                              \
-        SKINNY_KERNEL(SPLIT, UV, A2, NTV, false, MERGE_MAX_SPLITS, ONE, kv);                           \
+        SKINNY_PARTS(SPLIT, UV, A2, NTV, false, MERGE_MAX_SPLITS, ONE, false, 8, 16, 1, TURN, kv);     \
     } while (0)
+#define SKINNY_LAUNCH(SPLIT, UV, A2, NTV, ONE) SKINNY_TURNED(SPLIT, UV, A2, NTV, ONE, false)
 // one chunk of UV / 2 blocks, or several
-#define SKINNY_CHUNKS(UV, A2, NTV)                                                                     \
+#define SKINNY_CHUNKS(UV, A2, NTV, TURN)                                                               \
     do {                                                                                               \
-        if (per_wave <= UV / 2) SKINNY_LAUNCH(true, UV, A2, NTV, true);                                \
-        else SKINNY_LAUNCH(true, UV, A2, NTV, false);                                                  \
+        if (per_wave <= UV / 2) SKINNY_TURNED(true, UV, A2, NTV, true, TURN);                          \
+        else SKINNY_TURNED(true, UV, A2, NTV, false, TURN);                                            \
     } while (0)
 // the same with narrow column tiles: chunks of four blocks
 #define SKINNY_NARROW(WCV)                                                                              \
@@ -1510,7 +1520,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 #undef SKINNY_NORMED
         } else if (two_tiles) {
             // (two tiles per chunk slot: half the blocks per chunk)
-            SKINNY_CHUNKS(2, false, 2);
+            SKINNY_CHUNKS(2, false, 2, false);
         } else if (M <= 8) {
             switch (std::min(per_wave, 4)) {
                 case 1: SKINNY_LAUNCH(true, 2, false, 1, true); break;
@@ -1521,8 +1531,8 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
                         if (parts_inside) {
 #define SKINNY_INSIDE(UV)                                                                              \
     do {                                                                                               \
-        if (through != nullptr) SKINNY_PARTS(true, UV, false, 1, true, MERGE_MAX_SPLITS, true, false, 8, 8, 2, *through); \
-        else SKINNY_PARTS(true, UV, false, 1, false, MERGE_MAX_SPLITS, true, false, 8, 8, 2, kv);       \
+        if (through != nullptr) SKINNY_PARTS(true, UV, false, 1, true, MERGE_MAX_SPLITS, true, false, 8, 8, 2, false, *through); \
+        else SKINNY_PARTS(true, UV, false, 1, false, MERGE_MAX_SPLITS, true, false, 8, 8, 2, false, kv);       \
     } while (0)
                             if (per_wave <= 4) SKINNY_INSIDE(8); else SKINNY_INSIDE(12);
 #undef SKINNY_INSIDE
@@ -1531,14 +1541,21 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
                         if (cols_per_wg <= 4) { SKINNY_NARROW(4); break; }
                         if (cols_per_wg <= 8) { SKINNY_NARROW(8); break; }
                     }
-                    SKINNY_CHUNKS(8, false, 1);
+                    // (rows in turn. 8 rows, in turn > in front: 2,304 x 3,072 5.6 > 5.8 us, 3,072 x 3,072 6.1 > 6.4; with up to three blocks
+                    // 768 x 768 3.4 > 3.2, 1,600 x 1,600 4.4 > 4.1)
+                    SKINNY_CHUNKS(8, false, 1, true);
                     break;
             }
         } else {
             switch (std::min(per_wave, 3)) {
                 case 1: SKINNY_LAUNCH(true, 2, true, 1, true); break;
                 case 2: SKINNY_LAUNCH(true, 4, true, 1, true); break;
-                default: SKINNY_CHUNKS(6, true, 1); break;
+                default:
+                    // (In turn from two whole chunks on, in turn > in front: 16 rows of 1,024 x 4,096 13.1 > 13.5 us, 9 rows 12.5 > 13.0;
+                    // with four and five blocks 3,072 x 3,072 7.0 > 6.9, 1,600 x 6,400 10.5 > 9.5, 32 rows of 2,304 x 3,072 11.4 > 11.0)
+                    if (per_wave >= 6) SKINNY_TURNED(true, 6, true, 1, false, true);
+                    else SKINNY_CHUNKS(6, true, 1, false);
+                    break;
             }
         }
     } else {
@@ -1549,6 +1566,7 @@ static int launch_skinny(const void* A, int lda, const bf16_t* W, int ldw, const
 #undef SKINNY_NARROW
 #undef SKINNY_CHUNKS
 #undef SKINNY_LAUNCH
+#undef SKINNY_TURNED
 #undef SKINNY_KERNEL
 #undef SKINNY_ANY
 #undef SKINNY_PARTS

@@ -65,3 +65,14 @@ def test_decode_attention_of_shaped_scores_refuses_keys_outside_the_pages():
     null, some, shape = ctypes.c_void_p(None), ctypes.c_void_p(16), Shape()
     head = [some, 64, 0, some, some, 64, some, 1, null, some, 1, 1, 1, 64, 16, ctypes.c_float(0.125), 0, 1, 4, some, 64, some, some, 64, 128]
     assert f(*head, some, 0, 0, null, ctypes.byref(shape), null, 0) == -1
+
+
+def test_few_row_products_keep_no_more_registers_in_scratch():
+    """The products of a few rows: none but those with two chunks of loads in flight (43), and those that merge three or four splits for
+    more than 8 rows with two and three blocks of K a wavefront."""
+    merging = {"gemm_bf16_skinny<1,3,1,6,1,1,0,3,1,0,8,16,1,0>": 91, "gemm_bf16_skinny<1,3,1,4,1,1,0,4,1,0,8,16,1,0>": 36, "gemm_bf16_skinny<1,3,1,6,1,1,0,4,1,0,8,16,1,0>": 179}
+    found = {k: n for k, n in kernels("gemm_bf16").items() if k.startswith("gemm_bf16_skinny")}
+    assert len(found) >= 80 and set(merging) <= set(found)
+    for k, n in found.items():
+        one_chunk = k.split("<")[1].split(",")[8] == "1"
+        assert n <= merging.get(k, 0 if one_chunk else 43), k
