@@ -401,7 +401,9 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
     // the norm and a product that writes the pages itself are shorter: 17 and 32 rows 4,224 x 1,408 16.4 and 17.2 us inside, 12.9 and 14.0 apart, 4,800 x
     // 1,600 17.3 and 18.0, 13.8 and 15.2, 6,048 x 2,016 21.7 and 22.2, 16.5 and 18.7; 3,840 x 1,280 8.7 and 9.0, 10.0 and 10.9.)
     const bool kv_fits = kv == nullptr || (aligned(w.data, 16) && (M <= 16 || w.rows <= 4096));
-    if (w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
+    // (the norm inside is worked out by every workgroup, from rows that another one may have written its results over by then)
+    const bool in_place = overlap(x, out);
+    if (!in_place && w.dtype == BF16 && K % 8 == 0 && w.stride % 8 == 0 && M <= tuning().ln_fuse_max_rows && x.contiguous() && aligned(gamma, 16) &&
         (beta == nullptr || aligned(beta, 16)) && kv_fits && (tmp == nullptr || norm_inside_pays(M, w.rows, K))) {
         int rc;
         if (kv != nullptr) {
@@ -419,7 +421,7 @@ void ln_linear(const Tensor2& x, const float* gamma, const float* beta, float ep
         if (rc != -2) check(rc, "ln_linear");
     }
     // 32 bits: up to 8 rows of wide products (the others sum in another order, or take the rows in other shares)
-    if (w.dtype == F32 && rows == nullptr && kv == nullptr && M <= tuning().ln_fuse_max_rows && x.contiguous()) {
+    if (!in_place && w.dtype == F32 && rows == nullptr && kv == nullptr && M <= tuning().ln_fuse_max_rows && x.contiguous()) {
         const int rc = mllm_norm_gemm_f32(static_cast<const float*>(x.data), static_cast<int>(x.stride), gamma, beta, eps, 0, static_cast<const float*>(w.data),
                                           static_cast<int>(w.stride), bias, out.data, static_cast<int>(out.stride), static_cast<int>(M),
                                           static_cast<int>(w.rows), static_cast<int>(K), epilogue, stream);

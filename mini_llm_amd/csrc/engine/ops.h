@@ -50,6 +50,14 @@ struct Tensor2 {
     }
 };
 
+// Whether two views touch the same memory (from their first element to their last).
+inline bool overlap(const Tensor2& a, const Tensor2& b) {
+    const auto end = [](const Tensor2& t) {
+        return static_cast<const char*>(t.data) + (t.rows < 1 ? 0 : ((t.rows - 1) * t.stride + t.cols) * static_cast<int64_t>(t.esz()));
+    };
+    return static_cast<const char*>(a.data) < end(b) && static_cast<const char*>(b.data) < end(a);
+}
+
 // Second destination of a fused QKV product: the columns after the first q_cols are keys, then
 // values (kv_dim = k_pages.cols each); row m's also go to row slots[m] (>= 0) of the pages.
 struct KvScatter {

@@ -59,15 +59,16 @@ void rms_linear(const Tensor2& x, const float* weight, float eps, const Tensor2&
     if (rows == nullptr && x.rows != M) fail("rms_linear: out has %lld rows, the input %lld", (long long)M, (long long)x.rows);
     const bool f32_out = epilogue == ADD_RESIDUAL || epilogue == STORE_F32;
     if (out.dtype != (f32_out ? F32 : w.dtype)) fail("rms_linear: out must be %s", dtype_name(f32_out ? F32 : w.dtype));
-    // (more rows than that: the norm is a kernel of its own, as for the LayerNorm product)
-    if (w.dtype == BF16 && M <= tuning().ln_fuse_max_rows && K % 8 == 0 && w.stride % 8 == 0 && x.contiguous() &&
+    // (more rows than that, and results over the rows themselves: the norm is a kernel of its own, as for the LayerNorm product)
+    const bool in_place = overlap(x, out);
+    if (!in_place && w.dtype == BF16 && M <= tuning().ln_fuse_max_rows && K % 8 == 0 && w.stride % 8 == 0 && x.contiguous() &&
         (reinterpret_cast<uintptr_t>(weight) & 15) == 0 && (tmp == nullptr || norm_inside_pays(M, w.rows, K))) {
         const int rc = mllm_rms_gemm_bf16(static_cast<const float*>(x.data), i32(x.stride), rows, weight, eps, w.data, i32(w.stride), bias,
                                           out.data, i32(out.stride), i32(M), i32(w.rows), i32(K), epilogue, stream);
         if (rc == 0) return;
         if (rc != -2) check(rc, "rms_linear");
     }
-    if (w.dtype == F32 && rows == nullptr && M <= tuning().ln_fuse_max_rows && x.contiguous()) {      // (see ln_linear)
+    if (!in_place && w.dtype == F32 && rows == nullptr && M <= tuning().ln_fuse_max_rows && x.contiguous()) {      // (see ln_linear)
         const int rc = mllm_norm_gemm_f32(static_cast<const float*>(x.data), i32(x.stride), weight, nullptr, eps, 1, static_cast<const float*>(w.data),
                                           i32(w.stride), bias, out.data, i32(out.stride), i32(M), i32(w.rows), i32(K), epilogue, stream);
         if (rc == 0) return;

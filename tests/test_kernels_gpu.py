@@ -653,6 +653,21 @@ def test_ln_linear_fp32_inside_has_the_bits_of_norm_and_product(ops, monkeypatch
     assert (inside.cpu().double() - ref).abs().max().item() <= 3e-5
 
 
+@pytest.mark.parametrize("dtype,M,K", [(torch.float32, 1, 2048), (torch.float32, 8, 2048), (torch.bfloat16, 1, 768), (torch.bfloat16, 16, 768),
+                                       (torch.bfloat16, 32, 1600)])
+def test_ln_linear_over_its_own_rows(ops, dtype, M, K):
+    """x += norm(x) W^T in place: a norm inside the product would read rows that other workgroups have added their results to."""
+    g = torch.Generator().manual_seed(M + K)
+    x = _rand((M, K), torch.float32, g, std=2.0)
+    gamma, bias = (1 + 0.1 * _rand((K,), torch.float32, g)).to(DEV), (0.5 * _rand((K,), torch.float32, g)).to(DEV)
+    w = _rand((K, K), dtype, g, std=1.0 / math.sqrt(K)).to(DEV)
+    here, there = x.to(DEV), x.to(DEV)
+    ops.ln_linear(here, gamma, None, 1e-5, w, bias, here, "add_residual")
+    h = ops.layernorm(x.to(DEV), gamma, None, 1e-5, torch.empty(M, K, dtype=dtype, device=DEV))
+    ops.linear(h, w, bias, there, "add_residual")
+    assert torch.equal(here, there)
+
+
 def test_linear_fp32_is_true_fp32(ops):
     """Values that bf16 or tf32 inputs would destroy: 1 + 2^-20 differs from 1 only in true fp32."""
     K = 64
