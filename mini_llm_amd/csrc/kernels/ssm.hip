@@ -85,32 +85,24 @@ __global__ void conv_silu_vec_kernel(const float* __restrict__ in, int ld, int C
         make_float4(silu_precise(acc[0]), silu_precise(acc[1]), silu_precise(acc[2]), silu_precise(acc[3]));
 }
 
-// A step of one token a sequence, a workgroup per token and 64 channel quads: the token's own row and the taps are asked for at once, from
-// arguments that arrive with the wavefront and without a division; only the carried rows, which move up by one here, wait for the
-// slot. A chain of latencies: 8 tokens x 1,792 channels 3.5 > 2.8 us.
+// A step of one token a sequence (token t is sequence t: no slot belongs to two tokens), a workgroup per token and 64 channel quads: the token's
+// own row, the taps and the slot are asked for at once, from arguments that arrive with the wavefront and without a division; only the
+// carried rows, which move up by one here, wait for the slot. A chain of latencies: 8 tokens x 1,792 channels 3.5 > 2.8 us.
 template <int TAPS>
 __global__ void __launch_bounds__(64)
 conv_silu_single_kernel(const float* __restrict__ in, int ld, int C, const float* __restrict__ w, const float* __restrict__ bias,
-                        const int* __restrict__ token_seq, const int* __restrict__ state_slots, const int* __restrict__ cu_q,
-                        float* __restrict__ state, size_t slot_floats, float* __restrict__ out, int ldo) {
+                        const int* __restrict__ state_slots, float* __restrict__ state, size_t slot_floats, float* __restrict__ out, int ldo) {
     const int t = blockIdx.x, ch = (blockIdx.y * 64 + threadIdx.x) * 4;
     if (ch >= C) return;
     float4 wf[TAPS], v[TAPS];
     const float4 own = *reinterpret_cast<const float4*>(in + static_cast<size_t>(t) * ld + ch), b4 = *reinterpret_cast<const float4*>(bias + ch);
 #pragma unroll
     for (int j = 0; j < TAPS; ++j) wf[j] = *reinterpret_cast<const float4*>(w + static_cast<size_t>(ch) * TAPS + 4 * j);
-    const int b = token_seq[t];
-    int slot = state_slots[t], first = cu_q[t];          // (asked for beside the sequence: it is the token's number)
-    if (b != t) { slot = state_slots[b]; first = cu_q[b]; }
+    const int slot = state_slots[t];
     if (slot < 0) return;
     float* carried = state + static_cast<size_t>(slot) * slot_floats;
-    const int k = t - first;              // 0
 #pragma unroll
-    for (int j = 0; j < TAPS - 1; ++j) {
-        const int idx = k - (TAPS - 1 - j);
-        v[j] = idx >= 0 ? *reinterpret_cast<const float4*>(in + static_cast<size_t>(first + idx) * ld + ch)
-                        : *reinterpret_cast<const float4*>(carried + static_cast<size_t>(TAPS - 1 + idx) * C + ch);
-    }
+    for (int j = 0; j < TAPS - 1; ++j) v[j] = *reinterpret_cast<const float4*>(carried + static_cast<size_t>(j) * C + ch);
     v[TAPS - 1] = own;
     float wv[4 * TAPS];
 #pragma unroll
@@ -1100,8 +1092,8 @@ int mllm_conv_silu(const float* proj, int ld, int col0, int C, const float* w, c
 #undef CSR
         } else
         if (single) {
-#define CS1(TAPS) case TAPS: conv_silu_single_kernel<TAPS><<<dim3(T, (C / 4 + 63) / 64), 64, 0, stream>>>(proj + col0, ld, C, w, bias, token_seq, state_slots, \
-                                                                                                        cu_q, state, slot_floats, out, ldo); break
+#define CS1(TAPS) case TAPS: conv_silu_single_kernel<TAPS><<<dim3(T, (C / 4 + 63) / 64), 64, 0, stream>>>(proj + col0, ld, C, w, bias, state_slots, state, \
+                                                                                                        slot_floats, out, ldo); break
             switch (taps) { CS1(2); CS1(3); CS1(4); CS1(5); CS1(6); CS1(7); CS1(8); }
 #undef CS1
         } else
