@@ -137,6 +137,10 @@ __device__ __forceinline__ float rows_sum(float v) {
     return a + b;
 }
 
+// The sum of four squares, rounded alike wherever it stands: left to the compiler, which product of a pair goes into the fused addition differs
+// between the instances of a kernel, and a row's norm with it between launches of a few rows and of many.
+__device__ __forceinline__ float squares_sum(float x, float y, float z, float w) { return fmaf(x, x, y * y) + fmaf(z, z, w * w); }
+
 // a / b for whole numbers that are the same in all lanes, 0 <= a < 2^20, b >= 1: in floating point, where half a unit more than `a` lies
 // further from the next quotient than the reciprocal errs (2^-22 of it). An integer division takes 40 instructions one after the other,
 // about 0.1 us, which a short kernel's first load waits for.

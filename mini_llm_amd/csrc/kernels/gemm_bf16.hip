@@ -1099,8 +1099,7 @@ gemm_bf16_skinny(// The first 14 dwords arrive in registers with the wavefront, 
 #pragma unroll
             for (int u = 0; u < NU; ++u) {
                 if (u < NU - 1 || lane + 64 * u < nq) {
-                    const float a = v[j][u].x - mean[j], b = v[j][u].y - mean[j], c = v[j][u].z - mean[j], d = v[j][u].w - mean[j];
-                    q += (a * a + b * b) + (c * c + d * d);
+                    q += squares_sum(v[j][u].x - mean[j], v[j][u].y - mean[j], v[j][u].z - mean[j], v[j][u].w - mean[j]);
                 }
             }
             inv[j] = 1.0f / sqrtf(wave_sum(q) / static_cast<float>(K) + eps);

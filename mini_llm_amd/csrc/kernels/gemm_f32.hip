@@ -354,8 +354,7 @@ gemm_f32_normed_kernel(// (the 14 dwords that arrive in registers; K in the lowe
 #pragma unroll
         for (int u = 0; u < NU; ++u) {
             if (u < NU - 1 || lane + 64 * u < nq) {
-                const float a = v[u].x - mean, b = v[u].y - mean, c = v[u].z - mean, d = v[u].w - mean;
-                q += (a * a + b * b) + (c * c + d * d);
+                q += squares_sum(v[u].x - mean, v[u].y - mean, v[u].z - mean, v[u].w - mean);
             }
         }
         const float inv = 1.0f / sqrtf(wave_sum(q) / static_cast<float>(K) + eps);

@@ -322,7 +322,7 @@ rmsnorm_vec_kernel(const float* __restrict__ x, int ldx, int n, const int* __res
     float ss = 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u)
-        if (u < NU - 1 || lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
+        if (u < NU - 1 || lane + 64 * u < nq) ss += squares_sum(v[u].x, v[u].y, v[u].z, v[u].w);
     const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(Dg) + eps);
     OutT* yr = y + static_cast<size_t>(r) * ldy + g * Dg;
 #pragma unroll
@@ -383,7 +383,7 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, int n, int D, float* __restrict__ 
     float ss = 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u)
-        if (u < NU - 1 || lane + 64 * u < nq) ss += (v[u].x * v[u].x + v[u].y * v[u].y) + (v[u].z * v[u].z + v[u].w * v[u].w);
+        if (u < NU - 1 || lane + 64 * u < nq) ss += squares_sum(v[u].x, v[u].y, v[u].z, v[u].w);
     const float inv = 1.0f / sqrtf(wave_sum(ss) / static_cast<float>(D) + eps);
     float next_ss = 0.f;
 #pragma unroll
@@ -397,7 +397,7 @@ rmsnorm_add_vec_kernel(float* __restrict__ y, int n, int D, float* __restrict__ 
             xr[i] = now;
             if (NEXT) {
                 xx[u] = now;
-                next_ss += (now.x * now.x + now.y * now.y) + (now.z * now.z + now.w * now.w);
+                next_ss += squares_sum(now.x, now.y, now.z, now.w);
             } else if (copy) {
                 uint2 pk;
                 pk.x = pack_bf16x2(now.x, now.y);

@@ -1649,6 +1649,59 @@ def _entry(library, name, *args):
     return rc
 
 
+@pytest.mark.parametrize("D", [4, 64, 252, 256, 260, 512, 516, 768, 1024, 1600, 2048])
+def test_a_rows_norm_has_the_same_bits_among_few_and_many(D):
+    """The RMS norms and those that go into the stream, 8 rows and 600 (other instances), around the 256 columns that an instance has: the same
+    bits."""
+    import ctypes
+    g = torch.Generator().manual_seed(D)
+    x, res, w, gate, nx = (_rand(s, torch.float32, g, std=2.0).to(DEV) for s in ((600, D), (600, D), (D,), (600, D), (D,)))
+    eps, mult = ctypes.c_float(1e-5), ctypes.c_float(0.7)
+    for use_gate in (False, True):
+        outs = []
+        for n in (8, 600):
+            y = torch.zeros(n, D, device=DEV)
+            assert _entry("norm_gate", "mllm_rmsnorm", x, D, None, w, gate if use_gate else None, D, y, D, n, D, 1, eps, 0, 1, ctypes.c_size_t(0), None) == 0
+            outs.append(y)
+        assert torch.equal(outs[0], outs[1][:8])
+    for center in (0, 1):
+        outs = []
+        for n in (8, 600):
+            y, s = x[:n].clone(), res[:n].clone()
+            assert _entry("norm_gate", "mllm_norm_add", y, w, None, None, mult, eps, s, n, D, 0, center, None, None) == 0
+            outs.append(s)
+        assert torch.equal(outs[0], outs[1][:8])
+    outs = []
+    for n in (8, 600):
+        y, s, c = x[:n].clone(), res[:n].clone(), torch.zeros(n, D, dtype=torch.bfloat16, device=DEV)
+        assert _entry("norm_gate", "mllm_rmsnorm_add_norm", y, w, None, mult, eps, s, n, D, 0, nx, eps, c, None) == 0
+        outs.append((s, c))
+    assert torch.equal(outs[0][0], outs[1][0][:8]) and torch.equal(outs[0][1], outs[1][1][:8])
+
+
+@pytest.mark.parametrize("M", [1, 2, 3, 8])
+@pytest.mark.parametrize("N,K", [(2048, 4), (2050, 252), (2304, 256), (2048, 260), (2304, 768), (4096, 1024), (4097, 772), (4800, 1600), (2056, 2044),
+                                 (6400, 2048)])
+@pytest.mark.parametrize("epi", ["store", "gelu_tanh"])
+def test_rms_norm_fp32_inside_has_the_bits_of_norm_and_product(ops, M, N, K, epi):
+    """The RMS form of the 32-bit norm inside the few-row product, around every 256 columns of K, with one column a wavefront and with two."""
+    import ctypes
+    g = torch.Generator().manual_seed(M + N + K)
+    x = _rand((M, K), torch.float32, g, std=2.0) + 0.3
+    w, weight, bias = _rand((N, K), torch.float32, g, std=1.0 / math.sqrt(K)), 1 + 0.1 * _rand((K,), torch.float32, g), 0.5 * _rand((N,), torch.float32, g)
+    mode, eps = ops.EPILOGUES[epi], ctypes.c_float(1e-5)
+    for b in (bias.to(DEV), None):
+        inside, apart = (torch.full((M, N), 7.0, device=DEV) for _ in range(2))
+        h = torch.full((M, K), 7.0, device=DEV)
+        assert _entry("gemm_f32", "mllm_norm_gemm_f32", x.to(DEV), K, weight.to(DEV), None, eps, 1, w.to(DEV), K, b, inside, N, M, N, K, mode, None) == 0
+        assert _entry("norm_gate", "mllm_rmsnorm", x.to(DEV), K, None, weight.to(DEV), None, 0, h, K, M, K, 1, eps, 0, 1, ctypes.c_size_t(0), None) == 0
+        assert _entry("gemm_f32", "mllm_gemm_f32", h, K, w.to(DEV), K, b, apart, N, M, N, K, mode, None) == 0
+        assert torch.equal(inside, apart)
+    norm = x.double() / (x.double().square().mean(1, keepdim=True) + 1e-5).sqrt() * weight.double()
+    ref = plain_ops.linear(norm, w.double(), None, torch.zeros(M, N, dtype=torch.float64), epi)
+    assert (inside.cpu().double() - ref).abs().max().item() <= 3e-5          # (as for the LayerNorm)
+
+
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 63, 64, 65, 130])
 @pytest.mark.parametrize("H,Dn,Dr,R,Dv,rot,half", [(12, 64, 32, 256, 64, 32, 0), (5, 32, 16, 128, 96, 8, 1), (1, 96, 32, 512, 40, 32, 0), (7, 128, 64, 96, 128, 64, 1),
                                                    (6, 64, 0, 100, 72, 0, 0)])
