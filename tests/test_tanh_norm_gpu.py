@@ -82,6 +82,30 @@ def test_products_through_norms(ops, M, N, K):
             assert (copy.cpu().double() - want).abs().max() <= 0.01 * max(1.0, float(want.abs().max()))
 
 
+@pytest.mark.parametrize("M", [1, 3, 8])
+@pytest.mark.parametrize("N,K", [(768, 3072), (1020, 3080), (900, 4104), (1000, 5000),             # 4 columns a workgroup, 4 to 7 blocks of K a wavefront
+                                 (1030, 3072), (1500, 4104), (1500, 5000), (2040, 3080),           # 5 to 8 columns
+                                 (1361, 5128), (1600, 6400), (1500, 9216)])                        # both parts of K inside, a chunk of 4 to 6 blocks
+def test_few_rows_of_a_long_product_through_norms(ops, M, N, K):
+    """Up to 8 rows take narrow tiles, or both parts of K in one workgroup: next to the plain result, and with the bits that the same rows have
+    among nine, which other kernels of the same sums take."""
+    g = torch.Generator().manual_seed(M + N + K)
+    a, w = torch.randn(9, K, generator=g).to(BF16), (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16)
+    bias, x = torch.randn(N, generator=g), torch.randn(9, N, generator=g)
+    prod = a.to(F64) @ w.to(F64).T
+    for with_bias, n, nx in ((False, _norm(g, N), _norm(g, N)), (True, None, _norm(g, N)), (True, _norm(g, N), None)):
+        outs = []
+        for rows in (M, 9):
+            copy, y = torch.full((rows, N), float("nan"), dtype=BF16, device=DEV), torch.full((rows, N), float("nan"), device=DEV)
+            out = ops.linear_stream_add(a[:rows].to(DEV), w.to(DEV), x[:rows].to(DEV), bias.to(DEV) if with_bias else None, y, _dev(n), copy, _dev(nx))
+            outs.append((out.cpu(), copy.cpu()))
+        assert torch.equal(outs[0][0], outs[1][0][:M]) and torch.equal(outs[0][1], outs[1][1][:M])
+        ref = x.to(F64) + _plain(n, prod + (bias.to(F64) if with_bias else 0))
+        assert (outs[1][0].double() - ref).abs().max() <= 2e-4          # (as above)
+        want = _plain(nx, ref)
+        assert (outs[1][1].double() - want).abs().max() <= 0.01 * max(1.0, float(want.abs().max()))
+
+
 @pytest.mark.parametrize("D,dim", [(32, 1), (64, 16), (320, 13), (768, 64), (1024, 32), (1600, 40), (2048, 64)])
 @pytest.mark.parametrize("T", [1, 8, 9, 70, 400])
 def test_a_tokens_own_input(ops, D, dim, T):
