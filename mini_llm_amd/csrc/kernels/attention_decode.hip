@@ -289,7 +289,7 @@ decode_attention_kernel(// the first 14 dwords arrive in registers with the wave
         const float pj = SIGMOID ? 1.f / (1.f + exp2_for<T>(-(d + sbias * MLLM_LOG2E))) : exp2_for<T>(d - mn);
         l = l * a + pj;
 #pragma unroll
-        for (int e = 0; e < EPL; ++e) o[e] = o[e] * a + pj * vf[e];
+        for (int e = 0; e < EPL; ++e) o[e] = fmaf(pj, vf[e], o[e] * a);       // (as the keys of the pages are added)
         m = mn;
     }
     // Merges the states of all lane groups and wavefronts, in a fixed order: lane groups whose numbers differ in one bit, from the
