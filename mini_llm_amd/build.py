@@ -34,8 +34,8 @@ GPU_ARCH = "gfx950"
 HIPCC_FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "-shared", f"--offload-arch={GPU_ARCH}",
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
-    # the first 16 dwords of a kernel's arguments arrive in registers with the wavefront instead of
-    # being loaded by it: saves the load's latency at the head of every short kernel
+    # the first dwords of a kernel's arguments arrive in registers with the wavefront instead of being loaded by it (16
+    # registers, two of which hold the arguments' address): saves the load's latency at the head of every short kernel
     "-mllvm", "-amdgpu-kernarg-preload-count=16",
     # MFMA results go to ordinary vector registers, not to the accumulation registers: the kernels here
     # read every result with vector instructions (softmax, epilogues), and each such read or write of an

@@ -598,7 +598,10 @@ bool paged_attention(const AttentionArgs& a, AttentionSplits* splits, hipStream_
     }
     if (decode) {
         const int pairs = T * a.n_heads;
-        // (32 bits: where the product that follows merges, up to 8 rows of 3,072 columns)
+        // (32 bits: up to 8 rows of 3,072 columns. A product of fewer than 2,048 columns merges the splits itself; in front of a wider one a kernel
+        // does, and splitting still pays. Attention and output projection, one workgroup a pair > split, us: 16 heads of 128 and 2,048 columns,
+        // 1 row of 257 keys 19.3 > 16.2, of 1,024 33.8 > 20.7, 8 rows 21.3 > 20.0 and 39.2 > 35.0; 32 heads of 64 16.6 > 15.3, 25.5 > 16.8,
+        // 18.8 > 17.7 and 34.1 > 32.9; 24 heads of 128 and 3,072 columns, 8 rows of 2,048 keys 80.6 > 79.8.)
         bool unmerged = a.may_split && splits != nullptr && tuning().decode_nsplit == 0 &&
                         (a.q.dtype == BF16 ? T <= tuning().merge_max_rows && a.head_dim % 8 == 0
                                            : T <= std::min(8, tuning().merge_max_rows) && a.head_dim % 4 == 0 && a.n_heads * a.head_dim <= 3072);

@@ -176,8 +176,8 @@ gemm_f32_rows_kernel(// (the first 14 dwords arrive in registers with the wavefr
 // wavefronts and each waits for chunk after chunk of its column: two wavefronts share a column, 256 columns of K in turn, and
 // ask for all their weights of a pass of KP = 512 STEPS columns at once, behind the pass's activations, which lie in LDS whole. One
 // pass covers K up to 3,072; beyond, the next pass's weights are on their way while one is used. What the epilogue adds is asked for
-// first. Bound by the chain launch, activations, weights, sums: 8 x 768 x 768 and 8 x 768 x 3,072 in a decode step 4.1 and 5.4
-// us, together 17.1 with a column a wavefront, and 4.9 for the former with two splits of attention merged in it.
+// first. Bound by the chain launch, activations, weights, sums: 8 x 768 x 768 with two splits of attention merged in it and 8 x 768 x 3,072
+// take 4.8 and 5.8 us in a decode step; unmerged and with a column a wavefront they took 17.1 together.
 // RAGGED: K is no multiple of 256, and what lies beyond it has to be left out (8 x 1,600 x 1,600 7.4 us, 7.2 if it were not).
 // MS > 0: A is the output of split decode attention, the states of MS splits of every (token, head) pair as attention_decode.hip leaves them
 // (partial_out), merged while the rows are staged: weights over the full range of 32 bits, as the attention's own.
@@ -308,8 +308,8 @@ gemm_f32_narrow_kernel(// (the 14 dwords that arrive in registers)
 // a lane) into LDS while the weights of its CPW columns, all of them, are on their way; then every wavefront sums its columns as the few-row
 // kernel does, in the same order, so that the result has the bits of norm and product apart. Every workgroup normalises the rows again,
 // which costs it the rows and the norm's vectors from L2 (30 KB at K = 768) but no launch. RMS: the norm does not centre.
-// Bound by its chain: launch, rows, norm, products, sums. At 8 rows of K = 768: 5.7 us for 2,304
-// columns and 6.2 for 3,072, where the few-row kernel alone takes 6.2 and 6.5 behind a norm of 2.2 and a launch's gap of 1.2 (4.4 and 3.8 at one row).
+// Bound by its chain: launch, rows, norm, products, sums. At 8 rows of K = 768: 6.1 us for 2,304
+// columns and 6.5 for 3,072 in a decode step, where the few-row kernel alone took 6.2 and 6.5 behind a norm of 2.2 and a launch's gap of 1.2.
 template <int NU, int CPW, int ROWS>
 __global__ void __launch_bounds__(512)
 gemm_f32_normed_kernel(// (the 14 dwords that arrive in registers; K in the lower 12 bits of the last, rows (4), epilogue (4), the kind of norm)
@@ -775,7 +775,10 @@ int mllm_gemm_f32_merged(const float* split_o, const float* split_ml, int n_spli
 
 // The norm of the fp32 rows x [M, K] (a LayerNorm, or with rms != 0 an RMS norm) inside the product of up to 8 of them: C = epilogue(norm(x) W^T + bias).
 // -2: sizes the kernel does not take (more rows, K over 2,048 or no multiple of 4, operands that are not 16-byte aligned, or fewer columns than
-// the few-row kernel has in this order of sums); norm and product apart are right for those.
+// the few-row kernel has in this order of sums); norm and product apart are right for those. Inside / apart, back to back on cold weights, us, 1, 4 and 8
+// rows: 2,304 x 768 3.6 / 6.8, 4.9 / 6.5, 5.6 / 7.5; 4,096 x 1,024 4.7 / 8.5, 6.1 / 8.2, 6.7 / 9.2; 5,120 x 1,280 7.1 / 9.9, 9.1 / 10.7, 10.4 / 12.1; 6,400 x 1,600
+// 9.3 / 13.7, 12.7 / 14.7, 15.1 / 16.7; 8,192 x 2,048 13.4 / 16.7, 17.2 / 19.7, 19.1 / 20.3. Inside loses 2 to 6 % at 5 to 8 rows of 4,800 x 1,600 (14.6 / 14.0)
+// and a row count or two of 2,304 and 6,144 x 2,048 (6 rows 17.4 / 16.4): no line drawn for those. (GPT-2 XL, 8 rows, a step: 3.64 > 3.49 ms.)
 int mllm_norm_gemm_f32(const float* x, int ldx, const float* gamma, const float* beta, float eps, int rms, const float* W, int ldw, const float* bias,
                        void* C, int ldc, int M, int N, int K, int mode, hipStream_t stream) {
     if (M <= 0 || N <= 0) return 0;

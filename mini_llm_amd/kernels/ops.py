@@ -373,8 +373,9 @@ def ln_linear(x: torch.Tensor, gamma: torch.Tensor, beta: Optional[torch.Tensor]
     ``rows`` (int32 [M]) row m of the input is x[rows[m]]; ``kv_scatter`` as for ``linear``.
 
     For bfloat16 weights, at most 32 rows and fewer than 16384 columns the norm is fused into the
-    product (one kernel); otherwise the norm and the product run one after the other. Same numerics
-    either way: statistics in fp32, the normalised rows rounded to w's dtype before the product.
+    product (one kernel), and so it is for fp32 weights, at most 8 rows that are not gathered, K up to 2048 and
+    2048 columns and more. Otherwise, and where out shares memory with x, the norm and the product run one after the
+    other. Same numerics either way: statistics in fp32, the normalised rows rounded to w's dtype before the product.
     """
     _gpu(x, gamma, beta, w, bias, out, rows)
     if epilogue not in EPILOGUES:
