@@ -128,8 +128,8 @@ decode_attention_kernel(// the first 14 dwords arrive in registers with the wave
     const int* gtable_row = block_tables + static_cast<size_t>(b) * max_blocks;
     // Without a window the keys start at block 0 whatever the position is, and rows of the table are
     // filled to their end (zeros behind a sequence's last block): the whole row goes to LDS without
-    // waiting for the position.
-    const bool whole_row = !windowed && max_blocks <= DEC_TABLE_LDS;
+    // waiting for the position. (A table without entries, where every token stands alone with its own key, is not read.)
+    const bool whole_row = !windowed && static_cast<unsigned>(max_blocks - 1) < DEC_TABLE_LDS;
     const auto raw_q = load_raw16(q + static_cast<size_t>(t) * q_stride + h * DH + c * EPL);
     int entry = 0;
     if (whole_row) entry = gtable_row[min(static_cast<int>(threadIdx.x), max_blocks - 1)];

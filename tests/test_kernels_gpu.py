@@ -1702,6 +1702,22 @@ def test_rms_norm_fp32_inside_has_the_bits_of_norm_and_product(ops, M, N, K, epi
     assert (inside.cpu().double() - ref).abs().max().item() <= 3e-5          # (as for the LayerNorm)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+def test_decode_attention_of_first_tokens_without_a_table(dtype):
+    """Tokens at position 0 whose keys stand in their own rows alone: a table of no entries is not read, and the result is the value."""
+    import ctypes
+    T, H, dh = 3, 4, 64
+    D, g = H * dh, torch.Generator().manual_seed(5)
+    q = _rand((T, 3 * D), dtype, g)
+    qd, out, pages = q.to(DEV), torch.zeros(T, D, dtype=dtype, device=DEV), [torch.zeros(32, D, dtype=dtype, device=DEV) for _ in range(2)]
+    ws, counters = torch.zeros(T * H * (dh + 2), device=DEV), torch.zeros(T * H, dtype=torch.int32, device=DEV)
+    positions, slots = torch.zeros(T, dtype=torch.int32, device=DEV), torch.tensor([17, 3, -1], dtype=torch.int32, device=DEV)
+    assert _entry("attention_decode", "mllm_decode_attention", qd, 3 * D, 0, *pages, D, None, 0, None, positions, T, H, H, dh, 16, ctypes.c_float(dh ** -0.5), 0, 1, 4,
+                  out, D, ws, counters, D, 2 * D, slots, 0, 0 if dtype == torch.float32 else 1, None, None, None, 0) == 0
+    assert torch.equal(out.cpu(), q[:, 2 * D:])
+    assert torch.equal(pages[0][[17, 3]].cpu(), q[:2, D:2 * D]) and torch.equal(pages[1][[17, 3]].cpu(), q[:2, 2 * D:])
+
+
 @pytest.mark.parametrize("T", [1, 15, 16, 17, 63, 64, 65, 130])
 @pytest.mark.parametrize("H,Dn,Dr,R,Dv,rot,half", [(12, 64, 32, 256, 64, 32, 0), (5, 32, 16, 128, 96, 8, 1), (1, 96, 32, 512, 40, 32, 0), (7, 128, 64, 96, 128, 64, 1),
                                                    (6, 64, 0, 100, 72, 0, 0)])
